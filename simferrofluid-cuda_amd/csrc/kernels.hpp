@@ -76,12 +76,15 @@ void launch_coarsen(hipStream_t s, Dims df, Op64 Af, const float *diag32f, Dims 
 // Dense inverse of the coarsest operator (n = cells <= kMaxCoarse) into ainv (n*n floats).
 constexpr int kMaxCoarse = 64;
 
-// The coarse end of a V-cycle in one launch of one block: from level `first`
-// (cells <= kTailMaxCells) down to the coarsest and back, with the per-cell
-// arithmetic of the separate smoothing, restriction and dense-solve launches.
-// The level's result is left in lv[0].x1 (tail_result); the other level
-// vectors are not touched. The first level's b must already hold its
-// right-hand side.
+// The coarse end of a V-cycle in one launch of one block: from its first level
+// (cells, z rows padded to groups of four, <= kTailMaxCells) down to the
+// coarsest and back, with the per-cell arithmetic of the separate smoothing,
+// restriction and dense-solve launches. The level's result is left in lv[0].x1
+// (tail_result); the other level vectors are not touched. The first level's b
+// must already hold its right-hand side. The first level lives in registers (a
+// group of four cells for each of 1024 threads), the others in LDS. (Two groups
+// a thread, 8192 cells, spilled and took 33 us at 20^3, where two tile launches
+// and the tail from 10^3 take 17.)
 constexpr size_t kTailMaxCells = 4096;
 constexpr int kTailMaxLevels = 8;
 struct TailLevel {
@@ -97,17 +100,60 @@ struct TailArgs {
     float cd[2][8] = {}, cr[2][8] = {};
     const float *ainv = nullptr;
 };
-// The tail keeps 8 arrays of every level it covers in LDS (gfx950: up to
-// 160 KiB per block).
+// LDS of the levels below the first: 8 padded arrays each (two with guards).
+constexpr int kTailPoolFloats = 16384;
+constexpr int kInvStride = 68;  // row stride of the dense inverse in LDS
+constexpr __host__ __device__ int tail_level_floats(int padded_cells) { return 8 * padded_cells + 16; }
+// Whether levels lv[0..nlev) (first to coarsest) can run as a tail.
+bool tail_fits(const Dims *lv, int nlev);
+void launch_vcycle_tail(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
+// The buffer that holds the tail's result for its first level.
+inline float *tail_result(const TailArgs &t) { return t.lv[0].x1; }
+// The tail with every array of its levels (8 each, unpadded) in LDS: the one
+// for hierarchies whose coarsest level has 2 (mod 4) cells (18, of 2 x 3 x 3),
+// for which its staging of the dense inverse leaves the entries (r, 0) and
+// (r, 1) of odd rows r unset. The cycle it computes there is not the
+// level-by-level one, solves take one or two iterations more, and their
+// iterates are kept as they are.
+constexpr size_t kTailLdsMaxCells = 4096;
 constexpr size_t kTailLdsBytes = 149504;
 inline size_t tail_lds_bytes(const TailArgs &t) {
     size_t b = 0;
     for (int l = 0; l < t.nlev; l++) b += 8 * sizeof(float) * t.lv[l].d.cells();
     return b;
 }
-void launch_vcycle_tail(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
-// The buffer that holds the tail's result for its first level.
-inline float *tail_result(const TailArgs &t) { return t.lv[0].x1; }
+void launch_vcycle_tail_lds(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
+
+// Several Chebyshev steps of one level in one launch, over overlapping tiles
+// held in registers and LDS. start:
+//   TILE_FIRST    from x = c0 D^-1 b, which is also the previous direction
+//   TILE_PROLONG  from xin + P e (e on the coarse extents dc), cd[0] = 0
+//   TILE_CONTINUE from xin with direction din
+// then nsteps steps with coefficients cd[], cr[]; x to xout and, when dout is
+// given, the direction to dout; with bc the restriction of the residual (the
+// coarse right-hand side). Same results as launch_smooth and launch_restrict,
+// bit for bit. xout must not alias xin, nor dout din.
+enum TileStart : int { TILE_FIRST = 0, TILE_PROLONG = 1, TILE_CONTINUE = 2 };
+constexpr int kTileMaxGroups = 2048;
+struct TilePlan {
+    int tx = 0, ty = 0, tz = 0;  // own cells of a tile (even; tz a multiple of 4)
+    int hx = 0, hy = 0, hz = 0;  // halo (0 where one tile spans the axis)
+    int bx = 0, by = 0, bz = 0;  // tiles along each axis
+    int groups = 0;              // groups of four cells with the halo
+};
+struct TileArgs {
+    Dims d, dc;
+    Op32 A;
+    TilePlan plan;
+    const float *b = nullptr, *xin = nullptr, *din = nullptr, *e = nullptr;
+    float *xout = nullptr, *dout = nullptr, *bc = nullptr;
+    int start = TILE_FIRST, nsteps = 0;
+    float c0 = 0.f, cd[8] = {}, cr[8] = {};
+};
+// The tile of the least modelled cost for `steps` steps (and the restriction)
+// on level d; its cost in microseconds.
+TilePlan choose_tile(Dims d, int steps, bool restrict_after, double *cost = nullptr);
+void launch_tile_steps(hipStream_t s, const TileArgs &a, const double *gate = nullptr);
 void launch_coarse_invert(hipStream_t s, Dims d, Op64 A, float *ainv);
 // On every level l < nlev: v[l][0..3][c] = 0 (and on level 0 w[c] = 0 when
 // w is given) at the cells with diag32[l][c] == 0. start[l] is the first

@@ -2,7 +2,7 @@
 // coarse-grid correction fused into the first post-smoothing step, one-pass
 // pairs of steps (and of the last step with the restriction), residual +
 // restriction, FP64 Galerkin coarsening over 2x2x2 aggregates, the dense
-// coarsest solve, and the small levels of a cycle in one single-block launch.
+// coarsest solve. (The small levels' launches are in mg_tile.hip.)
 //
 // Threads map to cells with z (the unit-stride axis of the reference layout)
 // across the 64 lanes of a wavefront and y across the 4 wavefronts of a
@@ -1330,7 +1330,7 @@ __global__ __launch_bounds__(kBlock) void k_coarse_solve(int n, const float *ain
 
 // ---------------------------------------------------------------- V-cycle tail
 // One block runs the coarse end of the V-cycle (levels of at most
-// kTailMaxCells cells) with the levels' arrays in LDS: each sweep covers a
+// kTailLdsMaxCells cells) with the levels' arrays in LDS: each sweep covers a
 // level's cells with the block's threads and ends at a barrier. The per-cell
 // arithmetic is that of k_smooth, k_restrict and k_coarse_solve (neighbour
 // values equal to what those take from adjacent lanes), so the result is the
@@ -1561,7 +1561,7 @@ __device__ void tail_restrict(const TailLevel &F, const float *__restrict__ x, f
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kTailThreads) void k_vcycle_tail(TailArgs t, const double *gate) {
+__global__ __launch_bounds__(kTailThreads) void k_vcycle_tail_lds(TailArgs t, const double *gate) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     if (gated(gate)) return;
     // every array of the tail's levels lives in LDS for the whole cycle (8
@@ -1589,7 +1589,7 @@ __global__ __launch_bounds__(kTailThreads) void k_vcycle_tail(TailArgs t, const 
     if (ainv_lds && 4 * tid < nC * nC) ainv4 = *(const f4 *)(t.ainv + 4 * tid);
     // Copy-in: where every level has a multiple of 4 cells (16-byte aligned
     // LDS arrays and source arrays), each thread loads at most one 16-byte
-    // vector of each array (kTailMaxCells / 4 <= kTailThreads) of the first
+    // vector of each array (kTailLdsMaxCells / 4 <= kTailThreads) of the first
     // three levels, all in flight together, then stores them.
     bool vec = true;
     for (int l = 0; l < t.nlev; l++) {
@@ -1994,14 +1994,14 @@ void launch_coarse_solve(hipStream_t st, int n, const float *ainv, const float *
     SFP_LAUNCH_CHECK();
 }
 
-void launch_vcycle_tail(hipStream_t st, const TailArgs &t, const double *gate) {
+void launch_vcycle_tail_lds(hipStream_t st, const TailArgs &t, const double *gate) {
     if (t.nlev < 2 || t.nlev > kTailMaxLevels) throw ArgError("vcycle tail: bad level count");
     for (int k = 0; k < 2; k++)
         if (t.deg[k] < 1 || t.deg[k] > 8) throw ArgError("vcycle tail: bad degree");
-    if (t.lv[0].d.cells() > kTailMaxCells) throw ArgError("vcycle tail: level too large");
+    if (t.lv[0].d.cells() > kTailLdsMaxCells) throw ArgError("vcycle tail: level too large");
     if ((int)t.lv[t.nlev - 1].d.cells() > kMaxCoarse) throw ArgError("vcycle tail: coarsest too large");
     if (tail_lds_bytes(t) > kTailLdsBytes) throw ArgError("vcycle tail: levels exceed the LDS");
-    hipLaunchKernelGGL(k_vcycle_tail, dim3(1), dim3(kTailThreads), 0, st, t, gate);
+    hipLaunchKernelGGL(k_vcycle_tail_lds, dim3(1), dim3(kTailThreads), 0, st, t, gate);
     SFP_LAUNCH_CHECK();
 }
 

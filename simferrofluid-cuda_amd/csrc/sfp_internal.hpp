@@ -88,7 +88,9 @@ struct DevBuf {
         if (count <= n && p) return;
         release();
         if (count == 0) return;
-        SFP_HIP(hipMalloc(&p, count * sizeof(T)));
+        // (64 bytes more: a 16-byte access at an array's last elements may
+        // reach past them)
+        SFP_HIP(hipMalloc(&p, count * sizeof(T) + 64));
         n = count;
     }
     void release() {

@@ -155,6 +155,7 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
         }
         if ((int)lv_.back().d.cells() > kMaxCoarse) throw ArgError("coarsest level too large");
         ainv_.ensure((size_t)lv_.back().d.cells() * lv_.back().d.cells());
+        stages_.clear();
         built_coarsest_ = coarsest;
     }
     for (size_t l = 1; l < lv_.size(); l++) {
@@ -213,8 +214,11 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
 
 float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
     const int nlev = (int)lv_.size() - l;
-    if (!ws.vcycle_tail || nlev < 2 || nlev > kTailMaxLevels || lv_[l].d.cells() > kTailMaxCells)
-        return nullptr;
+    if (!ws.vcycle_tail || nlev < 2 || nlev > kTailMaxLevels) return nullptr;
+    Dims dims[kTailMaxLevels];
+    for (int q = 0; q < nlev; q++) dims[q] = lv_[l + q].d;
+    const bool lds = dims[nlev - 1].cells() % 4 == 2;  // (see launch_vcycle_tail_lds)
+    if (lds ? dims[0].cells() > kTailLdsMaxCells : !tail_fits(dims, nlev)) return nullptr;
     TailArgs t;
     t.nlev = nlev;
     for (int q = 0; q < nlev; q++) {
@@ -230,14 +234,59 @@ float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
         }
     }
     t.ainv = ainv_.p;
-    if (tail_lds_bytes(t) > kTailLdsBytes) return nullptr;
+    if (lds && tail_lds_bytes(t) > kTailLdsBytes) return nullptr;
     join_ainv(ws);
-    launch_vcycle_tail(ws.stream, t, ws.gate);
+    if (lds) launch_vcycle_tail_lds(ws.stream, t, ws.gate);
+    else launch_vcycle_tail(ws.stream, t, ws.gate);
     return tail_result(t);
 }
 
 // Grids whose kernels are bound by launch latency rather than bytes.
 static bool small_grid(Dims d) { return d.cells() <= ((size_t)1 << 19); }
+
+// One separate launch of a step or the restriction on a level (us): 3.1 us
+// up to 64^3 whatever it computes, 5.6 ns per thousand cells above (measured:
+// 32^3 and 64^3 3.0-3.2, 80^3 3.7-4.4, 96^3 5.1-7.0, 128^3 12.0-12.4 us).
+static double separate_cost(Dims d) { return std::max(3.1, 0.6 + 5.6e-6 * (double)d.cells()); }
+
+const System::TileStages &System::tile_stages(const Workspace &ws, int l, int steps, bool restrict_after) {
+    static const TileStages none;
+    if (!ws.vcycle_tail) return none;
+    if (stages_.size() != lv_.size()) stages_.assign(lv_.size(), {});
+    for (const TileStages &t : stages_[l])
+        if (t.steps == steps && t.restrict_after == restrict_after) return t;
+    TileStages t;
+    t.steps = steps;
+    t.restrict_after = restrict_after;
+    const Dims d = lv_[l].d;
+    // (above 2^19 cells the tiles' repeated loads are bound by the caches, which
+    // the model does not hold: 128^3, five steps 96 us against 60 us separately)
+    if (!small_grid(d)) return none;
+    double best = separate_cost(d) * (steps + (restrict_after ? 1 : 0));
+    double c = 0.0;
+    const TilePlan one = choose_tile(d, steps, restrict_after, &c);
+    if (c < best) {
+        best = c;
+        t.n = 1;
+        t.count[0] = steps;
+        t.plan[0] = one;
+    }
+    for (int a = 1; a < steps; a++) {
+        double c0 = 0.0, c1 = 0.0;
+        const TilePlan p0 = choose_tile(d, a, false, &c0), p1 = choose_tile(d, steps - a, restrict_after, &c1);
+        if (c0 + c1 < best) {
+            best = c0 + c1;
+            t.n = 2;
+            t.count[0] = a;
+            t.count[1] = steps - a;
+            t.plan[0] = p0;
+            t.plan[1] = p1;
+        }
+    }
+    stages_[l].push_back(t);
+    return stages_[l].back();
+}
+
 
 // Algorithmic bytes per cell of one single Chebyshev step: x, b, diag and 3
 // couplings in and x out, plus the direction in and out by mode and the
@@ -283,6 +332,39 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
         if (track) ws.timers[K_SMOOTH].end(st);
         std::swap(cur, oth);
     };
+    // the whole descent of a small level in one or two launches
+    if (const TileStages &T = tile_stages(ws, l, deg - 1, true); T.n > 0) {
+        if (r64) launch_smooth_first(st, L.d, A, r64, L.b.p, cur, cb.cr[0], ws.gate);  // (b)
+        Level &C = lv_[l + 1];
+        int s = 1;
+        for (int q = 0; q < T.n; q++) {
+            TileArgs t;
+            t.d = L.d;
+            t.dc = C.d;
+            t.A = A;
+            t.plan = T.plan[q];
+            t.b = L.b.p;
+            t.start = q == 0 ? TILE_FIRST : TILE_CONTINUE;
+            t.c0 = cb.cr[0];
+            t.nsteps = T.count[q];
+            for (int e = 0; e < t.nsteps; e++) {
+                t.cd[e] = cb.cd[s + e];
+                t.cr[e] = cb.cr[s + e];
+            }
+            s += t.nsteps;
+            if (q > 0) {
+                t.xin = cur;
+                t.din = L.dv.p;
+            }
+            t.xout = oth;
+            if (q + 1 < T.n) t.dout = L.dv.p;
+            else t.bc = C.b.p;
+            launch_tile_steps(st, t, ws.gate);
+            std::swap(cur, oth);
+        }
+        const float *e = vlevel(ws, sm, l + 1, nullptr, false);
+        return post_smooth(ws, sm, l, cur, e);
+    }
     // the last step and the restriction run as one pass where the grid pays
     // for the pass's tile overlap
     const bool fuse_restrict =
@@ -341,6 +423,32 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
     float *oth = cur == L.x0.p ? L.x1.p : L.x0.p;
     const int deg = cb.degree;
     const bool track = l == 0 && ws.profiling;
+    if (const TileStages &T = tile_stages(ws, l, deg, false); T.n > 0) {
+        int s = 0;
+        for (int q = 0; q < T.n; q++) {
+            TileArgs t;
+            t.d = L.d;
+            t.dc = lv_[l + 1].d;
+            t.A = A;
+            t.plan = T.plan[q];
+            t.b = L.b.p;
+            t.start = q == 0 ? TILE_PROLONG : TILE_CONTINUE;
+            t.nsteps = T.count[q];
+            for (int v = 0; v < t.nsteps; v++) {
+                t.cd[v] = s + v == 0 ? 0.f : cb.cd[s + v];
+                t.cr[v] = cb.cr[s + v];
+            }
+            s += t.nsteps;
+            t.xin = cur;
+            t.e = e;
+            if (q > 0) t.din = L.dv.p;
+            t.xout = oth;
+            if (q + 1 < T.n) t.dout = L.dv.p;
+            launch_tile_steps(st, t, ws.gate);
+            std::swap(cur, oth);
+        }
+        return cur;
+    }
     // the last two steps run as one pass where the grid is large enough to
     // pay for the pass's tile overlap (the direction they leave is not stored:
     // nothing reads it before the next cycle rewrites it)

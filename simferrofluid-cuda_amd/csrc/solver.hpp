@@ -108,7 +108,8 @@ struct Workspace {
     // &scalars->stop while a batched solve runs (iteration kernels return at
     // once when it is nonzero), null otherwise
     const double *gate = nullptr;
-    // run the V-cycle's small levels (<= kTailMaxCells cells) in one launch
+    // run the V-cycle's small levels (<= kTailMaxCells cells) in one launch, and
+    // the ones above them in a few (launch_tile_steps)
     bool vcycle_tail = true;
     // run as one pass on large grids: bit 0, the last pre-smoothing step with
     // the restriction; bit 1, the last two post-smoothing steps (the flat step
@@ -200,6 +201,18 @@ class System {
     // levels l .. coarsest in one launch (vlevel with r64 null), or null
     // where the tail does not apply
     float *vcycle_tail(Workspace &ws, const Smoothing &sm, int l);
+    // The steps of one half of level l's visit (steps, and the restriction
+    // after them) as one or two launches over tiles; n[0] = 0: separate
+    // launches are cheaper.
+    struct TileStages {
+        int steps = -1;
+        bool restrict_after = false;
+        int n = 0;  // launches
+        int count[2] = {0, 0};
+        TilePlan plan[2];
+    };
+    const TileStages &tile_stages(const Workspace &ws, int l, int steps, bool restrict_after);
+    std::vector<std::vector<TileStages>> stages_;  // by level
     void network_correction(Workspace &ws, float *x);
     void coarse_phi(Workspace &ws);
     DevBuf<double> phic_;  // level set restricted to the first coarse level
