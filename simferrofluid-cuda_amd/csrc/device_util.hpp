@@ -105,6 +105,38 @@ __device__ __forceinline__ void sum_partials(const double *partials, unsigned nb
     block_sum<N, T>(v);
 }
 
+// The sums of N arrays of nb block partials ([q * nb + b]) in every thread of
+// a block (of whole wavefronts), in the order of a 1024-thread sum_partials
+// for nb <= 15 * 1024: bit for bit the one-block finalize's. A kernel that
+// needs a reduction's result adds the partials itself where they are few,
+// which costs it one memory latency instead of a launch (3 to 4 us) between.
+template <int N>
+__device__ __forceinline__ void fold_partials(const double *__restrict__ partials, unsigned nb, double (&v)[N]) {
+    __shared__ double sh[N][16];
+    const unsigned tid = (unsigned)flat_tid(), nt = blockDim.x * blockDim.y * blockDim.z;
+    const unsigned waves = min((nb + 63u) / 64u, 16u);
+    for (unsigned vt = tid; vt < 64u * waves; vt += nt) {  // whole wavefronts (nt a multiple of 64)
+        double a[N];
+#pragma unroll
+        for (int q = 0; q < N; q++) a[q] = 0.0;
+        for (unsigned b = vt; b < nb; b += 1024u)
+#pragma unroll
+            for (int q = 0; q < N; q++) a[q] += partials[(size_t)q * nb + b];
+#pragma unroll
+        for (int q = 0; q < N; q++) a[q] = wave_sum(a[q]);
+        if ((tid & 63u) == 0)
+#pragma unroll
+            for (int q = 0; q < N; q++) sh[q][vt >> 6] = a[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        double s = sh[q][0];
+        for (unsigned w = 1; w < waves; w++) s += sh[q][w];
+        v[q] = s;
+    }
+}
+
 // Tile of a cell-parallel block: z index k (lanes), y index j (wavefronts)
 // and the first of its cg.planes consecutive x planes. Blocks are taken in
 // launch order (tiles of one plane, then the next chunk of planes); a

@@ -92,6 +92,14 @@ struct TailLevel {
     Op32 A;
     float *b, *x0, *x1, *dv;
 };
+// The ||r||^2 of the update before a cycle, added by the cycle's first launch:
+// nb partials (0: nothing to add), counted and compared to stop_rr as
+// launch_fcg_norm does; the launch returns when that raises `stop`.
+struct FoldArgs {
+    const double *partials = nullptr;
+    unsigned nb = 0;
+    KrylovScalars *sc = nullptr;
+};
 struct TailArgs {
     int nlev = 0;  // levels in the tail, the last the coarsest
     TailLevel lv[kTailMaxLevels];
@@ -99,6 +107,7 @@ struct TailArgs {
     int deg[2] = {3, 3};
     float cd[2][8] = {}, cr[2][8] = {};
     const float *ainv = nullptr;
+    FoldArgs fold;
 };
 // LDS of the levels below the first: 8 padded arrays each (two with guards).
 constexpr int kTailPoolFloats = 16384;
@@ -117,11 +126,7 @@ inline float *tail_result(const TailArgs &t) { return t.lv[0].x1; }
 // iterates are kept as they are.
 constexpr size_t kTailLdsMaxCells = 4096;
 constexpr size_t kTailLdsBytes = 149504;
-inline size_t tail_lds_bytes(const TailArgs &t) {
-    size_t b = 0;
-    for (int l = 0; l < t.nlev; l++) b += 8 * sizeof(float) * t.lv[l].d.cells();
-    return b;
-}
+inline size_t tail_lds_bytes(Dims d) { return 8 * sizeof(float) * d.cells(); }
 void launch_vcycle_tail_lds(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
 
 // Several Chebyshev steps of one level in one launch, over overlapping tiles
@@ -149,6 +154,7 @@ struct TileArgs {
     float *xout = nullptr, *dout = nullptr, *bc = nullptr;
     int start = TILE_FIRST, nsteps = 0;
     float c0 = 0.f, cd[8] = {}, cr[8] = {};
+    FoldArgs fold;
 };
 // The tile of the least modelled cost for `steps` steps (and the restriction)
 // on level d; its cost in microseconds.
@@ -188,33 +194,37 @@ void launch_batch_begin(hipStream_t s, KrylovScalars *sc, double stop_rr, double
 void launch_residual64(hipStream_t s, Dims d, Op64 A, const double *b, const double *x,
                        double *r, double *partials, KrylovScalars *sc, float *b32 = nullptr,
                        float *x0 = nullptr, const float *diag32 = nullptr, float c0 = 0.f);
-// w = A z; dots z.w, z.q_prev, z.r; the last block forms beta, p.q and alpha.
-// active: the FP32 diagonal (0 = inactive cell) to skip all-inactive
-// wavefronts, where z must be 0; null = every cell (any z).
+// w = A z; dots z.w, z.q_prev, z.r, and with them alpha, beta and p.q of
+// iteration number iter (scalars->alpha[iter % kCoefs], ...). fold: only the
+// partial sums (the update adds them).
+// active: the FP32 diagonal (0 = inactive cell, where z counts as 0) to skip
+// all-inactive wavefronts; null = every cell.
 void launch_fcg_matvec(hipStream_t s, Dims d, Op64 A, const float *active, const float *z,
-                       const double *r, const double *qprev, double *w, int first,
+                       const double *r, const double *qprev, double *w, int first, int iter, bool fold,
                        double *partials, KrylovScalars *sc, const double *gate = nullptr,
                        hipEvent_t kernel_done = nullptr);
-// The update of x in an FCG iteration: now (x += alpha p), later (left for
-// the next iteration or launch_fcg_flush), or both the previous iteration's
-// and this one's (x += alpha_prev p_prev + alpha p), so x is read and written
-// every other iteration.
-enum XUpdate : int { X_NOW = 0, X_LATER = 1, X_BOTH = 2 };
-// p = z - beta p; q = w - beta q; x per xmode; r -= alpha q; rr = r.r
-// (all-inactive wavefronts skipped when `active` is given); b32 (or null)
-// receives r rounded to FP32 and x0 (or null) the first Chebyshev iterate
-// c0 D^{-1} b32, with D the FP32 diagonal `active`.
-void launch_fcg_update(hipStream_t s, Dims d, const float *active, const float *z,
-                       const double *w, double *p, double *q, double *x, double *r, float *b32,
-                       float *x0, float c0, int first, int xmode, double *partials,
+// q = w - beta q; r -= alpha q; rr = r.r (all-inactive wavefronts skipped when
+// `active` is given); b32 (or null) receives r rounded to FP32 and x0 (or null)
+// the first Chebyshev iterate c0 D^{-1} b32, with D the FP32 diagonal
+// `active`. fold: the scalars are formed from the matvec's partials in the
+// kernel, and of rr only the partial sums (launch_fcg_norm, or the next cycle's
+// first launch, adds them).
+void launch_fcg_update(hipStream_t s, Dims d, const float *active, const double *w, double *q, double *r,
+                       float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate = nullptr,
                        hipEvent_t kernel_done = nullptr);
 // (kernel_done, if given, is recorded after the stencil kernel and before
 // the one-block finalize that forms the scalars.)
-// x += alpha p with the last iteration's alpha and direction (after an
-// X_LATER iteration), over the update's groups of cells.
-void launch_fcg_flush(hipStream_t s, Dims d, const float *active, const double *p, double *x,
-                      const KrylovScalars *sc);
+// rr from the update's partials; counts the update and raises `stop`.
+void launch_fcg_norm(hipStream_t s, Dims d, double *partials, KrylovScalars *sc, const double *gate = nullptr);
+// Grids whose reductions' partials the kernels that need the sums add
+// themselves.
+bool fold_pays(Dims d);
+FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc);
+// x += alpha_k p_k, p_k = z_k - beta_k p_{k-1} for the K <= kRing iterations
+// i0 .. i0 + K - 1 whose z_k are at z + (k - i0) stride (see k_fcg_flush).
+void launch_fcg_flush(hipStream_t s, Dims d, const float *active, const float *z, size_t stride, int K, int i0,
+                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc);
 // z = D^{-1} r on active cells (Jacobi preconditioner).
 void launch_jacobi(hipStream_t s, Dims d, Op32 A, const double *r, float *z,
                    const double *gate = nullptr);

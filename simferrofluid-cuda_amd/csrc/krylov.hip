@@ -204,9 +204,10 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
     block_partials<2>(v, partials);
 }
 
-// `active` (the FP32 diagonal, 0 = inactive cell) or null: with it, a
-// wavefront whose cells are all inactive is skipped (z is 0 there and the
-// vectors it would write are never read by active cells). The flag of the
+// `active` (the FP32 diagonal, 0 = inactive cell) or null: with it, z counts as
+// 0 at the inactive cells (a z buffer may hold an earlier solve's values in
+// groups that its writer skips), and a wavefront whose cells are all inactive
+// is skipped (the vectors it would write are never read by active cells). The flag of the
 // next plane is loaded one plane ahead, and every load of a plane is issued
 // before the lane exchange.
 __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64 A,
@@ -232,8 +233,9 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64
     bool primed = false;  // zm, zc, cxc hold this plane's values
     float act_next = (active && on) ? active[c] : 0.f;
     for (int i = i0; i < ie; i++, c += s.sx) {
+        float act = 1.f;
         if (active) {
-            const float act = act_next;
+            act = act_next;
             act_next = (on && i + 1 < ie) ? active[c + s.sx] : 0.f;
             if (!__any(on && act > 0.f)) {
                 primed = false;
@@ -273,7 +275,7 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64
             if (j + 1 < d.ny) off += cyp * (double)zyp;
             if (zlo) off += czm * (double)zzm;
             if (zhi) off += czp * (double)zzp;
-            const double zd = (double)zc;
+            const double zd = act > 0.f ? (double)zc : 0.0;
             const double wc = dg * zd - off;
             st_stream(w + c, wc);
             v[0] += zd * wc;
@@ -308,10 +310,12 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
     const size_t c = (size_t)blockIdx.x * kMatvecCells + 2 * (size_t)flat_tid();
     const bool on = c < d.cells();  // cells() is even: then c + 1 is a cell too
     double v[3] = {0.0, 0.0, 0.0};  // z.w, z.q_prev, z.r
-    bool act = on;
+    bool act = on, on0 = true, on1 = true;  // the pair's cells are active
     if (active && on) {
         const float2v a = *(const float2v *)(active + c);
-        act = a.x > 0.f || a.y > 0.f;
+        on0 = a.x > 0.f;
+        on1 = a.y > 0.f;
+        act = on0 || on1;
     }
     if (__any(act) && on) {
         // (i, j, k) of the first cell (the launcher keeps cells() < 2^32)
@@ -324,7 +328,8 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
         const bool zl = k > 0, zh = k + 2 < d.nz;  // neighbours below the first, above the second
         const float2v f0 = {0.f, 0.f};
         const double2v d0 = {0.0, 0.0};
-        const float2v zc = *(const float2v *)(z + c);
+        const float2v zl2 = *(const float2v *)(z + c);
+        const float2v zc = {on0 ? zl2.x : 0.f, on1 ? zl2.y : 0.f};
         const float2v zxm = xl ? *(const float2v *)(z + c - s.sx) : f0;
         const float2v zxp = xh ? *(const float2v *)(z + c + s.sx) : f0;
         const float2v zym = yl ? *(const float2v *)(z + c - s.sy) : f0;
@@ -382,28 +387,69 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
     block_partials<3>(v, partials);
 }
 
+// The iteration's scalars from its dots: p = z - beta p_prev with beta =
+// z.q_prev / p_prev.q_prev makes p A-orthogonal to p_prev; then p.q = z.w -
+// beta z.q_prev, and p.r = z.r because p_prev.r = 0 after the previous step.
+struct Recurrence {
+    double alpha, beta, pq;
+};
+__device__ __forceinline__ Recurrence recurrence(const double (&v)[3], double pq_prev, int first) {
+    Recurrence c{0.0, 0.0, v[0]};
+    if (!first && pq_prev != 0.0) {
+        c.beta = v[1] / pq_prev;
+        c.pq = v[0] - c.beta * v[1];
+    }
+    c.alpha = c.pq != 0.0 ? v[2] / c.pq : 0.0;
+    return c;
+}
+
 // The update is pointwise: it runs over the flat cell index with two
 // consecutive cells per lane (16-byte loads and stores of the FP64 vectors),
 // one pair per thread (kUpdateCells per block). A wavefront whose 128 cells
-// are all inactive is skipped (p, q, x, r stay 0 there). With b32 it also
+// are all inactive is skipped (q, r stay 0 there). With b32 it also
 // stores the new residual rounded to FP32: the right-hand side the next
 // V-cycle starts from, which then need not read the FP64 residual.
+//
+// Neither the direction p nor the solution x is formed here: both are sums of
+// the iterations' z with scalars, so the z are kept (FP32, as the V-cycle
+// stores them) and k_fcg_flush runs p = z - beta p, x += alpha p for up to
+// kRing iterations in one pass. The update then moves 40 B per cell and the
+// FP32 copies' 12 instead of 80 (z, p in and out, x every other iteration).
+//
+// kFold: the block adds the matvec's partials (mv, nb_mv of them) and forms
+// the scalars itself (and block 0 stores them) instead of a finalize launch
+// before it.
 constexpr unsigned kUpdateCells = 2 * kBlock;
 
+template <bool kFold>
 __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__restrict__ active,
-                                                       const float *z,  // may be x0: read before x0 is written
                                                        const double *__restrict__ w,
-                                                       double *__restrict__ p,
                                                        double *__restrict__ q,
-                                                       double *__restrict__ x,
                                                        double *__restrict__ r,
                                                        float *__restrict__ b32,
-                                                       float *x0, float c0, int first, int xmode,
+                                                       float *__restrict__ x0, float c0, int first, int iter,
+                                                       const double *__restrict__ mv, unsigned nb_mv,
                                                        double *__restrict__ partials,
-                                                       const KrylovScalars *__restrict__ sc,
+                                                       KrylovScalars *sc,
                                                        const double *gate) {
     if (gated(gate)) return;
-    const double alpha = sc->alpha, beta = sc->beta, alpha_prev = sc->alpha_prev;
+    const int ci = iter % kCoefs;
+    double alpha, beta;
+    if constexpr (kFold) {
+        double v[3];
+        fold_partials<3>(mv, nb_mv, v);
+        const Recurrence c = recurrence(v, first ? 0.0 : sc->pq[(iter + kCoefs - 1) % kCoefs], first);
+        alpha = c.alpha;
+        beta = c.beta;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            sc->alpha[ci] = alpha;
+            sc->beta[ci] = beta;
+            sc->pq[ci] = c.pq;
+        }
+    } else {
+        alpha = sc->alpha[ci];
+        beta = sc->beta[ci];
+    }
     double v[1] = {0.0};
     const size_t c = (size_t)blockIdx.x * kUpdateCells + 2 * (size_t)flat_tid();
     const bool pair = c + 1 < n;  // else at most the grid's last cell
@@ -416,38 +462,19 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
     }
     if (__any(act)) {
         if (pair) {
-            const float2v zf = *(const float2v *)(z + c);
-            const double2v zc = {(double)zf.x, (double)zf.y};
             const double2v wc = ld_stream((const double2v *)(w + c));
             const double2v r0 = ld_stream((const double2v *)(r + c));
-            double2v pc, qc, pp = {0.0, 0.0};
-            if (first) {
-                pc = zc;
-                qc = wc;
-            } else {
-                pp = ld_stream((const double2v *)(p + c));
+            double2v qc = wc;
+            if (!first) {
                 const double2v qq = ld_stream((const double2v *)(q + c));
-                pc.x = zc.x - beta * pp.x;
-                pc.y = zc.y - beta * pp.y;
                 qc.x = wc.x - beta * qq.x;
                 qc.y = wc.y - beta * qq.y;
             }
             double2v rc;
             rc.x = r0.x - alpha * qc.x;
             rc.y = r0.y - alpha * qc.y;
-            st_stream((double2v *)(p + c), pc);
             st_stream((double2v *)(q + c), qc);
             st_stream((double2v *)(r + c), rc);
-            if (xmode != X_LATER) {
-                double2v xn = ld_stream((const double2v *)(x + c));
-                if (xmode == X_BOTH) {
-                    xn.x += alpha_prev * pp.x;
-                    xn.y += alpha_prev * pp.y;
-                }
-                xn.x += alpha * pc.x;
-                xn.y += alpha * pc.y;
-                st_stream((double2v *)(x + c), xn);
-            }
             if (b32) {
                 const float2v bf = {(float)rc.x, (float)rc.y};
                 *(float2v *)(b32 + c) = bf;
@@ -459,18 +486,8 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
             v[0] += rc.x * rc.x;
             v[0] += rc.y * rc.y;
         } else if (c < n) {
-            const double zc = (double)z[c];
-            const double pp = first ? 0.0 : p[c];
-            const double pc = first ? zc : zc - beta * pp;
             const double qc = first ? w[c] : w[c] - beta * q[c];
-            p[c] = pc;
             q[c] = qc;
-            if (xmode != X_LATER) {
-                double xn = x[c];
-                if (xmode == X_BOTH) xn += alpha_prev * pp;
-                xn += alpha * pc;
-                x[c] = xn;
-            }
             const double rc = r[c] - alpha * qc;
             r[c] = rc;
             if (b32) {
@@ -483,31 +500,64 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
     block_partials<1>(v, partials);
 }
 
-// x += alpha p (the update an X_LATER iteration left pending), over the
-// update's groups of cells.
+// p = z_k - beta_k p, x += alpha_k p for K iterations (numbers i0 .. i0 + K - 1,
+// their z at z + k stride), in the order and arithmetic of an update per
+// iteration. has_p: p0 holds the direction before them; store_p: it receives
+// the last one. zero_x: x starts from 0 (and every cell is written); else a
+// wavefront without active cells is skipped. z counts as 0 at inactive cells.
+template <int K>
 __global__ __launch_bounds__(kBlock) void k_fcg_flush(size_t n, const float *__restrict__ active,
-                                                      const double *__restrict__ p,
-                                                      double *__restrict__ x,
+                                                      const float *__restrict__ z, size_t stride,
+                                                      double *__restrict__ p0, int has_p, int store_p,
+                                                      double *__restrict__ x, int zero_x, int i0,
                                                       const KrylovScalars *__restrict__ sc) {
-    const double alpha = sc->alpha;
     const size_t c = (size_t)blockIdx.x * kUpdateCells + 2 * (size_t)flat_tid();
     const bool pair = c + 1 < n;
     bool act = c < n;
+    float2v dg = {1.f, 1.f};
     if (active) {
-        float2v dg = {0.f, 0.f};
+        dg = float2v{0.f, 0.f};
         if (pair) dg = *(const float2v *)(active + c);
         else if (c < n) dg.x = active[c];
         act = dg.x > 0.f || dg.y > 0.f;
     }
-    if (!__any(act)) return;
+    if (zero_x ? !(c < n) : !__any(act)) return;
+    double alpha[K], beta[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        alpha[k] = sc->alpha[(i0 + k) % kCoefs];
+        beta[k] = sc->beta[(i0 + k) % kCoefs];
+    }
     if (pair) {
-        const double2v pc = ld_stream((const double2v *)(p + c));
-        double2v xn = ld_stream((const double2v *)(x + c));
-        xn.x += alpha * pc.x;
-        xn.y += alpha * pc.y;
+        float2v zk[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            zk[k] = act ? ld_stream((const float2v *)(z + k * stride + c)) : float2v{0.f, 0.f};
+            if (!(dg.x > 0.f)) zk[k].x = 0.f;
+            if (!(dg.y > 0.f)) zk[k].y = 0.f;
+        }
+        double2v p = {0.0, 0.0}, xn = {0.0, 0.0};
+        if (has_p) p = ld_stream((const double2v *)(p0 + c));
+        if (!zero_x) xn = ld_stream((const double2v *)(x + c));
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            p.x = (double)zk[k].x - beta[k] * p.x;
+            p.y = (double)zk[k].y - beta[k] * p.y;
+            xn.x += alpha[k] * p.x;
+            xn.y += alpha[k] * p.y;
+        }
+        if (store_p) st_stream((double2v *)(p0 + c), p);
         st_stream((double2v *)(x + c), xn);
     } else if (c < n) {
-        x[c] += alpha * p[c];
+        double p = has_p ? p0[c] : 0.0, xn = zero_x ? 0.0 : x[c];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const double zc = dg.x > 0.f ? (double)z[k * stride + c] : 0.0;
+            p = zc - beta[k] * p;
+            xn += alpha[k] * p;
+        }
+        if (store_p) p0[c] = p;
+        x[c] = xn;
     }
 }
 
@@ -555,7 +605,7 @@ __global__ __launch_bounds__(64) void k_batch_begin(KrylovScalars *sc, double st
     }
 }
 
-__global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned nb, int first,
+__global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned nb, int first, int iter,
                                                      const double *__restrict__ partials,
                                                      KrylovScalars *sc, const double *gate) {
     if (gated(gate)) return;
@@ -577,26 +627,16 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
         sc->rr = v[0];
         sc->bb = v[1];
     } else if (op == FIN_MATVEC) {
-        const double zw = v[0], zq = v[1], zr = v[2];
-        double beta = 0.0, pq = zw;
-        if (!first && sc->pq_prev != 0.0) {
-            // p = z - beta p_prev with beta = z.q_prev / p_prev.q_prev makes p
-            // A-orthogonal to p_prev; then p.q = z.w - beta z.q_prev, and
-            // p.r = z.r because p_prev.r = 0 after the previous step.
-            beta = zq / sc->pq_prev;
-            pq = zw - beta * zq;
-        }
-        sc->zw = zw;
-        sc->zq = zq;
-        sc->zr = zr;
-        sc->beta = beta;
-        sc->pq = pq;
-        sc->alpha_prev = sc->alpha;
-        sc->alpha = pq != 0.0 ? zr / pq : 0.0;
+        const Recurrence c = recurrence(v, first ? 0.0 : sc->pq[(iter + kCoefs - 1) % kCoefs], first);
+        sc->zw = v[0];
+        sc->zq = v[1];
+        sc->zr = v[2];
+        sc->alpha[iter % kCoefs] = c.alpha;
+        sc->beta[iter % kCoefs] = c.beta;
+        sc->pq[iter % kCoefs] = c.pq;
     } else if (op == FIN_UPDATE) {
         const double rr_prev = sc->rr;
         sc->rr = v[0];
-        sc->pq_prev = sc->pq;
         sc->iters += 1.0;
         if (gate && v[0] <= sc->stop_rr) sc->stop = 1.0;  // later gated kernels return at once
         if (gate && sc->stall_rr > 0.0 && v[0] > sc->stall_rr * rr_prev) {
@@ -632,7 +672,7 @@ __global__ __launch_bounds__(kStageThreads) void k_partials_stage(unsigned nb, u
 
 // `partials` holds the N sums of op for nb blocks ([q * nb + b]); the stage
 // writes its sums after them (reduction_partials leaves room).
-void finalize(hipStream_t st, int op, unsigned nb, int first, double *partials, KrylovScalars *sc,
+void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *partials, KrylovScalars *sc,
               const double *gate = nullptr) {
     const int N = op == FIN_MATVEC ? 3 : op == FIN_RESIDUAL ? 2 : 1;
     if (nb > kStageMin) {
@@ -652,8 +692,8 @@ void finalize(hipStream_t st, int op, unsigned nb, int first, double *partials, 
         partials = out;
         nb = G;
     }
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, st, op, nb, first, partials,
-                       sc, gate);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, st, op, nb, first, iter,
+                       partials, sc, gate);
     SFP_LAUNCH_CHECK();
 }
 
@@ -672,10 +712,20 @@ static unsigned matvec_blocks(Dims d) {
 static unsigned update_blocks(Dims d) { return (unsigned)((d.cells() + kUpdateCells - 1) / kUpdateCells); }
 
 size_t reduction_partials(Dims d) {
-    // The largest set of partials, then room for the two-stage finalize's chunk sums.
-    return std::max({3 * (size_t)cell_launch(d, kReducePlanes).blocks(),
-                     3 * (size_t)matvec_blocks(d), (size_t)update_blocks(d)}) +
+    // The matvec's partials, the update's after them (a folded update reads
+    // the former while it writes the latter) or the largest other set, then
+    // room for the two-stage finalize's chunk sums.
+    return std::max(3 * (size_t)cell_launch(d, kReducePlanes).blocks(),
+                    3 * (size_t)matvec_blocks(d) + (size_t)update_blocks(d)) +
            3 * (size_t)kStageMaxBlocks;
+}
+
+// Up to this many partials a kernel adds them itself (fold_partials): every
+// block reads them all, from L2 (64^3: 512 blocks, 12 KB each).
+constexpr unsigned kFoldMax = 2048;
+bool fold_pays(Dims d) { return std::max(matvec_blocks(d), update_blocks(d)) <= kFoldMax; }
+FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc) {
+    return FoldArgs{partials + 3 * (size_t)matvec_blocks(d), update_blocks(d), sc};
 }
 
 void launch_count_active(hipStream_t st, Dims d, const float *diag32, double *partials,
@@ -683,7 +733,7 @@ void launch_count_active(hipStream_t st, Dims d, const float *diag32, double *pa
     Launch L = cell_launch(d, kReducePlanes);
     hipLaunchKernelGGL(k_count_active, L.grid, L.block, 0, st, L.cg, d, diag32, partials);
     SFP_LAUNCH_CHECK();
-    finalize(st, FIN_COUNT, L.blocks(), 0, partials, sc);
+    finalize(st, FIN_COUNT, L.blocks(), 0, 0, partials, sc);
 }
 
 void launch_batch_begin(hipStream_t st, KrylovScalars *sc, double stop_rr, double stall_rr) {
@@ -705,19 +755,20 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
         hipLaunchKernelGGL(k_residual64_flat, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials, b32,
                            x0, diag32, c0);
         SFP_LAUNCH_CHECK();
-        finalize(st, FIN_RESIDUAL, nb, 0, partials, sc);
+        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc);
         return;
     }
     Launch L = cell_launch(d, kReducePlanes);
     hipLaunchKernelGGL(k_residual64, L.grid, L.block, 0, st, L.cg, d, A, b, x, r, partials, b32, x0,
                        diag32, c0);
     SFP_LAUNCH_CHECK();
-    finalize(st, FIN_RESIDUAL, L.blocks(), 0, partials, sc);
+    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc);
 }
 
 void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, const float *z,
-                       const double *r, const double *qprev, double *w, int first,
+                       const double *r, const double *qprev, double *w, int first, int iter, bool fold,
                        double *partials, KrylovScalars *sc, const double *gate, hipEvent_t kernel_done) {
+    unsigned nb = matvec_blocks(d);
     if (matvec_flat(d)) {
         // pairs of cells: 16-byte (8-byte for z and the flags) aligned vectors
         for (const void *a : {(const void *)A.diag, (const void *)A.cpl[0], (const void *)A.cpl[1],
@@ -725,45 +776,68 @@ void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, cons
             if ((uintptr_t)a % 16) throw ArgError("launch_fcg_matvec: FP64 array not 16-byte aligned");
         if ((uintptr_t)z % 8 || (uintptr_t)active % 8)
             throw ArgError("launch_fcg_matvec: z or the diagonal not 8-byte aligned");
-        const unsigned nb = matvec_blocks(d);
         hipLaunchKernelGGL(k_fcg_matvec_flat, dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r,
                            qprev, w, first, partials, gate);
-        SFP_LAUNCH_CHECK();
-        if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
-        finalize(st, FIN_MATVEC, nb, first, partials, sc, gate);
-        return;
+    } else {
+        const Launch L = matvec_launch(d);
+        hipLaunchKernelGGL(k_fcg_matvec, L.grid, L.block, 0, st, L.cg, d, A, active, z, r, qprev, w,
+                           first, partials, gate);
     }
-    Launch L = matvec_launch(d);
-    hipLaunchKernelGGL(k_fcg_matvec, L.grid, L.block, 0, st, L.cg, d, A, active, z, r, qprev, w,
-                       first, partials, gate);
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
-    finalize(st, FIN_MATVEC, L.blocks(), first, partials, sc, gate);
+    if (!fold) finalize(st, FIN_MATVEC, nb, first, iter, partials, sc, gate);
 }
 
-void launch_fcg_update(hipStream_t st, Dims d, const float *active, const float *z,
-                       const double *w, double *p, double *q, double *x, double *r, float *b32,
-                       float *x0, float c0, int first, int xmode, double *partials,
+void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double *w, double *q, double *r,
+                       float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate, hipEvent_t kernel_done) {
-    if (xmode == X_BOTH && first) throw ArgError("launch_fcg_update: X_BOTH needs a previous direction");
-    // two cells per lane: 16-byte (8-byte for z) aligned vectors
-    for (const void *a : {(const void *)w, (const void *)p, (const void *)q, (const void *)x, (const void *)r})
+    // two cells per lane: 16-byte (8-byte for the FP32 ones) aligned vectors
+    for (const void *a : {(const void *)w, (const void *)q, (const void *)r})
         if ((uintptr_t)a % 16) throw ArgError("launch_fcg_update: FP64 vector not 16-byte aligned");
-    if ((uintptr_t)z % 8 || (uintptr_t)b32 % 8 || (uintptr_t)x0 % 8)
-        throw ArgError("launch_fcg_update: z, b32 or x0 not 8-byte aligned");
+    if ((uintptr_t)active % 8 || (uintptr_t)b32 % 8 || (uintptr_t)x0 % 8)
+        throw ArgError("launch_fcg_update: the diagonal, b32 or x0 not 8-byte aligned");
     if (x0 && (!b32 || !active)) throw ArgError("launch_fcg_update: x0 needs b32 and the diagonal");
-    const unsigned nb = update_blocks(d);
-    hipLaunchKernelGGL(k_fcg_update, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, z, w, p, q,
-                       x, r, b32, x0, c0, first, xmode, partials, sc, gate);
+    const unsigned nb = update_blocks(d), nb_mv = matvec_blocks(d);
+    double *out = partials + 3 * (size_t)nb_mv;
+    if (fold)
+        hipLaunchKernelGGL(k_fcg_update<true>, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, w, q, r, b32, x0,
+                           c0, first, iter, partials, nb_mv, out, sc, gate);
+    else
+        hipLaunchKernelGGL(k_fcg_update<false>, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, w, q, r, b32, x0,
+                           c0, first, iter, partials, nb_mv, out, sc, gate);
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
-    finalize(st, FIN_UPDATE, nb, first, partials, sc, gate);
+    if (!fold) launch_fcg_norm(st, d, partials, sc, gate);
 }
 
-void launch_fcg_flush(hipStream_t st, Dims d, const float *active, const double *p, double *x,
-                      const KrylovScalars *sc) {
-    const unsigned nb = update_blocks(d);
-    hipLaunchKernelGGL(k_fcg_flush, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, p, x, sc);
+void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc, const double *gate) {
+    finalize(st, FIN_UPDATE, update_blocks(d), 0, 0, partials + 3 * (size_t)matvec_blocks(d), sc, gate);
+}
+
+void launch_fcg_flush(hipStream_t st, Dims d, const float *active, const float *z, size_t stride, int K, int i0,
+                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc) {
+    if (K < 1 || K > kRing) throw ArgError("launch_fcg_flush: bad iteration count");
+    if ((has_p || store_p) && !p) throw ArgError("launch_fcg_flush: no direction");
+    if ((uintptr_t)z % 8 || stride % 2 || (uintptr_t)active % 8 || (uintptr_t)p % 16 || (uintptr_t)x % 16)
+        throw ArgError("launch_fcg_flush: vectors not aligned");
+    const dim3 grid(update_blocks(d)), block(kBlock);
+#define SFP_FLUSH(N)                                                                                   \
+    case N:                                                                                            \
+        hipLaunchKernelGGL(k_fcg_flush<N>, grid, block, 0, st, d.cells(), active, z, stride, p,        \
+                           has_p ? 1 : 0, store_p ? 1 : 0, x, zero_x ? 1 : 0, i0, sc);                 \
+        break;
+    switch (K) {
+        SFP_FLUSH(1)
+        SFP_FLUSH(2)
+        SFP_FLUSH(3)
+        SFP_FLUSH(4)
+        SFP_FLUSH(5)
+        SFP_FLUSH(6)
+        SFP_FLUSH(7)
+        SFP_FLUSH(8)
+    }
+#undef SFP_FLUSH
+    static_assert(kRing == 8, "one instance per iteration count");
     SFP_LAUNCH_CHECK();
 }
 

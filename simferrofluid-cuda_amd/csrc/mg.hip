@@ -2000,7 +2000,9 @@ void launch_vcycle_tail_lds(hipStream_t st, const TailArgs &t, const double *gat
         if (t.deg[k] < 1 || t.deg[k] > 8) throw ArgError("vcycle tail: bad degree");
     if (t.lv[0].d.cells() > kTailLdsMaxCells) throw ArgError("vcycle tail: level too large");
     if ((int)t.lv[t.nlev - 1].d.cells() > kMaxCoarse) throw ArgError("vcycle tail: coarsest too large");
-    if (tail_lds_bytes(t) > kTailLdsBytes) throw ArgError("vcycle tail: levels exceed the LDS");
+    size_t bytes = 0;
+    for (int l = 0; l < t.nlev; l++) bytes += tail_lds_bytes(t.lv[l].d);
+    if (bytes > kTailLdsBytes) throw ArgError("vcycle tail: levels exceed the LDS");
     hipLaunchKernelGGL(k_vcycle_tail_lds, dim3(1), dim3(kTailThreads), 0, st, t, gate);
     SFP_LAUNCH_CHECK();
 }

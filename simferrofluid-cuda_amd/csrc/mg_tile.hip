@@ -31,6 +31,19 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ bool gated(const double *gate) { return gate && *gate != 0.0; }
 
+// The pending ||r||^2 (see FoldArgs): true when the solve stops here.
+__device__ __forceinline__ bool fold_stop(const FoldArgs &f) {
+    double v[1];
+    fold_partials<1>(f.partials, f.nb, v);
+    const bool stop = v[0] <= f.sc->stop_rr;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        f.sc->rr = v[0];
+        f.sc->iters += 1.0;
+        if (stop) f.sc->stop = 1.0;
+    }
+    return stop;
+}
+
 // Guard floats before and after an LDS iterate (the z neighbours of its first
 // and last group; any finite value, their coupling is 0).
 constexpr int kGuard = 4;
@@ -260,6 +273,7 @@ __global__ __launch_bounds__(1024) void k_tile_steps(TileArgs a, const double *g
         }
     }
     if (gated(gate)) return;  // (after the loads: the flag's latency is theirs)
+    if (a.fold.nb && fold_stop(a.fold)) return;  // uniform
     if (threadIdx.x < 2 * kGuard) {
         const int o = threadIdx.x < kGuard ? threadIdx.x : 4 * ng + threadIdx.x;
         lds[0][o] = lds[1][o] = 0.f;
@@ -450,6 +464,7 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(TailArgs t, const double *
         *(f4 *)(inv + r * kInvStride + c) = a4;
     }
     if (gated(gate)) return;  // (after the loads: the flag's latency is theirs)
+    if (t.fold.nb && fold_stop(t.fold)) return;  // uniform
     if (tid < 2 * kGuard) {
         const int o = tid < kGuard ? tid : 4 * ng + tid;
         lds[0][o] = lds[1][o] = 0.f;

@@ -146,20 +146,25 @@ struct Level {
     }
 };
 
+// Directions of FCG iterations kept as their FP32 preconditioned residuals z
+// until the solution is brought up to date (see launch_fcg_flush), and the
+// iterations whose coefficients are kept.
+constexpr int kRing = 8, kCoefs = 2 * kRing;
+
 // Scalars of the flexible-CG recurrences, resident on the device.
 struct KrylovScalars {
-    double zw, zq, zr, pq_prev;  // dots of the current iteration
-    double alpha, beta, pq;
+    double zw, zq, zr;           // dots of the current iteration
     double rr, bb;               // ||r||^2, ||b||^2
     double pad[4];               // scratch of single reductions (count, scales)
     // batched iterations: `stop` becomes nonzero when rr <= stop_rr after an
     // update, and every gated kernel of later iterations then returns at once;
     // `iters` counts the updates done
     double stop, iters, stop_rr;
-    double alpha_prev;  // the previous iteration's alpha (lagged solution update)
     // learned preconditioner in a batch: an update whose ||r||^2 exceeds
     // stall_rr times the previous one raises `stalled` and `stop` (0: off)
     double stall_rr, stalled;
+    // of iteration number i, at i mod kCoefs
+    double alpha[kCoefs], beta[kCoefs], pq[kCoefs];
 };
 
 // Per-kernel timing collected with HIP events on the context stream.

@@ -114,10 +114,13 @@ void System::allocate(Dims d) {
     rhs_.ensure(n);
     x_.ensure(n);
     r_.ensure(n);
-    p_.ensure(n);
     q_.ensure(n);
     w_.ensure(n);
-    for (auto *v : {&r_, &p_, &q_, &w_}) SFP_HIP(hipMemset(v->p, 0, n * sizeof(double)));
+    for (auto *v : {&r_, &q_, &w_}) SFP_HIP(hipMemset(v->p, 0, n * sizeof(double)));
+    zring_stride_ = (n + 63) / 64 * 64;
+    zring_.ensure(kRing * zring_stride_);
+    SFP_HIP(hipMemset(zring_.p, 0, kRing * zring_stride_ * sizeof(float)));
+    p_.release();
     SFP_HIP(hipMemset(x_.p, 0, n * sizeof(double)));
     built_coarsest_ = -1;
 }
@@ -191,9 +194,10 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     // A new operator may have a new active set, so the vectors are cleared at
     // the inactive cells (values left on cells that were active before would
     // otherwise leak into z, w, q and the inner products). Active cells are
-    // written before they are read in every cycle; p and q are written at
-    // every cell of the update's groups by the first iteration and read in
-    // those groups only.
+    // written before they are read in every cycle; q is written at every cell
+    // of the update's groups by the first iteration and read in those groups
+    // only. The ring of z needs none: z counts as 0 at inactive cells wherever
+    // it is read for its own cell, and elsewhere couples with weight 0.
     if (lv_.size() > (size_t)kClearMaxLevels) throw ArgError("too many multigrid levels");
     ClearArgs ca;
     ca.nlev = (int)lv_.size();
@@ -212,13 +216,30 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     launch_clear_inactive(ws.stream, ca);
 }
 
-float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
+// (see launch_vcycle_tail_lds)
+static bool lds_tail(Dims coarsest) { return coarsest.cells() % 4 == 2; }
+
+bool System::tail_at(const Workspace &ws, int l) const {
     const int nlev = (int)lv_.size() - l;
-    if (!ws.vcycle_tail || nlev < 2 || nlev > kTailMaxLevels) return nullptr;
+    if (!ws.vcycle_tail || nlev < 2 || nlev > kTailMaxLevels) return false;
     Dims dims[kTailMaxLevels];
     for (int q = 0; q < nlev; q++) dims[q] = lv_[l + q].d;
-    const bool lds = dims[nlev - 1].cells() % 4 == 2;  // (see launch_vcycle_tail_lds)
-    if (lds ? dims[0].cells() > kTailLdsMaxCells : !tail_fits(dims, nlev)) return nullptr;
+    if (!lds_tail(dims[nlev - 1])) return tail_fits(dims, nlev);
+    size_t bytes = 0;
+    for (int q = 0; q < nlev; q++) bytes += tail_lds_bytes(dims[q]);
+    return dims[0].cells() <= kTailLdsMaxCells && bytes <= kTailLdsBytes;
+}
+
+bool System::fold_at(const Workspace &ws, const Smoothing &sm, int l) {
+    if (!fold_pays(lv_[l].d) || l + 1 >= (int)lv_.size()) return false;
+    if (tail_at(ws, l)) return !lds_tail(lv_.back().d);
+    return tile_stages(ws, l, sm.at(l).degree - 1, true).n > 0;
+}
+
+float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
+    if (!tail_at(ws, l)) return nullptr;
+    const int nlev = (int)lv_.size() - l;
+    const bool lds = lds_tail(lv_.back().d);
     TailArgs t;
     t.nlev = nlev;
     for (int q = 0; q < nlev; q++) {
@@ -233,8 +254,9 @@ float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
             t.cr[set][q] = cb.cr[q];
         }
     }
+    t.lv[0].x1 = last_out(ws, l, t.lv[0].x1);
     t.ainv = ainv_.p;
-    if (lds && tail_lds_bytes(t) > kTailLdsBytes) return nullptr;
+    if (!lds && l == ws.z_level) t.fold = ws.fold;
     join_ainv(ws);
     if (lds) launch_vcycle_tail_lds(ws.stream, t, ws.gate);
     else launch_vcycle_tail(ws.stream, t, ws.gate);
@@ -314,8 +336,9 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
     if (l + 1 == (int)lv_.size()) {
         if (r64) launch_smooth_first(st, L.d, L.op32(), r64, L.b.p, L.x1.p, 0.f, ws.gate);
         join_ainv(ws);
-        launch_coarse_solve(st, (int)L.d.cells(), ainv_.p, L.b.p, L.x0.p, ws.gate);
-        return L.x0.p;
+        float *out = last_out(ws, l, L.x0.p);
+        launch_coarse_solve(st, (int)L.d.cells(), ainv_.p, L.b.p, out, ws.gate);
+        return out;
     }
     const Op32 A = L.op32();
     // the flat kernels (nz a multiple of 4) and the pair kernels rebuild a
@@ -357,6 +380,7 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
                 t.din = L.dv.p;
             }
             t.xout = oth;
+            if (q == 0 && l == ws.z_level) t.fold = ws.fold;
             if (q + 1 < T.n) t.dout = L.dv.p;
             else t.bc = C.b.p;
             launch_tile_steps(st, t, ws.gate);
@@ -442,8 +466,9 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
             t.xin = cur;
             t.e = e;
             if (q > 0) t.din = L.dv.p;
-            t.xout = oth;
             if (q + 1 < T.n) t.dout = L.dv.p;
+            else oth = last_out(ws, l, oth);
+            t.xout = oth;
             launch_tile_steps(st, t, ws.gate);
             std::swap(cur, oth);
         }
@@ -463,6 +488,7 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
         // step 0 adds the prolonged correction; the fine-level steps are timed
         const int mode = (s == 0 ? (add_first ? 0 : SM_PROLONG) : SM_READ_D) | (s < deg - 1 ? SM_WRITE_D : 0);
         const bool t = track;
+        if (s == deg - 1) oth = last_out(ws, l, oth);
         if (t) ws.timers[K_SMOOTH].begin(st, step_bytes(mode, L.pinned_rowsum && flat_step(L.d)) * (double)L.d.cells());
         launch_smooth(st, mode, L.d, A, nullptr, L.b.p, cur, oth, L.dv.p, cb.cr[0], s == 0 ? 0.f : cb.cd[s],
                       s == 0 ? cb.cr[0] : cb.cr[s], s == 0 ? e : nullptr, ws.gate);
@@ -471,6 +497,7 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
     }
     if (fused) {
         // reads x, b, d, diag (unless rebuilt), 3 couplings and writes x
+        oth = last_out(ws, l, oth);
         if (track) ws.timers[K_SMOOTH_PAIR].begin(st, (L.pinned_rowsum ? 28.0 : 32.0) * (double)L.d.cells());
         launch_smooth_pair(st, L.d, A, L.b.p, cur, oth, L.dv.p, cb.cd[deg - 2], cb.cr[deg - 2],
                            cb.cd[deg - 1], cb.cr[deg - 1], ws.gate, L.rowact.p);
@@ -482,8 +509,9 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
 
 float *System::precondition(Workspace &ws, const SolverConfig &cfg, const double *r64) {
     if (cfg.precond == 2) {  // SFP_PRECOND_JACOBI
-        launch_jacobi(ws.stream, d_, lv_[0].op32(), r64, lv_[0].x0.p, ws.gate);
-        return lv_[0].x0.p;
+        float *z = last_out(ws, 0, lv_[0].x0.p);
+        launch_jacobi(ws.stream, d_, lv_[0].op32(), r64, z, ws.gate);
+        return z;
     }
     if (cfg.precond == 3 && lv_.size() > 1) return learned_cycle(ws, cfg, r64, kCycleSmooth);
     return vlevel(ws, Smoothing::make(cfg), 0, r64);
@@ -494,7 +522,11 @@ float *System::learned_cycle(Workspace &ws, const SolverConfig &cfg, const doubl
     const Smoothing sm = Smoothing::make_learned(cfg);
     Level &L = lv_[0], &C = lv_[1];
     const hipStream_t st = ws.stream;
+    // (the V-cycle's result stays in the level; the last smoothing's goes to zout)
+    float *const zout = ws.zout;
+    ws.zout = nullptr;
     float *z = vlevel(ws, sm, 0, r64);
+    ws.zout = zout;
     // residual the V-cycle leaves, restricted to the first coarse level
     launch_restrict(st, L.d, L.op32(), L.b.p, z, C.b.p, ws.gate);
     if (c == kCycleRestrictOnly) return C.b.p;
@@ -569,7 +601,8 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     const Op64 A = lv_[level].op64();
     const bool fine = level == 0;
     const bool profiling = fine && ws.profiling;
-    if (!warm) SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));
+    // a cold solve's x is 0 until the first flush, which then does not read it
+    bool zero_x = !warm;
     // The V-cycle preconditioners start from the residual rounded to FP32 in
     // the level's b, with the cycle's first Chebyshev iterate in the level's
     // x0: the residual kernels and the FCG update store both, so no cycle
@@ -607,14 +640,26 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     // and iterations enqueued behind a stall would still launch every
     // kernel of the learned cycle (each returning at once)
     int next_batch = learned ? 1 : kBatch;
-    // x is updated every other iteration (X_LATER, then X_BOTH): `run` counts
-    // the updates since it was last current; an odd count leaves alpha p of
-    // the last one pending, added before anything reads x
-    int run = 0;
-    auto bring_x_up_to_date = [&]() {
-        if (run % 2) launch_fcg_flush(st, d, lv_[level].diag32.p, p_.p, x_.p, ws.scalars.p);
-        run = 0;
+    // iterations whose z is in the ring and whose alpha p is not yet in x, and
+    // the number of the next iteration (its scalars' place)
+    int pending = 0, iter = 0;
+    bool has_p = false;  // p_ holds the direction before the pending iterations
+    const float *flags = A.pinned_rowsum ? nullptr : lv_[level].diag32.p;
+    auto bring_x_up_to_date = [&](bool keep_p) {
+        if (pending > 0) {
+            if (keep_p) p_.ensure(d_.cells());
+            launch_fcg_flush(st, d, flags, zring_.p, zring_stride_, pending, iter - pending, p_.p,
+                             has_p, keep_p, x_.p, zero_x, ws.scalars.p);
+            zero_x = false;
+            has_p = keep_p;
+        }
+        pending = 0;
     };
+    // small grids: the reductions' partials are added by the launches that
+    // need the sums (the update, and the next cycle's first) instead of
+    // finalize launches between
+    const bool fold = !profiling && cfg.precond == 0 && fold_at(ws, plain, level);
+    ws.z_level = level;
     info.precond_used = learned ? 1 : (cfg.precond == 1 ? 0 : cfg.precond);
     while (true) {
         if (rel <= cfg.tol) {
@@ -622,7 +667,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             // recursive residual reached tol: recompute its norm from x in
             // FP64 (the sums only), and restart from the true residual if the
             // two have drifted apart
-            bring_x_up_to_date();
+            bring_x_up_to_date(false);
             launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p);
             ws.read_scalars();
             rel = std::sqrt(ws.host_sc->rr / bb);
@@ -643,7 +688,8 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
         // once an iteration reduced ||r|| by less than stall_ratio, and every
         // kernel of the remaining iterations of the batch then returns at
         // once (profiled launches among them are dropped from the timings).
-        const int batch = std::min(next_batch, cfg.max_iters - info.iterations);
+        if (pending == kRing) bring_x_up_to_date(true);
+        const int batch = std::min({next_batch, cfg.max_iters - info.iterations, kRing - pending});
         if (batch > 1) {
             launch_batch_begin(st, ws.scalars.p, cfg.tol * cfg.tol * bb,
                                learned ? cfg.stall_ratio * cfg.stall_ratio : 0.0);
@@ -652,6 +698,10 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
         for (int it = 0; it < batch; it++) {
             const double *r64 = b_ready ? nullptr : r_.p;  // null: the cycle reads b
             ws.x0_level = b_ready ? level : -1;
+            ws.zout = zring_.p + (size_t)(pending + it) * zring_stride_;
+            // (within a batch, the update before this cycle left its norm's
+            // partials)
+            ws.fold = fold && it > 0 ? update_fold(d, ws.partials.p, ws.scalars.p) : FoldArgs{};
             const float *z;
             if (learned)
                 z = precondition_learned(ws, cfg, r64);
@@ -670,30 +720,32 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
                                                  (first ? 0.0 : 8.0) + 8.0) * cells);
                 done = ws.timers[K_MATVEC64].pending_end();
             }
-            launch_fcg_matvec(st, d, A, A.pinned_rowsum ? nullptr : lv_[level].diag32.p, z, r_.p, q_.p,
-                              w_.p, first ? 1 : 0, ws.partials.p, ws.scalars.p, ws.gate, done);
+            ws.zout = nullptr;
+            ws.fold = FoldArgs{};
+            launch_fcg_matvec(st, d, A, flags, z, r_.p, q_.p, w_.p, first ? 1 : 0, iter + it, fold,
+                              ws.partials.p, ws.scalars.p, ws.gate, done);
             if (profiling) ws.timers[K_MATVEC64].end_recorded();
-            // z, w, p, q, r in; p, q, r out; x in and out every other
-            // iteration (and diag in, b and x0 out)
-            const int xmode = (run + it) % 2 == 0 ? X_LATER : X_BOTH;
+            // w, q, r in; q, r out (and diag in, b and x0 out)
             if (profiling) {
-                ws.timers[K_UPDATE64].begin(st, (4.0 + 8.0 * 4 + 8.0 * 3 + (xmode == X_LATER ? 0.0 : 16.0) +
-                                                 (b32 ? 4.0 + 4.0 + 4.0 : 0.0)) * cells);
+                ws.timers[K_UPDATE64].begin(st, (8.0 * 3 + 8.0 * 2 + (x0 ? 4.0 + 4.0 + 4.0 : 0.0)) * cells);
                 done = ws.timers[K_UPDATE64].pending_end();
             }
             ws.x0_level = -1;
-            launch_fcg_update(st, d, lv_[level].diag32.p, z, w_.p, p_.p, q_.p, x_.p, r_.p, b32,
-                              b32 ? lv_[level].x0.p : nullptr, c0, first ? 1 : 0, xmode, ws.partials.p,
-                              ws.scalars.p, ws.gate, done);
+            // (a cycle whose first launch folds forms its first iterate itself)
+            float *const x0_next = fold ? nullptr : x0;
+            launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, w_.p, q_.p, r_.p, b32, x0_next, c0,
+                              first ? 1 : 0, iter + it, fold, ws.partials.p, ws.scalars.p, ws.gate, done);
             if (profiling) ws.timers[K_UPDATE64].end_recorded();
             first = false;
             b_ready = b32 != nullptr;
         }
+        if (fold) launch_fcg_norm(st, d, ws.partials.p, ws.scalars.p, ws.gate);
         ws.read_scalars();
         const bool stalled = batch > 1 && ws.host_sc->stalled != 0.0;
         ws.gate = nullptr;
         const int done = batch > 1 ? (int)ws.host_sc->iters : 1;
-        run += done;
+        pending += done;
+        iter += done;
         info.iterations += done;
         if (!learned && cfg.precond == 1 && info.precond_used == 1) info.fallback += done;
         const double prev = rel;
@@ -715,7 +767,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             // iterate stored by the last update belongs to the learned
             // cycle's smoother
             learned = false;
-            bring_x_up_to_date();
+            bring_x_up_to_date(false);
             first = true;
             const float c0_plain = first_coef(false);
             if (c0_plain != c0) b_ready = false;
@@ -723,7 +775,8 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             next_batch = kBatch;
         }
     }
-    bring_x_up_to_date();
+    bring_x_up_to_date(false);
+    if (zero_x) SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));  // (no iteration)
     if (!checked) {
         launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p);
         ws.read_scalars();

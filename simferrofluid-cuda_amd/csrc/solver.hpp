@@ -124,6 +124,12 @@ struct Workspace {
     // level whose x0 holds the first Chebyshev iterate of its b (stored by
     // the FCG update for the next cycle), or -1
     int x0_level = -1;
+    // where the cycle from level z_level leaves its result (null: in one of
+    // the level's own iterates)
+    float *zout = nullptr;
+    int z_level = 0;
+    // the ||r||^2 the cycle's first launch adds (fold.nb 0: none)
+    FoldArgs fold;
     // a second stream (default priority) on which the coarsest level's dense
     // inverse is formed while `stream` runs the rest of the set-up; side_in
     // orders it after the coarsening, side_out orders its first use after it
@@ -201,6 +207,13 @@ class System {
     // levels l .. coarsest in one launch (vlevel with r64 null), or null
     // where the tail does not apply
     float *vcycle_tail(Workspace &ws, const Smoothing &sm, int l);
+    bool tail_at(const Workspace &ws, int l) const;
+    // the cycle from level l starts with a launch that takes ws.fold
+    bool fold_at(const Workspace &ws, const Smoothing &sm, int l);
+    // where the last launch of level l writes (a step's usual output or ws.zout)
+    float *last_out(const Workspace &ws, int l, float *usual) const {
+        return ws.zout && ws.z_level == l ? ws.zout : usual;
+    }
     // The steps of one half of level l's visit (steps, and the restriction
     // after them) as one or two launches over tiles; n[0] = 0: separate
     // launches are cheaper.
@@ -218,7 +231,13 @@ class System {
     DevBuf<double> phic_;  // level set restricted to the first coarse level
     Dims d_{};
     std::vector<Level> lv_;
-    DevBuf<double> rhs_, x_, r_, p_, q_, w_;
+    DevBuf<double> rhs_, x_, r_, q_, w_;
+    // the z of the iterations whose update of x is pending: kRing vectors,
+    // zring_stride_ apart; p_ (formed only where more than kRing iterations
+    // are pending): the direction before them
+    DevBuf<float> zring_;
+    size_t zring_stride_ = 0;
+    DevBuf<double> p_;
     DevBuf<float> ainv_;
     // the dense inverse is being formed on ws.side: join before reading it
     // (or before the coarsest operator it reads is rewritten)
