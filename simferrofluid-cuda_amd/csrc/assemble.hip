@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void k_pressure_assemble(CellGrid cg,
                 const double weight = 1 - fr[ord];
                 if (weight > 0) {
                     if (!nbv[ord]) {
-                        atomicExch(err, 1);
+                        *err = 1;  // (host memory, written only on an error)
                     } else {
                         if (pn[ord] <= 0) {
                             diag += weight;
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kBlock) void k_pressure_apply(CellGrid cg, Dims d, 
         if (!v0 || !v1) {
             // open face on the grid boundary: the reference reads outside the grid
             const int *in = v0 ? c0 : c1;
-            if (liquid[d.idx(in[0], in[1], in[2])]) atomicExch(err, 1);
+            if (liquid[d.idx(in[0], in[1], in[2])]) *err = 1;  // (host memory, written only on an error)
             continue;
         }
         const size_t i0 = d.idx(c0[0], c0[1], c0[2]), i1 = d.idx(c1[0], c1[1], c1[2]);

@@ -97,15 +97,14 @@ void fill_stats(sfp_stats *st, const SolveInfo &info, long long unknowns, float 
 }
 
 void check_err(sfp_context ctx, const char *msg) {
-    SFP_HIP(hipMemcpyAsync(ctx->ws.host_err, ctx->ws.err.p, sizeof(int), hipMemcpyDeviceToHost,
-                           ctx->ws.stream));
-    SFP_HIP(hipStreamSynchronize(ctx->ws.stream));
+    ctx->ws.wait();
     if (*ctx->ws.host_err) {
-        SFP_HIP(hipMemsetAsync(ctx->ws.err.p, 0, sizeof(int), ctx->ws.stream));
-        SFP_HIP(hipStreamSynchronize(ctx->ws.stream));
+        *ctx->ws.host_err = 0;
         throw InputError(msg);
     }
 }
+
+const char *const kOpenFace = "open (fraction < 1) face on the grid boundary next to a liquid cell";
 
 // ---------------------------------------------------------------- pressure
 void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
@@ -136,19 +135,10 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
         double *c64[3] = {L.cpl64[0].p, L.cpl64[1].p, L.cpl64[2].p};
         float *c32[3] = {L.cpl32[0].p, L.cpl32[1].p, L.cpl32[2].p};
         launch_pressure_assemble(s, d, phi, F, V, U, jump ? &J : nullptr, vol_error, L.diag64.p, c64,
-                                 sys.rhs().p, L.diag32.p, c32, ctx->liquid.p, ctx->ws.err.p);
-        check_err(ctx, "open (fraction < 1) face on the grid boundary next to a liquid cell");
-        const long long unknowns = sys.count_active(ctx->ws);
-        if (unknowns == 0) {  // Pressure::Project returns early
-            ctx->pressure_ready = true;
-            if (pressure) SFP_HIP(hipMemsetAsync(pressure, 0, d.cells() * sizeof(double), s));
-            SFP_HIP(hipStreamSynchronize(s));
-            fill_stats(st, SolveInfo{0, 0.0, true, 0, ctx->cfg.precond}, 0, 0.f, 0.f, 0.f);
-            return;
-        }
+                                 sys.rhs().p, L.diag32.p, c32, ctx->liquid.p, ctx->ws.host_err);
+        // (its input errors and the number of unknowns are read with the
+        // solve's first residual: nothing before that needs them)
         sys.build_hierarchy(ctx->ws, ctx->cfg.for_pressure());
-        ctx->pressure_unknowns = unknowns;
-        ctx->pressure_ready = true;
     } else {
         if (!ctx->pressure_ready) throw StateError("reproject before project");
         if (ctx->pressure_unknowns == 0) {
@@ -161,15 +151,26 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     ctx->ws.phi = phi;
     ctx->ws.spacing = ctx->spacing;
     SolveInfo info = sys.solve(ctx->ws, ctx->cfg.for_pressure(), reproject);
+    if (info.input_error) check_err(ctx, kOpenFace);
+    if (!reproject) {
+        ctx->pressure_unknowns = info.active;
+        ctx->pressure_ready = true;
+        if (info.active == 0) {  // Pressure::Project returns early
+            if (pressure) SFP_HIP(hipMemsetAsync(pressure, 0, d.cells() * sizeof(double), s));
+            SFP_HIP(hipStreamSynchronize(s));
+            fill_stats(st, SolveInfo{0, 0.0, true, 0, ctx->cfg.precond}, 0, 0.f, 0.f, 0.f);
+            return;
+        }
+    }
     SFP_HIP(hipEventRecord(ctx->ev[2], s));
     MutFaces Vm{{vel[0], vel[1], vel[2]}};
     launch_pressure_apply(s, d, phi, F, jump ? &J : nullptr, ctx->liquid.p, sys.x().p, Vm,
-                          ctx->ws.err.p);
+                          ctx->ws.host_err);
     if (pressure)
         SFP_HIP(hipMemcpyAsync(pressure, sys.x().p, d.cells() * sizeof(double),
                                hipMemcpyDeviceToDevice, s));
     SFP_HIP(hipEventRecord(ctx->ev[3], s));
-    check_err(ctx, "open (fraction < 1) face on the grid boundary next to a liquid cell");
+    check_err(ctx, kOpenFace);
     fill_stats(st, info, ctx->pressure_unknowns, elapsed(ctx->ev[0], ctx->ev[1]),
                elapsed(ctx->ev[1], ctx->ev[2]), elapsed(ctx->ev[2], ctx->ev[3]));
 }
@@ -498,11 +499,11 @@ sfp_status sfp_create(sfp_context *out, int nx, int ny, int nz, double spacing,
         for (auto &e : ctx->ev) SFP_HIP(hipEventCreate(&e));
         ctx->ws.partials.ensure(reduction_partials(ctx->d));
         ctx->ws.scalars.ensure(1);
-        ctx->ws.err.ensure(1);
         SFP_HIP(hipMemset(ctx->ws.scalars.p, 0, sizeof(KrylovScalars)));
-        SFP_HIP(hipMemset(ctx->ws.err.p, 0, sizeof(int)));
         SFP_HIP(hipHostMalloc((void **)&ctx->ws.host_sc, sizeof(KrylovScalars), hipHostMallocDefault));
         SFP_HIP(hipHostMalloc((void **)&ctx->ws.host_err, sizeof(int), hipHostMallocDefault));
+        *ctx->ws.host_sc = KrylovScalars{};
+        *ctx->ws.host_err = 0;
     } catch (const std::exception &e) {
         g_create_error = e.what();
         sfp_destroy(ctx);

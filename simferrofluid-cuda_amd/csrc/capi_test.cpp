@@ -152,9 +152,9 @@ sfp_status sfp_test_residual(sfp_context ctx, int which, const double *x, double
         dr.ensure(n);
         SFP_HIP(hipMemcpyAsync(dx.p, x, n * sizeof(double), hipMemcpyHostToDevice, ctx->ws.stream));
         launch_residual64(ctx->ws.stream, d, s.fine().op64(), s.rhs().p, dx.p, dr.p,
-                          ctx->ws.partials.p, ctx->ws.scalars.p);
+                          ctx->ws.partials.p, ctx->ws.scalars.p, ctx->ws.host_sc);
         d2h(ctx, r, dr.p, n);
-        ctx->ws.read_scalars();
+        ctx->ws.wait();
         if (rr) *rr = ctx->ws.host_sc->rr;
         if (bb) *bb = ctx->ws.host_sc->bb;
     });

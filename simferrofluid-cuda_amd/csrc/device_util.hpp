@@ -23,9 +23,53 @@ __device__ __forceinline__ float rcp_or_zero(float dg) {
     return dg > 0.f ? __builtin_amdgcn_rcpf(dg) : 0.f;
 }
 
+// A load whose value is used on one side of a branch only is moved down to
+// that side, and then its latency is not shared with the loads before the
+// branch. `pin` counts as a use where it stands: a kernel that wants all of its
+// loads in flight together pins them before its first branch on one of them.
+template <class T>
+__device__ __forceinline__ void pin(const T &v) {
+    asm volatile("" ::"v"(v));
+}
+// The gate of a batch of iterations (KrylovScalars::stop; null: open), without
+// a branch around the load: `other` is any readable address.
+__device__ __forceinline__ double load_gate(const double *gate, const void *other) {
+    const double v = *(gate ? gate : (const double *)other);
+    return gate ? v : 0.0;
+}
+
+// Sum over the wavefront, the same in every lane: halves 32 lanes apart, then
+// 16, 8, 4, 2 and 1, the tree of shuffles down in lane 0 (so the same bits
+// there). The exchanges are register moves (v_permlane32_swap,
+// v_permlane16_swap, DPP rotations of 16-lane rows and quads): a shuffle
+// through the LDS unit waits about 130 cycles, six of them for each sum.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    auto halves = [](double a) { return __builtin_bit_cast(u2, a); };
+    auto whole = [](unsigned lo, unsigned hi) { return __builtin_bit_cast(double, u2{lo, hi}); };
+    {
+        const u2 h = halves(v);
+        const auto l = __builtin_amdgcn_permlane32_swap(h.x, h.x, false, false);
+        const auto u = __builtin_amdgcn_permlane32_swap(h.y, h.y, false, false);
+        v = whole(l[0], u[0]) + whole(l[1], u[1]);
+    }
+    {
+        const u2 h = halves(v);
+        const auto l = __builtin_amdgcn_permlane16_swap(h.x, h.x, false, false);
+        const auto u = __builtin_amdgcn_permlane16_swap(h.y, h.y, false, false);
+        v = whole(l[0], u[0]) + whole(l[1], u[1]);
+    }
+#define SFP_DPP_ADD(CTRL)                                                                             \
+    {                                                                                                 \
+        const u2 h = halves(v);                                                                       \
+        v += whole((unsigned)__builtin_amdgcn_mov_dpp((int)h.x, CTRL, 0xf, 0xf, true),                \
+                   (unsigned)__builtin_amdgcn_mov_dpp((int)h.y, CTRL, 0xf, 0xf, true));               \
+    }
+    SFP_DPP_ADD(0x128)  // row_ror:8
+    SFP_DPP_ADD(0x124)  // row_ror:4 (the lanes 8 apart agree)
+    SFP_DPP_ADD(0x4e)   // quad_perm 2,3,0,1
+    SFP_DPP_ADD(0xb1)   // quad_perm 1,0,3,2
+#undef SFP_DPP_ADD
     return v;
 }
 
@@ -105,29 +149,59 @@ __device__ __forceinline__ void sum_partials(const double *partials, unsigned nb
     block_sum<N, T>(v);
 }
 
-// The sums of N arrays of nb block partials ([q * nb + b]) in every thread of
-// a block (of whole wavefronts), in the order of a 1024-thread sum_partials
-// for nb <= 15 * 1024: bit for bit the one-block finalize's. A kernel that
-// needs a reduction's result adds the partials itself where they are few,
-// which costs it one memory latency instead of a launch (3 to 4 us) between.
+// The sums of N arrays of nb <= kFoldMax block partials ([q * nb + b]) in every
+// thread of a block (of whole wavefronts, at least 64 kFoldMax / 1024 threads),
+// in the order of a 1024-thread sum_partials: bit for bit the one-block
+// finalize's. A kernel that needs a reduction's result adds the partials
+// itself where they are few, which costs it little beside its other loads
+// (fold_load, issued with them; then fold_sum) instead of a launch of 3 to 4
+// us between.
+constexpr unsigned kFoldMax = 1024;
+constexpr int kFoldLoads = 4;  // a thread's values of each array in registers (256 threads: all)
+
 template <int N>
-__device__ __forceinline__ void fold_partials(const double *__restrict__ partials, unsigned nb, double (&v)[N]) {
-    __shared__ double sh[N][16];
+struct FoldLoad {
+    double a[N][kFoldLoads];
+};
+template <int N>
+__device__ __forceinline__ void fold_load(const double *__restrict__ partials, unsigned nb, FoldLoad<N> &f) {
     const unsigned tid = (unsigned)flat_tid(), nt = blockDim.x * blockDim.y * blockDim.z;
-    const unsigned waves = min((nb + 63u) / 64u, 16u);
-    for (unsigned vt = tid; vt < 64u * waves; vt += nt) {  // whole wavefronts (nt a multiple of 64)
-        double a[N];
 #pragma unroll
-        for (int q = 0; q < N; q++) a[q] = 0.0;
-        for (unsigned b = vt; b < nb; b += 1024u)
+    for (int u = 0; u < kFoldLoads; u++) {
+        const unsigned b = tid + u * nt;
 #pragma unroll
-            for (int q = 0; q < N; q++) a[q] += partials[(size_t)q * nb + b];
-#pragma unroll
-        for (int q = 0; q < N; q++) a[q] = wave_sum(a[q]);
-        if ((tid & 63u) == 0)
-#pragma unroll
-            for (int q = 0; q < N; q++) sh[q][vt >> 6] = a[q];
+        for (int q = 0; q < N; q++) f.a[q][u] = partials[(size_t)q * nb + min(b, nb - 1)];
     }
+}
+template <int N>
+__device__ __forceinline__ void pin(const FoldLoad<N> &f) {
+#pragma unroll
+    for (int u = 0; u < kFoldLoads; u++)
+#pragma unroll
+        for (int q = 0; q < N; q++) pin(f.a[q][u]);
+}
+template <int N>
+__device__ __forceinline__ void fold_sum(const double *__restrict__ partials, unsigned nb, const FoldLoad<N> &f,
+                                         double (&v)[N]) {
+    __shared__ double sh[N][kFoldMax / 64];
+    const unsigned tid = (unsigned)flat_tid(), nt = blockDim.x * blockDim.y * blockDim.z;
+    const unsigned waves = (nb + 63u) / 64u;  // wavefronts of 64 partials
+#pragma unroll
+    for (int u = 0; u < kFoldLoads; u++) {
+        const unsigned vt = tid + u * nt;
+        if (vt >= 64u * waves) break;  // uniform over the wavefront
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const double a = wave_sum(vt < nb ? f.a[q][u] : 0.0);
+            if ((tid & 63u) == 0) sh[q][vt >> 6] = a;
+        }
+    }
+    for (unsigned vt = tid + kFoldLoads * nt; vt < 64u * waves; vt += nt)  // (blocks of fewer than 256 threads)
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            const double a = wave_sum(vt < nb ? partials[(size_t)q * nb + vt] : 0.0);
+            if ((tid & 63u) == 0) sh[q][vt >> 6] = a;
+        }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < N; q++) {

@@ -178,6 +178,10 @@ void launch_coarse_solve(hipStream_t s, int n, const float *ainv, const float *b
                          const double *gate = nullptr);
 
 // ---------------------------------------------------------------- Krylov (krylov.hip)
+// `host` (the residual, the update and the norm): a pinned copy of the scalars
+// that the launch's finalize fills in (rr, bb, active, iters, stalled; also
+// behind a closed gate), so that the host reads them after a stream
+// synchronization, without a copy (a launch of its own, 3 us, before it).
 // Reduction kernels cover this many x planes per block (fewer partials).
 constexpr int kReducePlanes = 0;  // automatic
 // Doubles of partial-sum scratch a reduction over grid d needs.
@@ -190,10 +194,12 @@ void launch_batch_begin(hipStream_t s, KrylovScalars *sc, double stop_rr, double
 // r may be null (only the sums).
 // With b32, also b32 = r rounded to FP32 and, with x0, x0 = c0 D32^-1 b32
 // (diag32: the FP32 diagonal): the right-hand side and first Chebyshev
-// iterate of a V-cycle on r, as the FCG update stores them.
+// iterate of a V-cycle on r, as the FCG update stores them. With diag32 the
+// active cells are counted too (scalars->active).
 void launch_residual64(hipStream_t s, Dims d, Op64 A, const double *b, const double *x,
-                       double *r, double *partials, KrylovScalars *sc, float *b32 = nullptr,
-                       float *x0 = nullptr, const float *diag32 = nullptr, float c0 = 0.f);
+                       double *r, double *partials, KrylovScalars *sc, KrylovScalars *host = nullptr,
+                       float *b32 = nullptr, float *x0 = nullptr, const float *diag32 = nullptr,
+                       float c0 = 0.f);
 // w = A z; dots z.w, z.q_prev, z.r, and with them alpha, beta and p.q of
 // iteration number iter (scalars->alpha[iter % kCoefs], ...). fold: only the
 // partial sums (the update adds them).
@@ -212,11 +218,12 @@ void launch_fcg_matvec(hipStream_t s, Dims d, Op64 A, const float *active, const
 void launch_fcg_update(hipStream_t s, Dims d, const float *active, const double *w, double *q, double *r,
                        float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate = nullptr,
-                       hipEvent_t kernel_done = nullptr);
+                       hipEvent_t kernel_done = nullptr, KrylovScalars *host = nullptr);
 // (kernel_done, if given, is recorded after the stencil kernel and before
 // the one-block finalize that forms the scalars.)
 // rr from the update's partials; counts the update and raises `stop`.
-void launch_fcg_norm(hipStream_t s, Dims d, double *partials, KrylovScalars *sc, const double *gate = nullptr);
+void launch_fcg_norm(hipStream_t s, Dims d, double *partials, KrylovScalars *sc, const double *gate = nullptr,
+                     KrylovScalars *host = nullptr);
 // Grids whose reductions' partials the kernels that need the sums add
 // themselves.
 bool fold_pays(Dims d);

@@ -12,7 +12,7 @@
 namespace sfp {
 namespace {
 
-enum FinalizeOp : int { FIN_RESIDUAL = 0, FIN_MATVEC = 1, FIN_UPDATE = 2, FIN_COUNT = 3 };
+enum FinalizeOp : int { FIN_RESIDUAL = 0, FIN_MATVEC = 1, FIN_UPDATE = 2 };
 
 // true when a batched solve has already converged (see KrylovScalars::stop)
 __device__ __forceinline__ bool gated(const double *gate) { return gate && *gate != 0.0; }
@@ -51,14 +51,16 @@ __global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64
     const bool on = k < d.nz && j < d.ny && i0 < d.nx;
     const bool zlo = k > 0, zhi = k + 1 < d.nz;
     const int ie = min(i0 + cg.planes, d.nx);
-    double v[2] = {0.0, 0.0};  // r.r, b.b
+    double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
     size_t c = on ? d.idx(i0, j, k) : 0;
     // the FP32 copy of r and the cycle's first iterate (the FCG update's arithmetic)
     auto store32 = [&](size_t q, double rq) {
+        const float dq = diag32 ? diag32[q] : 0.f;
+        if (dq > 0.f) v[2] += 1.0;
         if (!b32) return;
         const float bf = (float)rq;
         b32[q] = bf;
-        if (x0) x0[q] = c0 * rcp_or_zero(diag32[q]) * bf;
+        if (x0) x0[q] = c0 * rcp_or_zero(dq) * bf;
     };
     if (!x) {
         if (on)
@@ -69,7 +71,7 @@ __global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64
                 v[0] += bc * bc;
                 v[1] += bc * bc;
             }
-        block_partials<2>(v, partials);
+        block_partials<3>(v, partials);
         return;
     }
     double xm = (on && i0 > 0) ? x[c - s.sx] : 0.0;
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64
         xc = xp;
         cxc = cxp;
     }
-    block_partials<2>(v, partials);
+    block_partials<3>(v, partials);
 }
 
 // The same residual over the flat cell index, two consecutive cells of one z
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
                                                             float c0) {
     const Strides s(d);
     const size_t c = (size_t)blockIdx.x * kResidualCells + 2 * (size_t)flat_tid();
-    double v[2] = {0.0, 0.0};  // r.r, b.b
+    double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
     if (c < d.cells()) {       // cells() is even: then c + 1 is a cell too
         const double2v d0 = {0.0, 0.0};
         const double2v bc = ld_stream((const double2v *)(b + c));
@@ -189,11 +191,12 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
             rc.y = bc.y - (dg.y * xc.y - o1);
         }
         if (r) st_stream((double2v *)(r + c), rc);
+        const float2v dd = diag32 ? *(const float2v *)(diag32 + c) : float2v{0.f, 0.f};
+        v[2] = (dd.x > 0.f ? 1.0 : 0.0) + (dd.y > 0.f ? 1.0 : 0.0);
         if (b32) {
             const float2v bf = {(float)rc.x, (float)rc.y};
             *(float2v *)(b32 + c) = bf;
             if (x0) {
-                const float2v dd = *(const float2v *)(diag32 + c);
                 const float2v xf = {c0 * rcp_or_zero(dd.x) * bf.x, c0 * rcp_or_zero(dd.y) * bf.y};
                 *(float2v *)(x0 + c) = xf;
             }
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
         v[0] = rc.x * rc.x + rc.y * rc.y;
         v[1] = bc.x * bc.x + bc.y * bc.y;
     }
-    block_partials<2>(v, partials);
+    block_partials<3>(v, partials);
 }
 
 // `active` (the FP32 diagonal, 0 = inactive cell) or null: with it, z counts as
@@ -432,13 +435,31 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
                                                        double *__restrict__ partials,
                                                        KrylovScalars *sc,
                                                        const double *gate) {
-    if (gated(gate)) return;
     const int ci = iter % kCoefs;
+    const size_t c = (size_t)blockIdx.x * kUpdateCells + 2 * (size_t)flat_tid();
+    const bool pair = c + 1 < n;  // else at most the grid's last cell
     double alpha, beta;
+    double2v wc = {0.0, 0.0}, r0 = {0.0, 0.0}, qq = {0.0, 0.0};
     if constexpr (kFold) {
+        // every load at once: the vectors' beside the gate's and the partials'
+        const double stop = load_gate(gate, sc);
+        FoldLoad<3> f;
+        fold_load<3>(mv, nb_mv, f);
+        const double pq_prev = sc->pq[(iter + kCoefs - 1) % kCoefs];
+        const size_t cl = pair ? c : 0;  // (a grid of one cell: the allocations hold a pair)
+        wc = ld_stream((const double2v *)(w + cl));
+        r0 = ld_stream((const double2v *)(r + cl));
+        qq = ld_stream((const double2v *)(q + cl));
+        pin(stop);
+        pin(f);
+        pin(pq_prev);
+        pin(wc);
+        pin(r0);
+        pin(qq);
+        if (stop != 0.0) return;
         double v[3];
-        fold_partials<3>(mv, nb_mv, v);
-        const Recurrence c = recurrence(v, first ? 0.0 : sc->pq[(iter + kCoefs - 1) % kCoefs], first);
+        fold_sum<3>(mv, nb_mv, f, v);
+        const Recurrence c = recurrence(v, first ? 0.0 : pq_prev, first);
         alpha = c.alpha;
         beta = c.beta;
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -447,12 +468,11 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
             sc->pq[ci] = c.pq;
         }
     } else {
+        if (gated(gate)) return;
         alpha = sc->alpha[ci];
         beta = sc->beta[ci];
     }
     double v[1] = {0.0};
-    const size_t c = (size_t)blockIdx.x * kUpdateCells + 2 * (size_t)flat_tid();
-    const bool pair = c + 1 < n;  // else at most the grid's last cell
     bool act = c < n;
     float2v dg = {0.f, 0.f};  // FP32 diagonal (the activity flag)
     if (active) {
@@ -462,11 +482,13 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
     }
     if (__any(act)) {
         if (pair) {
-            const double2v wc = ld_stream((const double2v *)(w + c));
-            const double2v r0 = ld_stream((const double2v *)(r + c));
+            if constexpr (!kFold) {
+                wc = ld_stream((const double2v *)(w + c));
+                r0 = ld_stream((const double2v *)(r + c));
+                if (!first) qq = ld_stream((const double2v *)(q + c));
+            }
             double2v qc = wc;
             if (!first) {
-                const double2v qq = ld_stream((const double2v *)(q + c));
                 qc.x = wc.x - beta * qq.x;
                 qc.y = wc.y - beta * qq.y;
             }
@@ -575,19 +597,6 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(CellGrid cg, Dims d, Op32 A,
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_count_active(CellGrid cg, Dims d,
-                                                         const float *__restrict__ diag32,
-                                                         double *__restrict__ partials) {
-    int k, j, i0;
-    cell_tile(cg, k, j, i0);
-    double v[1] = {0.0};
-    if (k < d.nz && j < d.ny) {
-        for (int i = i0, ie = min(i0 + cg.planes, d.nx); i < ie; i++)
-            if (diag32[d.idx(i, j, k)] > 0.f) v[0] += 1.0;
-    }
-    block_partials<1>(v, partials);
-}
-
 // One block: add the partials and advance the scalar recurrences.
 // The finalize kernel is one block of kFinalizeThreads (wide, so the partial
 // sums of the largest grids take few rounds of loads).
@@ -607,16 +616,24 @@ __global__ __launch_bounds__(64) void k_batch_begin(KrylovScalars *sc, double st
 
 __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned nb, int first, int iter,
                                                      const double *__restrict__ partials,
-                                                     KrylovScalars *sc, const double *gate) {
-    if (gated(gate)) return;
+                                                     KrylovScalars *sc, const double *gate,
+                                                     KrylovScalars *host) {
+    // what the host reads after this launch (host: its pinned copy, or null)
+    auto tell_host = [&] {
+        if (!host) return;
+        host->rr = sc->rr;
+        host->bb = sc->bb;
+        host->active = sc->active;
+        host->iters = sc->iters;
+        host->stalled = sc->stalled;
+    };
+    if (gated(gate)) {
+        if (flat_tid() == 0) tell_host();
+        return;
+    }
     double v[3] = {0.0, 0.0, 0.0};
-    if (op == FIN_MATVEC) {
+    if (op != FIN_UPDATE) {
         sum_partials<3, kFinalizeThreads, 16>(partials, nb, v);
-    } else if (op == FIN_RESIDUAL) {
-        double t[2];
-        sum_partials<2, kFinalizeThreads, 16>(partials, nb, t);
-        v[0] = t[0];
-        v[1] = t[1];
     } else {
         double t[1];
         sum_partials<1, kFinalizeThreads, 16>(partials, nb, t);
@@ -626,6 +643,7 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
     if (op == FIN_RESIDUAL) {
         sc->rr = v[0];
         sc->bb = v[1];
+        sc->active = v[2];
     } else if (op == FIN_MATVEC) {
         const Recurrence c = recurrence(v, first ? 0.0 : sc->pq[(iter + kCoefs - 1) % kCoefs], first);
         sc->zw = v[0];
@@ -634,7 +652,7 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
         sc->alpha[iter % kCoefs] = c.alpha;
         sc->beta[iter % kCoefs] = c.beta;
         sc->pq[iter % kCoefs] = c.pq;
-    } else if (op == FIN_UPDATE) {
+    } else {
         const double rr_prev = sc->rr;
         sc->rr = v[0];
         sc->iters += 1.0;
@@ -643,9 +661,8 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
             sc->stalled = 1.0;  // the host switches to the plain V-cycle after the batch
             sc->stop = 1.0;
         }
-    } else {
-        sc->pad[0] = v[0];
     }
+    tell_host();
 }
 
 // Above kStageMin partials the sums take two launches: kStageThreads-wide
@@ -673,17 +690,14 @@ __global__ __launch_bounds__(kStageThreads) void k_partials_stage(unsigned nb, u
 // `partials` holds the N sums of op for nb blocks ([q * nb + b]); the stage
 // writes its sums after them (reduction_partials leaves room).
 void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *partials, KrylovScalars *sc,
-              const double *gate = nullptr) {
-    const int N = op == FIN_MATVEC ? 3 : op == FIN_RESIDUAL ? 2 : 1;
+              const double *gate = nullptr, KrylovScalars *host = nullptr) {
+    const int N = op == FIN_UPDATE ? 1 : 3;
     if (nb > kStageMin) {
         const unsigned chunk = std::max(kStageChunk, (nb + kStageMaxBlocks - 1) / kStageMaxBlocks);
         const unsigned G = (nb + chunk - 1) / chunk;
         double *out = partials + (size_t)N * nb;
         if (N == 3)
             hipLaunchKernelGGL(k_partials_stage<3>, dim3(G), dim3(kStageThreads), 0, st, nb, chunk, partials, out,
-                               gate);
-        else if (N == 2)
-            hipLaunchKernelGGL(k_partials_stage<2>, dim3(G), dim3(kStageThreads), 0, st, nb, chunk, partials, out,
                                gate);
         else
             hipLaunchKernelGGL(k_partials_stage<1>, dim3(G), dim3(kStageThreads), 0, st, nb, chunk, partials, out,
@@ -693,7 +707,7 @@ void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *
         nb = G;
     }
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, st, op, nb, first, iter,
-                       partials, sc, gate);
+                       partials, sc, gate, host);
     SFP_LAUNCH_CHECK();
 }
 
@@ -720,20 +734,9 @@ size_t reduction_partials(Dims d) {
            3 * (size_t)kStageMaxBlocks;
 }
 
-// Up to this many partials a kernel adds them itself (fold_partials): every
-// block reads them all, from L2 (64^3: 512 blocks, 12 KB each).
-constexpr unsigned kFoldMax = 2048;
 bool fold_pays(Dims d) { return std::max(matvec_blocks(d), update_blocks(d)) <= kFoldMax; }
 FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc) {
     return FoldArgs{partials + 3 * (size_t)matvec_blocks(d), update_blocks(d), sc};
-}
-
-void launch_count_active(hipStream_t st, Dims d, const float *diag32, double *partials,
-                         KrylovScalars *sc) {
-    Launch L = cell_launch(d, kReducePlanes);
-    hipLaunchKernelGGL(k_count_active, L.grid, L.block, 0, st, L.cg, d, diag32, partials);
-    SFP_LAUNCH_CHECK();
-    finalize(st, FIN_COUNT, L.blocks(), 0, 0, partials, sc);
 }
 
 void launch_batch_begin(hipStream_t st, KrylovScalars *sc, double stop_rr, double stall_rr) {
@@ -742,8 +745,8 @@ void launch_batch_begin(hipStream_t st, KrylovScalars *sc, double stop_rr, doubl
 }
 
 void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const double *x,
-                       double *r, double *partials, KrylovScalars *sc, float *b32, float *x0,
-                       const float *diag32, float c0) {
+                       double *r, double *partials, KrylovScalars *sc, KrylovScalars *host, float *b32,
+                       float *x0, const float *diag32, float c0) {
     if (x0 && (!b32 || !diag32)) throw ArgError("launch_residual64: x0 needs b32 and the diagonal");
     if (matvec_flat(d)) {
         for (const void *a : {(const void *)A.diag, (const void *)A.cpl[0], (const void *)A.cpl[1],
@@ -755,14 +758,14 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
         hipLaunchKernelGGL(k_residual64_flat, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials, b32,
                            x0, diag32, c0);
         SFP_LAUNCH_CHECK();
-        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc);
+        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host);
         return;
     }
     Launch L = cell_launch(d, kReducePlanes);
     hipLaunchKernelGGL(k_residual64, L.grid, L.block, 0, st, L.cg, d, A, b, x, r, partials, b32, x0,
                        diag32, c0);
     SFP_LAUNCH_CHECK();
-    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc);
+    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc, nullptr, host);
 }
 
 void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, const float *z,
@@ -790,7 +793,7 @@ void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, cons
 
 void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double *w, double *q, double *r,
                        float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
-                       KrylovScalars *sc, const double *gate, hipEvent_t kernel_done) {
+                       KrylovScalars *sc, const double *gate, hipEvent_t kernel_done, KrylovScalars *host) {
     // two cells per lane: 16-byte (8-byte for the FP32 ones) aligned vectors
     for (const void *a : {(const void *)w, (const void *)q, (const void *)r})
         if ((uintptr_t)a % 16) throw ArgError("launch_fcg_update: FP64 vector not 16-byte aligned");
@@ -807,11 +810,12 @@ void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double
                            c0, first, iter, partials, nb_mv, out, sc, gate);
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
-    if (!fold) launch_fcg_norm(st, d, partials, sc, gate);
+    if (!fold) launch_fcg_norm(st, d, partials, sc, gate, host);
 }
 
-void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc, const double *gate) {
-    finalize(st, FIN_UPDATE, update_blocks(d), 0, 0, partials + 3 * (size_t)matvec_blocks(d), sc, gate);
+void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc, const double *gate,
+                     KrylovScalars *host) {
+    finalize(st, FIN_UPDATE, update_blocks(d), 0, 0, partials + 3 * (size_t)matvec_blocks(d), sc, gate, host);
 }
 
 void launch_fcg_flush(hipStream_t st, Dims d, const float *active, const float *z, size_t stride, int K, int i0,

@@ -201,6 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
 // arithmetic is k_smooth's (same operands, same order), so the two give the
 // same bits. A wavefront whose 256 cells are all inactive writes nothing.
 constexpr unsigned kSmoothFlatCells = 4 * kBlock;
+constexpr size_t kEagerCells = (size_t)1 << 21;
 
 // Row-sum FP32 diagonal (Op32::pinned_rowsum) of one cell from its six
 // couplings in the order -x, +x, -y, +y, -z, +z (0 where there is no
@@ -226,7 +227,58 @@ __device__ __forceinline__ bool rowsum_group(const Op32 &A, size_t c, Dims d) {
     return A.pinned_rowsum && c != 0 && c != (size_t)d.nz && c != (size_t)d.ny * d.nz;
 }
 
-template <int MODE, bool kRowsum>
+// The operands of one group: every address is inside the grid (a missing
+// neighbour's is the group's own; its coupling is 0, the lower ones as
+// stored, the upper ones by selection), so the loads need no branches and are
+// all in flight together.
+struct GroupOperands {
+    f4v xc, xm, xp, ym, yp, cx, cxp, cy, cyp, cz, b;
+    float zlo, zhi, czhi;
+};
+__device__ __forceinline__ GroupOperands load_operands(const Op32 &A, const float *__restrict__ b,
+                                                       const float *__restrict__ x, Dims d, unsigned c, int i, int j,
+                                                       int k) {
+    const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy;
+    const bool xh = i + 1 < d.nx, yh = j + 1 < d.ny, zh = k + 4 < d.nz;
+    const unsigned cxm = i > 0 ? c - sx : c, cxu = xh ? c + sx : c, cym = j > 0 ? c - sy : c, cyu = yh ? c + sy : c;
+    const unsigned czl = k > 0 ? c - 1 : c, czu = zh ? c + 4 : c;
+    GroupOperands g;
+    g.xc = *(const f4v *)(x + c);
+    g.xm = *(const f4v *)(x + cxm);
+    g.xp = *(const f4v *)(x + cxu);
+    g.ym = *(const f4v *)(x + cym);
+    g.yp = *(const f4v *)(x + cyu);
+    g.cx = *(const f4v *)(A.cpl[0] + c);
+    g.cxp = *(const f4v *)(A.cpl[0] + cxu);
+    g.cy = *(const f4v *)(A.cpl[1] + c);
+    g.cyp = *(const f4v *)(A.cpl[1] + cyu);
+    g.cz = *(const f4v *)(A.cpl[2] + c);
+    g.b = *(const f4v *)(b + c);
+    g.zlo = x[czl];
+    g.zhi = x[czu];
+    g.czhi = A.cpl[2][czu];
+    return g;
+}
+__device__ __forceinline__ void pin(const GroupOperands &g) {
+    for (const f4v &v : {g.xc, g.xm, g.xp, g.ym, g.yp, g.cx, g.cxp, g.cy, g.cyp, g.cz, g.b}) sfp::pin(v);
+    sfp::pin(g.zlo);
+    sfp::pin(g.zhi);
+    sfp::pin(g.czhi);
+}
+// The upper couplings at the grid's end.
+__device__ __forceinline__ void end_couplings(GroupOperands &g, Dims d, int i, int j, int k) {
+    const f4v z4 = {0.f, 0.f, 0.f, 0.f};
+    if (!(i + 1 < d.nx)) g.cxp = z4;
+    if (!(j + 1 < d.ny)) g.cyp = z4;
+    if (!(k + 4 < d.nz)) g.czhi = 0.f;
+}
+
+// kEager (levels of at most kEagerCells cells, where a launch is one round of
+// wavefronts bound by its chain of memory latencies): the gate, the diagonal
+// and every operand are loaded at once and the launch leaves after them, on a
+// closed gate or an inactive wavefront; else (large levels, bound by the bytes)
+// before the operands' loads.
+template <int MODE, bool kRowsum, bool kEager>
 __global__ __launch_bounds__(kBlock) void k_smooth_flat(Dims d, Op32 A, const float *__restrict__ b,
                                                         const float *__restrict__ xin,
                                                         float *__restrict__ xout, float *dvec,
@@ -237,83 +289,89 @@ __global__ __launch_bounds__(kBlock) void k_smooth_flat(Dims d, Op32 A, const fl
     constexpr bool kProlong = (MODE & SM_PROLONG) != 0;
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef float f2 __attribute__((ext_vector_type(2)));
-    if (gated(gate)) return;
-    const Strides s(d);
-    const size_t c = (size_t)blockIdx.x * kSmoothFlatCells + 4 * (size_t)flat_tid();
-    const bool on = c < d.cells();  // cells() is a multiple of 4
-    const f4 z4 = {0.f, 0.f, 0.f, 0.f};
-    const bool rs = kRowsum && on && rowsum_group(A, c, d);  // every group there has an active cell
-    f4 dg = (on && !rs) ? *(const f4 *)(A.diag + c) : z4;
-    const bool act = rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f;
-    if (!__any(act) || !on) return;
-    // (i, j, k) of the first cell (the launcher keeps cells() < 2^32)
-    const unsigned cu = (unsigned)c;
-    const unsigned t = cu / (unsigned)d.nz;
-    const int k = (int)(cu - t * (unsigned)d.nz);
+    const double stop = load_gate(gate, A.diag);
+    const unsigned n = (unsigned)d.cells();  // a multiple of 4 below 2^32
+    const unsigned ct = blockIdx.x * kSmoothFlatCells + 4 * (unsigned)flat_tid();
+    const bool on = ct < n;
+    const unsigned c = on ? ct : n - 4;
+    const bool rs = kRowsum && rowsum_group(A, c, d);  // every group there has an active cell
+    f4 dg = {0.f, 0.f, 0.f, 0.f};
+    if (!rs) dg = *(const f4 *)(A.diag + c);
+    if constexpr (!kEager) {
+        if (stop != 0.0) return;
+        const bool act = on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f);
+        if (!__any(act)) return;
+    }
+    // (i, j, k) of the first cell
+    const unsigned t = c / (unsigned)d.nz;
+    const int k = (int)(c - t * (unsigned)d.nz);
     const unsigned iu = t / (unsigned)d.ny;
     const int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny);
-    const bool up = i + 1 < d.nx, ylo = j > 0, yhi = j + 1 < d.ny;
-    const bool zl = k > 0, zh = k + 4 < d.nz;  // neighbours below the first, above the last
-    f4 xc = *(const f4 *)(xin + c);
-    f4 xm = i > 0 ? *(const f4 *)(xin + c - s.sx) : z4;
-    f4 xp = up ? *(const f4 *)(xin + c + s.sx) : z4;
-    const f4 cxc = *(const f4 *)(A.cpl[0] + c);
-    const f4 cxp = up ? *(const f4 *)(A.cpl[0] + c + s.sx) : z4;
-    const f4 cym = ylo ? *(const f4 *)(A.cpl[1] + c) : z4;
-    f4 xym = ylo ? *(const f4 *)(xin + c - s.sy) : z4;
-    const f4 cyp = yhi ? *(const f4 *)(A.cpl[1] + c + s.sy) : z4;
-    f4 xyp = yhi ? *(const f4 *)(xin + c + s.sy) : z4;
-    const f4 cz = *(const f4 *)(A.cpl[2] + c);
-    float xzlo = zl ? xin[c - 1] : 0.f;
-    float xzhi = zh ? xin[c + 4] : 0.f;
-    const float czhi = zh ? A.cpl[2][c + 4] : 0.f;
-    if (rs) dg = rowsum_diag4(cxc, cxp, cym, cyp, cz, czhi);
-    const f4 bc = *(const f4 *)(b + c);
-    f4 dprev = z4;
+    GroupOperands g = load_operands(A, b, xin, d, c, i, j, k);
+    f4 dprev = {0.f, 0.f, 0.f, 0.f};
     if constexpr ((MODE & SM_READ_D) != 0) dprev = *(const f4 *)(dvec + c);
-    const f4 xin_c = xc;
+    f2 ec, e_xm, e_xp, e_ym, e_yp;
+    float ezlo = 0.f, ezhi = 0.f;
     if constexpr (kProlong) {
         // coarse values of the group's two coarse cells in this row and in the
         // neighbouring rows and planes (16-byte aligned groups: k >> 1 even)
-        const int kc = k >> 1;
-        auto e2 = [&](int ii, int jj) { return *(const f2 *)(e + dc.idx(ii >> 1, jj >> 1, kc)); };
-        const f2 ec = e2(i, j);
-        const f2 e_xm = i > 0 ? e2(i - 1, j) : f2{0.f, 0.f};
-        const f2 e_xp = up ? e2(i + 1, j) : f2{0.f, 0.f};
-        const f2 e_ym = ylo ? e2(i, j - 1) : f2{0.f, 0.f};
-        const f2 e_yp = yhi ? e2(i, j + 1) : f2{0.f, 0.f};
-        const float ezlo = zl ? e[dc.idx(i >> 1, j >> 1, kc - 1)] : 0.f;
-        const float ezhi = zh ? e[dc.idx(i >> 1, j >> 1, kc + 2)] : 0.f;
+        const int kc = k >> 1, jl = max(j - 1, 0) >> 1, jh = min(j + 1, d.ny - 1) >> 1, il = max(i - 1, 0) >> 1,
+                  ih = min(i + 1, d.nx - 1) >> 1;
+        auto e2 = [&](int ii, int jj) { return *(const f2 *)(e + dc.idx(ii, jj, kc)); };
+        ec = e2(i >> 1, j >> 1);
+        e_xm = e2(il, j >> 1);
+        e_xp = e2(ih, j >> 1);
+        e_ym = e2(i >> 1, jl);
+        e_yp = e2(i >> 1, jh);
+        ezlo = e[dc.idx(i >> 1, j >> 1, max(kc - 1, 0))];
+        ezhi = e[dc.idx(i >> 1, j >> 1, min(kc + 2, dc.nz - 1))];
+    }
+    if constexpr (kEager) {
+        pin(g);
+        sfp::pin(dg);
+        if constexpr ((MODE & SM_READ_D) != 0) sfp::pin(dprev);
+        if constexpr (kProlong) {
+            for (const f2 &v : {ec, e_xm, e_xp, e_ym, e_yp}) sfp::pin(v);
+            sfp::pin(ezlo);
+            sfp::pin(ezhi);
+        }
+        if (stop != 0.0) return;
+    }
+    end_couplings(g, d, i, j, k);
+    if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
+    const f4 xin_c = g.xc;
+    if constexpr (kProlong) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            xc[q] = xc[q] + ec[q >> 1];
-            xm[q] = xm[q] + e_xm[q >> 1];
-            xp[q] = xp[q] + e_xp[q >> 1];
-            xym[q] = xym[q] + e_ym[q >> 1];
-            xyp[q] = xyp[q] + e_yp[q >> 1];
+            g.xc[q] = g.xc[q] + ec[q >> 1];
+            g.xm[q] = g.xm[q] + e_xm[q >> 1];
+            g.xp[q] = g.xp[q] + e_xp[q >> 1];
+            g.ym[q] = g.ym[q] + e_ym[q >> 1];
+            g.yp[q] = g.yp[q] + e_yp[q >> 1];
         }
-        xzlo = xzlo + ezlo;
-        xzhi = xzhi + ezhi;
+        g.zlo = g.zlo + ezlo;
+        g.zhi = g.zhi + ezhi;
     }
     f4 xo, dno;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const float xzm = q > 0 ? xc[q - 1] : xzlo;
-        const float xzp = q < 3 ? xc[q + 1] : xzhi;
-        const float czp = q < 3 ? cz[q + 1] : czhi;
-        float off = fmaf(cxc[q], xm[q], cxp[q] * xp[q]);
-        if (ylo) off = fmaf(cym[q], xym[q], off);
-        if (yhi) off = fmaf(cyp[q], xyp[q], off);
-        if (q > 0 || zl) off = fmaf(cz[q], xzm, off);
-        if (q < 3 || zh) off = fmaf(czp, xzp, off);
+        const float xzm = q > 0 ? g.xc[q - 1] : g.zlo;
+        const float xzp = q < 3 ? g.xc[q + 1] : g.zhi;
+        const float czp = q < 3 ? g.cz[q + 1] : g.czhi;
+        float off = fmaf(g.cx[q], g.xm[q], g.cxp[q] * g.xp[q]);
+        off = fmaf(g.cy[q], g.ym[q], off);
+        off = fmaf(g.cyp[q], g.yp[q], off);
+        off = fmaf(g.cz[q], xzm, off);
+        off = fmaf(czp, xzp, off);
         // centre iterate: the coarse correction only lands on active cells
-        const float x0 = (kProlong && !(dg[q] > 0.f)) ? xin_c[q] : xc[q];
-        const float r = bc[q] - fmaf(dg[q], x0, -off);
+        const float x0 = (kProlong && !(dg[q] > 0.f)) ? xin_c[q] : g.xc[q];
+        const float r = g.b[q] - fmaf(dg[q], x0, -off);
         const float dp = (MODE & SM_XFIRST) != 0 ? x0 : dprev[q];
         const float dn = fmaf(cd, dp, cr * rcp_or_zero(dg[q]) * r);
         xo[q] = x0 + dn;
         dno[q] = dn;
     }
+    if (!on) return;
     *(f4 *)(xout + c) = xo;
     if constexpr ((MODE & SM_WRITE_D) != 0) *(f4 *)(dvec + c) = dno;
 }
@@ -911,7 +969,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict(CellGrid cg, Dims df, Op32 
 // stores zeros.
 constexpr int kRestrictFlatZ = 64;  // z cells per wavefront
 
-template <bool kRowsum>
+template <bool kRowsum, bool kEager>
 __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const float *__restrict__ b,
                                                           const float *__restrict__ x, Dims dc,
                                                           float *__restrict__ bc, float *__restrict__ x0c,
@@ -919,7 +977,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
                                                           const double *gate) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef float f2 __attribute__((ext_vector_type(2)));
-    if (gated(gate)) return;
+    const double stop = load_gate(gate, A.diag);
     const int lane = threadIdx.x & 63;
     const unsigned wave = (unsigned)(blockIdx.x * kBlock + threadIdx.x) >> 6;
     const unsigned zch = (unsigned)(df.nz + kRestrictFlatZ - 1) / kRestrictFlatZ;
@@ -927,47 +985,43 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
     const unsigned kz = wave % zch, t = wave / zch;
     const unsigned jp = t % yp, ip = t / yp;
     if (ip >= (unsigned)(df.nx + 1) / 2) return;  // uniform over the wavefront (no barriers follow)
-    const int i = 2 * (int)ip + (lane >> 5), j = 2 * (int)jp + ((lane >> 4) & 1);
-    const int k = kRestrictFlatZ * (int)kz + 4 * (lane & 15);
-    const bool on = i < df.nx && j < df.ny && k < df.nz;
-    const Strides s(df);
-    const size_t c = on ? df.idx(i, j, k) : 0;
-    const f4 z4 = {0.f, 0.f, 0.f, 0.f};
-    const bool rs = kRowsum && on && rowsum_group(A, c, df);  // every group there has an active cell
-    f4 dg = (on && !rs) ? *(const f4 *)(A.diag + c) : z4;
-    f4 r = z4;
-    if (__any(rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f) && on) {
-        const bool up = i + 1 < df.nx, ylo = j > 0, yhi = j + 1 < df.ny;
-        const bool zl = k > 0, zh = k + 4 < df.nz;
-        const f4 xc = *(const f4 *)(x + c);
-        const f4 xm = i > 0 ? *(const f4 *)(x + c - s.sx) : z4;
-        const f4 xp = up ? *(const f4 *)(x + c + s.sx) : z4;
-        const f4 cxc = *(const f4 *)(A.cpl[0] + c);
-        const f4 cxp = up ? *(const f4 *)(A.cpl[0] + c + s.sx) : z4;
-        const f4 cym = ylo ? *(const f4 *)(A.cpl[1] + c) : z4;
-        const f4 xym = ylo ? *(const f4 *)(x + c - s.sy) : z4;
-        const f4 cyp = yhi ? *(const f4 *)(A.cpl[1] + c + s.sy) : z4;
-        const f4 xyp = yhi ? *(const f4 *)(x + c + s.sy) : z4;
-        const f4 cz = *(const f4 *)(A.cpl[2] + c);
-        const float xzlo = zl ? x[c - 1] : 0.f;
-        const float xzhi = zh ? x[c + 4] : 0.f;
-        const float czhi = zh ? A.cpl[2][c + 4] : 0.f;
-        if (rs) dg = rowsum_diag4(cxc, cxp, cym, cyp, cz, czhi);
-        const f4 bv = *(const f4 *)(b + c);
+    const int iw = 2 * (int)ip + (lane >> 5), jw = 2 * (int)jp + ((lane >> 4) & 1);
+    const int kw = kRestrictFlatZ * (int)kz + 4 * (lane & 15);
+    const bool on = iw < df.nx && jw < df.ny && kw < df.nz;
+    // lanes outside the grid load the nearest cells and drop them
+    const int i = min(iw, df.nx - 1), j = min(jw, df.ny - 1), k = min(kw, df.nz - 4);
+    const unsigned c = (unsigned)df.idx(i, j, k);
+    const bool rs = kRowsum && rowsum_group(A, c, df);  // every group there has an active cell
+    f4 dg = {0.f, 0.f, 0.f, 0.f};
+    if (!rs) dg = *(const f4 *)(A.diag + c);
+    f4 r = {0.f, 0.f, 0.f, 0.f};
+    bool any = true;
+    if constexpr (!kEager) {
+        if (stop != 0.0) return;
+        any = __any(on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f));
+    }
+    if (any) {
+        GroupOperands g = load_operands(A, b, x, df, c, i, j, k);
+        if constexpr (kEager) {
+            pin(g);
+            sfp::pin(dg);
+            if (stop != 0.0) return;
+        }
+        end_couplings(g, df, i, j, k);
+        if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            if (!(dg[q] > 0.f)) continue;
-            const float xzm = q > 0 ? xc[q - 1] : xzlo;
-            const float xzp = q < 3 ? xc[q + 1] : xzhi;
-            const float czp = q < 3 ? cz[q + 1] : czhi;
-            float off = 0.f;
-            if (i > 0) off = fmaf(cxc[q], xm[q], off);
-            if (up) off = fmaf(cxp[q], xp[q], off);
-            if (ylo) off = fmaf(cym[q], xym[q], off);
-            if (yhi) off = fmaf(cyp[q], xyp[q], off);
-            if (q > 0 || zl) off = fmaf(cz[q], xzm, off);
-            if (q < 3 || zh) off = fmaf(czp, xzp, off);
-            r[q] = bv[q] - fmaf(dg[q], xc[q], -off);
+            const float xzm = q > 0 ? g.xc[q - 1] : g.zlo;
+            const float xzp = q < 3 ? g.xc[q + 1] : g.zhi;
+            const float czp = q < 3 ? g.cz[q + 1] : g.czhi;
+            float off = fmaf(g.cx[q], g.xm[q], 0.f);
+            off = fmaf(g.cxp[q], g.xp[q], off);
+            off = fmaf(g.cy[q], g.ym[q], off);
+            off = fmaf(g.cyp[q], g.yp[q], off);
+            off = fmaf(g.cz[q], xzm, off);
+            off = fmaf(czp, xzp, off);
+            const float rr = g.b[q] - fmaf(dg[q], g.xc[q], -off);
+            r[q] = on && dg[q] > 0.f ? rr : 0.f;
         }
     }
     float s0 = r.x + r.y, s1 = r.z + r.w;  // z pairs
@@ -1243,22 +1297,26 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_flat(Dims df, Op64 Af, const
 }
 
 // Dense inverse of the coarsest operator (n <= 64 cells; SPD up to
-// pure-Neumann blocks) by in-place Gauss-Jordan in LDS, rows stored with a
-// fixed stride of 64 so the element loops split an index with a shift and a
-// mask. Pivots below 1e-12 of the largest diagonal (the pure-Neumann
-// direction) are dropped: their row and column stay 0. One block of
-// kInvertThreads: every thread owns S * S / kInvertThreads matrix entries, so
-// a pivot step is a few FP64 operations per thread between two barriers.
-constexpr int kInvertThreads = 1024;
+// pure-Neumann blocks) by in-place Gauss-Jordan. Pivots below 1e-12 of the
+// largest diagonal (the pure-Neumann direction) are dropped: their row and
+// column stay 0.
+//
+// The 64 pivot steps are a serial chain, so what counts is the length of one:
+// the matrix is in registers, wavefront w of four holding rows 16 w .. 16 w +
+// 15 and lane c column c. A step takes the pivot row through LDS (its
+// wavefront writes it, and the pivot's reciprocal; two buffers, so one barrier)
+// and the pivot column of a wavefront's own rows from lane kk's registers. One
+// block at 4^3 cells: 77 us with the matrix in LDS and 1024 threads (two
+// barriers and three LDS latencies a step), 20 us so.
+constexpr int kInvertThreads = 256;
 
 __global__ __launch_bounds__(kInvertThreads) void k_coarse_invert(Dims d, Op64 A, float *ainv) {
-    constexpr int S = kMaxCoarse;  // row stride
-    static_assert(S == 64, "the element split below assumes a stride of 64");
+    constexpr int S = kMaxCoarse, R = S / (kInvertThreads / 64);  // rows per wavefront
+    static_assert(S == 64 && R == 16, "lane c holds column c");
     __shared__ double M[S * S];
-    __shared__ double rowk[S], colk[S];
-    __shared__ double scale_sh;
+    __shared__ double rowk[2][S], pivk[2][2];  // the pivot row; the pivot and its reciprocal
     const int n = (int)d.cells();
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const Strides s(d);
     for (int e = tid; e < S * S; e += kInvertThreads) M[e] = 0.0;
     __syncthreads();
@@ -1273,45 +1331,56 @@ __global__ __launch_bounds__(kInvertThreads) void k_coarse_invert(Dims d, Op64 A
         if (k + 1 < d.nz) M[c * S + (c + 1)] = -A.cpl[2][c + 1];
     }
     __syncthreads();
-    if (tid == 0) {
-        double m = 0.0;
-        for (int c = 0; c < n; c++) m = fmax(m, fabs(M[c * S + c]));
-        scale_sh = m;
-    }
-    __syncthreads();
-    const double tiny = 1e-12 * scale_sh;
-    for (int kk = 0; kk < n; kk++) {
-        const double p = M[kk * S + kk];
-        if (tid < n) {
-            rowk[tid] = M[kk * S + tid];
-            colk[tid] = M[tid * S + kk];
-        }
-        __syncthreads();
-        if (fabs(p) <= tiny) {
-            if (tid < n) {
-                M[kk * S + tid] = 0.0;
-                M[tid * S + kk] = 0.0;
+    double m = fabs(M[lane * S + lane]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    const double tiny = 1e-12 * m;
+    double a[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) a[r] = M[(R * wave + r) * S + lane];
+    auto at_lane = [](double v, int l) {
+        typedef int i2 __attribute__((ext_vector_type(2)));
+        const i2 h = __builtin_bit_cast(i2, v);
+        return __builtin_bit_cast(double, i2{__builtin_amdgcn_readlane(h.x, l), __builtin_amdgcn_readlane(h.y, l)});
+    };
+    for (int w = 0; w < S / R; w++) {
+#pragma unroll
+        for (int ki = 0; ki < R; ki++) {
+            const int kk = R * w + ki;
+            if (kk >= n) break;  // uniform over the block
+            const int buf = ki & 1;
+            if (wave == w) {
+                const double p = at_lane(a[ki], kk);
+                rowk[buf][lane] = a[ki];
+                if (lane == 0) {
+                    pivk[buf][0] = p;
+                    pivk[buf][1] = 1.0 / p;
+                }
             }
-        } else {
-            const double pinv = 1.0 / p;  // the same value in every thread
-            for (int e = tid; e < S * S; e += kInvertThreads) {
-                const int r = e >> 6, c = e & (S - 1);
-                if (r >= n || c >= n) continue;
+            __syncthreads();
+            const double p = pivk[buf][0], pinv = pivk[buf][1], rk = rowk[buf][lane];
+            const bool drop = fabs(p) <= tiny;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const double ck = at_lane(a[r], kk);
+                const bool row = wave == w && r == ki;
                 double v;
-                if (r == kk && c == kk)
-                    v = pinv;
-                else if (r == kk)
-                    v = rowk[c] * pinv;
-                else if (c == kk)
-                    v = -colk[r] * pinv;
-                else
-                    v = M[e] - colk[r] * rowk[c] * pinv;
-                M[e] = v;
+                if (drop) {
+                    v = row || lane == kk ? 0.0 : a[r];
+                } else if (row) {
+                    v = lane == kk ? pinv : rk * pinv;
+                } else {
+                    v = lane == kk ? -ck * pinv : a[r] - ck * rk * pinv;
+                }
+                a[r] = v;
             }
         }
-        __syncthreads();
     }
-    for (int e = tid; e < n * n; e += kInvertThreads) ainv[e] = (float)M[(e / n) * S + (e % n)];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int row = R * wave + r;
+        if (row < n && lane < n) ainv[row * n + lane] = (float)a[r];
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_coarse_solve(int n, const float *ainv, const float *b,
@@ -1762,14 +1831,17 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
     if (smooth_flat(d, mode, r64, ecoarse, {A.diag, A.cpl[0], A.cpl[1], A.cpl[2], b, xin, xout, dvec})) {
         const unsigned nb = (unsigned)((d.cells() + kSmoothFlatCells - 1) / kSmoothFlatCells);
         const Dims dc = d.coarse();
+        const bool eager = d.cells() <= kEagerCells;
+#define SFP_FLAT_LAUNCH(M, RS, EA)                                                                 \
+    hipLaunchKernelGGL((k_smooth_flat<M, RS, EA>), dim3(nb), dim3(kBlock), 0, st, d, A, b, xin,    \
+                       xout, dvec, cd, cr, ecoarse, dc, gate)
 #define SFP_FLAT_CASE(M)                                                                           \
     case M:                                                                                        \
-        if (A.pinned_rowsum)                                                                       \
-            hipLaunchKernelGGL((k_smooth_flat<M, true>), dim3(nb), dim3(kBlock), 0, st, d, A, b,   \
-                               xin, xout, dvec, cd, cr, ecoarse, dc, gate);                        \
-        else                                                                                       \
-            hipLaunchKernelGGL((k_smooth_flat<M, false>), dim3(nb), dim3(kBlock), 0, st, d, A, b,  \
-                               xin, xout, dvec, cd, cr, ecoarse, dc, gate);                        \
+        if (A.pinned_rowsum) {                                                                     \
+            if (eager) SFP_FLAT_LAUNCH(M, true, true); else SFP_FLAT_LAUNCH(M, true, false);       \
+        } else {                                                                                   \
+            if (eager) SFP_FLAT_LAUNCH(M, false, true); else SFP_FLAT_LAUNCH(M, false, false);     \
+        }                                                                                          \
         break;
         switch (mode) {
             SFP_FLAT_CASE(SM_PROLONG)
@@ -1784,6 +1856,7 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
                 throw ArgError("unsupported smoother mode");
         }
 #undef SFP_FLAT_CASE
+#undef SFP_FLAT_LAUNCH
         SFP_LAUNCH_CHECK();
         return;
     }
@@ -1943,12 +2016,16 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
         const size_t waves = (size_t)((df.nz + kRestrictFlatZ - 1) / kRestrictFlatZ) *
                              ((df.ny + 1) / 2) * ((df.nx + 1) / 2);
         const unsigned nb = (unsigned)((waves * 64 + kBlock - 1) / kBlock);
-        if (A.pinned_rowsum)
-            hipLaunchKernelGGL(k_restrict_flat<true>, dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,
-                               bc, x0c, diag32c, c0, gate);
-        else
-            hipLaunchKernelGGL(k_restrict_flat<false>, dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,
-                               bc, x0c, diag32c, c0, gate);
+        const bool eager = df.cells() <= kEagerCells;
+#define SFP_RESTRICT_LAUNCH(RS, EA)                                                                \
+    hipLaunchKernelGGL((k_restrict_flat<RS, EA>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,  \
+                       bc, x0c, diag32c, c0, gate)
+        if (A.pinned_rowsum) {
+            if (eager) SFP_RESTRICT_LAUNCH(true, true); else SFP_RESTRICT_LAUNCH(true, false);
+        } else {
+            if (eager) SFP_RESTRICT_LAUNCH(false, true); else SFP_RESTRICT_LAUNCH(false, false);
+        }
+#undef SFP_RESTRICT_LAUNCH
         SFP_LAUNCH_CHECK();
         return;
     }

@@ -29,13 +29,12 @@ namespace {
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ bool gated(const double *gate) { return gate && *gate != 0.0; }
-
-// The pending ||r||^2 (see FoldArgs): true when the solve stops here.
-__device__ __forceinline__ bool fold_stop(const FoldArgs &f) {
+// The pending ||r||^2 (see FoldArgs): true when the solve stops here. (stop_rr:
+// f.sc->stop_rr, loaded with the partials.)
+__device__ __forceinline__ bool fold_stop(const FoldArgs &f, const FoldLoad<1> &l, double stop_rr) {
     double v[1];
-    fold_partials<1>(f.partials, f.nb, v);
-    const bool stop = v[0] <= f.sc->stop_rr;
+    fold_sum<1>(f.partials, f.nb, l, v);
+    const bool stop = v[0] <= stop_rr;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         f.sc->rr = v[0];
         f.sc->iters += 1.0;
@@ -56,17 +55,18 @@ struct Geo {
     __device__ int groups() const { return nx * (sx >> 2); }
 };
 
-// Four values of a z row from element offset o, of which the first m are in
-// the row; 0 for the others. Rows need not be aligned (gfx950 loads 16 bytes
+// Four values of a z row from element offset o, and those past the row's end
+// (all but the first m) set to 0. Rows need not be aligned (gfx950 loads 16 bytes
 // from any multiple of four), and the up to three values read past the last
 // row are inside the buffer's allocation (DevBuf::ensure).
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f4 ld_row(const float *__restrict__ p, unsigned o, int m) {
-    const f4 v = *(const f4u *)((const char *)p + 4u * o);
-    f4 w;
+__device__ __forceinline__ f4 ld_row(const float *__restrict__ p, unsigned o) {
+    return *(const f4u *)((const char *)p + 4u * o);
+}
+__device__ __forceinline__ f4 in_row(f4 v, int m) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) w[q] = q < m ? v[q] : 0.f;
-    return w;
+    for (int q = 0; q < 4; q++) v[q] = q < m ? v[q] : 0.f;
+    return v;
 }
 __device__ __forceinline__ void st_row(float *__restrict__ p, unsigned o, int m, f4 v) {
     if (m >= 4) {
@@ -89,27 +89,45 @@ struct Groups {
     unsigned nx[G], ny[G];
 };
 
-// The operator and right-hand side of group q at grid cell (i, j, k), element
-// offset o; `in`: inside the grid (else all 0).
+// The operator (but rd) and right-hand side of group q at grid cell (i, j, k),
+// element offset o (0 outside the grid), as stored; mask_group then zeroes what
+// lies outside the grid (m: its cells inside the z row, 0 outside the grid).
+// Loads first, selections after: the loads of all of a thread's groups are
+// then in flight together.
 template <int G>
 __device__ __forceinline__ void load_group(Groups<G> &g, int q, const Op32 &A, const float *__restrict__ b, Dims d,
-                                           int i, int j, int k, unsigned o, bool in) {
-    const f4 z4 = {0.f, 0.f, 0.f, 0.f};
-    g.cx[q] = g.cxp[q] = g.cy[q] = g.cyp[q] = g.cz[q] = g.dg[q] = g.rd[q] = g.b[q] = g.d[q] = g.x[q] = z4;
-    g.czp[q] = 0.f;
-    if (!in) return;
+                                           int i, int j, unsigned o, int m) {
     const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy;
-    const int m = d.nz - k;
-    const bool xh = i + 1 < d.nx, yh = j + 1 < d.ny;
-    g.dg[q] = ld_row(A.diag, o, m);
-    g.cx[q] = ld_row(A.cpl[0], o, m);
-    g.cxp[q] = ld_row(A.cpl[0], xh ? o + sx : o, xh ? m : 0);
-    g.cy[q] = ld_row(A.cpl[1], o, m);
-    g.cyp[q] = ld_row(A.cpl[1], yh ? o + sy : o, yh ? m : 0);
-    g.cz[q] = ld_row(A.cpl[2], o, m);
-    const float u = A.cpl[2][m > 4 ? o + 4 : o];
-    g.czp[q] = m > 4 ? u : 0.f;
-    g.b[q] = ld_row(b, o, m);
+    g.dg[q] = ld_row(A.diag, o);
+    g.cx[q] = ld_row(A.cpl[0], o);
+    g.cxp[q] = ld_row(A.cpl[0], m > 0 && i + 1 < d.nx ? o + sx : o);
+    g.cy[q] = ld_row(A.cpl[1], o);
+    g.cyp[q] = ld_row(A.cpl[1], m > 0 && j + 1 < d.ny ? o + sy : o);
+    g.cz[q] = ld_row(A.cpl[2], o);
+    g.czp[q] = A.cpl[2][m > 4 ? o + 4 : o];
+    g.b[q] = ld_row(b, o);
+}
+template <int G>
+__device__ __forceinline__ void pin_group(const Groups<G> &g, int q) {
+    pin(g.dg[q]);
+    pin(g.cx[q]);
+    pin(g.cxp[q]);
+    pin(g.cy[q]);
+    pin(g.cyp[q]);
+    pin(g.cz[q]);
+    pin(g.czp[q]);
+    pin(g.b[q]);
+}
+template <int G>
+__device__ __forceinline__ void mask_group(Groups<G> &g, int q, Dims d, int i, int j, int m) {
+    g.dg[q] = in_row(g.dg[q], m);
+    g.cx[q] = in_row(g.cx[q], m);
+    g.cxp[q] = in_row(g.cxp[q], i + 1 < d.nx ? m : 0);
+    g.cy[q] = in_row(g.cy[q], m);
+    g.cyp[q] = in_row(g.cyp[q], j + 1 < d.ny ? m : 0);
+    g.cz[q] = in_row(g.cz[q], m);
+    g.czp[q] = m > 4 ? g.czp[q] : 0.f;
+    g.b[q] = in_row(g.b[q], m);
 #pragma unroll
     for (int s = 0; s < 4; s++) g.rd[q][s] = rcp_or_zero(g.dg[q][s]);
 }
@@ -231,7 +249,7 @@ __device__ __forceinline__ float child_sum(const float *S, int i, int j, int K, 
 // the tile holds whole rows), computes every step on all of it (the outer
 // cells of the halo go wrong by one layer a step, the tile's own cells never
 // see them) and stores its own cells.
-template <int G>
+template <int G, int START>
 __global__ __launch_bounds__(1024) void k_tile_steps(TileArgs a, const double *gate) {
     __shared__ __attribute__((aligned(16))) float lds[2][G * 4096 + 2 * kGuard];
     const Dims d = a.d;
@@ -243,37 +261,62 @@ __global__ __launch_bounds__(1024) void k_tile_steps(TileArgs a, const double *g
     const int i0 = ib * P.tx - P.hx, j0 = jb * P.ty - P.hy, k0 = kb * P.tz - P.hz;
     const Geo e(P.tx + 2 * P.hx, P.ty + 2 * P.hy, P.tz + 2 * P.hz);
     const int ng = e.groups();
+    // every load is issued before any is waited for: the gate's and the pending
+    // norm's, the operator's, the iterate's and the coarse correction's
+    const double stop = load_gate(gate, a.b);
+    FoldLoad<1> fl;
+    double stop_rr = 0.0;
+    if (START == TILE_FIRST && a.fold.nb) {
+        fold_load<1>(a.fold.partials, a.fold.nb, fl);
+        stop_rr = a.fold.sc->stop_rr;
+    }
     Groups<G> g;
+    float e0[G], e1[G];
+    int gi[G], gj[G], m[G];
 #pragma unroll
     for (int q = 0; q < G; q++) {
         const int t = (int)threadIdx.x + q * (int)blockDim.x;
-        g.c[q] = -1;
-        if (t >= ng) continue;
         int i, j, k;
-        place_group(g, q, t, e, i, j, k);
-        const int gi = i0 + i, gj = j0 + j, gk = k0 + k;
-        const bool in = gi >= 0 && gi < d.nx && gj >= 0 && gj < d.ny && gk >= 0 && gk < d.nz;
-        const unsigned o = in ? ((unsigned)gi * d.ny + gj) * (unsigned)d.nz + gk : 0u;
-        load_group(g, q, a.A, a.b, d, gi, gj, gk, o, in);
-        if (in && a.start != TILE_FIRST) {
-            g.x[q] = ld_row(a.xin, o, d.nz - gk);
-            if (a.start == TILE_CONTINUE) g.d[q] = ld_row(a.din, o, d.nz - gk);
-            if (a.start == TILE_PROLONG) {
-                const unsigned er = ((unsigned)(gi >> 1) * a.dc.ny + (gj >> 1)) * (unsigned)a.dc.nz + (gk >> 1);
-                const float e0 = a.e[er], e1 = gk + 2 < d.nz ? a.e[er + 1] : 0.f;
-#pragma unroll
-                for (int s = 0; s < 4; s++)
-                    if (g.dg[q][s] > 0.f) g.x[q][s] = g.x[q][s] + (s < 2 ? e0 : e1);
-            }
-        }
-        if (a.start == TILE_FIRST) {
-#pragma unroll
-            for (int s = 0; s < 4; s++) g.x[q][s] = a.c0 * g.rd[q][s] * g.b[q][s];
-            g.d[q] = g.x[q];
+        place_group(g, q, min(t, ng - 1), e, i, j, k);
+        if (t >= ng) g.c[q] = -1;
+        gi[q] = i0 + i;
+        gj[q] = j0 + j;
+        const int gk = k0 + k;
+        const bool in = t < ng && gi[q] >= 0 && gi[q] < d.nx && gj[q] >= 0 && gj[q] < d.ny && gk >= 0 && gk < d.nz;
+        const unsigned o = in ? ((unsigned)gi[q] * d.ny + gj[q]) * (unsigned)d.nz + gk : 0u;
+        m[q] = in ? d.nz - gk : 0;
+        load_group(g, q, a.A, a.b, d, gi[q], gj[q], o, m[q]);
+        if constexpr (START != TILE_FIRST) g.x[q] = ld_row(a.xin, o);
+        if constexpr (START == TILE_CONTINUE) g.d[q] = ld_row(a.din, o);
+        if constexpr (START == TILE_PROLONG) {
+            const unsigned er =
+                in ? ((unsigned)(gi[q] >> 1) * a.dc.ny + (gj[q] >> 1)) * (unsigned)a.dc.nz + (gk >> 1) : 0u;
+            e0[q] = a.e[er];
+            e1[q] = a.e[m[q] > 2 ? er + 1 : er];
         }
     }
-    if (gated(gate)) return;  // (after the loads: the flag's latency is theirs)
-    if (a.fold.nb && fold_stop(a.fold)) return;  // uniform
+#pragma unroll
+    for (int q = 0; q < G; q++) {
+        pin_group(g, q);
+        if constexpr (START != TILE_FIRST) pin(g.x[q]);
+        if constexpr (START == TILE_CONTINUE) pin(g.d[q]);
+        if constexpr (START == TILE_PROLONG) pin(e0[q]), pin(e1[q]);
+    }
+    if (stop != 0.0) return;
+    if (START == TILE_FIRST && a.fold.nb && fold_stop(a.fold, fl, stop_rr)) return;  // uniform
+#pragma unroll
+    for (int q = 0; q < G; q++) {
+        mask_group(g, q, d, gi[q], gj[q], m[q]);
+        if constexpr (START != TILE_FIRST) g.x[q] = in_row(g.x[q], m[q]);
+        if constexpr (START == TILE_CONTINUE) g.d[q] = in_row(g.d[q], m[q]);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (START == TILE_FIRST) g.x[q][s] = a.c0 * g.rd[q][s] * g.b[q][s];
+            if (START == TILE_PROLONG && g.dg[q][s] > 0.f) g.x[q][s] = g.x[q][s] + (s < 2 ? e0[q] : e1[q]);
+        }
+        if (START == TILE_FIRST) g.d[q] = g.x[q];
+        if (START == TILE_PROLONG) g.d[q] = f4{0.f, 0.f, 0.f, 0.f};  // (cd[0] is 0)
+    }
     if (threadIdx.x < 2 * kGuard) {
         const int o = threadIdx.x < kGuard ? threadIdx.x : 4 * ng + threadIdx.x;
         lds[0][o] = lds[1][o] = 0.f;
@@ -429,11 +472,19 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(TailArgs t, const double *
     const int ng = e.groups();
     // every load of the copy-in is issued before any is waited for: the first
     // level's operator and b into registers, the others' into LDS
+    const double stop = load_gate(gate, t.ainv);
+    FoldLoad<1> fl;
+    double stop_rr = 0.0;
+    if (t.fold.nb) {
+        fold_load<1>(t.fold.partials, t.fold.nb, fl);
+        stop_rr = t.fold.sc->stop_rr;
+    }
     Groups<1> g;
-    int gi = 0, gj = 0, gk = 0;
-    g.c[0] = -1;
-    if (tid < ng) place_group(g, 0, tid, e, gi, gj, gk);
-    load_group(g, 0, t.lv[0].A, t.lv[0].b, d, gi, gj, gk, (unsigned)((gi * d.ny + gj) * d.nz + gk), tid < ng);
+    int gi, gj, gk;
+    place_group(g, 0, min(tid, ng - 1), e, gi, gj, gk);
+    if (tid >= ng) g.c[0] = -1;
+    const int gm = tid < ng ? d.nz - gk : 0;
+    load_group(g, 0, t.lv[0].A, t.lv[0].b, d, gi, gj, tid < ng ? (unsigned)((gi * d.ny + gj) * d.nz + gk) : 0u, gm);
     {
         const int nC = (int)t.lv[last].d.cells();
         f4 a4 = {0.f, 0.f, 0.f, 0.f};  // row r, columns c .. c + 3
@@ -463,8 +514,10 @@ __global__ __launch_bounds__(1024) void k_vcycle_tail(TailArgs t, const double *
         }
         *(f4 *)(inv + r * kInvStride + c) = a4;
     }
-    if (gated(gate)) return;  // (after the loads: the flag's latency is theirs)
-    if (t.fold.nb && fold_stop(t.fold)) return;  // uniform
+    pin_group(g, 0);
+    if (stop != 0.0) return;
+    if (t.fold.nb && fold_stop(t.fold, fl, stop_rr)) return;  // uniform
+    mask_group(g, 0, d, gi, gj, gm);
     if (tid < 2 * kGuard) {
         const int o = tid < kGuard ? tid : 4 * ng + tid;
         lds[0][o] = lds[1][o] = 0.f;
@@ -623,14 +676,25 @@ void launch_tile_steps(hipStream_t st, const TileArgs &a, const double *gate) {
     if ((P.bx > 1 && P.hx < reach) || (P.by > 1 && P.hy < reach) || (P.bz > 1 && P.hz < reach))
         throw ArgError("tile steps: halo narrower than the steps");
     if (a.d.cells() >= ((size_t)1 << 30)) throw ArgError("tile steps: level too large");
+    if (!a.b || !a.xout || (a.start != TILE_FIRST && !a.xin) || (a.start == TILE_PROLONG && !a.e) ||
+        (a.start == TILE_CONTINUE && !a.din) || a.start < TILE_FIRST || a.start > TILE_CONTINUE)
+        throw ArgError("tile steps: missing input");
+    if (a.fold.nb > kFoldMax || (a.fold.nb && a.start != TILE_FIRST)) throw ArgError("tile steps: bad fold");
     if (a.xout == a.xin || (a.dout && a.dout == a.din) || (a.bc && a.dout))
         throw ArgError("tile steps: outputs alias inputs");
     const unsigned nb = (unsigned)(P.bx * P.by * P.bz);
+    const dim3 grid(nb), block(((P.groups <= 1024 ? P.groups : (P.groups + 1) / 2) + 63) / 64 * 64);
+#define SFP_TILE(G, S) hipLaunchKernelGGL((k_tile_steps<G, S>), grid, block, 0, st, a, gate)
     if (P.groups <= 1024) {
-        hipLaunchKernelGGL(k_tile_steps<1>, dim3(nb), dim3((P.groups + 63) / 64 * 64), 0, st, a, gate);
+        if (a.start == TILE_FIRST) SFP_TILE(1, TILE_FIRST);
+        else if (a.start == TILE_PROLONG) SFP_TILE(1, TILE_PROLONG);
+        else SFP_TILE(1, TILE_CONTINUE);
     } else {
-        hipLaunchKernelGGL(k_tile_steps<2>, dim3(nb), dim3(((P.groups + 1) / 2 + 63) / 64 * 64), 0, st, a, gate);
+        if (a.start == TILE_FIRST) SFP_TILE(2, TILE_FIRST);
+        else if (a.start == TILE_PROLONG) SFP_TILE(2, TILE_PROLONG);
+        else SFP_TILE(2, TILE_CONTINUE);
     }
+#undef SFP_TILE
     SFP_LAUNCH_CHECK();
 }
 

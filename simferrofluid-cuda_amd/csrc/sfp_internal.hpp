@@ -155,7 +155,8 @@ constexpr int kRing = 8, kCoefs = 2 * kRing;
 struct KrylovScalars {
     double zw, zq, zr;           // dots of the current iteration
     double rr, bb;               // ||r||^2, ||b||^2
-    double pad[4];               // scratch of single reductions (count, scales)
+    double active;               // active cells counted by the last residual kernel given the diagonal
+    double pad[4];               // scratch of single reductions (scales)
     // batched iterations: `stop` becomes nonzero when rr <= stop_rr after an
     // update, and every gated kernel of later iterations then returns at once;
     // `iters` counts the updates done

@@ -79,11 +79,6 @@ KernelTimer::~KernelTimer() {
     for (auto e : ev) (void)hipEventDestroy(e);
 }
 
-void Workspace::read_scalars() {
-    SFP_HIP(hipMemcpyAsync(host_sc, scalars.p, sizeof(KrylovScalars), hipMemcpyDeviceToHost, stream));
-    SFP_HIP(hipStreamSynchronize(stream));
-}
-
 // ---------------------------------------------------------------- System
 // The stencil kernels skip wavefront rows whose cells are all inactive; the
 // skipped cells of the level vectors then keep the zeros written here.
@@ -586,12 +581,6 @@ const float *System::restrict_smoothed(Workspace &ws, const SolverConfig &cfg, c
     return learned_cycle(ws, cfg, r64, kCycleRestrictOnly);
 }
 
-long long System::count_active(Workspace &ws) {
-    launch_count_active(ws.stream, d_, lv_[0].diag32.p, ws.partials.p, ws.scalars.p);
-    ws.read_scalars();
-    return (long long)ws.host_sc->pad[0];
-}
-
 SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm) {
     SolveInfo info;
     info.precond_used = cfg.precond;
@@ -620,8 +609,13 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     };
     float c0 = first_coef(learned);
     launch_residual64(st, d, A, rhs_.p, warm ? x_.p : nullptr, r_.p, ws.partials.p,
-                      ws.scalars.p, b32, x0, lv_[level].diag32.p, c0);
-    ws.read_scalars();
+                      ws.scalars.p, ws.host_sc, b32, x0, lv_[level].diag32.p, c0);
+    ws.wait();
+    info.active = (long long)ws.host_sc->active;
+    if (*ws.host_err) {
+        info.input_error = true;
+        return info;
+    }
     const double bb = ws.host_sc->bb;
     if (bb == 0.0) {  // zero right-hand side: x = 0
         SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));
@@ -668,13 +662,13 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             // FP64 (the sums only), and restart from the true residual if the
             // two have drifted apart
             bring_x_up_to_date(false);
-            launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p);
-            ws.read_scalars();
+            launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p, ws.host_sc);
+            ws.wait();
             rel = std::sqrt(ws.host_sc->rr / bb);
             checked = true;
             if (rel > cfg.tol) {
                 launch_residual64(st, d, A, rhs_.p, x_.p, r_.p, ws.partials.p,
-                                  ws.scalars.p, b32, x0, lv_[level].diag32.p, c0);
+                                  ws.scalars.p, nullptr, b32, x0, lv_[level].diag32.p, c0);
                 first = true;
                 b_ready = b32 != nullptr;
             }
@@ -734,13 +728,14 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             // (a cycle whose first launch folds forms its first iterate itself)
             float *const x0_next = fold ? nullptr : x0;
             launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, w_.p, q_.p, r_.p, b32, x0_next, c0,
-                              first ? 1 : 0, iter + it, fold, ws.partials.p, ws.scalars.p, ws.gate, done);
+                              first ? 1 : 0, iter + it, fold, ws.partials.p, ws.scalars.p, ws.gate, done,
+                              it + 1 == batch ? ws.host_sc : nullptr);
             if (profiling) ws.timers[K_UPDATE64].end_recorded();
             first = false;
             b_ready = b32 != nullptr;
         }
-        if (fold) launch_fcg_norm(st, d, ws.partials.p, ws.scalars.p, ws.gate);
-        ws.read_scalars();
+        if (fold) launch_fcg_norm(st, d, ws.partials.p, ws.scalars.p, ws.gate, ws.host_sc);
+        ws.wait();
         const bool stalled = batch > 1 && ws.host_sc->stalled != 0.0;
         ws.gate = nullptr;
         const int done = batch > 1 ? (int)ws.host_sc->iters : 1;
@@ -778,8 +773,8 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     bring_x_up_to_date(false);
     if (zero_x) SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));  // (no iteration)
     if (!checked) {
-        launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p);
-        ws.read_scalars();
+        launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p, ws.host_sc);
+        ws.wait();
         rel = std::sqrt(ws.host_sc->rr / bb);
     }
     info.rel = rel;

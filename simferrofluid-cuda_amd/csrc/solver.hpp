@@ -95,9 +95,10 @@ struct Workspace {
     hipStream_t stream = nullptr;
     DevBuf<double> partials;
     DevBuf<KrylovScalars> scalars;
-    DevBuf<int> err;
-    KrylovScalars *host_sc = nullptr;  // pinned
-    int *host_err = nullptr;           // pinned
+    // pinned, and written by kernels: the scalars the host reads, and the
+    // input-error flag of the assembly and the velocity update
+    KrylovScalars *host_sc = nullptr;
+    int *host_err = nullptr;
     bool profiling = false;
     std::array<KernelTimer, K_COUNT> timers;
     // learned preconditioner: the context's network and the level set and
@@ -135,7 +136,7 @@ struct Workspace {
     // orders it after the coarsening, side_out orders its first use after it
     hipStream_t side = nullptr;
     hipEvent_t side_in = nullptr, side_out = nullptr;
-    void read_scalars();               // synchronous copy of *scalars to host_sc
+    void wait() { SFP_HIP(hipStreamSynchronize(stream)); }
 };
 
 struct SolveInfo {
@@ -144,6 +145,8 @@ struct SolveInfo {
     bool converged = false;
     int fallback = 0;
     int precond_used = 0;
+    long long active = 0;  // rows of the system
+    bool input_error = false;  // the assembly before the solve raised it: nothing was solved
 };
 
 class System {
@@ -186,8 +189,6 @@ class System {
     SolveInfo solve_level(Workspace &ws, const SolverConfig &cfg, int level) {
         return fcg(ws, cfg, level, false);
     }
-    // Number of active rows (sets ws.scalars->pad[0]); synchronous.
-    long long count_active(Workspace &ws);
     // The operator is a Neumann problem made definite by one eliminated cell
     // (the magnetic potential's pin at cell 0). Its coarse levels then scale
     // only the couplings by coarse_scale and keep each aggregate's row sum
@@ -245,8 +246,5 @@ class System {
     void join_ainv(Workspace &ws);
     int built_coarsest_ = -1;
 };
-
-void launch_count_active(hipStream_t s, Dims d, const float *diag32, double *partials,
-                         KrylovScalars *sc);
 
 }  // namespace sfp
