@@ -200,13 +200,16 @@ __global__ __launch_bounds__(kBlock) void k_pressure_apply(CellGrid cg, Dims d, 
                                                            const double *__restrict__ jump,
                                                            const unsigned char *__restrict__ liquid,
                                                            const double *__restrict__ p,
-                                                           double *__restrict__ vel, int *err) {
+                                                           double *__restrict__ vel, int *err,
+                                                           double *__restrict__ p_out, const double *need) {
+    if (need && *need == 0.0) return;
     const Dims fd = d.face(axis);
     int k, j, i0;
     cell_tile(cg, k, j, i0);
     if (k >= fd.nz || j >= fd.ny) return;
     for (int i = i0, ie = min(i0 + cg.planes, fd.nx); i < ie; i++) {
         const size_t fidx = fd.idx(i, j, k);
+        if (p_out && i < d.nx && j < d.ny && k < d.nz) p_out[d.idx(i, j, k)] = p[d.idx(i, j, k)];
         const double weight = 1. - frac[fidx];
         if (weight == 0.) continue;
         int c1[3] = {i, j, k};
@@ -345,8 +348,11 @@ __global__ __launch_bounds__(kBlock) void k_magnetic_assemble(CellGrid cg, Dims 
 
 __global__ __launch_bounds__(kBlock) void k_magnetic_total_field(CellGrid cg, Dims d, int axis, double inv,
                                                                  const double *__restrict__ pot,
-                                                                 const double *__restrict__ hext,
-                                                                 double *__restrict__ htot) {
+                                                                 const double *hext,
+                                                                 double *__restrict__ htot,
+                                                                 double *__restrict__ pot_out,
+                                                                 double *out, const double *need) {
+    if (need && *need == 0.0) return;
     const Dims fd = d.face(axis);
     int k, j, i0;
     cell_tile(cg, k, j, i0);
@@ -356,6 +362,7 @@ __global__ __launch_bounds__(kBlock) void k_magnetic_total_field(CellGrid cg, Di
         int c0[3] = {i, j, k};
         c0[axis] -= 1;
         const int c1[3] = {i, j, k};
+        if (pot_out && valid(d, c1)) pot_out[d.idx(i, j, k)] = pot[d.idx(i, j, k)];
         double h;
         if (valid(d, c0) && valid(d, c1))
             h = (pot[d.idx(c0[0], c0[1], c0[2])] - pot[d.idx(c1[0], c1[1], c1[2])]) * inv;
@@ -363,6 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_magnetic_total_field(CellGrid cg, Di
             h = 0.;
         h += hext[fidx];
         htot[fidx] = h;
+        if (out) out[fidx] = h;
     }
 }
 
@@ -411,11 +419,11 @@ void launch_pressure_rhs(hipStream_t st, Dims d, const unsigned char *liquid, Fa
 
 void launch_pressure_apply(hipStream_t st, Dims d, const double *phi, Faces frac,
                            const Faces *jump, const unsigned char *liquid, const double *p,
-                           MutFaces vel, int *err) {
+                           MutFaces vel, int *err, double *p_out, const double *need) {
     for (int a = 0; a < 3; a++) {
         Launch L = cell_launch(d.face(a), 0, kAssemblyPlanes);
         hipLaunchKernelGGL(k_pressure_apply, L.grid, L.block, 0, st, L.cg, d, a, phi, frac.a[a],
-                           jump ? jump->a[a] : nullptr, liquid, p, vel.a[a], err);
+                           jump ? jump->a[a] : nullptr, liquid, p, vel.a[a], err, a == 0 ? p_out : nullptr, need);
         SFP_LAUNCH_CHECK();
     }
 }
@@ -440,11 +448,12 @@ void launch_magnetic_assemble(hipStream_t st, Dims d, Faces mu, Faces hext, doub
 }
 
 void launch_magnetic_total_field(hipStream_t st, Dims d, double inv, const double *pot,
-                                 Faces hext, MutFaces htot) {
+                                 Faces hext, MutFaces htot, double *pot_out, MutFaces out,
+                                 const double *need) {
     for (int a = 0; a < 3; a++) {
         Launch L = cell_launch(d.face(a), 0, kAssemblyPlanes);
         hipLaunchKernelGGL(k_magnetic_total_field, L.grid, L.block, 0, st, L.cg, d, a, inv, pot,
-                           hext.a[a], htot.a[a]);
+                           hext.a[a], htot.a[a], a == 0 ? pot_out : nullptr, out.a[a], need);
         SFP_LAUNCH_CHECK();
     }
 }

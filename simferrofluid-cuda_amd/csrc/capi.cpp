@@ -104,6 +104,11 @@ void check_err(sfp_context ctx, const char *msg) {
     }
 }
 
+// whether two arrays share memory (null: no)
+bool meet(const double *a, size_t na, const double *b, size_t nb) {
+    return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 const char *const kOpenFace = "open (fraction < 1) face on the grid boundary next to a liquid cell";
 
 // ---------------------------------------------------------------- pressure
@@ -150,7 +155,22 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     SFP_HIP(hipEventRecord(ctx->ev[1], s));
     ctx->ws.phi = phi;
     ctx->ws.spacing = ctx->spacing;
-    SolveInfo info = sys.solve(ctx->ws, ctx->cfg.for_pressure(), reproject);
+    MutFaces Vm{{vel[0], vel[1], vel[2]}};
+    // the update stores the caller's copy of the pressure too, unless that lies
+    // over an array it reads
+    const size_t nb = d.cells() * sizeof(double);
+    bool apart = !meet(pressure, nb, phi, nb);
+    for (int a = 0; a < 3; a++) {
+        const size_t fb = face_count(d, a) * sizeof(double);
+        for (const double *p : {frac[a], (const double *)vel[a], J.a[a]}) apart = apart && !meet(pressure, nb, p, fb);
+    }
+    const Finish apply = [&](const double *need) {
+        SFP_HIP(hipEventRecord(ctx->ev[2], s));
+        launch_pressure_apply(s, d, phi, F, jump ? &J : nullptr, ctx->liquid.p, sys.x().p, Vm,
+                              ctx->ws.host_err, apart ? pressure : nullptr, need);
+        SFP_HIP(hipEventRecord(ctx->ev[3], s));
+    };
+    SolveInfo info = sys.solve(ctx->ws, ctx->cfg.for_pressure(), reproject, apply);
     if (info.input_error) check_err(ctx, kOpenFace);
     if (!reproject) {
         ctx->pressure_unknowns = info.active;
@@ -162,14 +182,8 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
             return;
         }
     }
-    SFP_HIP(hipEventRecord(ctx->ev[2], s));
-    MutFaces Vm{{vel[0], vel[1], vel[2]}};
-    launch_pressure_apply(s, d, phi, F, jump ? &J : nullptr, ctx->liquid.p, sys.x().p, Vm,
-                          ctx->ws.host_err);
-    if (pressure)
-        SFP_HIP(hipMemcpyAsync(pressure, sys.x().p, d.cells() * sizeof(double),
-                               hipMemcpyDeviceToDevice, s));
-    SFP_HIP(hipEventRecord(ctx->ev[3], s));
+    if (!info.finished) apply(nullptr);
+    if (pressure && !apart) SFP_HIP(hipMemcpyAsync(pressure, sys.x().p, nb, hipMemcpyDeviceToDevice, s));
     check_err(ctx, kOpenFace);
     fill_stats(st, info, ctx->pressure_unknowns, elapsed(ctx->ev[0], ctx->ev[1]),
                elapsed(ctx->ev[1], ctx->ev[2]), elapsed(ctx->ev[2], ctx->ev[3]));
@@ -207,22 +221,38 @@ void magnetic_dev(sfp_context ctx, const double *phi, const double *const hext[3
     SFP_HIP(hipEventRecord(ctx->ev[1], s));
     ctx->ws.phi = phi;
     ctx->ws.spacing = ctx->spacing;
-    SolveInfo info = sys.solve(ctx->ws, ctx->cfg, ctx->magnetic_warm);
-    ctx->magnetic_warm = true;
-    SFP_HIP(hipEventRecord(ctx->ev[2], s));
-    MutFaces T{{ctx->htot[0].p, ctx->htot[1].p, ctx->htot[2].p}};
-    launch_magnetic_total_field(s, d, ctx->mg.inv, sys.x().p, H, T);
-    ctx->field_ready = true;
-    if (potential)
-        SFP_HIP(hipMemcpyAsync(potential, sys.x().p, d.cells() * sizeof(double),
-                               hipMemcpyDeviceToDevice, s));
+    MutFaces T{{ctx->htot[0].p, ctx->htot[1].p, ctx->htot[2].p}}, out{{nullptr, nullptr, nullptr}};
     if (htot_out)
+        for (int a = 0; a < 3; a++) out.a[a] = htot_out[a];
+    // the caller's copies are stored with the field, unless they lie over an
+    // array it is formed from (the face's own external field apart)
+    const size_t nb = d.cells() * sizeof(double);
+    bool apart = true;
+    for (int a = 0; a < 3; a++) {
+        const size_t fb = face_count(d, a) * sizeof(double);
+        apart = apart && !meet(potential, nb, hext[a], fb);
+        for (int b = 0; b < 3; b++)
+            if (a != b || out.a[b] != hext[a])
+                apart = apart && !meet(out.a[b], face_count(d, b) * sizeof(double), hext[a], fb);
+    }
+    const Finish assign = [&](const double *need) {
+        SFP_HIP(hipEventRecord(ctx->ev[2], s));
+        launch_magnetic_total_field(s, d, ctx->mg.inv, sys.x().p, H, T, apart ? potential : nullptr,
+                                    apart ? out : MutFaces{{nullptr, nullptr, nullptr}}, need);
+        SFP_HIP(hipEventRecord(ctx->ev[3], s));
+    };
+    SolveInfo info = sys.solve(ctx->ws, ctx->cfg, ctx->magnetic_warm, assign);
+    ctx->magnetic_warm = true;
+    if (!info.finished) assign(nullptr);
+    if (!apart) {
+        if (potential) SFP_HIP(hipMemcpyAsync(potential, sys.x().p, nb, hipMemcpyDeviceToDevice, s));
         for (int a = 0; a < 3; a++)
-            if (htot_out[a])
-                SFP_HIP(hipMemcpyAsync(htot_out[a], ctx->htot[a].p, face_count(d, a) * sizeof(double),
+            if (out.a[a])
+                SFP_HIP(hipMemcpyAsync(out.a[a], T.a[a], face_count(d, a) * sizeof(double),
                                        hipMemcpyDeviceToDevice, s));
-    SFP_HIP(hipEventRecord(ctx->ev[3], s));
-    SFP_HIP(hipStreamSynchronize(s));
+    }
+    ctx->ws.wait();
+    ctx->field_ready = true;
     fill_stats(st, info, (long long)d.cells() - (dirichlet ? 0 : 1), elapsed(ctx->ev[0], ctx->ev[1]),
                elapsed(ctx->ev[1], ctx->ev[2]), elapsed(ctx->ev[2], ctx->ev[3]));
 }
@@ -291,7 +321,6 @@ void extrapolate_velocity_dev(sfp_context ctx, double *const vel[3], const doubl
         launch_velocity_valid(s, d, a, phi, frac[a], ctx->post_valid[0][a].p);
         launch_extrapolate(s, fd, vel[a], ctx->post_valid[0][a].p, ctx->post_valid[1][a].p, 0.0, steps);
     }
-    SFP_HIP(hipStreamSynchronize(s));
 }
 
 void collider_enforce_dev(sfp_context ctx, double *const vel[3], const double *const frac[3],
@@ -311,7 +340,6 @@ void collider_enforce_dev(sfp_context ctx, double *const vel[3], const double *c
     launch_collider_enforce(s, d, ctx->spacing, ctx->origin, old, Faces{{frac[0], frac[1], frac[2]}},
                             Faces{{normal[0], normal[1], normal[2]}},
                             Faces{{colvel[0], colvel[1], colvel[2]}}, MutFaces{{vel[0], vel[1], vel[2]}});
-    SFP_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace
@@ -416,7 +444,10 @@ sfp_status sfp_projection_substep(sfp_context ctx, double *const velocity[3], co
             du[a] = up(ctx, ctx->s_face[2][a], solid_velocity[a], n);
             dj[a] = jump ? up(ctx, ctx->s_face[3][a], jump[a], n) : nullptr;
             dn[a] = up(ctx, ctx->s_face[4][a], normal[a], n);
-            dc[a] = up(ctx, ctx->s_face[5][a], collider_velocity[a], n);
+            // (the collider is often the solid of the projection: one upload)
+            dc[a] = collider_velocity[a] == solid_velocity[a]
+                        ? du[a]
+                        : up(ctx, ctx->s_face[5][a], collider_velocity[a], n);
         }
         const double *dphi = up(ctx, ctx->s_phi, level_set, d.cells());
         double *dp = nullptr;
@@ -436,14 +467,20 @@ sfp_status sfp_projection_substep(sfp_context ctx, double *const velocity[3], co
 sfp_status sfp_extrapolate_velocity_device(sfp_context ctx, double *const velocity[3],
                                            const double *level_set,
                                            const double *const fraction[3], int steps) {
-    return guarded(ctx, [&] { extrapolate_velocity_dev(ctx, velocity, level_set, fraction, steps); });
+    return guarded(ctx, [&] {
+        extrapolate_velocity_dev(ctx, velocity, level_set, fraction, steps);
+        ctx->ws.wait();
+    });
 }
 
 sfp_status sfp_collider_enforce_device(sfp_context ctx, double *const velocity[3],
                                        const double *const fraction[3],
                                        const double *const normal[3],
                                        const double *const collider_velocity[3]) {
-    return guarded(ctx, [&] { collider_enforce_dev(ctx, velocity, fraction, normal, collider_velocity); });
+    return guarded(ctx, [&] {
+        collider_enforce_dev(ctx, velocity, fraction, normal, collider_velocity);
+        ctx->ws.wait();
+    });
 }
 
 const char *sfp_status_string(sfp_status s) {

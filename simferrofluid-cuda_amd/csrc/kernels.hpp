@@ -179,27 +179,29 @@ void launch_coarse_solve(hipStream_t s, int n, const float *ainv, const float *b
 
 // ---------------------------------------------------------------- Krylov (krylov.hip)
 // `host` (the residual, the update and the norm): a pinned copy of the scalars
-// that the launch's finalize fills in (rr, bb, active, iters, stalled; also
+// that the launch's finalize fills in (all but the recurrences' scalars; also
 // behind a closed gate), so that the host reads them after a stream
 // synchronization, without a copy (a launch of its own, 3 us, before it).
 // Reduction kernels cover this many x planes per block (fewer partials).
 constexpr int kReducePlanes = 0;  // automatic
 // Doubles of partial-sum scratch a reduction over grid d needs.
 size_t reduction_partials(Dims d);
-// Before a batch of gated iterations: scalars->stop = 0, ->iters = 0,
-// ->stop_rr = stop_rr, ->stall_rr = stall_rr (0: no stall test),
-// ->stalled = 0.
-void launch_batch_begin(hipStream_t s, KrylovScalars *sc, double stop_rr, double stall_rr = 0.0);
+// Before a batch of gated iterations: scalars->stop_rr = tol2 ||b||^2,
+// ->stall_rr = stall_rr (0: no stall test), ->iters, ->ok, ->stalled and ->stop
+// = 0; first (batch of a solve): stop is raised where ||r||^2 needs no iteration.
+void launch_batch_begin(hipStream_t s, KrylovScalars *sc, double tol2, double stall_rr, bool first);
 // r = b - A x (x may be null = 0); scalars->rr = r.r, scalars->bb = b.b;
 // r may be null (only the sums).
 // With b32, also b32 = r rounded to FP32 and, with x0, x0 = c0 D32^-1 b32
 // (diag32: the FP32 diagonal): the right-hand side and first Chebyshev
 // iterate of a V-cycle on r, as the FCG update stores them. With diag32 the
-// active cells are counted too (scalars->active).
+// active cells are counted too (scalars->active). scalars->check_rr = r.r, ->ok
+// whether its root over ||b|| is at most tol. need: the launches return while
+// *need is 0.
 void launch_residual64(hipStream_t s, Dims d, Op64 A, const double *b, const double *x,
                        double *r, double *partials, KrylovScalars *sc, KrylovScalars *host = nullptr,
                        float *b32 = nullptr, float *x0 = nullptr, const float *diag32 = nullptr,
-                       float c0 = 0.f);
+                       float c0 = 0.f, const double *need = nullptr, double tol = 0.0);
 // w = A z; dots z.w, z.q_prev, z.r, and with them alpha, beta and p.q of
 // iteration number iter (scalars->alpha[iter % kCoefs], ...). fold: only the
 // partial sums (the update adds them).
@@ -229,9 +231,11 @@ void launch_fcg_norm(hipStream_t s, Dims d, double *partials, KrylovScalars *sc,
 bool fold_pays(Dims d);
 FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc);
 // x += alpha_k p_k, p_k = z_k - beta_k p_{k-1} for the K <= kRing iterations
-// i0 .. i0 + K - 1 whose z_k are at z + (k - i0) stride (see k_fcg_flush).
+// i0 .. i0 + K - 1 whose z_k are at z + (k - i0) stride (see k_fcg_flush; need:
+// K counts those before the current batch).
 void launch_fcg_flush(hipStream_t s, Dims d, const float *active, const float *z, size_t stride, int K, int i0,
-                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc);
+                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc,
+                      const double *need = nullptr);
 // z = D^{-1} r on active cells (Jacobi preconditioner).
 void launch_jacobi(hipStream_t s, Dims d, Op32 A, const double *r, float *z,
                    const double *gate = nullptr);
@@ -271,10 +275,11 @@ void launch_pressure_assemble(hipStream_t s, Dims d, const double *phi, Faces fr
 // Pressure::SetRightHandSide on the stored unknowns.
 void launch_pressure_rhs(hipStream_t s, Dims d, const unsigned char *liquid, Faces frac,
                          Faces vel, Faces us, double vol_error, double *rhs);
-// Pressure::ApplyProjection (p on the full grid, 0 at air cells).
+// Pressure::ApplyProjection (p on the full grid, 0 at air cells); p_out (or
+// null) receives a copy of p. need: the launches return while *need is 0.
 void launch_pressure_apply(hipStream_t s, Dims d, const double *phi, Faces frac,
                            const Faces *jump, const unsigned char *liquid, const double *p,
-                           MutFaces vel, int *err);
+                           MutFaces vel, int *err, double *p_out, const double *need);
 // MagneticField::BuildMatrix coefficients, matrix and AssembleRHS.
 void launch_magnetic_mu(hipStream_t s, Dims d, const MagGeom &g, const double *phi, double chi,
                         double band, MutFaces mu);
@@ -283,9 +288,11 @@ void launch_magnetic_mu(hipStream_t s, Dims d, const MagGeom &g, const double *p
 void launch_magnetic_assemble(hipStream_t s, Dims d, Faces mu, Faces hext, double spacing,
                               double *diag64, double *const cpl64[3], double *rhs,
                               float *diag32, float *const cpl32[3], int dirichlet = 0);
-// MagneticField::AssignTotalField.
+// MagneticField::AssignTotalField; copies of the potential to pot_out and of
+// the field to out (each null: none). need as above.
 void launch_magnetic_total_field(hipStream_t s, Dims d, double inv, const double *pot,
-                                 Faces hext, MutFaces htot);
+                                 Faces hext, MutFaces htot, double *pot_out, MutFaces out,
+                                 const double *need);
 // MagneticField::CalculateVertexPressures.
 void launch_vertex_pressures(hipStream_t s, Dims d, const MagGeom &g, Faces htot, double chi,
                              int nverts, const double *pos, const double *nrm, double *out);

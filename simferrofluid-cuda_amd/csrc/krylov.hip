@@ -43,7 +43,8 @@ __global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64
                                                        float *__restrict__ b32,
                                                        float *__restrict__ x0,
                                                        const float *__restrict__ diag32,
-                                                       float c0) {
+                                                       float c0, const double *need) {
+    if (need && *need == 0.0) return;
     int k, j, i0;
     cell_tile(cg, k, j, i0);
     const Strides s(d);
@@ -130,7 +131,8 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
                                                             float *__restrict__ b32,
                                                             float *__restrict__ x0,
                                                             const float *__restrict__ diag32,
-                                                            float c0) {
+                                                            float c0, const double *need) {
+    if (need && *need == 0.0) return;
     const Strides s(d);
     const size_t c = (size_t)blockIdx.x * kResidualCells + 2 * (size_t)flat_tid();
     double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
@@ -524,15 +526,18 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
 
 // p = z_k - beta_k p, x += alpha_k p for K iterations (numbers i0 .. i0 + K - 1,
 // their z at z + k stride), in the order and arithmetic of an update per
-// iteration. has_p: p0 holds the direction before them; store_p: it receives
-// the last one. zero_x: x starts from 0 (and every cell is written); else a
-// wavefront without active cells is skipped. z counts as 0 at inactive cells.
-template <int K>
+// iteration. K is k0 or, with `need` (the stop flag: the launch returns while
+// it is down), k0 plus the iterations of the batch before it. has_p: p0 holds
+// the direction before them; store_p: it receives the last one. zero_x: x
+// starts from 0 (and every cell is written); else a wavefront without active
+// cells is skipped. z counts as 0 at inactive cells.
 __global__ __launch_bounds__(kBlock) void k_fcg_flush(size_t n, const float *__restrict__ active,
                                                       const float *__restrict__ z, size_t stride,
                                                       double *__restrict__ p0, int has_p, int store_p,
-                                                      double *__restrict__ x, int zero_x, int i0,
-                                                      const KrylovScalars *__restrict__ sc) {
+                                                      double *__restrict__ x, int zero_x, int i0, int k0,
+                                                      const KrylovScalars *__restrict__ sc, const double *need) {
+    if (need && *need == 0.0) return;
+    const int K = min(need ? k0 + (int)sc->iters : k0, kRing);  // uniform
     const size_t c = (size_t)blockIdx.x * kUpdateCells + 2 * (size_t)flat_tid();
     const bool pair = c + 1 < n;
     bool act = c < n;
@@ -544,39 +549,31 @@ __global__ __launch_bounds__(kBlock) void k_fcg_flush(size_t n, const float *__r
         act = dg.x > 0.f || dg.y > 0.f;
     }
     if (zero_x ? !(c < n) : !__any(act)) return;
-    double alpha[K], beta[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        alpha[k] = sc->alpha[(i0 + k) % kCoefs];
-        beta[k] = sc->beta[(i0 + k) % kCoefs];
-    }
     if (pair) {
-        float2v zk[K];
+        float2v zk[kRing];
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            zk[k] = act ? ld_stream((const float2v *)(z + k * stride + c)) : float2v{0.f, 0.f};
-            if (!(dg.x > 0.f)) zk[k].x = 0.f;
-            if (!(dg.y > 0.f)) zk[k].y = 0.f;
-        }
+        for (int k = 0; k < kRing; k++)
+            zk[k] = k < K && act ? ld_stream((const float2v *)(z + k * stride + c)) : float2v{0.f, 0.f};
         double2v p = {0.0, 0.0}, xn = {0.0, 0.0};
         if (has_p) p = ld_stream((const double2v *)(p0 + c));
         if (!zero_x) xn = ld_stream((const double2v *)(x + c));
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            p.x = (double)zk[k].x - beta[k] * p.x;
-            p.y = (double)zk[k].y - beta[k] * p.y;
-            xn.x += alpha[k] * p.x;
-            xn.y += alpha[k] * p.y;
+        for (int k = 0; k < kRing; k++) {
+            if (k >= K) break;
+            const double alpha = sc->alpha[(i0 + k) % kCoefs], beta = sc->beta[(i0 + k) % kCoefs];
+            p.x = (double)(dg.x > 0.f ? zk[k].x : 0.f) - beta * p.x;
+            p.y = (double)(dg.y > 0.f ? zk[k].y : 0.f) - beta * p.y;
+            xn.x += alpha * p.x;
+            xn.y += alpha * p.y;
         }
         if (store_p) st_stream((double2v *)(p0 + c), p);
         st_stream((double2v *)(x + c), xn);
     } else if (c < n) {
         double p = has_p ? p0[c] : 0.0, xn = zero_x ? 0.0 : x[c];
-#pragma unroll
         for (int k = 0; k < K; k++) {
             const double zc = dg.x > 0.f ? (double)z[k * stride + c] : 0.0;
-            p = zc - beta[k] * p;
-            xn += alpha[k] * p;
+            p = zc - sc->beta[(i0 + k) % kCoefs] * p;
+            xn += sc->alpha[(i0 + k) % kCoefs] * p;
         }
         if (store_p) p0[c] = p;
         x[c] = xn;
@@ -602,13 +599,17 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(CellGrid cg, Dims d, Op32 A,
 // sums of the largest grids take few rounds of loads).
 constexpr int kFinalizeThreads = 1024;
 
-// Start of a batch of gated iterations: clear the stop flag and the iteration
-// count, set the threshold on ||r||^2 (one thread; no host copy needed).
-__global__ __launch_bounds__(64) void k_batch_begin(KrylovScalars *sc, double stop_rr, double stall_rr) {
+// Start of a batch of gated iterations: the threshold on ||r||^2 (tol2 times
+// the ||b||^2 of the solve's first residual), the counters and the stop flag
+// cleared (one thread; the host need not know ||b|| yet). first: nor has it
+// seen that residual, so the flag is up where no iteration is needed.
+__global__ __launch_bounds__(64) void k_batch_begin(KrylovScalars *sc, double tol2, double stall_rr, int first) {
     if (threadIdx.x == 0) {
-        sc->stop = 0.0;
-        sc->iters = 0.0;
+        const double stop_rr = tol2 * sc->bb;
+        sc->stop = first && (sc->bb == 0.0 || sc->rr <= stop_rr) ? 1.0 : 0.0;
         sc->stop_rr = stop_rr;
+        sc->iters = 0.0;
+        sc->ok = 0.0;
         sc->stall_rr = stall_rr;
         sc->stalled = 0.0;
     }
@@ -617,7 +618,8 @@ __global__ __launch_bounds__(64) void k_batch_begin(KrylovScalars *sc, double st
 __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned nb, int first, int iter,
                                                      const double *__restrict__ partials,
                                                      KrylovScalars *sc, const double *gate,
-                                                     KrylovScalars *host) {
+                                                     KrylovScalars *host, const double *need, double tol) {
+    if (need && *need == 0.0) return;
     // what the host reads after this launch (host: its pinned copy, or null)
     auto tell_host = [&] {
         if (!host) return;
@@ -626,6 +628,9 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
         host->active = sc->active;
         host->iters = sc->iters;
         host->stalled = sc->stalled;
+        host->stop = sc->stop;
+        host->check_rr = sc->check_rr;
+        host->ok = sc->ok;
     };
     if (gated(gate)) {
         if (flat_tid() == 0) tell_host();
@@ -644,6 +649,8 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(int op, unsigned 
         sc->rr = v[0];
         sc->bb = v[1];
         sc->active = v[2];
+        sc->check_rr = v[0];
+        sc->ok = sqrt(v[0] / v[1]) <= tol ? 1.0 : 0.0;
     } else if (op == FIN_MATVEC) {
         const Recurrence c = recurrence(v, first ? 0.0 : sc->pq[(iter + kCoefs - 1) % kCoefs], first);
         sc->zw = v[0];
@@ -690,7 +697,8 @@ __global__ __launch_bounds__(kStageThreads) void k_partials_stage(unsigned nb, u
 // `partials` holds the N sums of op for nb blocks ([q * nb + b]); the stage
 // writes its sums after them (reduction_partials leaves room).
 void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *partials, KrylovScalars *sc,
-              const double *gate = nullptr, KrylovScalars *host = nullptr) {
+              const double *gate = nullptr, KrylovScalars *host = nullptr, const double *need = nullptr,
+              double tol = 0.0) {
     const int N = op == FIN_UPDATE ? 1 : 3;
     if (nb > kStageMin) {
         const unsigned chunk = std::max(kStageChunk, (nb + kStageMaxBlocks - 1) / kStageMaxBlocks);
@@ -707,7 +715,7 @@ void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *
         nb = G;
     }
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalizeThreads), 0, st, op, nb, first, iter,
-                       partials, sc, gate, host);
+                       partials, sc, gate, host, need, tol);
     SFP_LAUNCH_CHECK();
 }
 
@@ -739,14 +747,14 @@ FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc) {
     return FoldArgs{partials + 3 * (size_t)matvec_blocks(d), update_blocks(d), sc};
 }
 
-void launch_batch_begin(hipStream_t st, KrylovScalars *sc, double stop_rr, double stall_rr) {
-    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(64), 0, st, sc, stop_rr, stall_rr);
+void launch_batch_begin(hipStream_t st, KrylovScalars *sc, double tol2, double stall_rr, bool first) {
+    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(64), 0, st, sc, tol2, stall_rr, first ? 1 : 0);
     SFP_LAUNCH_CHECK();
 }
 
 void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const double *x,
                        double *r, double *partials, KrylovScalars *sc, KrylovScalars *host, float *b32,
-                       float *x0, const float *diag32, float c0) {
+                       float *x0, const float *diag32, float c0, const double *need, double tol) {
     if (x0 && (!b32 || !diag32)) throw ArgError("launch_residual64: x0 needs b32 and the diagonal");
     if (matvec_flat(d)) {
         for (const void *a : {(const void *)A.diag, (const void *)A.cpl[0], (const void *)A.cpl[1],
@@ -756,16 +764,16 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
             throw ArgError("launch_residual64: b32, x0 or the diagonal not 8-byte aligned");
         const unsigned nb = (unsigned)((d.cells() + kResidualCells - 1) / kResidualCells);
         hipLaunchKernelGGL(k_residual64_flat, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials, b32,
-                           x0, diag32, c0);
+                           x0, diag32, c0, need);
         SFP_LAUNCH_CHECK();
-        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host);
+        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host, need, tol);
         return;
     }
     Launch L = cell_launch(d, kReducePlanes);
     hipLaunchKernelGGL(k_residual64, L.grid, L.block, 0, st, L.cg, d, A, b, x, r, partials, b32, x0,
-                       diag32, c0);
+                       diag32, c0, need);
     SFP_LAUNCH_CHECK();
-    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc, nullptr, host);
+    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc, nullptr, host, need, tol);
 }
 
 void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, const float *z,
@@ -819,29 +827,14 @@ void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc
 }
 
 void launch_fcg_flush(hipStream_t st, Dims d, const float *active, const float *z, size_t stride, int K, int i0,
-                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc) {
-    if (K < 1 || K > kRing) throw ArgError("launch_fcg_flush: bad iteration count");
+                      double *p, bool has_p, bool store_p, double *x, bool zero_x, const KrylovScalars *sc,
+                      const double *need) {
+    if (K < (need ? 0 : 1) || K > kRing) throw ArgError("launch_fcg_flush: bad iteration count");
     if ((has_p || store_p) && !p) throw ArgError("launch_fcg_flush: no direction");
     if ((uintptr_t)z % 8 || stride % 2 || (uintptr_t)active % 8 || (uintptr_t)p % 16 || (uintptr_t)x % 16)
         throw ArgError("launch_fcg_flush: vectors not aligned");
-    const dim3 grid(update_blocks(d)), block(kBlock);
-#define SFP_FLUSH(N)                                                                                   \
-    case N:                                                                                            \
-        hipLaunchKernelGGL(k_fcg_flush<N>, grid, block, 0, st, d.cells(), active, z, stride, p,        \
-                           has_p ? 1 : 0, store_p ? 1 : 0, x, zero_x ? 1 : 0, i0, sc);                 \
-        break;
-    switch (K) {
-        SFP_FLUSH(1)
-        SFP_FLUSH(2)
-        SFP_FLUSH(3)
-        SFP_FLUSH(4)
-        SFP_FLUSH(5)
-        SFP_FLUSH(6)
-        SFP_FLUSH(7)
-        SFP_FLUSH(8)
-    }
-#undef SFP_FLUSH
-    static_assert(kRing == 8, "one instance per iteration count");
+    hipLaunchKernelGGL(k_fcg_flush, dim3(update_blocks(d)), dim3(kBlock), 0, st, d.cells(), active, z, stride, p,
+                       has_p ? 1 : 0, store_p ? 1 : 0, x, zero_x ? 1 : 0, i0, K, sc, need);
     SFP_LAUNCH_CHECK();
 }
 

@@ -1307,7 +1307,7 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_flat(Dims df, Op64 Af, const
 // wavefront writes it, and the pivot's reciprocal; two buffers, so one barrier)
 // and the pivot column of a wavefront's own rows from lane kk's registers. One
 // block at 4^3 cells: 77 us with the matrix in LDS and 1024 threads (two
-// barriers and three LDS latencies a step), 20 us so.
+// barriers and three LDS latencies a step), 66 us so (3^3 cells 31 us).
 constexpr int kInvertThreads = 256;
 
 __global__ __launch_bounds__(kInvertThreads) void k_coarse_invert(Dims d, Op64 A, float *ainv) {

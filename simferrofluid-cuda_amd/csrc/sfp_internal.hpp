@@ -149,7 +149,7 @@ struct Level {
 // Directions of FCG iterations kept as their FP32 preconditioned residuals z
 // until the solution is brought up to date (see launch_fcg_flush), and the
 // iterations whose coefficients are kept.
-constexpr int kRing = 8, kCoefs = 2 * kRing;
+constexpr int kRing = 12, kCoefs = 2 * kRing;
 
 // Scalars of the flexible-CG recurrences, resident on the device.
 struct KrylovScalars {
@@ -161,6 +161,9 @@ struct KrylovScalars {
     // update, and every gated kernel of later iterations then returns at once;
     // `iters` counts the updates done
     double stop, iters, stop_rr;
+    // ||b - A x||^2 of the last residual formed, and whether it met the
+    // tolerance (a batch's own check: see System::fcg)
+    double check_rr, ok;
     // learned preconditioner in a batch: an update whose ||r||^2 exceeds
     // stall_rr times the previous one raises `stalled` and `stop` (0: off)
     double stall_rr, stalled;

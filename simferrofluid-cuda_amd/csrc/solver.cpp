@@ -581,7 +581,7 @@ const float *System::restrict_smoothed(Workspace &ws, const SolverConfig &cfg, c
     return learned_cycle(ws, cfg, r64, kCycleRestrictOnly);
 }
 
-SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm) {
+SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm, const Finish &finish) {
     SolveInfo info;
     info.precond_used = cfg.precond;
     const hipStream_t st = ws.stream;
@@ -610,22 +610,13 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     float c0 = first_coef(learned);
     launch_residual64(st, d, A, rhs_.p, warm ? x_.p : nullptr, r_.p, ws.partials.p,
                       ws.scalars.p, ws.host_sc, b32, x0, lv_[level].diag32.p, c0);
-    ws.wait();
-    info.active = (long long)ws.host_sc->active;
-    if (*ws.host_err) {
-        info.input_error = true;
-        return info;
-    }
-    const double bb = ws.host_sc->bb;
-    if (bb == 0.0) {  // zero right-hand side: x = 0
-        SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));
-        info.converged = true;
-        info.rel = 0.0;
-        return info;
-    }
-    double rel = std::sqrt(ws.host_sc->rr / bb);
+    // The host reads the first residual (||b||, the system's size and its input
+    // errors) with the first batch's, which the device gates where no
+    // iteration is needed.
+    bool known = false;
+    double bb = 0.0, rel = 0.0;
     bool first = true;
-    bool checked = true;  // rel is a true residual
+    bool checked = false;  // rel is a true residual
     const double cells = (double)n;
     if (learned) prepare_learned(ws);
     bool b_ready = b32 != nullptr;  // lv_[level].b holds r rounded (and lv_[level].x0 its first iterate)
@@ -634,6 +625,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     // and iterations enqueued behind a stall would still launch every
     // kernel of the learned cycle (each returning at once)
     int next_batch = learned ? 1 : kBatch;
+    bool predicted = false;  // next_batch is expected to reach the tolerance
     // iterations whose z is in the ring and whose alpha p is not yet in x, and
     // the number of the next iteration (its scalars' place)
     int pending = 0, iter = 0;
@@ -649,6 +641,13 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
         }
         pending = 0;
     };
+    // the recurrence restarts from the true residual
+    auto restart = [&] {
+        launch_residual64(st, d, A, rhs_.p, x_.p, r_.p, ws.partials.p, ws.scalars.p, nullptr, b32, x0,
+                          lv_[level].diag32.p, c0);
+        first = true;
+        b_ready = b32 != nullptr;
+    };
     // small grids: the reductions' partials are added by the launches that
     // need the sums (the update, and the next cycle's first) instead of
     // finalize launches between
@@ -656,7 +655,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     ws.z_level = level;
     info.precond_used = learned ? 1 : (cfg.precond == 1 ? 0 : cfg.precond);
     while (true) {
-        if (rel <= cfg.tol) {
+        if (known && rel <= cfg.tol) {
             if (checked) break;
             // recursive residual reached tol: recompute its norm from x in
             // FP64 (the sums only), and restart from the true residual if the
@@ -666,27 +665,27 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             ws.wait();
             rel = std::sqrt(ws.host_sc->rr / bb);
             checked = true;
-            if (rel > cfg.tol) {
-                launch_residual64(st, d, A, rhs_.p, x_.p, r_.p, ws.partials.p,
-                                  ws.scalars.p, nullptr, b32, x0, lv_[level].diag32.p, c0);
-                first = true;
-                b_ready = b32 != nullptr;
-            }
+            if (rel > cfg.tol) restart();
             continue;
         }
-        if (info.iterations >= cfg.max_iters) break;
-        // Up to kBatch iterations are enqueued before the host looks at the
-        // residual (after the first batch, as many as the residual's rate of
-        // decrease predicts are left): the update's finalize raises `stop` on
-        // the device once ||r|| <= tol ||b||, or (learned preconditioner)
-        // once an iteration reduced ||r|| by less than stall_ratio, and every
-        // kernel of the remaining iterations of the batch then returns at
-        // once (profiled launches among them are dropped from the timings).
-        if (pending == kRing) bring_x_up_to_date(true);
-        const int batch = std::min({next_batch, cfg.max_iters - info.iterations, kRing - pending});
-        if (batch > 1) {
-            launch_batch_begin(st, ws.scalars.p, cfg.tol * cfg.tol * bb,
-                               learned ? cfg.stall_ratio * cfg.stall_ratio : 0.0);
+        if (known && info.iterations >= cfg.max_iters) break;
+        // Iterations are enqueued in batches (the first kBatch, then as many
+        // as the residual's rate of decrease predicts are left) before the host
+        // looks at the residual: the update's finalize raises `stop` on the
+        // device once ||r|| <= tol ||b||, or (learned preconditioner) once an
+        // iteration reduced ||r|| by less than stall_ratio, and every kernel
+        // of the remaining iterations of the batch then returns at once
+        // (profiled launches among them are dropped from the timings).
+        if (pending + next_batch > kRing) bring_x_up_to_date(true);
+        const int batch = std::min(next_batch, cfg.max_iters - info.iterations);
+        // Behind a batch expected to be the last, the check above and what
+        // follows the solve are enqueued too, behind the stop flag and the
+        // check's own result: one wait instead of three (each leaves the GPU
+        // idle for some 20 us).
+        const bool check_here = predicted && finish && !learned && !profiling && batch == next_batch;
+        if (batch > 0) {
+            launch_batch_begin(st, ws.scalars.p, cfg.tol * cfg.tol,
+                               learned ? cfg.stall_ratio * cfg.stall_ratio : 0.0, !known);
             ws.gate = &ws.scalars.p->stop;
         }
         for (int it = 0; it < batch; it++) {
@@ -734,28 +733,79 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             first = false;
             b_ready = b32 != nullptr;
         }
-        if (fold) launch_fcg_norm(st, d, ws.partials.p, ws.scalars.p, ws.gate, ws.host_sc);
-        ws.wait();
-        const bool stalled = batch > 1 && ws.host_sc->stalled != 0.0;
+        if (fold && batch > 0) launch_fcg_norm(st, d, ws.partials.p, ws.scalars.p, ws.gate, ws.host_sc);
         ws.gate = nullptr;
-        const int done = batch > 1 ? (int)ws.host_sc->iters : 1;
+        if (check_here) {
+            const double *stop = &ws.scalars.p->stop;
+            launch_fcg_flush(st, d, flags, zring_.p, zring_stride_, pending, iter - pending, p_.p, has_p, false,
+                             x_.p, zero_x, ws.scalars.p, stop);
+            launch_residual64(st, d, A, rhs_.p, x_.p, nullptr, ws.partials.p, ws.scalars.p, ws.host_sc, nullptr,
+                              nullptr, nullptr, 0.f, stop, cfg.tol);
+            finish(&ws.scalars.p->ok);
+        }
+        ws.wait();
+        const KrylovScalars &h = *ws.host_sc;
+        if (!known) {
+            known = true;
+            info.active = (long long)h.active;
+            // (launches that returned at once are no measurement)
+            if (profiling && (h.iters == 0.0 || *ws.host_err))
+                for (auto &t : ws.timers) t.used = 0;
+            if (*ws.host_err) {
+                info.input_error = true;
+                return info;
+            }
+            bb = h.bb;
+            if (bb == 0.0) {  // zero right-hand side: x = 0
+                SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));
+                info.converged = true;
+                info.rel = 0.0;
+                info.precond_used = cfg.precond;
+                return info;
+            }
+            rel = std::sqrt(h.check_rr / bb);
+            checked = true;
+            if (batch == 0) continue;
+        }
+        const bool stalled = h.stalled != 0.0;
+        const int done = (int)h.iters;
         pending += done;
         iter += done;
         info.iterations += done;
         if (!learned && cfg.precond == 1 && info.precond_used == 1) info.fallback += done;
         const double prev = rel;
-        rel = std::sqrt(ws.host_sc->rr / bb);
-        checked = false;
-        // the next batch: as many iterations as the last ones' mean residual
-        // reduction predicts are left (iterations enqueued past convergence
-        // still launch every kernel, which returns at once)
+        if (done > 0) {
+            rel = std::sqrt(h.rr / bb);
+            checked = false;
+        }
+        if (check_here && h.stop != 0.0) {  // the flush and the check have run
+            zero_x = has_p = false;
+            pending = 0;
+            rel = std::sqrt(h.check_rr / bb);
+            checked = true;
+            info.finished = h.ok != 0.0;
+            if (info.finished) break;
+            restart();
+            continue;
+        }
+        // The next batch: as many iterations as the last ones' mean residual
+        // reduction predicts are left. Enqueued past convergence an iteration
+        // still launches every kernel, which returns at once: some 10 launches
+        // or 25 us where the levels run in tiles, 45 launches or 110 us on
+        // larger grids (a magnetic 256^3 solve predicts 7 where 4 are left),
+        // so there a batch is kBatch at most and the host waits again. A wait
+        // costs some 20 us, as do the check and the Finish behind a batch that
+        // then needs another.
         next_batch = kBatch;
+        predicted = false;
         if (done > 0 && rel > 0.0 && rel < prev) {
             const double rate = std::pow(rel / prev, 1.0 / done);
             const double left = std::log(cfg.tol / rel) / std::log(rate);
-            if (left < kBatch) next_batch = std::max(1, (int)std::ceil(left));
+            const int cap = small_grid(d) ? kRing : kBatch;
+            if (left <= cap) next_batch = std::max(1, (int)std::ceil(left));
+            predicted = left <= 1.5 * next_batch;
         }
-        if (learned && (stalled || (batch == 1 && rel > cfg.stall_ratio * prev))) {
+        if (learned && (stalled || (batch == 1 && done == 1 && rel > cfg.stall_ratio * prev))) {
             // fall back to the plain V-cycle, restarting the recurrence from
             // the current iterate (a direction built with the other
             // preconditioner slows the V-cycle's iterations down); the first
@@ -768,6 +818,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             if (c0_plain != c0) b_ready = false;
             c0 = c0_plain;
             next_batch = kBatch;
+            predicted = false;
         }
     }
     bring_x_up_to_date(false);

@@ -7,11 +7,13 @@
 #include "unet.hpp"
 
 #include <array>
+#include <functional>
 #include <vector>
 
 namespace sfp {
 
-// FCG iterations enqueued between two reads of the residual on the host.
+// FCG iterations enqueued before the host first reads the residual (and later
+// where their number cannot be predicted).
 constexpr int kBatch = 4;
 
 struct SolverConfig {
@@ -147,7 +149,12 @@ struct SolveInfo {
     int precond_used = 0;
     long long active = 0;  // rows of the system
     bool input_error = false;  // the assembly before the solve raised it: nothing was solved
+    bool finished = false;     // the solve's Finish has run
 };
+
+// Enqueues what follows a solve (the velocity or field update) behind a flag:
+// its launches must return while *need is 0.
+using Finish = std::function<void(const double *need)>;
 
 class System {
   public:
@@ -180,14 +187,16 @@ class System {
     const float *restrict_smoothed(Workspace &ws, const SolverConfig &cfg, const double *r64);
     // Features of the first coarse level into f3 ([cells][3] FP32).
     void learned_features(Workspace &ws, float *f3);
-    // Flexible CG on A x = rhs; x holds the start when warm.
-    SolveInfo solve(Workspace &ws, const SolverConfig &cfg, bool warm) {
-        return fcg(ws, cfg, 0, warm);
+    // Flexible CG on A x = rhs; x holds the start when warm. `finish` (or
+    // null) is enqueued behind the batch expected to be the last, to run there
+    // if that meets the tolerance; SolveInfo::finished tells.
+    SolveInfo solve(Workspace &ws, const SolverConfig &cfg, bool warm, const Finish &finish = nullptr) {
+        return fcg(ws, cfg, 0, warm, finish);
     }
     // Flexible CG with level `level`'s FP64 operator and the V-cycle from that
     // level down, on the first cells of rhs/x (from x = 0).
     SolveInfo solve_level(Workspace &ws, const SolverConfig &cfg, int level) {
-        return fcg(ws, cfg, level, false);
+        return fcg(ws, cfg, level, false, nullptr);
     }
     // The operator is a Neumann problem made definite by one eliminated cell
     // (the magnetic potential's pin at cell 0). Its coarse levels then scale
@@ -203,7 +212,7 @@ class System {
     enum Cycle { kCycleLearned, kCycleSmooth, kCycleRestrictOnly };
     float *learned_cycle(Workspace &ws, const SolverConfig &cfg, const double *r64, Cycle c);
     float *post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur, const float *e);
-    SolveInfo fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm);
+    SolveInfo fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm, const Finish &finish);
     float *vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r64, bool x0_ready = false);
     // levels l .. coarsest in one launch (vlevel with r64 null), or null
     // where the tail does not apply

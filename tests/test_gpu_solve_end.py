@@ -1,0 +1,87 @@
+"""GPU test of how a solve ends: the check of its true residual, the velocity
+or field update and the caller's copies are enqueued behind the batch that is
+expected to converge, and run by the host's decision everywhere else. With the
+kernel timings on, a solve never does the former."""
+import numpy as np
+import pytest
+import torch
+
+import sfp
+from sfp import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def passes(sc, kind, profiled, params):
+    """Two passes (the second from a warm start: Reproject, or the next
+    magnetic solve of the same scene), each (arrays, stats)."""
+    out = []
+    with sfp.Context.for_scene(sc, **params) as ctx:
+        ctx.profile(profiled)
+        for warm in (False, True):
+            if kind == "pressure":
+                vel, x, st = ctx.pressure_project(sc, reproject=warm)
+            else:
+                x, vel, st = ctx.magnetic_solve(sc)
+            out.append(([x, *vel], st))
+    return out
+
+
+# a small grid (batches of any length) and a larger one (batches of four); a
+# tolerance met at once, within, at the end of and after the first batch, and
+# never; as many iterations as allowed, and none
+@pytest.mark.parametrize("kind,n", [("pressure", (19, 21, 23)), ("magnetic", (24, 20, 28)),
+                                    ("magnetic", (90, 88, 86))])
+@pytest.mark.parametrize("tol,max_iters", [(0.9, 50), (1e-2, 50), (1e-4, 50), (1e-8, 50), (1e-8, 6),
+                                           (1e-8, 0), (1e-300, 14)])
+def test_ends_alike(kind, n, tol, max_iters):
+    """The two ways run the same kernels in the same order: equal results."""
+    print(f"[case] solve end {kind} {n} {tol} {max_iters}", flush=True)
+    sc = scenes.random_pressure_scene(n, 9) if kind == "pressure" else scenes.magnetic_scene(n, seed=9)
+    params = dict(tol=tol, max_iters=max_iters)
+    for (got, st), (want, st0) in zip(passes(sc, kind, False, params), passes(sc, kind, True, params)):
+        for key in ("iterations", "converged", "rel_residual", "unknowns"):
+            assert st[key] == st0[key], key
+        assert st["iterations"] <= max_iters and st["converged"] == (st["rel_residual"] <= tol)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, b)
+
+
+def test_zero_right_hand_side_and_shared_outputs():
+    """A zero field gives a zero potential from a warm start too; outputs that
+    lie over inputs get the values of separate ones."""
+    print("[case] solve end, zero right-hand side, shared outputs", flush=True)
+    sc = scenes.magnetic_scene((24, 20, 28), seed=9)
+    ptr = lambda ts: [t.data_ptr() for t in ts]  # noqa: E731
+    dev = lambda a: torch.tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")  # noqa: E731
+    with sfp.Context.for_scene(sc, tol=1e-8) as ctx:
+        want_x, want_f, _ = ctx.magnetic_solve(sc)
+        phi = dev(sc["phi"])
+        field = [dev(h) for h in sc["hext"]]
+        zero = [torch.zeros_like(h) for h in field]
+        x = torch.full_like(phi, 3.0)
+        torch.cuda.synchronize()
+        st = ctx.magnetic_solve_device(phi.data_ptr(), ptr(zero), sc["chi"], sc["band"], x.data_ptr())
+        assert st["iterations"] == 0 and st["converged"] and not x.any()
+        ctx.reset_warm_start()
+        # the field over the external field, the potential over its first array
+        ctx.magnetic_solve_device(phi.data_ptr(), ptr(field), sc["chi"], sc["band"], None, ptr(field))
+        for a, b in zip(field, want_f):
+            np.testing.assert_array_equal(a.cpu().numpy(), b)
+        field = [dev(h) for h in sc["hext"]]
+        torch.cuda.synchronize()
+        ctx.reset_warm_start()
+        ctx.magnetic_solve_device(phi.data_ptr(), ptr(field), sc["chi"], sc["band"], field[0].data_ptr())
+        np.testing.assert_array_equal(field[0].flatten()[:phi.numel()].cpu().numpy(), want_x.flatten())
+    sc = scenes.random_pressure_scene((19, 21, 23), 9)
+    with sfp.Context.for_scene(sc, tol=1e-8) as ctx:
+        want_v, want_p, _ = ctx.pressure_project(sc)
+        phi, frac, us = dev(sc["phi"]), [dev(a) for a in sc["fraction"]], [dev(a) for a in sc["solid_velocity"]]
+        vel = [dev(a) for a in sc["velocity"]]
+        jump = [dev(a) for a in sc["jump"]] if sc.get("jump") is not None else None
+        torch.cuda.synchronize()
+        ctx.pressure_project_device(ptr(vel), phi.data_ptr(), ptr(frac), ptr(us),
+                                    None if jump is None else ptr(jump), sc["vol_error"], phi.data_ptr())
+        np.testing.assert_array_equal(phi.cpu().numpy(), want_p)
+        for a, b in zip(vel, want_v):
+            np.testing.assert_array_equal(a.cpu().numpy(), b)
