@@ -1303,18 +1303,21 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_flat(Dims df, Op64 Af, const
 //
 // The 64 pivot steps are a serial chain, so what counts is the length of one:
 // the matrix is in registers, wavefront w of four holding rows 16 w .. 16 w +
-// 15 and lane c column c. A step takes the pivot row through LDS (its
-// wavefront writes it, and the pivot's reciprocal; two buffers, so one barrier)
-// and the pivot column of a wavefront's own rows from lane kk's registers. One
-// block at 4^3 cells: 77 us with the matrix in LDS and 1024 threads (two
-// barriers and three LDS latencies a step), 66 us so (3^3 cells 31 us).
+// 15 and lane c column c. A step reads the pivot row and the pivot's
+// reciprocal from LDS and the pivot column of its own rows from lane kk's
+// registers; the wavefront with the next pivot row updates that one first and
+// publishes it (two buffers, one barrier), so its division overlaps the other
+// rows' updates. In column kk the row counts as 1 and the matrix as 0, which
+// leaves one product and one sum per element whatever its place. One block at
+// 4^3 cells: 36 us (66 with the division between the rows' updates and the
+// barrier and a choice of four forms per element; 77 with the matrix in LDS).
 constexpr int kInvertThreads = 256;
 
 __global__ __launch_bounds__(kInvertThreads) void k_coarse_invert(Dims d, Op64 A, float *ainv) {
     constexpr int S = kMaxCoarse, R = S / (kInvertThreads / 64);  // rows per wavefront
     static_assert(S == 64 && R == 16, "lane c holds column c");
     __shared__ double M[S * S];
-    __shared__ double rowk[2][S], pivk[2][2];  // the pivot row; the pivot and its reciprocal
+    __shared__ double rowk[2][S], pivk[2];  // the pivot row; the pivot's reciprocal, 0 for a dropped one
     const int n = (int)d.cells();
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const Strides s(d);
@@ -1343,37 +1346,40 @@ __global__ __launch_bounds__(kInvertThreads) void k_coarse_invert(Dims d, Op64 A
         const i2 h = __builtin_bit_cast(i2, v);
         return __builtin_bit_cast(double, i2{__builtin_amdgcn_readlane(h.x, l), __builtin_amdgcn_readlane(h.y, l)});
     };
+    auto publish = [&](double row, int kk) {
+        const double p = at_lane(row, kk);
+        rowk[kk & 1][lane] = row;
+        const double pinv = fabs(p) <= tiny ? 0.0 : 1.0 / p;
+        if (lane == 0) pivk[kk & 1] = pinv;
+    };
+    if (wave == 0) publish(a[0], 0);
+    __syncthreads();
     for (int w = 0; w < S / R; w++) {
 #pragma unroll
         for (int ki = 0; ki < R; ki++) {
             const int kk = R * w + ki;
             if (kk >= n) break;  // uniform over the block
-            const int buf = ki & 1;
-            if (wave == w) {
-                const double p = at_lane(a[ki], kk);
-                rowk[buf][lane] = a[ki];
-                if (lane == 0) {
-                    pivk[buf][0] = p;
-                    pivk[buf][1] = 1.0 / p;
-                }
+            const int kn = (ki + 1) % R;  // the next pivot row's place in its wavefront
+            const bool next = wave == (ki + 1 < R ? w : w + 1) && kk + 1 < n;
+            const double pinv = pivk[kk & 1], row = rowk[kk & 1][lane];
+            const double rk = lane == kk ? 1.0 : row;
+            auto step = [&](double v) {
+                const double ck = at_lane(v, kk);
+                const double v0 = lane == kk ? 0.0 : v;
+                return pinv == 0.0 ? v0 : v0 - ck * rk * pinv;
+            };
+            if (next) {
+                a[kn] = step(a[kn]);
+                publish(a[kn], kk + 1);
             }
-            __syncthreads();
-            const double p = pivk[buf][0], pinv = pivk[buf][1], rk = rowk[buf][lane];
-            const bool drop = fabs(p) <= tiny;
+            // (the pivot row itself, and the next one where it is done, are put
+            // right after the loop)
+            const double done = a[kn];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const double ck = at_lane(a[r], kk);
-                const bool row = wave == w && r == ki;
-                double v;
-                if (drop) {
-                    v = row || lane == kk ? 0.0 : a[r];
-                } else if (row) {
-                    v = lane == kk ? pinv : rk * pinv;
-                } else {
-                    v = lane == kk ? -ck * pinv : a[r] - ck * rk * pinv;
-                }
-                a[r] = v;
-            }
+            for (int r = 0; r < R; r++) a[r] = step(a[r]);
+            if (next) a[kn] = done;
+            if (wave == w) a[ki] = pinv == 0.0 ? 0.0 : rk * pinv;
+            __syncthreads();
         }
     }
 #pragma unroll
