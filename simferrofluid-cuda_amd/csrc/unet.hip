@@ -437,122 +437,204 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
     }
 }
 
-// Weight gradient partials as an implicit GEMM on MFMA: for tap blockIdx.y
-// and voxel chunk blockIdx.x, part[chunk][tap][cout][cin] =
-// sum_v g[v][cout] x[v + tap][cin] (M = output channels, N = input channels,
-// K = the chunk's voxels; BF16 products, exact in FP32, FP32 accumulation);
-// the centre-tap blocks also store bias partials bpart[chunk][cout] =
-// sum_v g[v][cout]. Every K step stages 128 voxels of g and of the shifted
-// x in LDS, transposed (channel-major, 8 consecutive voxels per 16-byte
-// fragment); wavefront w takes the step's voxels 32 w .. 32 w + 31 for every
-// output tile, and the four partial sets are added in a fixed order at the
-// end, so the result does not depend on timing. Input channels below 16 are
-// padded with zeros.
+// Weight gradient partials as an implicit GEMM on MFMA (M = 16 output channels,
+// N = 16 input channels, K = voxels; BF16 products, exact in FP32, FP32
+// accumulation): part[chunk][tile][tap][co][ci] = sum_v g[v][co] x[v + tap][ci]
+// for the voxels of a chunk and the channel tile blockIdx.y; "tap" 27 has x = 1
+// and gives the bias sums.
+//
+// A block stages one plane of a column (yt x zt voxels, up to kDwVoxels) of g
+// and three planes of x with their one-voxel frame in LDS, as the tensors lie
+// (16 channels of a voxel together), and marches along x, a plane's loads in
+// flight while the one before is used: x is read from memory 1.3 times and once
+// more per run instead of 27 times. Both MFMA operands need 8 voxels of one
+// channel per lane; ds_read_b64_tr_b16 transposes on the way (a 16-lane group
+// reads 4 voxels x 16 channels, lane n gets channel n's 4), so a tap is an
+// address offset. The 28 taps are split over 7 wavefronts, which all pass over
+// every voxel: no sum over wavefronts, 16 accumulator registers each. What
+// bounds it is LDS reads, 68 of 512 B per 32 voxels for 28 MFMAs. Voxels past
+// the volume, or past the column in its last 32, read the zero row in both.
+//
+// 32^3 x 8 crops, all ten convolutions: 127 us (607 with a block per tap and
+// both tensors transposed by 2-byte LDS stores), their partials' sums 15 us in
+// one launch (305 in twenty).
+constexpr int kDwVoxels = 256;  // voxels of a column plane
+constexpr int kDwFramed = 340;  // the most with the frame: sides up to 32, product up to 256
+constexpr int kDwThreads = 448, kDwTaps = 28;
+constexpr int kDwPart = kDwTaps * 256;  // floats of a partial tile
+
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+
 template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void k_conv_dw(const uint16_t *__restrict__ x,
-                                                 const uint16_t *__restrict__ g, int B, int X,
-                                                 int Y, int Z, int chunk_len,
-                                                 float *__restrict__ part,
-                                                 float *__restrict__ bpart) {
-    constexpr int KV = 128;                       // voxels per K step (4 x 32)
-    constexpr int CINP = CIN < 16 ? 16 : CIN;     // padded to the MFMA's 16 columns
-    constexpr int MB = COUT / 16, NB = CINP / 16, T = MB * NB;
-    constexpr int PAIRS = CIN * COUT;
-    __shared__ __attribute__((aligned(16))) uint16_t sg[COUT][KV];
-    __shared__ __attribute__((aligned(16))) uint16_t sx[CINP][KV];
-    __shared__ float red[4][T][4][64];            // each wavefront's partial tiles
-    const int tap = blockIdx.y;
-    const int dx = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
-    const size_t nv = (size_t)B * X * Y * Z;
-    const size_t v0 = (size_t)blockIdx.x * chunk_len;
-    const size_t v1 = v0 + chunk_len < nv ? v0 + chunk_len : nv;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int gq = lane >> 4, r16 = lane & 15;
-    v4f acc[T];
+__global__ __launch_bounds__(kDwThreads) void k_conv_dw(const uint16_t *__restrict__ x,
+                                                        const uint16_t *__restrict__ g, DwPlan p,
+                                                        float *__restrict__ part) {
+    constexpr int NB = CIN < 16 ? 1 : CIN / 16;
+    constexpr int kZero = 3 * kDwFramed;  // the zero row
+    __shared__ __attribute__((aligned(16))) uint16_t sx[kZero + 1][16];
+    __shared__ __attribute__((aligned(16))) uint16_t sg[kDwVoxels][16];
+    typedef __attribute__((address_space(3))) v4s *lds4;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int mb = (int)blockIdx.y / NB, nb = (int)blockIdx.y % NB;
+    const int fz = p.zt + 2, framed = (p.yt + 2) * fz, voxels = p.yt * p.zt;
+    // this lane's voxels in a unit of 32: kq and kq + 16 (any assignment of
+    // voxels to K will do, as long as both operands have it)
+    const int kq = 4 * (lane >> 4) + ((lane & 15) >> 2), pc = 4 * (lane & 3);
+    if (tid < 16) sx[kZero][tid] = 0;
+    // pieces of 16 bytes: (voxel, half) = (e / 2, e % 2)
+    constexpr int RX = (2 * kDwFramed + kDwThreads - 1) / kDwThreads;
+    constexpr int RG = (2 * kDwVoxels + kDwThreads - 1) / kDwThreads;
+    uint4 rx[RX], rg[RG];
+    v4f acc[4];
 #pragma unroll
-    for (int t = 0; t < T; t++) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    float bacc = 0.f;
-    if (CINP > CIN) {  // the padding columns stay zero
-        for (int e = tid; e < (CINP - CIN) * KV; e += 256) sx[CIN + e / KV][e % KV] = 0;
-    }
-    for (size_t vb = v0; vb < v1; vb += KV) {
-        __syncthreads();  // the previous step's fragments are read
-        // g: 8 channels (16 bytes) of one voxel per thread and round
-        for (int e = tid; e < KV * (COUT / 8); e += 256) {
-            const int vi = e / (COUT / 8), q = e - vi * (COUT / 8);
-            const size_t v = vb + vi;
-            uint4 u = make_uint4(0, 0, 0, 0);
-            if (v < v1) u = *reinterpret_cast<const uint4 *>(g + v * COUT + 8 * q);
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&u);
+    for (int j = 0; j < 4; j++) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+    const uint4 none = make_uint4(0, 0, 0, 0);
+    for (int item = blockIdx.x; item < p.items; item += gridDim.x) {
+        const int col = item / p.segs, seg = item - col * p.segs;
+        const int tz = col % p.nzt, ty = (col / p.nzt) % p.nyt, bb = col / (p.nzt * p.nyt);
+        const int y0 = ty * p.yt, z0 = tz * p.zt;
+        const int xa = seg * p.seg, xe = min(xa + p.seg, p.X);
+        auto load_x = [&](int plane) {
+            const uint16_t *px = x + (size_t)(bb * (long long)p.X + plane) * p.Y * p.Z * CIN + 16 * nb;
 #pragma unroll
-            for (int c = 0; c < 8; c++) sg[8 * q + c][vi] = h[c];
-        }
-        // x at the tapped voxel (zero outside the volume)
-        for (int e = tid; e < KV * (CIN / 8); e += 256) {
-            const int vi = e / (CIN / 8), q = e - vi * (CIN / 8);
-            const size_t v = vb + vi;
-            uint4 u = make_uint4(0, 0, 0, 0);
-            if (v < v1) {
-                size_t r = v;
-                const int z = (int)(r % Z);
-                r /= Z;
-                const int y = (int)(r % Y);
-                r /= Y;
-                const int xx = (int)(r % X);
-                const size_t bb = r / X;
-                const int jx = xx + dx, jy = y + dy, jz = z + dz;
-                if (jx >= 0 && jy >= 0 && jz >= 0 && jx < X && jy < Y && jz < Z)
-                    u = *reinterpret_cast<const uint4 *>(x + (((bb * X + jx) * Y + jy) * Z + jz) * CIN + 8 * q);
+            for (int r = 0; r < RX; r++) {
+                const int e = tid + r * kDwThreads, vi = e >> 1;
+                const int yy = (int)(((unsigned)vi * p.magic_f) >> 16), zz = vi - yy * fz;
+                const int gy = y0 + yy - 1, gz = z0 + zz - 1;
+                rx[r] = none;
+                if (vi < framed && (CIN >= 16 || !(e & 1)) && plane >= 0 && plane < p.X && gy >= 0 && gy < p.Y &&
+                    gz >= 0 && gz < p.Z)
+                    rx[r] = *reinterpret_cast<const uint4 *>(px + ((size_t)gy * p.Z + gz) * CIN + 8 * (e & 1));
             }
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&u);
+        };
+        auto store_x = [&](int plane) {
+            const int base = ((plane + 1) % 3) * kDwFramed;
 #pragma unroll
-            for (int c = 0; c < 8; c++) sx[8 * q + c][vi] = h[c];
-        }
-        __syncthreads();
-        // this wavefront's 32 voxels of the step: k = 32 wave + 8 gq .. + 7
-        const int k0 = 32 * wave + 8 * gq;
-        v8bf af[MB], bf[NB];
+            for (int r = 0; r < RX; r++) {
+                const int e = tid + r * kDwThreads;
+                if (e >> 1 < framed) *reinterpret_cast<uint4 *>(&sx[base + (e >> 1)][8 * (e & 1)]) = rx[r];
+            }
+        };
+        auto load_g = [&](int plane) {
+            const uint16_t *pg = g + (size_t)(bb * (long long)p.X + plane) * p.Y * p.Z * COUT + 16 * mb;
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-            af[mb] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(&sg[16 * mb + r16][k0]));
+            for (int r = 0; r < RG; r++) {
+                const int e = tid + r * kDwThreads, vi = e >> 1;
+                const int yy = (int)(((unsigned)vi * p.magic) >> 16), zz = vi - yy * p.zt;
+                const int gy = y0 + yy, gz = z0 + zz;
+                rg[r] = none;
+                if (vi < voxels && gy < p.Y && gz < p.Z)
+                    rg[r] = *reinterpret_cast<const uint4 *>(pg + ((size_t)gy * p.Z + gz) * COUT + 8 * (e & 1));
+            }
+        };
+        auto store_g = [&] {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-            bf[nb] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(&sx[16 * nb + r16][k0]));
+            for (int r = 0; r < RG; r++) {
+                const int e = tid + r * kDwThreads;
+                if (e < 2 * kDwVoxels) *reinterpret_cast<uint4 *>(&sg[e >> 1][8 * (e & 1)]) = rg[r];
+            }
+        };
+        // the corner (tap 0) of each of this lane's voxels in a staged plane
+        int corner[kDwVoxels / 32][2];
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
+        for (int u = 0; u < kDwVoxels / 32; u++)
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-                acc[mb * NB + nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mb], bf[nb], acc[mb * NB + nb], 0, 0, 0);
-        if (tap == 13 && tid < COUT) {
-            float sb = 0.f;
-            for (int i = 0; i < KV; i++) sb += bf2f(sg[tid][i]);
-            bacc += sb;
+            for (int h = 0; h < 2; h++) {
+                const int q = 32 * u + kq + 16 * h;
+                const int yy = (int)(((unsigned)q * p.magic) >> 16), zz = q - yy * p.zt;
+                const bool in = q < voxels && y0 + yy < p.Y && z0 + zz < p.Z;
+                corner[u][h] = in ? (yy * fz + zz) * 16 + pc : -1;
+            }
+        load_x(xa - 1);
+        __syncthreads();  // the item before is done with LDS
+        store_x(xa - 1);
+        load_x(xa);
+        store_x(xa);
+        load_x(xa + 1);
+        load_g(xa);
+        for (int xp = xa; xp < xe; xp++) {
+            __syncthreads();  // the plane before is done with
+            store_x(xp + 1);
+            store_g();
+            __syncthreads();
+            if (xp + 1 < xe) {
+                load_x(xp + 2);
+                load_g(xp + 1);
+            }
+            int off[4];  // this wavefront's taps: the plane's slot and the offset in it (uniform)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int t = 4 * wave + j, dx = t / 9, dy = (t / 3) % 3, dz = t % 3;
+                off[j] = (((xp + dx) % 3) * kDwFramed + dy * fz + dz) * 16;
+            }
+#pragma unroll
+            for (int u = 0; u < kDwVoxels / 32; u++) {
+                if (32 * u >= voxels) break;  // uniform
+                auto read = [](const uint16_t *a, const uint16_t *b) {
+                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)a);
+                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)b);
+                    return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                };
+                const uint16_t *sgu = &sg[0][0] + (32 * u + kq) * 16 + pc, *sxu = &sx[0][0];
+                const v8bf ga = read(sgu, sgu + 256);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    v8bf xb;
+                    if (j == 3 && wave == 6) {  // the bias: x = 1
+                        const short one = 0x3f80;
+                        xb = __builtin_bit_cast(v8bf, v8s{one, one, one, one, one, one, one, one});
+                    } else {
+                        const int c0 = corner[u][0], c1 = corner[u][1];
+                        xb = read(sxu + (c0 < 0 ? kZero * 16 + pc : c0 + off[j]),
+                                  sxu + (c1 < 0 ? kZero * 16 + pc : c1 + off[j]));
+                    }
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, xb, acc[j], 0, 0, 0);
+                }
+            }
         }
     }
-    // add the four wavefronts' tiles in a fixed order
+    // D[co][ci]: row 4 (lane / 16) + i, column lane % 16
+    float *out = part + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * kDwPart;
 #pragma unroll
-    for (int t = 0; t < T; t++)
+    for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) red[wave][t][j][lane] = acc[t][j];
-    __syncthreads();
-    for (int e = tid; e < T * 4 * 64; e += 256) {
-        const int t = e / 256, j = (e / 64) & 3, l = e & 63;
-        const float sum = ((red[0][t][j][l] + red[1][t][j][l]) + red[2][t][j][l]) + red[3][t][j][l];
-        // C[row][col] of tile t: row = 4 (l >> 4) + j (output channel), col = l & 15 (input channel)
-        const int co = 16 * (t / NB) + 4 * (l >> 4) + j, ci = 16 * (t % NB) + (l & 15);
-        if (ci < CIN) part[((size_t)blockIdx.x * 27 + tap) * PAIRS + co * CIN + ci] = sum;
-    }
-    if (tap == 13 && tid < COUT) bpart[(size_t)blockIdx.x * COUT + tid] = bacc;
+        for (int i = 0; i < 4; i++)
+            out[(4 * wave + j) * 256 + (4 * (lane >> 4) + i) * 16 + (lane & 15)] = acc[j][i];
 }
 
-// out[i] += sum over chunks of part[chunk][i] (fixed order).
-__global__ __launch_bounds__(256) void k_reduce_chunks(const float *__restrict__ part, int chunks,
-                                                       size_t n, float *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int c = 0; c < chunks; c++) s += part[(size_t)c * n + i];
-    out[i] += s;
+// The sums over the chunks of every convolution's partials, in a fixed order: a
+// block per tap of a tile, wavefront w adding the chunks w, w + 8, .. and their
+// eight sums added at the end.
+constexpr int kDwSumWaves = 8;
+__global__ __launch_bounds__(64 * kDwSumWaves) void k_dw_sums(DwSums s, const float *__restrict__ part,
+                                                              float *__restrict__ grad) {
+    __shared__ v4f red[kDwSumWaves][64];
+    int k = 0;
+    while (k + 1 < kUNetConvs && (int)blockIdx.x >= s.first[k + 1]) k++;
+    const int rem = (int)blockIdx.x - s.first[k], tile = rem / kDwTaps, t = rem % kDwTaps;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nb = tile % s.nb[k], mb = tile / s.nb[k];
+    const float *src = part + s.off[k] + (size_t)tile * kDwPart + t * 256 + 4 * lane;
+    const size_t stride = (size_t)s.tiles[k] * kDwPart;
+    v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int c = wave; c < s.chunks[k]; c += kDwSumWaves) sum += *reinterpret_cast<const v4f *>(src + c * stride);
+    red[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0) {
+        for (int w = 1; w < kDwSumWaves; w++) sum += red[w][lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = 4 * lane + i, co = 16 * mb + e / 16, ci = 16 * nb + e % 16;
+            if (t < 27) {
+                if (ci < s.cin[k]) grad[s.off_w[k] + ((size_t)t * s.cout[k] + co) * s.cin[k] + ci] = sum[i];
+            } else if (ci == 0) {
+                grad[s.off_b[k] + co] = sum[i];
+            }
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_pool2(const uint16_t *__restrict__ in, int B, int X, int Y,
@@ -809,10 +891,8 @@ void conv_dispatch(hipStream_t st, const ConvArgs &a) {
 }
 
 template <int CIN, int COUT>
-void dw_dispatch(hipStream_t st, const uint16_t *x, const uint16_t *g, int B, int X, int Y, int Z,
-                 float *part, float *bpart, int chunks, int chunk_len) {
-    hipLaunchKernelGGL((k_conv_dw<CIN, COUT>), dim3(chunks, 27), dim3(256), 0, st, x, g, B, X, Y, Z,
-                       chunk_len, part, bpart);
+void dw_dispatch(hipStream_t st, const uint16_t *x, const uint16_t *g, const DwPlan &p, float *part) {
+    hipLaunchKernelGGL((k_conv_dw<CIN, COUT>), dim3(p.chunks, p.tiles), dim3(kDwThreads), 0, st, x, g, p, part);
     SFP_LAUNCH_CHECK();
 }
 
@@ -843,15 +923,42 @@ void unet_conv(hipStream_t st, int cin, int cout, const uint16_t *in, const uint
     throw ArgError("unsupported convolution shape");
 }
 
-void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, int B,
-                  int X, int Y, int Z, float *part, float *dw, float *db) {
-    const size_t nv = (size_t)B * X * Y * Z;
-    const int chunks = (int)std::min<size_t>(kDwChunks, nv);
-    const int chunk_len = (int)((nv + chunks - 1) / chunks);
-    const size_t n = 27 * (size_t)cin * cout;
-    float *bpart = part + (size_t)chunks * n;
+DwPlan unet_dw_plan(int cin, int cout, int B, int X, int Y, int Z) {
+    DwPlan p{};
+    p.X = X, p.Y = Y, p.Z = Z;
+    const auto share = [](int n, int most) {  // the size of equal parts of at most `most`
+        const int parts = (n + most - 1) / most;
+        return (n + parts - 1) / parts;
+    };
+    p.zt = share(Z, 32);
+    p.yt = share(Y, std::min(32, kDwVoxels / p.zt));
+    p.nyt = (Y + p.yt - 1) / p.yt;
+    p.nzt = (Z + p.zt - 1) / p.zt;
+    // q / zt as q * magic >> 16: exact for q < 1024 and divisors up to 34
+    p.magic = 65536u / (unsigned)p.zt + 1;
+    p.magic_f = 65536u / (unsigned)(p.zt + 2) + 1;
+    p.tiles = (cout / 16) * std::max(1, cin / 16);
+    const long long columns = (long long)B * p.nyt * p.nzt;
+    // blocks: one per CU (each more adds its partial tile's 28 KB to write and
+    // sum; a run's first plane costs three of x)
+    const int want = std::max(1, kDwBlocks / p.tiles);
+    const int segs = (int)std::min<long long>(X, std::max<long long>(1, (want + columns - 1) / columns));
+    p.seg = (X + segs - 1) / segs;
+    p.segs = (X + p.seg - 1) / p.seg;
+    if (columns * p.segs > 0x7fffffff) throw ArgError("weight gradient: volume too large");
+    p.items = (int)(columns * p.segs);
+    const int rounds = (p.items + want - 1) / want;
+    p.chunks = (p.items + rounds - 1) / rounds;
+    return p;
+}
+
+size_t unet_dw_part(const DwPlan &p) { return (size_t)p.chunks * p.tiles * kDwPart; }
+
+void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, const DwPlan &p,
+                  float *part) {
+    if (p.yt > 32 || p.zt > 32 || p.yt * p.zt > kDwVoxels) throw ArgError("weight gradient: plane too large");
 #define SFP_DW(CI, CO) \
-    if (cin == CI && cout == CO) dw_dispatch<CI, CO>(st, x, g, B, X, Y, Z, part, bpart, chunks, chunk_len); else
+    if (cin == CI && cout == CO) return dw_dispatch<CI, CO>(st, x, g, p, part);
     SFP_DW(8, 16)
     SFP_DW(16, 16)
     SFP_DW(16, 32)
@@ -860,11 +967,27 @@ void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const ui
     SFP_DW(32, 64)
     SFP_DW(64, 32)
     SFP_DW(64, 64)
-    throw ArgError("unsupported convolution shape");
 #undef SFP_DW
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(blocks_for(n)), dim3(256), 0, st, part, chunks, n, dw);
-    SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(256), 0, st, bpart, chunks, (size_t)cout, db);
+    throw ArgError("unsupported convolution shape");
+}
+
+void unet_dw_sums(hipStream_t st, const DwPlan plan[kUNetConvs], const long long off_w[kUNetConvs],
+                  const long long off_b[kUNetConvs], const float *part, float *grad) {
+    DwSums s{};
+    size_t off = 0;
+    for (int k = 0; k < kUNetConvs; k++) {
+        s.off[k] = off;
+        off += unet_dw_part(plan[k]);
+        s.chunks[k] = plan[k].chunks;
+        s.tiles[k] = plan[k].tiles;
+        s.cin[k] = kConvCin[k];
+        s.cout[k] = kConvCout[k];
+        s.nb[k] = std::max(1, kConvCin[k] / 16);
+        s.off_w[k] = off_w[k];
+        s.off_b[k] = off_b[k];
+        s.first[k + 1] = s.first[k] + plan[k].tiles * kDwTaps;
+    }
+    hipLaunchKernelGGL(k_dw_sums, dim3(s.first[kUNetConvs]), dim3(64 * kDwSumWaves), 0, st, s, part, grad);
     SFP_LAUNCH_CHECK();
 }
 

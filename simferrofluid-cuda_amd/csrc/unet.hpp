@@ -21,7 +21,8 @@ namespace sfp {
 constexpr int kUNetConvs = 10;
 constexpr int kConvCin[kUNetConvs] = {8, 16, 16, 32, 32, 64, 64, 32, 32, 16};
 constexpr int kConvCout[kUNetConvs] = {16, 16, 32, 32, 64, 64, 32, 32, 16, 16};
-constexpr int kDwChunks = 64;  // voxel chunks of the weight-gradient reduction
+constexpr int kConvLevel[kUNetConvs] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0};
+constexpr int kDwBlocks = 256;  // blocks a weight gradient's launch aims at
 
 // Taps stored for a convolution with `cin` input channels: padded so that the
 // 32-wide K chunks of the MFMA cover whole taps.
@@ -38,8 +39,29 @@ void unet_conv(hipStream_t st, int cin, int cout, const uint16_t *in, const uint
                const float *bias, const uint16_t *skip, uint16_t *out, float *out32,
                uint16_t *relu_copy, int B, int X, int Y, int Z, bool relu, bool up_input = false,
                const double *gate = nullptr);
-void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, int B,
-                  int X, int Y, int Z, float *part, float *dw, float *db);
+// Weight gradients of a convolution, in two launches: partial sums over chunks
+// of the volume (unet_dw_part(plan) floats), and the sums over all ten
+// convolutions' partials (which follow each other in `part`) into the gradient.
+struct DwPlan {
+    int X, Y, Z;
+    int yt, zt, nyt, nzt;  // the volume's columns along x: nyt x nzt of yt x zt voxels per batch entry
+    int seg, segs;         // runs of `seg` planes in a column
+    int items, chunks;     // columns times runs; blocks they are dealt to
+    int tiles;             // 16 x 16 channel tiles
+    unsigned magic, magic_f;
+};
+struct DwSums {
+    size_t off[kUNetConvs];
+    long long off_w[kUNetConvs], off_b[kUNetConvs];
+    int chunks[kUNetConvs], tiles[kUNetConvs], cin[kUNetConvs], cout[kUNetConvs], nb[kUNetConvs];
+    int first[kUNetConvs + 1];
+};
+DwPlan unet_dw_plan(int cin, int cout, int B, int X, int Y, int Z);
+size_t unet_dw_part(const DwPlan &plan);
+void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, const DwPlan &plan,
+                  float *part);
+void unet_dw_sums(hipStream_t st, const DwPlan plan[kUNetConvs], const long long off_w[kUNetConvs],
+                  const long long off_b[kUNetConvs], const float *part, float *grad);
 void unet_pool2(hipStream_t st, const uint16_t *in, int B, int X, int Y, int Z, int C, uint16_t *out,
                 const double *gate = nullptr);
 void unet_pool2_bwd(hipStream_t st, const float *g, const float *add, int B, int X, int Y, int Z,
@@ -107,6 +129,7 @@ class UNet {
     // backward scratch
     DevBuf<float> gA_, gB_, gC_, gs0_, gs1_, part_;
     DevBuf<uint16_t> g16_;
+    DwPlan dw_plan_[kUNetConvs];
     DevBuf<double> dpart_, dsums_;
 };
 

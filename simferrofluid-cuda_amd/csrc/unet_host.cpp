@@ -107,7 +107,13 @@ void UNet::ensure(const UNetShape &s, bool training) {
         gs0_.ensure(n0 * 16);
         gs1_.ensure(n1 * 32);
         g16_.ensure(n0 * 16);
-        part_.ensure((size_t)kDwChunks * (27 * 64 * 64 + 64));
+        size_t floats = 0;
+        for (int k = 0; k < kUNetConvs; k++) {
+            const int l = kConvLevel[k];
+            dw_plan_[k] = unet_dw_plan(kConvCin[k], kConvCout[k], s.B, s.X >> l, s.Y >> l, s.Z >> l);
+            floats += unet_dw_part(dw_plan_[k]);
+        }
+        part_.ensure(floats);
     }
     dpart_.ensure(17 * ((n0 + 255) / 256) + 17);
     dsums_.ensure(17);
@@ -157,16 +163,16 @@ double UNet::loss_and_backward(hipStream_t st, const uint16_t *x8, const float *
     const int B = shape_.B;
     const size_t n0 = shape_.voxels(0), n1 = shape_.voxels(1), n2 = shape_.voxels(2);
     forward(st, x8, z_.p);
-    SFP_HIP(hipMemsetAsync(grad_.p, 0, grad_.n * sizeof(float), st));
     unet_mse(st, z_.p, t, m, n0, dpart_.p, dsums_.p, dz_.p);
     double mse[2];
     SFP_HIP(hipMemcpyAsync(mse, dsums_.p, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     SFP_HIP(hipStreamSynchronize(st));
     unet_head_bwd(st, d0_.p, w_.p + off_head_, dz_.p, n0, gA_.p, dpart_.p, dsums_.p, grad_.p + off_head_);
     auto L = [&](int level, int a) { return dims(level, a); };
-    auto dw = [&](int k, int level, const uint16_t *x, const uint16_t *g) {
-        unet_conv_dw(st, kConvCin[k], kConvCout[k], x, g, B, L(level, 0), L(level, 1), L(level, 2), part_.p,
-                     grad_.p + off_w_[k], grad_.p + off_b_[k]);
+    float *part[kUNetConvs] = {part_.p};
+    for (int k = 1; k < kUNetConvs; k++) part[k] = part[k - 1] + unet_dw_part(dw_plan_[k - 1]);
+    auto dw = [&](int k, const uint16_t *x, const uint16_t *g) {
+        unet_conv_dw(st, kConvCin[k], kConvCout[k], x, g, dw_plan_[k], part[k]);
     };
     auto dx = [&](int k, int level, const uint16_t *g, float *out) {
         unet_conv(st, kConvCout[k], kConvCin[k], g, wt_[k].p, nullptr, nullptr, nullptr, out, nullptr, B,
@@ -174,42 +180,43 @@ double UNet::loss_and_backward(hipStream_t st, const uint16_t *x8, const float *
     };
     // level 0 decoder
     unet_relu_mask(st, gA_.p, d0_.p, n0 * 16, g16_.p);
-    dw(9, 0, s0_.p, g16_.p);
+    dw(9, s0_.p, g16_.p);
     dx(9, 0, g16_.p, gs0_.p);
     unet_relu_mask(st, gs0_.p, r8_.p, n0 * 16, g16_.p);
-    dw(8, 0, u0_.p, g16_.p);
+    dw(8, u0_.p, g16_.p);
     dx(8, 0, g16_.p, gB_.p);
     // level 1 decoder
     unet_up2_bwd(st, gB_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, gA_.p);
     unet_relu_mask(st, gA_.p, d1_.p, n1 * 32, g16_.p);
-    dw(7, 1, s1_.p, g16_.p);
+    dw(7, s1_.p, g16_.p);
     dx(7, 1, g16_.p, gs1_.p);
     unet_relu_mask(st, gs1_.p, r6_.p, n1 * 32, g16_.p);
-    dw(6, 1, u1_.p, g16_.p);
+    dw(6, u1_.p, g16_.p);
     dx(6, 1, g16_.p, gB_.p);
     // level 2
     unet_up2_bwd(st, gB_.p, B, L(2, 0), L(2, 1), L(2, 2), 64, gA_.p);
     unet_relu_mask(st, gA_.p, e2_.p, n2 * 64, g16_.p);
-    dw(5, 2, a2_.p, g16_.p);
+    dw(5, a2_.p, g16_.p);
     dx(5, 2, g16_.p, gB_.p);
     unet_relu_mask(st, gB_.p, a2_.p, n2 * 64, g16_.p);
-    dw(4, 2, p1_.p, g16_.p);
+    dw(4, p1_.p, g16_.p);
     dx(4, 2, g16_.p, gA_.p);
     // level 1 encoder (the skip into s1 adds gs1)
     unet_pool2_bwd(st, gA_.p, gs1_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, gB_.p);
     unet_relu_mask(st, gB_.p, e1_.p, n1 * 32, g16_.p);
-    dw(3, 1, a1_.p, g16_.p);
+    dw(3, a1_.p, g16_.p);
     dx(3, 1, g16_.p, gA_.p);
     unet_relu_mask(st, gA_.p, a1_.p, n1 * 32, g16_.p);
-    dw(2, 1, p0_.p, g16_.p);
+    dw(2, p0_.p, g16_.p);
     dx(2, 1, g16_.p, gB_.p);
     // level 0 encoder (the skip into s0 adds gs0)
     unet_pool2_bwd(st, gB_.p, gs0_.p, B, L(0, 0), L(0, 1), L(0, 2), 16, gA_.p);
     unet_relu_mask(st, gA_.p, e0_.p, n0 * 16, g16_.p);
-    dw(1, 0, a0_.p, g16_.p);
+    dw(1, a0_.p, g16_.p);
     dx(1, 0, g16_.p, gB_.p);
     unet_relu_mask(st, gB_.p, a0_.p, n0 * 16, g16_.p);
-    dw(0, 0, x8, g16_.p);
+    dw(0, x8, g16_.p);
+    unet_dw_sums(st, dw_plan_, off_w_, off_b_, part_.p, grad_.p);
     if (host_sums) {
         host_sums[0] = mse[0];
         host_sums[1] = mse[1];
