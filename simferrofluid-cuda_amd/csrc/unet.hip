@@ -32,12 +32,14 @@ struct ConvArgs {
     const uint16_t *in;   // [B][X][Y][Z][CIN]
     const uint16_t *w;    // [tap][COUT][CIN]
     const float *bias;    // [COUT] or null
-    const uint16_t *skip; // [B][X][Y][Z][COUT] or null: added after the ReLU
+    const uint16_t *skip; // [B][X][Y][Z][COUT] or null: added after the ReLU, or (mask) an activation
+                          // whose ReLU the gradient passes: out is 0 where it is not positive
     uint16_t *out;        // BF16 output or null
     float *out32;         // FP32 output or null
     uint16_t *relu_copy;  // relu(acc + bias) before the skip, or null
     int B, X, Y, Z;
     int relu;
+    int mask;
     int up;  // 1: `in` is [B][X/2][Y/2][Z/2][CIN], read nearest-up-sampled
     const double *gate;  // nonzero *gate: return at once (a stopped batch of FCG iterations)
     unsigned in_bytes;   // size of `in` (at most kInLimit)
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
     const auto rout32 = buf_rsrc(a.out32, a.out32 ? 4 * a.out_elems : 0);
     const auto rrelu = buf_rsrc(a.relu_copy, a.relu_copy ? 2 * a.out_elems : 0);
     const bool has_skip = a.skip != nullptr, has_relu_copy = a.relu_copy != nullptr;
-    const bool relu = a.relu != 0, f32 = a.out32 != nullptr;
+    const bool relu = a.relu != 0, f32 = a.out32 != nullptr, mask = a.mask != 0;
     // Two fragment buffers alternate with the step's parity and three
     // accumulator slots rotate with the step mod 3: the march is unrolled by
     // six, so every index is a constant and no fragment is copied. Step t
@@ -371,11 +373,14 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
                     float v = acc[S][oy][j] + bias;
                     if (relu) v = v > 0.f ? v : 0.f;
                     if (has_relu_copy) __builtin_amdgcn_raw_buffer_store_b16(bf16_bits(v), rrelu, o, 0, 0);
-                    if (has_skip) v += bf2f(skv[oy][j]);
+                    if (has_skip && !mask) v += bf2f(skv[oy][j]);
+                    if (mask)
+                        __builtin_amdgcn_raw_buffer_store_b16(
+                            bf2f(skv[oy][j]) > 0.f ? bf16_bits(v) : (uint16_t)0, rout, o, 0, 0);
                     if (f32)  // (FP32 output: twice the 16-bit offset)
                         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rout32,
                                                               ob[oy][j] == kOutOutside ? kOutOutside : 2 * o, 0, 0);
-                    else
+                    else if (!mask)
                         __builtin_amdgcn_raw_buffer_store_b16(bf16_bits(v), rout, o, 0, 0);
                 }
                 acc[S][oy] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -441,7 +446,8 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
 // N = 16 input channels, K = voxels; BF16 products, exact in FP32, FP32
 // accumulation): part[chunk][tile][tap][co][ci] = sum_v g[v][co] x[v + tap][ci]
 // for the voxels of a chunk and the channel tile blockIdx.y; "tap" 27 has x = 1
-// and gives the bias sums.
+// and gives the bias sums. up: x has half the resolution and is read
+// nearest-up-sampled.
 //
 // A block stages one plane of a column (yt x zt voxels, up to kDwVoxels) of g
 // and three planes of x with their one-voxel frame in LDS, as the tensors lie
@@ -468,7 +474,7 @@ typedef short v8s __attribute__((ext_vector_type(8)));
 
 template <int CIN, int COUT>
 __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const uint16_t *__restrict__ x,
-                                                        const uint16_t *__restrict__ g, DwPlan p,
+                                                        const uint16_t *__restrict__ g, DwPlan p, int up,
                                                         float *__restrict__ part) {
     constexpr int NB = CIN < 16 ? 1 : CIN / 16;
     constexpr int kZero = 3 * kDwFramed;  // the zero row
@@ -487,6 +493,7 @@ __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const uint16_t *__restri
     constexpr int RX = (2 * kDwFramed + kDwThreads - 1) / kDwThreads;
     constexpr int RG = (2 * kDwVoxels + kDwThreads - 1) / kDwThreads;
     uint4 rx[RX], rg[RG];
+    const int Xs = p.X >> up, Ys = p.Y >> up, Zs = p.Z >> up;
     v4f acc[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const uint16_t *__restri
         const int y0 = ty * p.yt, z0 = tz * p.zt;
         const int xa = seg * p.seg, xe = min(xa + p.seg, p.X);
         auto load_x = [&](int plane) {
-            const uint16_t *px = x + (size_t)(bb * (long long)p.X + plane) * p.Y * p.Z * CIN + 16 * nb;
+            const uint16_t *px = x + (size_t)(bb * (long long)Xs + (plane >> up)) * Ys * Zs * CIN + 16 * nb;
 #pragma unroll
             for (int r = 0; r < RX; r++) {
                 const int e = tid + r * kDwThreads, vi = e >> 1;
@@ -506,7 +513,8 @@ __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const uint16_t *__restri
                 rx[r] = none;
                 if (vi < framed && (CIN >= 16 || !(e & 1)) && plane >= 0 && plane < p.X && gy >= 0 && gy < p.Y &&
                     gz >= 0 && gz < p.Z)
-                    rx[r] = *reinterpret_cast<const uint4 *>(px + ((size_t)gy * p.Z + gz) * CIN + 8 * (e & 1));
+                    rx[r] = *reinterpret_cast<const uint4 *>(px + ((size_t)(gy >> up) * Zs + (gz >> up)) * CIN +
+                                                              8 * (e & 1));
             }
         };
         auto store_x = [&](int plane) {
@@ -637,102 +645,112 @@ __global__ __launch_bounds__(64 * kDwSumWaves) void k_dw_sums(DwSums s, const fl
     }
 }
 
-__global__ __launch_bounds__(256) void k_pool2(const uint16_t *__restrict__ in, int B, int X, int Y,
-                                               int Z, int C, uint16_t *__restrict__ out,
-                                               const double *gate) {
+// The passes between the convolutions are bound by the bytes they move: a
+// thread takes 8 channels of a voxel (16-byte loads and stores), and the
+// backward ones end with the activation's ReLU and the rounding the next
+// convolution reads, so no FP32 gradient is stored for a pass of its own.
+struct Voxel8 {
+    int c, z, y, x, b;  // first channel; position in a volume of the pass's own extents
+};
+__device__ __forceinline__ Voxel8 voxel8(unsigned i, int X, int Y, int Z, int C) {
+    Voxel8 v;
+    unsigned r = i;
+    const unsigned c8 = (unsigned)C / 8;
+    v.c = 8 * (int)(r % c8);
+    r /= c8;
+    v.z = (int)(r % (unsigned)Z);
+    r /= (unsigned)Z;
+    v.y = (int)(r % (unsigned)Y);
+    r /= (unsigned)Y;
+    v.x = (int)(r % (unsigned)X);
+    v.b = (int)(r / (unsigned)X);
+    return v;
+}
+struct Half8 {
+    uint16_t h[8];
+};
+__device__ __forceinline__ Half8 load_half8(const uint16_t *p) {
+    return __builtin_bit_cast(Half8, *reinterpret_cast<const uint4 *>(p));
+}
+__device__ __forceinline__ void store_half8(uint16_t *p, const Half8 &v) {
+    *reinterpret_cast<uint4 *>(p) = __builtin_bit_cast(uint4, v);
+}
+struct Float8 {
+    float f[8];
+};
+__device__ __forceinline__ Float8 load_float8(const float *p) {
+    Float8 v;
+    const v4f a = reinterpret_cast<const v4f *>(p)[0], b = reinterpret_cast<const v4f *>(p)[1];
+#pragma unroll
+    for (int c = 0; c < 4; c++) v.f[c] = a[c], v.f[4 + c] = b[c];
+    return v;
+}
+// bf16(g) where the activation is positive, else 0
+__device__ __forceinline__ Half8 relu_masked(const Float8 &g, const Half8 &act) {
+    Half8 o;
+#pragma unroll
+    for (int c = 0; c < 8; c++) o.h[c] = bf2f(act.h[c]) > 0.f ? f2bf(g.f[c]) : (uint16_t)0;
+    return o;
+}
+// child d of a coarse voxel, as an offset into the fine tensor
+__device__ __forceinline__ size_t child8(const Voxel8 &v, int d, int X, int Y, int Z, int C) {
+    return ((((size_t)v.b * X + 2 * v.x + (d >> 2)) * Y + 2 * v.y + ((d >> 1) & 1)) * Z + 2 * v.z + (d & 1)) * C +
+           v.c;
+}
+
+__global__ __launch_bounds__(256) void k_pool2(const uint16_t *__restrict__ in, unsigned n8, int X, int Y,
+                                               int Z, int C, uint16_t *__restrict__ out, const double *gate) {
     if (gate && *gate != 0.0) return;
-    const int Xo = X / 2, Yo = Y / 2, Zo = Z / 2;
-    const size_t n = (size_t)B * Xo * Yo * Zo * C;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    size_t r = i;
-    const int c = (int)(r % C);
-    r /= C;
-    const int z = (int)(r % Zo);
-    r /= Zo;
-    const int y = (int)(r % Yo);
-    r /= Yo;
-    const int x = (int)(r % Xo);
-    const size_t b = r / Xo;
-    float s = 0.f;
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const Voxel8 v = voxel8(i, X / 2, Y / 2, Z / 2, C);
+    Half8 o;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
     for (int d = 0; d < 8; d++) {
-        const size_t v = ((b * X + 2 * x + (d >> 2)) * Y + 2 * y + ((d >> 1) & 1)) * Z + 2 * z + (d & 1);
-        s += bf2f(in[v * C + c]);
+        const Half8 h = load_half8(in + child8(v, d, X, Y, Z, C));
+#pragma unroll
+        for (int c = 0; c < 8; c++) s[c] += bf2f(h.h[c]);
     }
-    out[i] = f2bf(s * 0.125f);
+#pragma unroll
+    for (int c = 0; c < 8; c++) o.h[c] = f2bf(s[c] * 0.125f);
+    store_half8(out + 8 * (size_t)i, o);
 }
 
-// gin[fine] = g[coarse] / 8, optionally plus add[fine]
+// g16[fine] = g[coarse] / 8 + add[fine], through the ReLU of act[fine]
 __global__ __launch_bounds__(256) void k_pool2_bwd(const float *__restrict__ g, const float *__restrict__ add,
-                                                   int B, int X, int Y, int Z, int C,
-                                                   float *__restrict__ gin) {
-    const size_t n = (size_t)B * X * Y * Z * C;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    size_t r = i;
-    const int c = (int)(r % C);
-    r /= C;
-    const int z = (int)(r % Z);
-    r /= Z;
-    const int y = (int)(r % Y);
-    r /= Y;
-    const int x = (int)(r % X);
-    const size_t b = r / X;
-    const size_t vc = ((b * (X / 2) + x / 2) * (Y / 2) + y / 2) * (Z / 2) + z / 2;
-    float v = 0.125f * g[vc * C + c];
-    if (add) v += add[i];
-    gin[i] = v;
-}
-
-__global__ __launch_bounds__(256) void k_up2(const uint16_t *__restrict__ in, int B, int Xc, int Yc,
-                                             int Zc, int C, uint16_t *__restrict__ out) {
-    const int X = 2 * Xc, Y = 2 * Yc, Z = 2 * Zc;
-    const size_t n = (size_t)B * X * Y * Z * C;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    size_t r = i;
-    const int c = (int)(r % C);
-    r /= C;
-    const int z = (int)(r % Z);
-    r /= Z;
-    const int y = (int)(r % Y);
-    r /= Y;
-    const int x = (int)(r % X);
-    const size_t b = r / X;
-    out[i] = in[(((b * Xc + x / 2) * Yc + y / 2) * Zc + z / 2) * C + c];
-}
-
-// gcoarse = sum of the 8 children of g (fine)
-__global__ __launch_bounds__(256) void k_up2_bwd(const float *__restrict__ g, int B, int Xc, int Yc,
-                                                 int Zc, int C, float *__restrict__ gc) {
-    const size_t n = (size_t)B * Xc * Yc * Zc * C;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    size_t r = i;
-    const int c = (int)(r % C);
-    r /= C;
-    const int z = (int)(r % Zc);
-    r /= Zc;
-    const int y = (int)(r % Yc);
-    r /= Yc;
-    const int x = (int)(r % Xc);
-    const size_t b = r / Xc;
-    const int X = 2 * Xc, Y = 2 * Yc, Z = 2 * Zc;
-    float s = 0.f;
-    for (int d = 0; d < 8; d++) {
-        const size_t v = ((b * X + 2 * x + (d >> 2)) * Y + 2 * y + ((d >> 1) & 1)) * Z + 2 * z + (d & 1);
-        s += g[v * C + c];
+                                                   const uint16_t *__restrict__ act, unsigned n8, int X, int Y,
+                                                   int Z, int C, uint16_t *__restrict__ g16) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const Voxel8 v = voxel8(i, X, Y, Z, C);
+    const size_t vc = (((size_t)v.b * (X / 2) + v.x / 2) * (Y / 2) + v.y / 2) * (Z / 2) + v.z / 2;
+    const Float8 gc = load_float8(g + vc * C + v.c), ad = load_float8(add + 8 * (size_t)i);
+    Float8 o;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        float t = 0.125f * gc.f[c];
+        t += ad.f[c];
+        o.f[c] = t;
     }
-    gc[i] = s;
+    store_half8(g16 + 8 * (size_t)i, relu_masked(o, load_half8(act + 8 * (size_t)i)));
 }
 
-// g16 = bf16(g * (act > 0))
-__global__ __launch_bounds__(256) void k_relu_mask(const float *__restrict__ g,
-                                                   const uint16_t *__restrict__ act, size_t n,
-                                                   uint16_t *__restrict__ g16) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    g16[i] = bf2f(act[i]) > 0.f ? f2bf(g[i]) : (uint16_t)0;
+// g16[coarse] = the sum of the 8 children of g[fine], through the ReLU of act[coarse]
+__global__ __launch_bounds__(256) void k_up2_bwd(const float *__restrict__ g, const uint16_t *__restrict__ act,
+                                                 unsigned n8, int Xc, int Yc, int Zc, int C,
+                                                 uint16_t *__restrict__ g16) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const Voxel8 v = voxel8(i, Xc, Yc, Zc, C);
+    Float8 s = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int d = 0; d < 8; d++) {
+        const Float8 h = load_float8(g + child8(v, d, 2 * Xc, 2 * Yc, 2 * Zc, C));
+#pragma unroll
+        for (int c = 0; c < 8; c++) s.f[c] += h.f[c];
+    }
+    store_half8(g16 + 8 * (size_t)i, relu_masked(s, load_half8(act + 8 * (size_t)i)));
 }
 
 // z[v] = bo + sum_c wo[c] d0[v][c]
@@ -742,16 +760,20 @@ __global__ __launch_bounds__(256) void k_head_fwd(const uint16_t *__restrict__ d
     const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (v >= nv) return;
     float s = wb[16];
-    const uint16_t *p = d0 + v * 16;
 #pragma unroll
-    for (int c = 0; c < 16; c++) s += wb[c] * bf2f(p[c]);
+    for (int q = 0; q < 2; q++) {
+        const Half8 h = load_half8(d0 + v * 16 + 8 * q);
+#pragma unroll
+        for (int c = 0; c < 8; c++) s += wb[8 * q + c] * bf2f(h.h[c]);
+    }
     z[v] = s;
 }
 
-// gd0[v][c] = dz[v] wo[c]; per-block partials of sum dz d0[v][c] (16) and sum dz
+// g16[v][c] = dz[v] wo[c] through the ReLU of d0; per-block partials of sum dz
+// d0[v][c] (16) and sum dz
 __global__ __launch_bounds__(256) void k_head_bwd(const uint16_t *__restrict__ d0, const float *__restrict__ wb,
                                                   const float *__restrict__ dz, size_t nv,
-                                                  float *__restrict__ gd0, double *__restrict__ part) {
+                                                  uint16_t *__restrict__ g16, double *__restrict__ part) {
     const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
     double acc[17];
 #pragma unroll
@@ -759,9 +781,15 @@ __global__ __launch_bounds__(256) void k_head_bwd(const uint16_t *__restrict__ d
     if (v < nv) {
         const float d = dz[v];
 #pragma unroll
-        for (int c = 0; c < 16; c++) {
-            gd0[v * 16 + c] = d * wb[c];
-            acc[c] = (double)d * bf2f(d0[v * 16 + c]);
+        for (int q = 0; q < 2; q++) {
+            const Half8 h = load_half8(d0 + v * 16 + 8 * q);
+            Float8 gd;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                gd.f[c] = d * wb[8 * q + c];
+                acc[8 * q + c] = (double)d * bf2f(h.h[c]);
+            }
+            store_half8(g16 + v * 16 + 8 * q, relu_masked(gd, h));
         }
         acc[16] = d;
     }
@@ -783,20 +811,19 @@ __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ z, const 
     block_partials<2>(acc, part);
 }
 
+// out[q] = the sum of column q's nb partials (a block per column); out32 (or
+// null) receives it rounded
 __global__ __launch_bounds__(256) void k_sum_partials(const double *__restrict__ part, unsigned nb,
-                                                      int n, double *__restrict__ out) {
-    // n <= 17 columns, each of nb partials
-    for (int q = 0; q < n; q++) {
-        double v[1] = {0.0};
-        for (unsigned b = threadIdx.x; b < nb; b += 256) v[0] += part[(size_t)q * nb + b];
-        block_sum<1>(v);
-        if (threadIdx.x == 0) out[q] = v[0];
+                                                      double *__restrict__ out, float *__restrict__ out32) {
+    const int q = blockIdx.x;
+    double v[1] = {0.0};
+#pragma unroll 4
+    for (unsigned b = threadIdx.x; b < nb; b += 256) v[0] += part[(size_t)q * nb + b];
+    block_sum<1>(v);
+    if (threadIdx.x == 0) {
+        out[q] = v[0];
+        if (out32) out32[q] = (float)v[0];
     }
-}
-
-__global__ __launch_bounds__(256) void k_cast_sums(const double *__restrict__ sums, int n,
-                                                   float *__restrict__ out) {
-    if ((int)threadIdx.x < n) out[threadIdx.x] = (float)sums[threadIdx.x];
 }
 
 __global__ __launch_bounds__(256) void k_mse_grad(const float *__restrict__ z, const float *__restrict__ t,
@@ -846,11 +873,12 @@ __global__ __launch_bounds__(256) void k_cast_weights(const float *__restrict__ 
 // FP32 [nv][4] -> BF16 [nv][8] (channels 4..7 zero)
 __global__ __launch_bounds__(256) void k_pack_input(const float *__restrict__ in, size_t nv,
                                                     uint16_t *__restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nv * 8) return;
-    const size_t v = i >> 3;
-    const int c = (int)(i & 7);
-    out[i] = c < 4 ? f2bf(in[v * 4 + c]) : (uint16_t)0;
+    const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (v >= nv) return;
+    Half8 o = {{0, 0, 0, 0, 0, 0, 0, 0}};
+#pragma unroll
+    for (int c = 0; c < 4; c++) o.h[c] = f2bf(in[v * 4 + c]);
+    store_half8(out + v * 8, o);
 }
 
 unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -891,8 +919,9 @@ void conv_dispatch(hipStream_t st, const ConvArgs &a) {
 }
 
 template <int CIN, int COUT>
-void dw_dispatch(hipStream_t st, const uint16_t *x, const uint16_t *g, const DwPlan &p, float *part) {
-    hipLaunchKernelGGL((k_conv_dw<CIN, COUT>), dim3(p.chunks, p.tiles), dim3(kDwThreads), 0, st, x, g, p, part);
+void dw_dispatch(hipStream_t st, const uint16_t *x, const uint16_t *g, const DwPlan &p, int up, float *part) {
+    hipLaunchKernelGGL((k_conv_dw<CIN, COUT>), dim3(p.chunks, p.tiles), dim3(kDwThreads), 0, st, x, g, p, up,
+                       part);
     SFP_LAUNCH_CHECK();
 }
 
@@ -901,13 +930,15 @@ void dw_dispatch(hipStream_t st, const uint16_t *x, const uint16_t *g, const DwP
 void unet_conv(hipStream_t st, int cin, int cout, const uint16_t *in, const uint16_t *w,
                const float *bias, const uint16_t *skip, uint16_t *out, float *out32,
                uint16_t *relu_copy, int B, int X, int Y, int Z, bool relu, bool up_input,
-               const double *gate) {
+               const double *gate, const uint16_t *mask) {
+    if (mask && (skip || relu_copy)) throw ArgError("a masked convolution has no skip tensor");
     if (up_input && (X % 2 || Y % 2 || Z % 2)) throw ArgError("up-sampled input needs even extents");
     const size_t in_bytes = (size_t)B * (up_input ? (size_t)(X / 2) * (Y / 2) * (Z / 2) : (size_t)X * Y * Z) * cin * 2;
     const size_t out_elems = (size_t)B * X * Y * Z * cout;
     if (in_bytes > kInLimit || out_elems * 4 > kOutOutside)
         throw ArgError("convolution tensors too large for 32-bit buffer offsets");
-    ConvArgs a{in, w, bias, skip, out, out32, relu_copy, B, X, Y, Z, relu ? 1 : 0, up_input ? 1 : 0, gate,
+    ConvArgs a{in, w, bias, mask ? mask : skip, out, out32, relu_copy, B, X, Y, Z, relu ? 1 : 0, mask ? 1 : 0,
+               up_input ? 1 : 0, gate,
                (unsigned)in_bytes, (unsigned)out_elems};
 #define SFP_CONV(CI, CO) \
     if (cin == CI && cout == CO) return conv_dispatch<CI, CO>(st, a);
@@ -955,10 +986,11 @@ DwPlan unet_dw_plan(int cin, int cout, int B, int X, int Y, int Z) {
 size_t unet_dw_part(const DwPlan &p) { return (size_t)p.chunks * p.tiles * kDwPart; }
 
 void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, const DwPlan &p,
-                  float *part) {
+                  bool up_input, float *part) {
+    if (up_input && (p.X % 2 || p.Y % 2 || p.Z % 2)) throw ArgError("up-sampled input needs even extents");
     if (p.yt > 32 || p.zt > 32 || p.yt * p.zt > kDwVoxels) throw ArgError("weight gradient: plane too large");
 #define SFP_DW(CI, CO) \
-    if (cin == CI && cout == CO) return dw_dispatch<CI, CO>(st, x, g, p, part);
+    if (cin == CI && cout == CO) return dw_dispatch<CI, CO>(st, x, g, p, up_input ? 1 : 0, part);
     SFP_DW(8, 16)
     SFP_DW(16, 16)
     SFP_DW(16, 32)
@@ -991,34 +1023,31 @@ void unet_dw_sums(hipStream_t st, const DwPlan plan[kUNetConvs], const long long
     SFP_LAUNCH_CHECK();
 }
 
+// 8-channel groups of a tensor (the passes over them index in 32 bits)
+static unsigned groups8(int B, int X, int Y, int Z, int C) {
+    const size_t n = (size_t)B * X * Y * Z * (C / 8);
+    if (C % 8 || n > 0xffffff00u) throw ArgError("U-Net tensor too large");
+    return (unsigned)n;
+}
+
 void unet_pool2(hipStream_t st, const uint16_t *in, int B, int X, int Y, int Z, int C, uint16_t *out,
                 const double *gate) {
-    const size_t n = (size_t)B * (X / 2) * (Y / 2) * (Z / 2) * C;
-    hipLaunchKernelGGL(k_pool2, dim3(blocks_for(n)), dim3(256), 0, st, in, B, X, Y, Z, C, out, gate);
+    const unsigned n = groups8(B, X / 2, Y / 2, Z / 2, C);
+    hipLaunchKernelGGL(k_pool2, dim3(blocks_for(n)), dim3(256), 0, st, in, n, X, Y, Z, C, out, gate);
     SFP_LAUNCH_CHECK();
 }
 
-void unet_pool2_bwd(hipStream_t st, const float *g, const float *add, int B, int X, int Y, int Z,
-                    int C, float *gin) {
-    const size_t n = (size_t)B * X * Y * Z * C;
-    hipLaunchKernelGGL(k_pool2_bwd, dim3(blocks_for(n)), dim3(256), 0, st, g, add, B, X, Y, Z, C, gin);
+void unet_pool2_bwd(hipStream_t st, const float *g, const float *add, const uint16_t *act, int B, int X, int Y,
+                    int Z, int C, uint16_t *g16) {
+    const unsigned n = groups8(B, X, Y, Z, C);
+    hipLaunchKernelGGL(k_pool2_bwd, dim3(blocks_for(n)), dim3(256), 0, st, g, add, act, n, X, Y, Z, C, g16);
     SFP_LAUNCH_CHECK();
 }
 
-void unet_up2(hipStream_t st, const uint16_t *in, int B, int Xc, int Yc, int Zc, int C, uint16_t *out) {
-    const size_t n = (size_t)B * 8 * Xc * Yc * Zc * C;
-    hipLaunchKernelGGL(k_up2, dim3(blocks_for(n)), dim3(256), 0, st, in, B, Xc, Yc, Zc, C, out);
-    SFP_LAUNCH_CHECK();
-}
-
-void unet_up2_bwd(hipStream_t st, const float *g, int B, int Xc, int Yc, int Zc, int C, float *gc) {
-    const size_t n = (size_t)B * Xc * Yc * Zc * C;
-    hipLaunchKernelGGL(k_up2_bwd, dim3(blocks_for(n)), dim3(256), 0, st, g, B, Xc, Yc, Zc, C, gc);
-    SFP_LAUNCH_CHECK();
-}
-
-void unet_relu_mask(hipStream_t st, const float *g, const uint16_t *act, size_t n, uint16_t *g16) {
-    hipLaunchKernelGGL(k_relu_mask, dim3(blocks_for(n)), dim3(256), 0, st, g, act, n, g16);
+void unet_up2_bwd(hipStream_t st, const float *g, const uint16_t *act, int B, int Xc, int Yc, int Zc, int C,
+                  uint16_t *g16) {
+    const unsigned n = groups8(B, Xc, Yc, Zc, C);
+    hipLaunchKernelGGL(k_up2_bwd, dim3(blocks_for(n)), dim3(256), 0, st, g, act, n, Xc, Yc, Zc, C, g16);
     SFP_LAUNCH_CHECK();
 }
 
@@ -1029,13 +1058,11 @@ void unet_head_fwd(hipStream_t st, const uint16_t *d0, const float *wb, size_t n
 }
 
 void unet_head_bwd(hipStream_t st, const uint16_t *d0, const float *wb, const float *dz, size_t nv,
-                   float *gd0, double *part, double *sums, float *gwb) {
+                   uint16_t *g16, double *part, double *sums, float *gwb) {
     const unsigned nb = blocks_for(nv);
-    hipLaunchKernelGGL(k_head_bwd, dim3(nb), dim3(256), 0, st, d0, wb, dz, nv, gd0, part);
+    hipLaunchKernelGGL(k_head_bwd, dim3(nb), dim3(256), 0, st, d0, wb, dz, nv, g16, part);
     SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, part, nb, 17, sums);
-    SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_cast_sums, dim3(1), dim3(256), 0, st, sums, 17, gwb);
+    hipLaunchKernelGGL(k_sum_partials, dim3(17), dim3(256), 0, st, part, nb, sums, gwb);
     SFP_LAUNCH_CHECK();
 }
 
@@ -1044,7 +1071,7 @@ void unet_mse(hipStream_t st, const float *z, const float *t, const float *m, si
     const unsigned nb = blocks_for(nv);
     hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, st, z, t, m, nv, part);
     SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, part, nb, 2, sums);
+    hipLaunchKernelGGL(k_sum_partials, dim3(2), dim3(256), 0, st, part, nb, sums, (float *)nullptr);
     SFP_LAUNCH_CHECK();
     if (dz) {
         hipLaunchKernelGGL(k_mse_grad, dim3(nb), dim3(256), 0, st, z, t, m, nv, sums, dz);
@@ -1068,7 +1095,7 @@ void unet_cast_weights(hipStream_t st, const float *w, int cin, int cout, uint16
 }
 
 void unet_pack_input(hipStream_t st, const float *in, size_t nv, uint16_t *out) {
-    hipLaunchKernelGGL(k_pack_input, dim3(blocks_for(nv * 8)), dim3(256), 0, st, in, nv, out);
+    hipLaunchKernelGGL(k_pack_input, dim3(blocks_for(nv)), dim3(256), 0, st, in, nv, out);
     SFP_LAUNCH_CHECK();
 }
 

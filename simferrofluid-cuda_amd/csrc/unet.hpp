@@ -34,11 +34,12 @@ long long unet_param_count();
 // up_input: `in` holds the half-resolution tensor, read nearest-up-sampled
 // (the up-sampling fused into the staging). gate (the forward's kernels): the
 // launch returns at once while *gate is nonzero (a stopped batch of FCG
-// iterations).
+// iterations). mask (of the output's shape): out = bf16 of the result where
+// mask > 0 and 0 elsewhere, next to the FP32 output if there is one.
 void unet_conv(hipStream_t st, int cin, int cout, const uint16_t *in, const uint16_t *w,
                const float *bias, const uint16_t *skip, uint16_t *out, float *out32,
                uint16_t *relu_copy, int B, int X, int Y, int Z, bool relu, bool up_input = false,
-               const double *gate = nullptr);
+               const double *gate = nullptr, const uint16_t *mask = nullptr);
 // Weight gradients of a convolution, in two launches: partial sums over chunks
 // of the volume (unet_dw_part(plan) floats), and the sums over all ten
 // convolutions' partials (which follow each other in `part`) into the gradient.
@@ -59,20 +60,21 @@ struct DwSums {
 DwPlan unet_dw_plan(int cin, int cout, int B, int X, int Y, int Z);
 size_t unet_dw_part(const DwPlan &plan);
 void unet_conv_dw(hipStream_t st, int cin, int cout, const uint16_t *x, const uint16_t *g, const DwPlan &plan,
-                  float *part);
+                  bool up_input, float *part);
 void unet_dw_sums(hipStream_t st, const DwPlan plan[kUNetConvs], const long long off_w[kUNetConvs],
                   const long long off_b[kUNetConvs], const float *part, float *grad);
 void unet_pool2(hipStream_t st, const uint16_t *in, int B, int X, int Y, int Z, int C, uint16_t *out,
                 const double *gate = nullptr);
-void unet_pool2_bwd(hipStream_t st, const float *g, const float *add, int B, int X, int Y, int Z,
-                    int C, float *gin);
-void unet_up2(hipStream_t st, const uint16_t *in, int B, int Xc, int Yc, int Zc, int C, uint16_t *out);
-void unet_up2_bwd(hipStream_t st, const float *g, int B, int Xc, int Yc, int Zc, int C, float *gc);
-void unet_relu_mask(hipStream_t st, const float *g, const uint16_t *act, size_t n, uint16_t *g16);
+// gradients through a pooling (plus the FP32 gradient `add` of a skip) or an
+// up-sampling, then the ReLU of `act`, rounded to BF16
+void unet_pool2_bwd(hipStream_t st, const float *g, const float *add, const uint16_t *act, int B, int X, int Y,
+                    int Z, int C, uint16_t *g16);
+void unet_up2_bwd(hipStream_t st, const float *g, const uint16_t *act, int B, int Xc, int Yc, int Zc, int C,
+                  uint16_t *g16);
 void unet_head_fwd(hipStream_t st, const uint16_t *d0, const float *wb, size_t nv, float *z,
                    const double *gate = nullptr);
 void unet_head_bwd(hipStream_t st, const uint16_t *d0, const float *wb, const float *dz, size_t nv,
-                   float *gd0, double *part, double *sums, float *gwb);
+                   uint16_t *g16, double *part, double *sums, float *gwb);
 void unet_mse(hipStream_t st, const float *z, const float *t, const float *m, size_t nv,
               double *part, double *sums, float *dz);
 void unet_adam(hipStream_t st, float *w, const float *g, float *m, float *v, size_t n, float lr,
@@ -124,11 +126,11 @@ class UNet {
     bool training_ = false;
     int step_ = 0;
     // activations (BF16)
-    DevBuf<uint16_t> x8_, a0_, e0_, p0_, a1_, e1_, p1_, a2_, e2_, u1_, r6_, s1_, d1_, u0_, r8_, s0_, d0_;
+    DevBuf<uint16_t> x8_, a0_, e0_, p0_, a1_, e1_, p1_, a2_, e2_, r6_, s1_, d1_, r8_, s0_, d0_;
     DevBuf<float> z_, dz_;
     // backward scratch
-    DevBuf<float> gA_, gB_, gC_, gs0_, gs1_, part_;
-    DevBuf<uint16_t> g16_;
+    DevBuf<float> gB_, gs0_, gs1_, part_;
+    DevBuf<uint16_t> g16_, h16_;
     DwPlan dw_plan_[kUNetConvs];
     DevBuf<double> dpart_, dsums_;
 };

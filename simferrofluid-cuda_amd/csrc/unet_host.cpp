@@ -92,21 +92,19 @@ void UNet::ensure(const UNetShape &s, bool training) {
     const size_t n0 = s.voxels(0), n1 = s.voxels(1), n2 = s.voxels(2);
     x8_.ensure(n0 * 8);
     for (auto *b : {&a0_, &e0_, &r8_, &s0_, &d0_}) b->ensure(n0 * 16);
-    if (training) u0_.ensure(n0 * 32);
     p0_.ensure(n1 * 16);
     for (auto *b : {&a1_, &e1_, &r6_, &s1_, &d1_}) b->ensure(n1 * 32);
-    if (training) u1_.ensure(n1 * 64);
     p1_.ensure(n2 * 32);
     a2_.ensure(n2 * 64);
     e2_.ensure(n2 * 64);
     z_.ensure(n0);
     if (training) {
         dz_.ensure(n0);
-        gA_.ensure(n0 * 16);
         gB_.ensure(n0 * 32);
         gs0_.ensure(n0 * 16);
         gs1_.ensure(n1 * 32);
         g16_.ensure(n0 * 16);
+        h16_.ensure(n0 * 16);
         size_t floats = 0;
         for (int k = 0; k < kUNetConvs; k++) {
             const int l = kConvLevel[k];
@@ -116,7 +114,7 @@ void UNet::ensure(const UNetShape &s, bool training) {
         part_.ensure(floats);
     }
     dpart_.ensure(17 * ((n0 + 255) / 256) + 17);
-    dsums_.ensure(17);
+    dsums_.ensure(2 + 17);  // the loss, the head's gradient
 }
 
 void UNet::conv(hipStream_t st, int k, int level, const uint16_t *in, const uint16_t *skip,
@@ -138,21 +136,11 @@ void UNet::forward(hipStream_t st, const uint16_t *x8, float *z, const double *g
     unet_pool2(st, e1_.p, B, dims(1, 0), dims(1, 1), dims(1, 2), 32, p1_.p, gate);
     conv(st, 4, 2, p1_.p, nullptr, a2_.p, nullptr, false, gate);
     conv(st, 5, 2, a2_.p, nullptr, e2_.p, nullptr, false, gate);
-    // training keeps the up-sampled tensors (the weight gradients read them);
-    // inference reads the half-resolution ones through the convolution
-    if (training_) {
-        unet_up2(st, e2_.p, B, dims(2, 0), dims(2, 1), dims(2, 2), 64, u1_.p);
-        conv(st, 6, 1, u1_.p, e1_.p, s1_.p, keep6, false, gate);
-    } else {
-        conv(st, 6, 1, e2_.p, e1_.p, s1_.p, keep6, true, gate);
-    }
+    // (the up-sampled tensors are never formed: the convolution and its weight
+    // gradient read the half-resolution ones)
+    conv(st, 6, 1, e2_.p, e1_.p, s1_.p, keep6, true, gate);
     conv(st, 7, 1, s1_.p, nullptr, d1_.p, nullptr, false, gate);
-    if (training_) {
-        unet_up2(st, d1_.p, B, dims(1, 0), dims(1, 1), dims(1, 2), 32, u0_.p);
-        conv(st, 8, 0, u0_.p, e0_.p, s0_.p, keep8, false, gate);
-    } else {
-        conv(st, 8, 0, d1_.p, e0_.p, s0_.p, keep8, true, gate);
-    }
+    conv(st, 8, 0, d1_.p, e0_.p, s0_.p, keep8, true, gate);
     conv(st, 9, 0, s0_.p, nullptr, d0_.p, nullptr, false, gate);
     unet_head_fwd(st, d0_.p, w_.p + off_head_, shape_.voxels(0), z, gate);
 }
@@ -161,62 +149,47 @@ double UNet::loss_and_backward(hipStream_t st, const uint16_t *x8, const float *
                                double *host_sums) {
     if (!training_) throw StateError("network buffers were sized for inference");
     const int B = shape_.B;
-    const size_t n0 = shape_.voxels(0), n1 = shape_.voxels(1), n2 = shape_.voxels(2);
+    const size_t n0 = shape_.voxels(0);
     forward(st, x8, z_.p);
     unet_mse(st, z_.p, t, m, n0, dpart_.p, dsums_.p, dz_.p);
+    float *part[kUNetConvs] = {part_.p};
+    for (int k = 1; k < kUNetConvs; k++) part[k] = part[k - 1] + unet_dw_part(dw_plan_[k - 1]);
+    auto L = [&](int level, int a) { return dims(level, a); };
+    // One layer back: the weight gradients from the layer's input x and output
+    // gradient g, then its input's gradient, FP32 in out32 and, through the ReLU
+    // of `act`, BF16 in out16 (either may be null).
+    auto back = [&](int k, int level, const uint16_t *x, bool up, const uint16_t *g, float *out32,
+                    const uint16_t *act, uint16_t *out16) {
+        unet_conv_dw(st, kConvCin[k], kConvCout[k], x, g, dw_plan_[k], up, part[k]);
+        if (out32 || out16)
+            unet_conv(st, kConvCout[k], kConvCin[k], g, wt_[k].p, nullptr, nullptr, out16, out32, nullptr, B,
+                      L(level, 0), L(level, 1), L(level, 2), false, false, nullptr, act);
+    };
+    uint16_t *g = g16_.p, *h = h16_.p;
+    unet_head_bwd(st, d0_.p, w_.p + off_head_, dz_.p, n0, g, dpart_.p, dsums_.p + 2, grad_.p + off_head_);
+    // level 0 decoder
+    back(9, 0, s0_.p, false, g, gs0_.p, r8_.p, h);
+    back(8, 0, d1_.p, true, h, gB_.p, nullptr, nullptr);
+    // level 1 decoder
+    unet_up2_bwd(st, gB_.p, d1_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, g);
+    back(7, 1, s1_.p, false, g, gs1_.p, r6_.p, h);
+    back(6, 1, e2_.p, true, h, gB_.p, nullptr, nullptr);
+    // level 2
+    unet_up2_bwd(st, gB_.p, e2_.p, B, L(2, 0), L(2, 1), L(2, 2), 64, g);
+    back(5, 2, a2_.p, false, g, nullptr, a2_.p, h);
+    back(4, 2, p1_.p, false, h, gB_.p, nullptr, nullptr);
+    // level 1 encoder (the skip into s1 adds gs1)
+    unet_pool2_bwd(st, gB_.p, gs1_.p, e1_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, g);
+    back(3, 1, a1_.p, false, g, nullptr, a1_.p, h);
+    back(2, 1, p0_.p, false, h, gB_.p, nullptr, nullptr);
+    // level 0 encoder (the skip into s0 adds gs0)
+    unet_pool2_bwd(st, gB_.p, gs0_.p, e0_.p, B, L(0, 0), L(0, 1), L(0, 2), 16, g);
+    back(1, 0, a0_.p, false, g, nullptr, a0_.p, h);
+    back(0, 0, x8, false, h, nullptr, nullptr, nullptr);
+    unet_dw_sums(st, dw_plan_, off_w_, off_b_, part_.p, grad_.p);
     double mse[2];
     SFP_HIP(hipMemcpyAsync(mse, dsums_.p, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     SFP_HIP(hipStreamSynchronize(st));
-    unet_head_bwd(st, d0_.p, w_.p + off_head_, dz_.p, n0, gA_.p, dpart_.p, dsums_.p, grad_.p + off_head_);
-    auto L = [&](int level, int a) { return dims(level, a); };
-    float *part[kUNetConvs] = {part_.p};
-    for (int k = 1; k < kUNetConvs; k++) part[k] = part[k - 1] + unet_dw_part(dw_plan_[k - 1]);
-    auto dw = [&](int k, const uint16_t *x, const uint16_t *g) {
-        unet_conv_dw(st, kConvCin[k], kConvCout[k], x, g, dw_plan_[k], part[k]);
-    };
-    auto dx = [&](int k, int level, const uint16_t *g, float *out) {
-        unet_conv(st, kConvCout[k], kConvCin[k], g, wt_[k].p, nullptr, nullptr, nullptr, out, nullptr, B,
-                  L(level, 0), L(level, 1), L(level, 2), false);
-    };
-    // level 0 decoder
-    unet_relu_mask(st, gA_.p, d0_.p, n0 * 16, g16_.p);
-    dw(9, s0_.p, g16_.p);
-    dx(9, 0, g16_.p, gs0_.p);
-    unet_relu_mask(st, gs0_.p, r8_.p, n0 * 16, g16_.p);
-    dw(8, u0_.p, g16_.p);
-    dx(8, 0, g16_.p, gB_.p);
-    // level 1 decoder
-    unet_up2_bwd(st, gB_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, gA_.p);
-    unet_relu_mask(st, gA_.p, d1_.p, n1 * 32, g16_.p);
-    dw(7, s1_.p, g16_.p);
-    dx(7, 1, g16_.p, gs1_.p);
-    unet_relu_mask(st, gs1_.p, r6_.p, n1 * 32, g16_.p);
-    dw(6, u1_.p, g16_.p);
-    dx(6, 1, g16_.p, gB_.p);
-    // level 2
-    unet_up2_bwd(st, gB_.p, B, L(2, 0), L(2, 1), L(2, 2), 64, gA_.p);
-    unet_relu_mask(st, gA_.p, e2_.p, n2 * 64, g16_.p);
-    dw(5, a2_.p, g16_.p);
-    dx(5, 2, g16_.p, gB_.p);
-    unet_relu_mask(st, gB_.p, a2_.p, n2 * 64, g16_.p);
-    dw(4, p1_.p, g16_.p);
-    dx(4, 2, g16_.p, gA_.p);
-    // level 1 encoder (the skip into s1 adds gs1)
-    unet_pool2_bwd(st, gA_.p, gs1_.p, B, L(1, 0), L(1, 1), L(1, 2), 32, gB_.p);
-    unet_relu_mask(st, gB_.p, e1_.p, n1 * 32, g16_.p);
-    dw(3, a1_.p, g16_.p);
-    dx(3, 1, g16_.p, gA_.p);
-    unet_relu_mask(st, gA_.p, a1_.p, n1 * 32, g16_.p);
-    dw(2, p0_.p, g16_.p);
-    dx(2, 1, g16_.p, gB_.p);
-    // level 0 encoder (the skip into s0 adds gs0)
-    unet_pool2_bwd(st, gB_.p, gs0_.p, B, L(0, 0), L(0, 1), L(0, 2), 16, gA_.p);
-    unet_relu_mask(st, gA_.p, e0_.p, n0 * 16, g16_.p);
-    dw(1, a0_.p, g16_.p);
-    dx(1, 0, g16_.p, gB_.p);
-    unet_relu_mask(st, gB_.p, a0_.p, n0 * 16, g16_.p);
-    dw(0, x8, g16_.p);
-    unet_dw_sums(st, dw_plan_, off_w_, off_b_, part_.p, grad_.p);
     if (host_sums) {
         host_sums[0] = mse[0];
         host_sums[1] = mse[1];
