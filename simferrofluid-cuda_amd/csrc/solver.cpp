@@ -581,6 +581,14 @@ const float *System::restrict_smoothed(Workspace &ws, const SolverConfig &cfg, c
     return learned_cycle(ws, cfg, r64, kCycleRestrictOnly);
 }
 
+// A z of infinities or NaN (from input that holds them) must not outlive its
+// solve: on cells that are active there and inactive in a later system, which
+// skips writing them, their neighbours couple with weight 0, and 0 times them
+// is NaN.
+void System::clear_ring(Workspace &ws) {
+    SFP_HIP(hipMemsetAsync(zring_.p, 0, kRing * zring_stride_ * sizeof(float), ws.stream));
+}
+
 SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm, const Finish &finish) {
     SolveInfo info;
     info.precond_used = cfg.precond;
@@ -753,6 +761,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
                 for (auto &t : ws.timers) t.used = 0;
             if (*ws.host_err) {
                 info.input_error = true;
+                clear_ring(ws);
                 return info;
             }
             bb = h.bb;
@@ -830,6 +839,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     }
     info.rel = rel;
     info.converged = rel <= cfg.tol;
+    if (!std::isfinite(rel)) clear_ring(ws);
     if (info.fallback > 0) info.precond_used = 0;
     if (profiling)
         for (auto &t : ws.timers) t.harvest();

@@ -212,6 +212,7 @@ class System {
     enum Cycle { kCycleLearned, kCycleSmooth, kCycleRestrictOnly };
     float *learned_cycle(Workspace &ws, const SolverConfig &cfg, const double *r64, Cycle c);
     float *post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur, const float *e);
+    void clear_ring(Workspace &ws);
     SolveInfo fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm, const Finish &finish);
     float *vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r64, bool x0_ready = false);
     // levels l .. coarsest in one launch (vlevel with r64 null), or null

@@ -85,3 +85,24 @@ def test_zero_right_hand_side_and_shared_outputs():
         np.testing.assert_array_equal(phi.cpu().numpy(), want_p)
         for a, b in zip(vel, want_v):
             np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+# grids whose kernels write every cell, and skip groups of inactive ones
+@pytest.mark.parametrize("n", [(64, 64, 64), (128, 132, 128)])
+def test_non_finite_input_leaves_nothing_behind(n):
+    """A projection of NaN velocities on a full container fails to converge;
+    the next one, on a pool, is that of a new context."""
+    print(f"[case] solve end after NaN {n}", flush=True)
+    pool = scenes.random_pressure_scene(n, 9)
+    full = dict(pool, phi=np.full_like(pool["phi"], -1.0), velocity=[np.full_like(v, np.nan) for v in pool["velocity"]])
+    with sfp.Context.for_scene(pool, tol=1e-8) as ctx:
+        want_v, want_p, want = ctx.pressure_project(pool)
+    with sfp.Context.for_scene(pool, tol=1e-8, max_iters=5) as ctx:
+        bad = ctx.pressure_project(full)[2]
+        assert not bad["converged"]
+        ctx.set_params(max_iters=200)
+        vel, p, st = ctx.pressure_project(pool)
+    assert st["converged"] and st["iterations"] == want["iterations"]
+    np.testing.assert_array_equal(p, want_p)
+    for a, b in zip(vel, want_v):
+        np.testing.assert_array_equal(a, b)
