@@ -67,7 +67,10 @@ sfp_status sfp_test_set_vcycle_tail(sfp_context ctx, int enable);
  * restriction and (bit 1) the last two post-smoothing steps on large grids,
  * (bits 2 and 3) the same on small grids, (bit 4) the first two
  * pre-smoothing passes of a degree-3 cycle on large grids, or each as
- * separate launches. Results are the same bit for bit. */
+ * separate launches. Bit 5 (from the next assembly on): run the kernels over
+ * the flat cell index on every chunk of cells instead of the active ones'
+ * list. A V-cycle's results are the same bit for bit; with bit 5 the solver's
+ * FP64 sums take another order. */
 sfp_status sfp_test_set_fused_pairs(sfp_context ctx, int mask); /* default 18 */
 /* Let the stencil kernels of the magnetic system (FCG matvec, smoothing
  * steps, restriction) rebuild the FP64 and FP32 diagonals from the couplings

@@ -125,6 +125,7 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     const Dims d = ctx->d;
     System &sys = ctx->pressure;
     sys.allocate(d);
+    sys.sparse_ = true;
     ctx->liquid.ensure(d.cells());
     const Faces F{{frac[0], frac[1], frac[2]}}, V{{vel[0], vel[1], vel[2]}}, U{{us[0], us[1], us[2]}};
     Faces J{{nullptr, nullptr, nullptr}};
@@ -533,6 +534,7 @@ sfp_status sfp_create(sfp_context *out, int nx, int ny, int nz, double spacing,
         SFP_HIP(hipStreamCreateWithFlags(&ctx->ws.side, hipStreamNonBlocking));
         SFP_HIP(hipEventCreateWithFlags(&ctx->ws.side_in, hipEventDisableTiming));
         SFP_HIP(hipEventCreateWithFlags(&ctx->ws.side_out, hipEventDisableTiming));
+        SFP_HIP(hipEventCreateWithFlags(&ctx->ws.side_lists, hipEventDisableTiming));
         for (auto &e : ctx->ev) SFP_HIP(hipEventCreate(&e));
         ctx->ws.partials.ensure(reduction_partials(ctx->d));
         ctx->ws.scalars.ensure(1);
@@ -557,7 +559,7 @@ void sfp_destroy(sfp_context ctx) {
     if (ctx->ws.side) (void)hipStreamSynchronize(ctx->ws.side);
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
-    for (hipEvent_t e : {ctx->ws.side_in, ctx->ws.side_out})
+    for (hipEvent_t e : {ctx->ws.side_in, ctx->ws.side_out, ctx->ws.side_lists})
         if (e) (void)hipEventDestroy(e);
     if (ctx->ws.host_sc) (void)hipHostFree(ctx->ws.host_sc);
     if (ctx->ws.host_err) (void)hipHostFree(ctx->ws.host_err);

@@ -243,7 +243,7 @@ sfp_status sfp_test_smooth_pair(sfp_context ctx, int which, int level, const flo
         if (x3_pair) {
             SFP_HIP(hipMemcpyAsync(dd.p, d1, n * sizeof(float), hipMemcpyHostToDevice, st));
             launch_smooth_pair(st, L.d, A, db.p, dx1.p, dx3.p, from_x1 ? dx1.p : dd.p, cdA, crA, cdB, crB,
-                               nullptr, L.rowact.p);
+                               nullptr, L.rowact.p, L.sparse ? L.segments.p : nullptr);
             d2h(ctx, x3_pair, dx3.p, n);
             SFP_HIP(hipStreamSynchronize(st));
         }
@@ -309,7 +309,7 @@ sfp_status sfp_test_set_vcycle_tail(sfp_context ctx, int enable) {
 
 sfp_status sfp_test_set_fused_pairs(sfp_context ctx, int mask) {
     return run(ctx, [&] {
-        if (mask < 0 || mask > 31) throw ArgError("fused pairs: mask is 0..31");
+        if (mask < 0 || mask > 63) throw ArgError("fused pairs: mask is 0..63");
         ctx->ws.fused_pairs = mask;
     });
 }

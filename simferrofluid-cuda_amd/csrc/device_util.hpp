@@ -38,6 +38,24 @@ __device__ __forceinline__ double load_gate(const double *gate, const void *othe
     return gate ? v : 0.0;
 }
 
+// The wavefront's number in the grid of a kernel over the flat cell index
+// (uniform), and a grid's number of them.
+__device__ __forceinline__ unsigned flat_wave() {
+    return blockIdx.x * (kBlock / 64) + (unsigned)__builtin_amdgcn_readfirstlane((int)(flat_tid() >> 6));
+}
+__device__ __forceinline__ unsigned flat_waves() { return gridDim.x * (kBlock / 64); }
+// The first of this lane's N consecutive cells, 64 N of a listed chunk to a
+// unit of work: unit `u` of list[0] * list_units<N>().
+template <int N>
+constexpr unsigned list_units() {
+    return kChunk / (64 * N);
+}
+template <int N>
+__device__ __forceinline__ unsigned list_cell(const unsigned *list, unsigned u) {
+    constexpr unsigned per = list_units<N>();
+    return list[1 + u / per] * kChunk + (u % per) * 64 * N + N * (flat_tid() & 63);
+}
+
 // Sum over the wavefront, the same in every lane: halves 32 lanes apart, then
 // 16, 8, 4, 2 and 1, the tree of shuffles down in lane 0 (so the same bits
 // there). The exchanges are register moves (v_permlane32_swap,

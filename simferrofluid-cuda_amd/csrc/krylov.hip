@@ -120,10 +120,12 @@ __global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64
 // off-diagonal sum keeps k_residual64's order, so r is the same to the bit; a
 // row-sum diagonal is rebuilt from the couplings as in the matvec. r, and b32
 // with x0, may be null (then not stored: a convergence check needs only the
-// sums).
+// sums, and with kList takes them over the listed chunks: b and x are 0 in the
+// others).
 constexpr unsigned kResidualCells = 2 * kBlock;
 
-__global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
+template <bool kList>
+__global__ __launch_bounds__(kBlock, kList ? 8 : 1) void k_residual64_flat(Dims d, Op64 A,
                                                             const double *__restrict__ b,
                                                             const double *__restrict__ x,
                                                             double *__restrict__ r,
@@ -134,9 +136,8 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
                                                             float c0, const double *need) {
     if (need && *need == 0.0) return;
     const Strides s(d);
-    const size_t c = (size_t)blockIdx.x * kResidualCells + 2 * (size_t)flat_tid();
     double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
-    if (c < d.cells()) {       // cells() is even: then c + 1 is a cell too
+    auto pair = [&](size_t c) {  // cells() is even: c + 1 is a cell too
         const double2v d0 = {0.0, 0.0};
         const double2v bc = ld_stream((const double2v *)(b + c));
         double2v rc = bc;
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
         }
         if (r) st_stream((double2v *)(r + c), rc);
         const float2v dd = diag32 ? *(const float2v *)(diag32 + c) : float2v{0.f, 0.f};
-        v[2] = (dd.x > 0.f ? 1.0 : 0.0) + (dd.y > 0.f ? 1.0 : 0.0);
+        v[2] += (dd.x > 0.f ? 1.0 : 0.0) + (dd.y > 0.f ? 1.0 : 0.0);
         if (b32) {
             const float2v bf = {(float)rc.x, (float)rc.y};
             *(float2v *)(b32 + c) = bf;
@@ -203,8 +204,19 @@ __global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A,
                 *(float2v *)(x0 + c) = xf;
             }
         }
-        v[0] = rc.x * rc.x + rc.y * rc.y;
-        v[1] = bc.x * bc.x + bc.y * bc.y;
+        v[0] += rc.x * rc.x + rc.y * rc.y;
+        v[1] += bc.x * bc.x + bc.y * bc.y;
+    };
+    const size_t n = d.cells();
+    if constexpr (kList) {
+        const unsigned units = A.chunks.list[0] * list_units<2>(), waves = flat_waves();
+        for (unsigned u = flat_wave(); u < units; u += waves) {
+            const unsigned c = list_cell<2>(A.chunks.list, u);
+            if (c < n) pair(c);
+        }
+    } else {
+        const size_t c = (size_t)blockIdx.x * kResidualCells + 2 * (size_t)flat_tid();
+        if (c < n) pair(c);
     }
     block_partials<3>(v, partials);
 }
@@ -299,10 +311,13 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64
 // vectors, 8-byte loads of z and its x and y neighbours, one extra z value and
 // z coupling at each end of the pair. Every cell's w and dot terms are formed
 // in the tiled kernel's order, so w is the same to the bit. A wavefront whose
-// 128 cells are all inactive is skipped.
+// 128 cells are all inactive is skipped; kList: kListBlocks blocks share the
+// listed chunks (256^3 pool, 26 % of the rows active: 80 us a wavefront per 128
+// cells of the grid, 69 so, and its fewer partial sums need one launch less).
 constexpr unsigned kMatvecCells = 2 * kBlock;
 
-__global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
+template <bool kList>
+__global__ __launch_bounds__(kBlock, kList ? 8 : 1) void k_fcg_matvec_flat(Dims d, Op64 A,
                                                             const float *__restrict__ active,
                                                             const float *__restrict__ z,
                                                             const double *__restrict__ r,
@@ -312,17 +327,18 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
                                                             const double *gate) {
     if (gated(gate)) return;
     const Strides s(d);
-    const size_t c = (size_t)blockIdx.x * kMatvecCells + 2 * (size_t)flat_tid();
-    const bool on = c < d.cells();  // cells() is even: then c + 1 is a cell too
     double v[3] = {0.0, 0.0, 0.0};  // z.w, z.q_prev, z.r
-    bool act = on, on0 = true, on1 = true;  // the pair's cells are active
-    if (active && on) {
-        const float2v a = *(const float2v *)(active + c);
-        on0 = a.x > 0.f;
-        on1 = a.y > 0.f;
-        act = on0 || on1;
-    }
-    if (__any(act) && on) {
+    // one pair of cells (cells() is even: c + 1 is a cell where c is; every lane
+    // of the wavefront comes here)
+    auto pair = [&](size_t c, bool on) {
+        bool act = on, on0 = true, on1 = true;  // the pair's cells are active
+        if (active && on) {
+            const float2v a = *(const float2v *)(active + c);
+            on0 = a.x > 0.f;
+            on1 = a.y > 0.f;
+            act = on0 || on1;
+        }
+        if (!(on && (kList || __any(act)))) return;
         // (i, j, k) of the first cell (the launcher keeps cells() < 2^32)
         const unsigned cu = (unsigned)c;
         const unsigned t = cu / (unsigned)d.nz;
@@ -385,9 +401,20 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec_flat(Dims d, Op64 A,
         wc.x = dg.x * z0 - o0;
         wc.y = dg.y * z1 - o1;
         st_stream((double2v *)(w + c), wc);
-        v[0] = z0 * wc.x + z1 * wc.y;
-        if (!first) v[1] = z0 * qp.x + z1 * qp.y;
-        v[2] = z0 * rc.x + z1 * rc.y;
+        v[0] += z0 * wc.x + z1 * wc.y;
+        if (!first) v[1] += z0 * qp.x + z1 * qp.y;
+        v[2] += z0 * rc.x + z1 * rc.y;
+    };
+    const size_t n = d.cells();
+    if constexpr (kList) {
+        const unsigned units = A.chunks.list[0] * list_units<2>(), waves = flat_waves();
+        for (unsigned u = flat_wave(); u < units; u += waves) {
+            const unsigned c = list_cell<2>(A.chunks.list, u);
+            pair(c, c < n);
+        }
+    } else {
+        const size_t c = (size_t)blockIdx.x * kMatvecCells + 2 * (size_t)flat_tid();
+        pair(c, c < n);
     }
     block_partials<3>(v, partials);
 }
@@ -520,6 +547,50 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
             }
             v[0] += rc * rc;
         }
+    }
+    block_partials<1>(v, partials);
+}
+
+// The same update on the listed chunks (kListBlocks blocks share them; cells()
+// is a multiple of 4), the scalars from a finalize launch.
+__global__ __launch_bounds__(kBlock) void k_fcg_update_list(size_t n, const unsigned *__restrict__ list,
+                                                            const float *__restrict__ active,
+                                                            const double *__restrict__ w, double *__restrict__ q,
+                                                            double *__restrict__ r, float *__restrict__ b32,
+                                                            float *__restrict__ x0, float c0, int first, int iter,
+                                                            double *__restrict__ partials,
+                                                            const KrylovScalars *__restrict__ sc,
+                                                            const double *gate) {
+    if (gated(gate)) return;
+    const double alpha = sc->alpha[iter % kCoefs], beta = sc->beta[iter % kCoefs];
+    double v[1] = {0.0};
+    const unsigned units = list[0] * list_units<2>(), waves = flat_waves();
+    for (unsigned u = flat_wave(); u < units; u += waves) {
+        const unsigned c = list_cell<2>(list, u);
+        if (c >= n) continue;
+        const float2v dg = x0 ? *(const float2v *)(active + c) : float2v{0.f, 0.f};
+        const double2v wc = ld_stream((const double2v *)(w + c)), r0 = ld_stream((const double2v *)(r + c));
+        double2v qc = wc;
+        if (!first) {
+            const double2v qq = ld_stream((const double2v *)(q + c));
+            qc.x = wc.x - beta * qq.x;
+            qc.y = wc.y - beta * qq.y;
+        }
+        double2v rc;
+        rc.x = r0.x - alpha * qc.x;
+        rc.y = r0.y - alpha * qc.y;
+        st_stream((double2v *)(q + c), qc);
+        st_stream((double2v *)(r + c), rc);
+        if (b32) {
+            const float2v bf = {(float)rc.x, (float)rc.y};
+            *(float2v *)(b32 + c) = bf;
+            if (x0) {
+                const float2v xf = {c0 * rcp_or_zero(dg.x) * bf.x, c0 * rcp_or_zero(dg.y) * bf.y};
+                *(float2v *)(x0 + c) = xf;
+            }
+        }
+        v[0] += rc.x * rc.x;
+        v[0] += rc.y * rc.y;
     }
     block_partials<1>(v, partials);
 }
@@ -731,6 +802,10 @@ static unsigned matvec_blocks(Dims d) {
     return matvec_flat(d) ? (unsigned)((d.cells() + kMatvecCells - 1) / kMatvecCells)
                           : matvec_launch(d).blocks();
 }
+// Blocks of a kernel over the listed chunks: as many as run at once (eight of
+// four wavefronts per CU), or the grid's where that is less.
+constexpr unsigned kListBlocks = 2048;
+static unsigned list_blocks(Dims d) { return std::min(kListBlocks, matvec_blocks(d)); }
 static unsigned update_blocks(Dims d) { return (unsigned)((d.cells() + kUpdateCells - 1) / kUpdateCells); }
 
 size_t reduction_partials(Dims d) {
@@ -762,9 +837,14 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
             if ((uintptr_t)a % 16) throw ArgError("launch_residual64: FP64 array not 16-byte aligned");
         if ((uintptr_t)b32 % 8 || (uintptr_t)x0 % 8 || (uintptr_t)diag32 % 8)
             throw ArgError("launch_residual64: b32, x0 or the diagonal not 8-byte aligned");
-        const unsigned nb = (unsigned)((d.cells() + kResidualCells - 1) / kResidualCells);
-        hipLaunchKernelGGL(k_residual64_flat, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials, b32,
-                           x0, diag32, c0, need);
+        const bool list = A.chunks.list && !r && !b32;  // (a residual that is stored covers every cell)
+        const unsigned nb = list ? list_blocks(d) : (unsigned)((d.cells() + kResidualCells - 1) / kResidualCells);
+        if (list)
+            hipLaunchKernelGGL(k_residual64_flat<true>, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials,
+                               b32, x0, diag32, c0, need);
+        else
+            hipLaunchKernelGGL(k_residual64_flat<false>, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials,
+                               b32, x0, diag32, c0, need);
         SFP_LAUNCH_CHECK();
         finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host, need, tol);
         return;
@@ -779,7 +859,8 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
 void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, const float *z,
                        const double *r, const double *qprev, double *w, int first, int iter, bool fold,
                        double *partials, KrylovScalars *sc, const double *gate, hipEvent_t kernel_done) {
-    unsigned nb = matvec_blocks(d);
+    const bool list = A.chunks.list != nullptr;
+    unsigned nb = list ? list_blocks(d) : matvec_blocks(d);
     if (matvec_flat(d)) {
         // pairs of cells: 16-byte (8-byte for z and the flags) aligned vectors
         for (const void *a : {(const void *)A.diag, (const void *)A.cpl[0], (const void *)A.cpl[1],
@@ -787,8 +868,12 @@ void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, cons
             if ((uintptr_t)a % 16) throw ArgError("launch_fcg_matvec: FP64 array not 16-byte aligned");
         if ((uintptr_t)z % 8 || (uintptr_t)active % 8)
             throw ArgError("launch_fcg_matvec: z or the diagonal not 8-byte aligned");
-        hipLaunchKernelGGL(k_fcg_matvec_flat, dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r,
-                           qprev, w, first, partials, gate);
+        if (list)
+            hipLaunchKernelGGL(k_fcg_matvec_flat<true>, dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r, qprev,
+                               w, first, partials, gate);
+        else
+            hipLaunchKernelGGL(k_fcg_matvec_flat<false>, dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r, qprev,
+                               w, first, partials, gate);
     } else {
         const Launch L = matvec_launch(d);
         hipLaunchKernelGGL(k_fcg_matvec, L.grid, L.block, 0, st, L.cg, d, A, active, z, r, qprev, w,
@@ -799,7 +884,7 @@ void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, cons
     if (!fold) finalize(st, FIN_MATVEC, nb, first, iter, partials, sc, gate);
 }
 
-void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double *w, double *q, double *r,
+void launch_fcg_update(hipStream_t st, Dims d, const float *active, const unsigned *chunks, const double *w, double *q, double *r,
                        float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate, hipEvent_t kernel_done, KrylovScalars *host) {
     // two cells per lane: 16-byte (8-byte for the FP32 ones) aligned vectors
@@ -808,9 +893,13 @@ void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double
     if ((uintptr_t)active % 8 || (uintptr_t)b32 % 8 || (uintptr_t)x0 % 8)
         throw ArgError("launch_fcg_update: the diagonal, b32 or x0 not 8-byte aligned");
     if (x0 && (!b32 || !active)) throw ArgError("launch_fcg_update: x0 needs b32 and the diagonal");
+    if (chunks && (fold || d.cells() % 4)) throw ArgError("launch_fcg_update: no list here");
     const unsigned nb = update_blocks(d), nb_mv = matvec_blocks(d);
     double *out = partials + 3 * (size_t)nb_mv;
-    if (fold)
+    if (chunks)
+        hipLaunchKernelGGL(k_fcg_update_list, dim3(list_blocks(d)), dim3(kBlock), 0, st, d.cells(), chunks, active,
+                           w, q, r, b32, x0, c0, first, iter, out, sc, gate);
+    else if (fold)
         hipLaunchKernelGGL(k_fcg_update<true>, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, w, q, r, b32, x0,
                            c0, first, iter, partials, nb_mv, out, sc, gate);
     else
@@ -818,7 +907,8 @@ void launch_fcg_update(hipStream_t st, Dims d, const float *active, const double
                            c0, first, iter, partials, nb_mv, out, sc, gate);
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
-    if (!fold) launch_fcg_norm(st, d, partials, sc, gate, host);
+    if (!fold)
+        finalize(st, FIN_UPDATE, chunks ? list_blocks(d) : nb, 0, 0, out, sc, gate, host);
 }
 
 void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc, const double *gate,

@@ -273,13 +273,23 @@ __device__ __forceinline__ void end_couplings(GroupOperands &g, Dims d, int i, i
     if (!(k + 4 < d.nz)) g.czhi = 0.f;
 }
 
-// kEager (levels of at most kEagerCells cells, where a launch is one round of
+// kEagerRun (levels of at most kEagerCells cells, where a launch is one round of
 // wavefronts bound by its chain of memory latencies): the gate, the diagonal
 // and every operand are loaded at once and the launch leaves after them, on a
 // closed gate or an inactive wavefront; else (large levels, bound by the bytes)
-// before the operands' loads.
-template <int MODE, bool kRowsum, bool kEager>
-__global__ __launch_bounds__(kBlock) void k_smooth_flat(Dims d, Op32 A, const float *__restrict__ b,
+// before the operands' loads. kListRun (levels with a list of active chunks):
+// as many blocks as run at once share the listed chunks, a
+// wavefront one at a time; with a wavefront per chunk of the grid those of the
+// inactive chunks have to be dispatched and to wait for a diagonal (256^3 pool,
+// 26 % active: 61 us a first post-smoothing step, 43 so, the list's bytes at the
+// copy rate being 31; its 128^3 level 11.8, 6.5 so).
+enum FlatRun { kBytesRun, kEagerRun, kListRun };
+// (wavefronts per SIMD the registers of a mode allow: blocks of a list run per CU)
+constexpr int list_waves(int mode) { return (mode & SM_PROLONG) ? 7 : 8; }
+
+template <int MODE, bool kRowsum, FlatRun kRun>
+__global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE) : 1) void k_smooth_flat(
+                                                        Dims d, Op32 A, const float *__restrict__ b,
                                                         const float *__restrict__ xin,
                                                         float *__restrict__ xout, float *dvec,
                                                         float cd, float cr,
@@ -289,91 +299,101 @@ __global__ __launch_bounds__(kBlock) void k_smooth_flat(Dims d, Op32 A, const fl
     constexpr bool kProlong = (MODE & SM_PROLONG) != 0;
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef float f2 __attribute__((ext_vector_type(2)));
+    constexpr bool kEager = kRun == kEagerRun;
+    static_assert(kRun != kListRun || !kRowsum, "no list where every cell is active");
     const double stop = load_gate(gate, A.diag);
     const unsigned n = (unsigned)d.cells();  // a multiple of 4 below 2^32
-    const unsigned ct = blockIdx.x * kSmoothFlatCells + 4 * (unsigned)flat_tid();
-    const bool on = ct < n;
-    const unsigned c = on ? ct : n - 4;
-    const bool rs = kRowsum && rowsum_group(A, c, d);  // every group there has an active cell
-    f4 dg = {0.f, 0.f, 0.f, 0.f};
-    if (!rs) dg = *(const f4 *)(A.diag + c);
-    if constexpr (!kEager) {
-        if (stop != 0.0) return;
-        const bool act = on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f);
-        if (!__any(act)) return;
-    }
-    // (i, j, k) of the first cell
-    const unsigned t = c / (unsigned)d.nz;
-    const int k = (int)(c - t * (unsigned)d.nz);
-    const unsigned iu = t / (unsigned)d.ny;
-    const int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny);
-    GroupOperands g = load_operands(A, b, xin, d, c, i, j, k);
-    f4 dprev = {0.f, 0.f, 0.f, 0.f};
-    if constexpr ((MODE & SM_READ_D) != 0) dprev = *(const f4 *)(dvec + c);
-    f2 ec, e_xm, e_xp, e_ym, e_yp;
-    float ezlo = 0.f, ezhi = 0.f;
-    if constexpr (kProlong) {
-        // coarse values of the group's two coarse cells in this row and in the
-        // neighbouring rows and planes (16-byte aligned groups: k >> 1 even)
-        const int kc = k >> 1, jl = max(j - 1, 0) >> 1, jh = min(j + 1, d.ny - 1) >> 1, il = max(i - 1, 0) >> 1,
-                  ih = min(i + 1, d.nx - 1) >> 1;
-        auto e2 = [&](int ii, int jj) { return *(const f2 *)(e + dc.idx(ii, jj, kc)); };
-        ec = e2(i >> 1, j >> 1);
-        e_xm = e2(il, j >> 1);
-        e_xp = e2(ih, j >> 1);
-        e_ym = e2(i >> 1, jl);
-        e_yp = e2(i >> 1, jh);
-        ezlo = e[dc.idx(i >> 1, j >> 1, max(kc - 1, 0))];
-        ezhi = e[dc.idx(i >> 1, j >> 1, min(kc + 2, dc.nz - 1))];
-    }
-    if constexpr (kEager) {
-        pin(g);
-        sfp::pin(dg);
-        if constexpr ((MODE & SM_READ_D) != 0) sfp::pin(dprev);
+    auto group = [&](unsigned ct) {  // the group of cells from ct on
+        const bool on = ct < n;
+        const unsigned c = on ? ct : n - 4;
+        const bool rs = kRowsum && rowsum_group(A, c, d);  // every group there has an active cell
+        f4 dg = {0.f, 0.f, 0.f, 0.f};
+        if (!rs) dg = *(const f4 *)(A.diag + c);
+        if constexpr (kRun == kBytesRun) {
+            if (stop != 0.0) return;
+            const bool act = on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f);
+            if (!__any(act)) return;
+        }
+        // (i, j, k) of the first cell
+        const unsigned t = c / (unsigned)d.nz;
+        const int k = (int)(c - t * (unsigned)d.nz);
+        const unsigned iu = t / (unsigned)d.ny;
+        const int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny);
+        GroupOperands g = load_operands(A, b, xin, d, c, i, j, k);
+        f4 dprev = {0.f, 0.f, 0.f, 0.f};
+        if constexpr ((MODE & SM_READ_D) != 0) dprev = *(const f4 *)(dvec + c);
+        f2 ec, e_xm, e_xp, e_ym, e_yp;
+        float ezlo = 0.f, ezhi = 0.f;
         if constexpr (kProlong) {
-            for (const f2 &v : {ec, e_xm, e_xp, e_ym, e_yp}) sfp::pin(v);
-            sfp::pin(ezlo);
-            sfp::pin(ezhi);
+            // coarse values of the group's two coarse cells in this row and in the
+            // neighbouring rows and planes (16-byte aligned groups: k >> 1 even)
+            const int kc = k >> 1, jl = max(j - 1, 0) >> 1, jh = min(j + 1, d.ny - 1) >> 1, il = max(i - 1, 0) >> 1,
+                      ih = min(i + 1, d.nx - 1) >> 1;
+            auto e2 = [&](int ii, int jj) { return *(const f2 *)(e + dc.idx(ii, jj, kc)); };
+            ec = e2(i >> 1, j >> 1);
+            e_xm = e2(il, j >> 1);
+            e_xp = e2(ih, j >> 1);
+            e_ym = e2(i >> 1, jl);
+            e_yp = e2(i >> 1, jh);
+            ezlo = e[dc.idx(i >> 1, j >> 1, max(kc - 1, 0))];
+            ezhi = e[dc.idx(i >> 1, j >> 1, min(kc + 2, dc.nz - 1))];
         }
-        if (stop != 0.0) return;
-    }
-    end_couplings(g, d, i, j, k);
-    if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
-    const f4 xin_c = g.xc;
-    if constexpr (kProlong) {
-#pragma unroll
+        if constexpr (kEager) {
+            pin(g);
+            sfp::pin(dg);
+            if constexpr ((MODE & SM_READ_D) != 0) sfp::pin(dprev);
+            if constexpr (kProlong) {
+                for (const f2 &v : {ec, e_xm, e_xp, e_ym, e_yp}) sfp::pin(v);
+                sfp::pin(ezlo);
+                sfp::pin(ezhi);
+            }
+            if (stop != 0.0) return;
+        }
+        end_couplings(g, d, i, j, k);
+        if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
+        const f4 xin_c = g.xc;
+        if constexpr (kProlong) {
+    #pragma unroll
+            for (int q = 0; q < 4; q++) {
+                g.xc[q] = g.xc[q] + ec[q >> 1];
+                g.xm[q] = g.xm[q] + e_xm[q >> 1];
+                g.xp[q] = g.xp[q] + e_xp[q >> 1];
+                g.ym[q] = g.ym[q] + e_ym[q >> 1];
+                g.yp[q] = g.yp[q] + e_yp[q >> 1];
+            }
+            g.zlo = g.zlo + ezlo;
+            g.zhi = g.zhi + ezhi;
+        }
+        f4 xo, dno;
+    #pragma unroll
         for (int q = 0; q < 4; q++) {
-            g.xc[q] = g.xc[q] + ec[q >> 1];
-            g.xm[q] = g.xm[q] + e_xm[q >> 1];
-            g.xp[q] = g.xp[q] + e_xp[q >> 1];
-            g.ym[q] = g.ym[q] + e_ym[q >> 1];
-            g.yp[q] = g.yp[q] + e_yp[q >> 1];
+            const float xzm = q > 0 ? g.xc[q - 1] : g.zlo;
+            const float xzp = q < 3 ? g.xc[q + 1] : g.zhi;
+            const float czp = q < 3 ? g.cz[q + 1] : g.czhi;
+            float off = fmaf(g.cx[q], g.xm[q], g.cxp[q] * g.xp[q]);
+            off = fmaf(g.cy[q], g.ym[q], off);
+            off = fmaf(g.cyp[q], g.yp[q], off);
+            off = fmaf(g.cz[q], xzm, off);
+            off = fmaf(czp, xzp, off);
+            // centre iterate: the coarse correction only lands on active cells
+            const float x0 = (kProlong && !(dg[q] > 0.f)) ? xin_c[q] : g.xc[q];
+            const float r = g.b[q] - fmaf(dg[q], x0, -off);
+            const float dp = (MODE & SM_XFIRST) != 0 ? x0 : dprev[q];
+            const float dn = fmaf(cd, dp, cr * rcp_or_zero(dg[q]) * r);
+            xo[q] = x0 + dn;
+            dno[q] = dn;
         }
-        g.zlo = g.zlo + ezlo;
-        g.zhi = g.zhi + ezhi;
+        if (!on) return;
+        *(f4 *)(xout + c) = xo;
+        if constexpr ((MODE & SM_WRITE_D) != 0) *(f4 *)(dvec + c) = dno;
+    };
+    if constexpr (kRun == kListRun) {
+        if (stop != 0.0) return;
+        const unsigned units = A.chunks.list[0], waves = flat_waves();
+        for (unsigned u = flat_wave(); u < units; u += waves) group(list_cell<4>(A.chunks.list, u));
+    } else {
+        group(blockIdx.x * kSmoothFlatCells + 4 * (unsigned)flat_tid());
     }
-    f4 xo, dno;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const float xzm = q > 0 ? g.xc[q - 1] : g.zlo;
-        const float xzp = q < 3 ? g.xc[q + 1] : g.zhi;
-        const float czp = q < 3 ? g.cz[q + 1] : g.czhi;
-        float off = fmaf(g.cx[q], g.xm[q], g.cxp[q] * g.xp[q]);
-        off = fmaf(g.cy[q], g.ym[q], off);
-        off = fmaf(g.cyp[q], g.yp[q], off);
-        off = fmaf(g.cz[q], xzm, off);
-        off = fmaf(czp, xzp, off);
-        // centre iterate: the coarse correction only lands on active cells
-        const float x0 = (kProlong && !(dg[q] > 0.f)) ? xin_c[q] : g.xc[q];
-        const float r = g.b[q] - fmaf(dg[q], x0, -off);
-        const float dp = (MODE & SM_XFIRST) != 0 ? x0 : dprev[q];
-        const float dn = fmaf(cd, dp, cr * rcp_or_zero(dg[q]) * r);
-        xo[q] = x0 + dn;
-        dno[q] = dn;
-    }
-    if (!on) return;
-    *(f4 *)(xout + c) = xo;
-    if constexpr ((MODE & SM_WRITE_D) != 0) *(f4 *)(dvec + c) = dno;
 }
 
 // Two passes over the grid in one (temporal blocking). Step A is a
@@ -621,10 +641,12 @@ template <bool kRowsum, bool kDx>
 __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     Dims d, Op32 A, const float *__restrict__ b, const float *__restrict__ x1,
     float *__restrict__ xo, const float *__restrict__ d1, float cdA, float crA, float cdB,
-    float crB, const unsigned char *__restrict__ rowact, int planes, unsigned ytiles,
-    const double *gate) {
+    float crB, const unsigned char *__restrict__ rowact, const int *__restrict__ segments, int planes,
+    unsigned ytiles, const double *gate) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     if (gated(gate)) return;
+    const unsigned runs = segments ? (unsigned)segments[0] : gridDim.x;
+    if (blockIdx.x >= runs) return;
     __shared__ f4 sx1[2][kRowPairRows + 2][64];  // x1 of rows -1 .. kRowPairRows (index row + 1)
     __shared__ f4 scy[4][kRowPairRows + 1][64];  // cpl_y of rows 0 .. kRowPairRows
     __shared__ f4 sx2[3][kRowPairRows][64];      // x2 of rows 0 .. kRowPairRows - 1
@@ -632,13 +654,17 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     // a contiguous run of them, so the rows two tiles share meet in one L2
     unsigned L = blockIdx.x;
     {
-        const unsigned q = gridDim.x / 8;
+        const unsigned q = runs / 8;
         if (L < 8 * q) L = (L % 8) * q + L / 8;
     }
-    const unsigned by = L % ytiles, bx = L / ytiles;
-    const int i0 = (int)bx * planes;
+    unsigned by = L % ytiles;
+    int i0 = (int)(L / ytiles) * planes, ie = min(i0 + planes, d.nx);
+    if (segments) {
+        by = (unsigned)segments[1 + 3 * L];
+        i0 = segments[2 + 3 * L];
+        ie = segments[3 + 3 * L];
+    }
     if (i0 >= d.nx) return;  // uniform over the block
-    const int ie = min(i0 + planes, d.nx);
     const int lane = threadIdx.x, row = threadIdx.y;
     const int k = 4 * lane;
     const int j = (int)by * kRowPairY - 1 + row;
@@ -969,7 +995,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict(CellGrid cg, Dims df, Op32 
 // stores zeros.
 constexpr int kRestrictFlatZ = 64;  // z cells per wavefront
 
-template <bool kRowsum, bool kEager>
+template <bool kRowsum, bool kEager, bool kList>
 __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const float *__restrict__ b,
                                                           const float *__restrict__ x, Dims dc,
                                                           float *__restrict__ bc, float *__restrict__ x0c,
@@ -979,7 +1005,11 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
     typedef float f2 __attribute__((ext_vector_type(2)));
     const double stop = load_gate(gate, A.diag);
     const int lane = threadIdx.x & 63;
-    const unsigned wave = (unsigned)(blockIdx.x * kBlock + threadIdx.x) >> 6;
+    unsigned wave = flat_wave();
+    if constexpr (kList) {  // (an inactive coarse cell's values are 0 already)
+        if (stop != 0.0 || wave >= A.chunks.quads[0]) return;
+        wave = A.chunks.quads[1 + wave];
+    }
     const unsigned zch = (unsigned)(df.nz + kRestrictFlatZ - 1) / kRestrictFlatZ;
     const unsigned yp = (unsigned)(df.ny + 1) / 2;
     const unsigned kz = wave % zch, t = wave / zch;
@@ -996,7 +1026,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
     if (!rs) dg = *(const f4 *)(A.diag + c);
     f4 r = {0.f, 0.f, 0.f, 0.f};
     bool any = true;
-    if constexpr (!kEager) {
+    if constexpr (!kEager && !kList) {
         if (stop != 0.0) return;
         any = __any(on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f));
     }
@@ -1817,6 +1847,11 @@ void launch_smooth_first(hipStream_t st, Dims d, Op32 A, const double *r64, floa
     SFP_LAUNCH_CHECK();
 }
 
+unsigned restrict_quads(Dims d) {
+    return (unsigned)((d.nz + kRestrictFlatZ - 1) / kRestrictFlatZ) * (unsigned)((d.ny + 1) / 2) *
+           (unsigned)((d.nx + 1) / 2);
+}
+
 bool flat_step(Dims d) { return d.nz % 4 == 0 && d.cells() < (size_t(1) << 32); }
 
 // The flat step where it applies: no fused first step, z rows of whole
@@ -1838,15 +1873,18 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
         const unsigned nb = (unsigned)((d.cells() + kSmoothFlatCells - 1) / kSmoothFlatCells);
         const Dims dc = d.coarse();
         const bool eager = d.cells() <= kEagerCells;
-#define SFP_FLAT_LAUNCH(M, RS, EA)                                                                 \
-    hipLaunchKernelGGL((k_smooth_flat<M, RS, EA>), dim3(nb), dim3(kBlock), 0, st, d, A, b, xin,    \
-                       xout, dvec, cd, cr, ecoarse, dc, gate)
+#define SFP_FLAT_LAUNCH(M, RS, RUN)                                                                  \
+    hipLaunchKernelGGL((k_smooth_flat<M, RS, RUN>),                                                  \
+                       dim3(RUN == kListRun ? std::min(nb, 256u * list_waves(M)) : nb), dim3(kBlock), 0, st, d, A, b, \
+                       xin, xout, dvec, cd, cr, ecoarse, dc, gate)
 #define SFP_FLAT_CASE(M)                                                                           \
     case M:                                                                                        \
         if (A.pinned_rowsum) {                                                                     \
-            if (eager) SFP_FLAT_LAUNCH(M, true, true); else SFP_FLAT_LAUNCH(M, true, false);       \
+            if (eager) SFP_FLAT_LAUNCH(M, true, kEagerRun); else SFP_FLAT_LAUNCH(M, true, kBytesRun); \
+        } else if (A.chunks.list) {                                                                \
+            SFP_FLAT_LAUNCH(M, false, kListRun);                                                   \
         } else {                                                                                   \
-            if (eager) SFP_FLAT_LAUNCH(M, false, true); else SFP_FLAT_LAUNCH(M, false, false);     \
+            if (eager) SFP_FLAT_LAUNCH(M, false, kEagerRun); else SFP_FLAT_LAUNCH(M, false, kBytesRun); \
         }                                                                                          \
         break;
         switch (mode) {
@@ -1942,9 +1980,180 @@ void launch_row_activity(hipStream_t st, Dims d, const float *diag32, unsigned c
     SFP_LAUNCH_CHECK();
 }
 
+// flags[q]: whether chunk q (256 cells) holds an active cell. A wavefront per
+// chunk; cells() is a multiple of 4.
+__global__ __launch_bounds__(kBlock) void k_chunk_flags(unsigned n, const float *__restrict__ diag32,
+                                                        unsigned char *__restrict__ flags) {
+    const unsigned q = (blockIdx.x * kBlock + threadIdx.x) / 64, lane = threadIdx.x & 63;
+    const unsigned c = q * kChunk + 4 * lane;
+    bool a = false;
+    if (c < n) {
+        const f4v v = *(const f4v *)(diag32 + c);
+        a = v.x > 0.f || v.y > 0.f || v.z > 0.f || v.w > 0.f;
+    }
+    const unsigned long long m = __ballot(a);
+    if (lane == 0 && q * kChunk < n) flags[q] = m != 0ull ? 1 : 0;
+}
+
+// The set flags' indices in ascending order (so sums over the listed chunks
+// have a fixed order), list[0] their number. A block for either list: a thread counts a run
+// of flags, 16 at a time, the counts are summed over the threads before it, and
+// it writes its run's (65536 chunks of a 256^3 grid: 12 us, beside the clears).
+constexpr int kListThreads = 1024;
+__global__ __launch_bounds__(kListThreads) void k_chunk_list(unsigned nch, const unsigned char *__restrict__ flags,
+                                                             unsigned *__restrict__ list, unsigned nq,
+                                                             const unsigned char *__restrict__ quad_flags,
+                                                             unsigned *__restrict__ quads) {
+    if (blockIdx.x == 1) {
+        nch = nq;
+        flags = quad_flags;
+        list = quads;
+    }
+    __shared__ unsigned sums[kListThreads / 64];
+    const unsigned tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const unsigned per = ((nch + kListThreads - 1) / kListThreads + 15) / 16 * 16;
+    const unsigned b0 = tid * per, b1 = min(b0 + per, nch);
+    auto each = [&](auto f) {
+        for (unsigned b = b0; b < b1; b += 16) {  // (an allocation reaches 64 bytes past its array)
+            const uint4 v = *(const uint4 *)(flags + b);
+            const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (unsigned k = 0; k < 16; k++)
+                if (b + k < b1 && ((w[k / 4] >> (8 * (k % 4))) & 0xffu)) f(b + k);
+        }
+    };
+    unsigned own = 0;
+    each([&](unsigned) { own++; });
+    unsigned sum = own;  // inclusive over the wavefront
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned v = __shfl_up(sum, o, 64);
+        if ((int)lane >= o) sum += v;
+    }
+    if (lane == 63) sums[wave] = sum;
+    __syncthreads();
+    unsigned before = 0, total = 0;
+    for (unsigned w = 0; w < kListThreads / 64; w++) {
+        if (w < wave) before += sums[w];
+        total += sums[w];
+    }
+    unsigned at = 1 + before + sum - own;
+    each([&](unsigned q) { list[at++] = q; });
+    if (tid == 0) list[0] = total;
+}
+
+// flags[u]: whether quad u of the restriction (k_restrict_flat's 64 cells of z
+// in two rows and two planes) meets an active chunk.
+__global__ __launch_bounds__(kBlock) void k_quad_flags(Dims d, unsigned quads,
+                                                       const unsigned char *__restrict__ chunk_flags,
+                                                       unsigned char *__restrict__ flags) {
+    const unsigned u = blockIdx.x * kBlock + threadIdx.x;
+    if (u >= quads) return;
+    const unsigned zch = (unsigned)(d.nz + kRestrictFlatZ - 1) / kRestrictFlatZ, yp = (unsigned)(d.ny + 1) / 2;
+    const int k0 = kRestrictFlatZ * (int)(u % zch), k1 = min(k0 + kRestrictFlatZ, d.nz) - 1;
+    const int j0 = 2 * (int)(u / zch % yp), i0 = 2 * (int)(u / zch / yp);
+    unsigned char a = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int i = min(i0 + (q >> 1), d.nx - 1), j = min(j0 + (q & 1), d.ny - 1);
+        a |= chunk_flags[(unsigned)d.idx(i, j, k0) / kChunk] | chunk_flags[(unsigned)d.idx(i, j, k1) / kChunk];
+    }
+    flags[u] = a;
+}
+
+void launch_active_chunks(hipStream_t st, Dims d, const float *diag32, unsigned char *flags, unsigned *list,
+                          unsigned char *quad_flags, unsigned *quads) {
+    if (!flat_step(d)) throw ArgError("launch_active_chunks: not a flat level");
+    const unsigned n = (unsigned)d.cells(), nch = (n + kChunk - 1) / kChunk, nq = restrict_quads(d);
+    hipLaunchKernelGGL(k_chunk_flags, dim3((nch + kBlock / 64 - 1) / (kBlock / 64)), dim3(kBlock), 0, st, n, diag32,
+                       flags);
+    SFP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_quad_flags, dim3((nq + kBlock - 1) / kBlock), dim3(kBlock), 0, st, d, nq, flags, quad_flags);
+    SFP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_chunk_list, dim3(2), dim3(kListThreads), 0, st, nch, flags, list, nq, quad_flags, quads);
+    SFP_LAUNCH_CHECK();
+}
+
+// The runs of planes that hold k_smooth_pair_rows' work where z rows are
+// inactive: one block per compute unit runs at a time and marches over its run,
+// so equal runs of whole tile columns leave the CUs of the air idle while the
+// liquid's set the time (256^3 pool, 26 % of the rows active: 76 us a pair, 40
+// with this). Runs start at an active plane of their column and take P planes,
+// P the least with which there are no more runs than CUs.
+constexpr int kSegTiles = 128, kSegPlanes = 1024, kSegMin = 8, kSegMax = 56;
+unsigned pair_segments_max(Dims d) {
+    const unsigned ytiles = (unsigned)((d.ny + kRowPairY - 1) / kRowPairY);
+    if (!row_pair(d) || ytiles > (unsigned)kSegTiles || d.nx > kSegPlanes) return 0;
+    return ytiles * (unsigned)((d.nx + kSegMin - 1) / kSegMin);
+}
+__global__ __launch_bounds__(kListThreads) void k_pair_segments(Dims d, int ytiles, int cus,
+                                                                const unsigned char *__restrict__ rowact,
+                                                                int *__restrict__ segments) {
+    __shared__ unsigned long long mask[kSegTiles][kSegPlanes / 64];
+    __shared__ int count[kSegTiles];
+    __shared__ int total;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int words = (d.nx + 63) / 64;
+    if (tid == 0) total = 0;
+    __syncthreads();
+    for (int e = wave; e < ytiles * words; e += kListThreads / 64) {
+        const int by = e / words, w = e % words, q = 64 * w + lane;
+        const int j1 = min((by + 1) * kRowPairY, d.ny);
+        bool a = false;
+        if (q < d.nx)
+            for (int j = by * kRowPairY; j < j1; j++) a |= rowact[(size_t)q * d.ny + j] != 0;
+        const unsigned long long m = __ballot(a);
+        if (lane == 0) {
+            mask[by][w] = m;
+            atomicAdd(&total, __popcll(m));
+        }
+    }
+    __syncthreads();
+    int P = min(kSegMax, max(kSegMin, (total + cus - 1) / cus));
+    auto next_active = [&](int q) {  // the first active plane from q on, or nx
+        for (int w = q / 64; w < words; w++) {
+            const unsigned long long m = mask[tid][w] & (w == q / 64 ? ~0ull << (q % 64) : ~0ull);
+            if (m) return 64 * w + __ffsll(m) - 1;
+        }
+        return d.nx;
+    };
+    while (true) {
+        __syncthreads();
+        if (tid == 0) total = 0;
+        __syncthreads();
+        if (tid < ytiles) {
+            int n = 0;
+            for (int q = next_active(0); q < d.nx; q = q + P < d.nx ? next_active(q + P) : d.nx) n++;
+            count[tid] = n;
+            atomicAdd(&total, n);
+        }
+        __syncthreads();
+        if (total <= cus || P >= kSegMax) break;  // uniform
+        P++;
+    }
+    if (tid < ytiles) {
+        int at = 0;
+        for (int y = 0; y < tid; y++) at += count[y];
+        for (int q = next_active(0); q < d.nx; q = q + P < d.nx ? next_active(q + P) : d.nx) {
+            segments[1 + 3 * at] = tid;
+            segments[2 + 3 * at] = q;
+            segments[3 + 3 * at] = min(q + P, d.nx);
+            at++;
+        }
+        if (tid == ytiles - 1) segments[0] = at;
+    }
+}
+void launch_pair_segments(hipStream_t st, Dims d, const unsigned char *rowact, int *segments) {
+    const int ytiles = (d.ny + kRowPairY - 1) / kRowPairY;
+    if (!pair_segments_max(d)) throw ArgError("launch_pair_segments: not a row-pair level");
+    hipLaunchKernelGGL(k_pair_segments, dim3(1), dim3(kListThreads), 0, st, d, ytiles, device_cus(), rowact,
+                       segments);
+    SFP_LAUNCH_CHECK();
+}
+
 void launch_smooth_pair(hipStream_t st, Dims d, Op32 A, const float *b, const float *x1, float *x3,
                         const float *d1, float cdA, float crA, float cdB, float crB,
-                        const double *gate, const unsigned char *rowact) {
+                        const double *gate, const unsigned char *rowact, const int *segments) {
     if (x1 == x3) throw ArgError("launch_smooth_pair: x3 aliases x1");
     bool rows = row_pair(d);
     for (const float *a : {A.diag, A.cpl[0], A.cpl[1], A.cpl[2], b, x1, (const float *)x3, d1})
@@ -1957,12 +2166,13 @@ void launch_smooth_pair(hipStream_t st, Dims d, Op32 A, const float *b, const fl
         const int runs_max = std::max(1, device_cus() / (int)ytiles);
         int planes = std::min(56, std::max(1, (d.nx + runs_max - 1) / runs_max));
         const unsigned runs = (unsigned)((d.nx + planes - 1) / planes);
-        const dim3 grid(ytiles * runs), block(64, kRowPairRows);
         const bool dx = d1 == x1;
         const unsigned char *ra = A.pinned_rowsum ? nullptr : rowact;
+        const int *sg = ra ? segments : nullptr;
+        const dim3 grid(sg ? pair_segments_max(d) : ytiles * runs), block(64, kRowPairRows);
 #define SFP_ROWPAIR(RS, DX)                                                                      \
     hipLaunchKernelGGL((k_smooth_pair_rows<RS, DX>), grid, block, 0, st, d, A, b, x1, x3, d1, cdA, \
-                       crA, cdB, crB, ra, planes, ytiles, gate)
+                       crA, cdB, crB, ra, sg, planes, ytiles, gate)
         if (A.pinned_rowsum) {
             if (dx) SFP_ROWPAIR(true, true); else SFP_ROWPAIR(true, false);
         } else {
@@ -2019,17 +2229,17 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
                 (uintptr_t)diag32c % 8 == 0;
     for (const float *a : {A.diag, A.cpl[0], A.cpl[1], A.cpl[2], b, x}) flat = flat && (uintptr_t)a % 16 == 0;
     if (flat) {
-        const size_t waves = (size_t)((df.nz + kRestrictFlatZ - 1) / kRestrictFlatZ) *
-                             ((df.ny + 1) / 2) * ((df.nx + 1) / 2);
-        const unsigned nb = (unsigned)((waves * 64 + kBlock - 1) / kBlock);
+        const unsigned nb = (unsigned)(((size_t)restrict_quads(df) * 64 + kBlock - 1) / kBlock);
         const bool eager = df.cells() <= kEagerCells;
-#define SFP_RESTRICT_LAUNCH(RS, EA)                                                                \
-    hipLaunchKernelGGL((k_restrict_flat<RS, EA>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,  \
+#define SFP_RESTRICT_LAUNCH(RS, EA, LI)                                                            \
+    hipLaunchKernelGGL((k_restrict_flat<RS, EA, LI>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,  \
                        bc, x0c, diag32c, c0, gate)
         if (A.pinned_rowsum) {
-            if (eager) SFP_RESTRICT_LAUNCH(true, true); else SFP_RESTRICT_LAUNCH(true, false);
+            if (eager) SFP_RESTRICT_LAUNCH(true, true, false); else SFP_RESTRICT_LAUNCH(true, false, false);
+        } else if (A.chunks.quads) {
+            SFP_RESTRICT_LAUNCH(false, false, true);
         } else {
-            if (eager) SFP_RESTRICT_LAUNCH(false, true); else SFP_RESTRICT_LAUNCH(false, false);
+            if (eager) SFP_RESTRICT_LAUNCH(false, true, false); else SFP_RESTRICT_LAUNCH(false, false, false);
         }
 #undef SFP_RESTRICT_LAUNCH
         SFP_LAUNCH_CHECK();

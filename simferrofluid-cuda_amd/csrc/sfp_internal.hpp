@@ -106,6 +106,15 @@ struct DevBuf {
 // cpl_a[c] >= 0 couples c - e_a and c (0 on the lower boundary, at inactive
 // cells and across solid faces). Inactive cells are identity rows (diag 1)
 // with zero right-hand side and zero solution.
+// The chunks of 256 consecutive cells that hold an active cell (null: every
+// chunk is taken): list[0] is their number, list[1 ..] their indices,
+// ascending. The kernels over the flat cell index then run on the listed chunks
+// only: an inactive chunk's cells are 0 and stay so. quads: the same of the
+// restriction's units of 64 cells in two rows and two planes.
+struct Chunks {
+    const unsigned *list = nullptr, *quads = nullptr;
+};
+constexpr unsigned kChunk = 256;
 struct Op64 {
     const double *diag;
     const double *cpl[3];
@@ -116,6 +125,7 @@ struct Op64 {
     // diagonal). Kernels may then rebuild the diagonal from the couplings
     // they load anyway instead of reading it.
     int pinned_rowsum = 0;
+    Chunks chunks = {};
 };
 struct Op32 {
     const float *diag;  // diagonal for active cells, 0 marks an inactive cell
@@ -123,6 +133,7 @@ struct Op32 {
     // 1: as Op64::pinned_rowsum, with the FP32 sums (cell 0's rebuilt
     // diagonal is 0, an inactive cell, as stored; cells 1, nz and nz*ny differ)
     int pinned_rowsum = 0;
+    Chunks chunks = {};
 };
 
 // One multigrid level: FP64 operator (setup, and the fine level's outer
@@ -135,14 +146,20 @@ struct Level {
     // z rows (i, j) holding an active cell (levels whose step pairs run over
     // whole rows; null elsewhere and where every row is active)
     DevBuf<unsigned char> rowact;
+    // the active chunks (sparse: kept and used), and the step pairs' segments
+    DevBuf<unsigned> chunk_list, quad_list;
+    DevBuf<unsigned char> chunk_flags, quad_flags;
+    DevBuf<int> segments;
+    bool sparse = false;
+    Chunks chunks() const { return sparse ? Chunks{chunk_list.p, quad_list.p} : Chunks{}; }
     // both operators have the row-sum structure of Op64::pinned_rowsum and
     // Op32::pinned_rowsum, and kernels may rebuild the diagonals
     bool pinned_rowsum = false;
     Op64 op64() const {
-        return Op64{diag64.p, {cpl64[0].p, cpl64[1].p, cpl64[2].p}, pinned_rowsum ? 1 : 0};
+        return Op64{diag64.p, {cpl64[0].p, cpl64[1].p, cpl64[2].p}, pinned_rowsum ? 1 : 0, chunks()};
     }
     Op32 op32() const {
-        return Op32{diag32.p, {cpl32[0].p, cpl32[1].p, cpl32[2].p}, pinned_rowsum ? 1 : 0};
+        return Op32{diag32.p, {cpl32[0].p, cpl32[1].p, cpl32[2].p}, pinned_rowsum ? 1 : 0, chunks()};
     }
 };
 

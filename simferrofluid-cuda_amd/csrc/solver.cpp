@@ -80,6 +80,9 @@ KernelTimer::~KernelTimer() {
 }
 
 // ---------------------------------------------------------------- System
+// Grids whose kernels are bound by launch latency rather than bytes.
+static bool small_grid(Dims d) { return d.cells() <= ((size_t)1 << 19); }
+
 // The stencil kernels skip wavefront rows whose cells are all inactive; the
 // skipped cells of the level vectors then keep the zeros written here.
 static void zero_vectors(Level &L) {
@@ -164,24 +167,46 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
         launch_coarsen(ws.stream, F.d, F.op64(), F.diag32.p, C.d, cfg.coarse_scale,
                        pinned_ ? 1.0 : cfg.coarse_scale, C.diag64.p, c64, C.diag32.p, c32);
     }
-    // The dense inverse of the coarsest level (a one-block kernel bound by its
-    // pivot steps) runs on the side stream, overlapping the clears below, the
-    // initial residual and the host's read of it; its first reader joins it.
+    // On the side stream, overlapping the clears below: which rows and chunks of
+    // cells are active (one-block kernels but for the flags), then the dense
+    // inverse of the coarsest level (one block bound by its pivot steps), which
+    // overlaps the initial residual too; the first reader of the inverse joins it.
+    const hipStream_t side = ws.side ? ws.side : ws.stream;
     if (ws.side) {
         SFP_HIP(hipEventRecord(ws.side_in, ws.stream));
-        SFP_HIP(hipStreamWaitEvent(ws.side, ws.side_in, 0));
-        launch_coarse_invert(ws.side, lv_.back().d, lv_.back().op64(), ainv_.p);
-        SFP_HIP(hipEventRecord(ws.side_out, ws.side));
-        ainv_pending_ = true;
-    } else {
-        launch_coarse_invert(ws.stream, lv_.back().d, lv_.back().op64(), ainv_.p);
+        SFP_HIP(hipStreamWaitEvent(side, ws.side_in, 0));
     }
-    // the row-tiled step pairs skip the loads of z rows without active cells
+    bool lists = false;
     for (Level &L : lv_) {
+        // the row-tiled step pairs skip the loads of z rows without active cells
         if (row_pair(L.d) && !L.pinned_rowsum) {
             L.rowact.ensure((size_t)L.d.nx * L.d.ny);
-            launch_row_activity(ws.stream, L.d, L.diag32.p, L.rowact.p);
+            launch_row_activity(side, L.d, L.diag32.p, L.rowact.p);
+            lists = true;
         }
+        // a system of part of the grid: the flat kernels run on the chunks that
+        // hold an active cell (small grids' launches cost the same either way)
+        L.sparse = sparse_ && !(ws.fused_pairs & 32) && flat_step(L.d) && !small_grid(L.d);
+        if (L.sparse) {
+            const size_t nch = (L.d.cells() + kChunk - 1) / kChunk;
+            L.chunk_flags.ensure(nch);
+            L.chunk_list.ensure(nch + 1);
+            L.quad_flags.ensure(restrict_quads(L.d));
+            L.quad_list.ensure(restrict_quads(L.d) + 1);
+            launch_active_chunks(side, L.d, L.diag32.p, L.chunk_flags.p, L.chunk_list.p, L.quad_flags.p,
+                                 L.quad_list.p);
+            if (const unsigned segs = L.pinned_rowsum ? 0 : pair_segments_max(L.d)) {
+                L.segments.ensure(1 + 3 * (size_t)segs);
+                launch_pair_segments(side, L.d, L.rowact.p, L.segments.p);
+            }
+            lists = true;
+        }
+    }
+    if (ws.side && lists) SFP_HIP(hipEventRecord(ws.side_lists, side));
+    launch_coarse_invert(side, lv_.back().d, lv_.back().op64(), ainv_.p);
+    if (ws.side) {
+        SFP_HIP(hipEventRecord(ws.side_out, side));
+        ainv_pending_ = true;
     }
     // Every kernel skips groups of inactive cells (rows, tiles, pairs of
     // rows) and writes 0 at the inactive cells of the groups it processes
@@ -209,6 +234,7 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     }
     ca.w = w_.p;
     launch_clear_inactive(ws.stream, ca);
+    if (ws.side && lists) SFP_HIP(hipStreamWaitEvent(ws.stream, ws.side_lists, 0));
 }
 
 // (see launch_vcycle_tail_lds)
@@ -257,9 +283,6 @@ float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
     else launch_vcycle_tail(ws.stream, t, ws.gate);
     return tail_result(t);
 }
-
-// Grids whose kernels are bound by launch latency rather than bytes.
-static bool small_grid(Dims d) { return d.cells() <= ((size_t)1 << 19); }
 
 // One separate launch of a step or the restriction on a level (us): 3.1 us
 // up to 64^3 whatever it computes, 5.6 ns per thousand cells above (measured:
@@ -402,7 +425,7 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
             // reads x0, b, diag, 3 couplings; writes x
             if (fine && ws.profiling) ws.timers[K_SMOOTH_PAIR].begin(st, (24.0 + pair_diag_bytes) * cells);
             launch_smooth_pair(st, L.d, A, L.b.p, cur, oth, cur, cb.cd[1], cb.cr[1], cb.cd[2], cb.cr[2],
-                               ws.gate, L.rowact.p);
+                               ws.gate, L.rowact.p, L.sparse ? L.segments.p : nullptr);
             if (fine && ws.profiling) ws.timers[K_SMOOTH_PAIR].end(st);
             std::swap(cur, oth);
         } else {
@@ -495,7 +518,7 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
         oth = last_out(ws, l, oth);
         if (track) ws.timers[K_SMOOTH_PAIR].begin(st, (L.pinned_rowsum ? 28.0 : 32.0) * (double)L.d.cells());
         launch_smooth_pair(st, L.d, A, L.b.p, cur, oth, L.dv.p, cb.cd[deg - 2], cb.cr[deg - 2],
-                           cb.cd[deg - 1], cb.cr[deg - 1], ws.gate, L.rowact.p);
+                           cb.cd[deg - 1], cb.cr[deg - 1], ws.gate, L.rowact.p, L.sparse ? L.segments.p : nullptr);
         if (track) ws.timers[K_SMOOTH_PAIR].end(st);
         std::swap(cur, oth);
     }
@@ -734,7 +757,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             ws.x0_level = -1;
             // (a cycle whose first launch folds forms its first iterate itself)
             float *const x0_next = fold ? nullptr : x0;
-            launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, w_.p, q_.p, r_.p, b32, x0_next, c0,
+            launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, A.chunks.list, w_.p, q_.p, r_.p, b32, x0_next, c0,
                               first ? 1 : 0, iter + it, fold, ws.partials.p, ws.scalars.p, ws.gate, done,
                               it + 1 == batch ? ws.host_sc : nullptr);
             if (profiling) ws.timers[K_UPDATE64].end_recorded();

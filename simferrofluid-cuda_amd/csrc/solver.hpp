@@ -137,7 +137,8 @@ struct Workspace {
     // inverse is formed while `stream` runs the rest of the set-up; side_in
     // orders it after the coarsening, side_out orders its first use after it
     hipStream_t side = nullptr;
-    hipEvent_t side_in = nullptr, side_out = nullptr;
+    // (side_lists: the lists of active cells before it)
+    hipEvent_t side_in = nullptr, side_out = nullptr, side_lists = nullptr;
     void wait() { SFP_HIP(hipStreamSynchronize(stream)); }
 };
 
@@ -207,6 +208,9 @@ class System {
     // level, the coarse problems would approach the singular Neumann one,
     // and the V-cycle would overshoot the near-constant mode.
     bool pinned_ = false;
+    // Inactive cells are expected (the air of a pressure system): levels over
+    // the flat cell index keep the list of their active chunks.
+    bool sparse_ = false;
 
   private:
     enum Cycle { kCycleLearned, kCycleSmooth, kCycleRestrictOnly };
