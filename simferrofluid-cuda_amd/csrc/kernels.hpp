@@ -38,8 +38,10 @@ void launch_smooth(hipStream_t s, int mode, Dims d, Op32 A, const double *r64, f
 // tiles overlap by one cell per side; measured equal at 128^3, faster above).
 inline bool pair_pays(Dims d) { return d.nz >= 64 && d.cells() > ((size_t)1 << 21); }
 // Grids on which launch_smooth runs its steps (all but the fused first step)
-// over the flat cell index: nz a multiple of 4, fewer than 2^32 cells.
+// over the flat cell index: fewer than 2^32 cells. whole_groups: with the
+// prolongation too (nz a multiple of 4).
 bool flat_step(Dims d);
+bool whole_groups(Dims d);
 // Grids with z rows of 193..256 cells in groups of four run it over whole
 // rows (k_smooth_pair_rows); rowact (null: all active) marks the z rows
 // holding an active cell (launch_row_activity), whose loads the others skip.
@@ -68,8 +70,8 @@ void launch_smooth_restrict(hipStream_t s, Dims d, Op32 A, const float *b, const
                             float *x2, const float *d1, float cd, float cr, float *bc,
                             const double *gate = nullptr);
 // x += P e on active cells (diag32 > 0), in place.
-void launch_prolong_add(hipStream_t s, Dims d, const float *diag32, const float *ecoarse, float *x,
-                        const double *gate = nullptr);
+void launch_prolong_add(hipStream_t s, Dims d, const float *diag32, const unsigned *list, const float *ecoarse,
+                        float *x, const double *gate = nullptr);
 // bc = R (b - A x): sum of the residuals of the (up to 8) children. With
 // x0c, also x0c = c0 Dc^-1 bc (diag32c: the coarse FP32 diagonal), the first
 // Chebyshev iterate of the coarse level's cycle, as the FCG update stores it

@@ -221,39 +221,79 @@ __device__ __forceinline__ f4v rowsum_diag4(f4v cxc, f4v cxp, f4v cym, f4v cyp, 
     for (int q = 0; q < 4; q++) dg[q] = rowsum_diag(cxc[q], cxp[q], cym[q], cyp[q], cz[q], q < 3 ? cz[q + 1] : czhi);
     return dg;
 }
-// The group starting at cell c (c a multiple of 4, nz a multiple of 4) holds
-// none of the cells whose diagonal is not the row sum (1, nz, nz*ny).
+// The group of four cells from c on holds none of the cells whose diagonal is
+// not the row sum (0, 1, nz, nz*ny); kAny: it may start at any cell.
+template <bool kAny = false>
 __device__ __forceinline__ bool rowsum_group(const Op32 &A, size_t c, Dims d) {
-    return A.pinned_rowsum && c != 0 && c != (size_t)d.nz && c != (size_t)d.ny * d.nz;
+    if constexpr (!kAny) return A.pinned_rowsum && c != 0 && c != (size_t)d.nz && c != (size_t)d.ny * d.nz;
+    const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy, cu = (unsigned)c;
+    return A.pinned_rowsum && cu > 1 && sy - cu >= 4 && sx - cu >= 4;  // (differences below 0 are large)
 }
 
-// The operands of one group: every address is inside the grid (a missing
-// neighbour's is the group's own; its coupling is 0, the lower ones as
-// stored, the upper ones by selection), so the loads need no branches and are
-// all in flight together.
+// The operands of one group, which (kAny: nz no multiple of 4) need not lie
+// within a z row: a neighbour is sx, sy or 1 cells on in the array wherever the
+// row or the plane ends, since the coupling to what lies across an end is 0 as
+// stored (the lower one of the first cell there). A missing neighbour group's
+// address is the group's own, and the upper couplings past the array are put to
+// 0 by selection, so the loads need no branches and are all in flight together.
+// With kAny a neighbour's group is at any 4-byte address. One that crosses the
+// array's end is loaded past it (an allocation reaches 64 bytes past its array)
+// and one that crosses its start is loaded from the start and moved; the cells
+// outside are put to 0 (end_cells). (Branches of the lanes here, on these rare
+// groups, cost 20 registers; with a uniform part in their condition they were
+// compiled to loads at undefined addresses.)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 struct GroupOperands {
     f4v xc, xm, xp, ym, yp, cx, cxp, cy, cyp, cz, b;
     float zlo, zhi, czhi;
 };
+// the first `k` cells of a group stay, the others are put to 0
+__device__ __forceinline__ f4v first_cells(f4v v, unsigned k) {
+#pragma unroll
+    for (unsigned q = 0; q < 4; q++) v[q] = q < k ? v[q] : 0.f;
+    return v;
+}
+// a group moved up by k cells, 0 below
+__device__ __forceinline__ f4v moved_up(f4v v, unsigned k) {
+    if (k & 1) v = f4v{0.f, v.x, v.y, v.z};
+    if (k & 2) v = f4v{0.f, 0.f, v.x, v.y};
+    return k < 4 ? v : f4v{0.f, 0.f, 0.f, 0.f};
+}
+// a group's own cells of an array, 0 past its end
+template <bool kAny>
+__device__ __forceinline__ f4v own_cells(const float *__restrict__ a, unsigned c, unsigned n) {
+    const f4v v = *(const f4u *)(a + c);
+    return kAny ? first_cells(v, n - c) : v;
+}
+template <bool kAny>
+__device__ __forceinline__ void store_cells(float *__restrict__ a, unsigned c, unsigned n, f4v v) {
+    if (!kAny || n - c >= 4) {
+        *(f4u *)(a + c) = v;
+    } else {
+#pragma unroll
+        for (unsigned q = 0; q < 4; q++)
+            if (c + q < n) a[c + q] = v[q];
+    }
+}
+template <bool kAny>
 __device__ __forceinline__ GroupOperands load_operands(const Op32 &A, const float *__restrict__ b,
-                                                       const float *__restrict__ x, Dims d, unsigned c, int i, int j,
-                                                       int k) {
-    const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy;
-    const bool xh = i + 1 < d.nx, yh = j + 1 < d.ny, zh = k + 4 < d.nz;
-    const unsigned cxm = i > 0 ? c - sx : c, cxu = xh ? c + sx : c, cym = j > 0 ? c - sy : c, cyu = yh ? c + sy : c;
-    const unsigned czl = k > 0 ? c - 1 : c, czu = zh ? c + 4 : c;
+                                                       const float *__restrict__ x, Dims d, unsigned c) {
+    const unsigned n = (unsigned)d.cells(), sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy, left = n - c;
+    const unsigned cxm = c >= sx ? c - sx : 0, cym = c >= sy ? c - sy : 0;
+    const unsigned cxu = left > sx ? c + sx : c, cyu = left > sy ? c + sy : c;
+    const unsigned czl = c > 0 ? c - 1 : c, czu = left > 4 ? c + 4 : c;
     GroupOperands g;
-    g.xc = *(const f4v *)(x + c);
-    g.xm = *(const f4v *)(x + cxm);
-    g.xp = *(const f4v *)(x + cxu);
-    g.ym = *(const f4v *)(x + cym);
-    g.yp = *(const f4v *)(x + cyu);
-    g.cx = *(const f4v *)(A.cpl[0] + c);
-    g.cxp = *(const f4v *)(A.cpl[0] + cxu);
-    g.cy = *(const f4v *)(A.cpl[1] + c);
-    g.cyp = *(const f4v *)(A.cpl[1] + cyu);
-    g.cz = *(const f4v *)(A.cpl[2] + c);
-    g.b = *(const f4v *)(b + c);
+    g.xc = *(const f4u *)(x + c);
+    g.xm = *(const f4u *)(x + cxm);
+    g.xp = *(const f4u *)(x + cxu);
+    g.ym = *(const f4u *)(x + cym);
+    g.yp = *(const f4u *)(x + cyu);
+    g.cx = *(const f4u *)(A.cpl[0] + c);
+    g.cxp = *(const f4u *)(A.cpl[0] + cxu);
+    g.cy = *(const f4u *)(A.cpl[1] + c);
+    g.cyp = *(const f4u *)(A.cpl[1] + cyu);
+    g.cz = *(const f4u *)(A.cpl[2] + c);
+    g.b = *(const f4u *)(b + c);
     g.zlo = x[czl];
     g.zhi = x[czu];
     g.czhi = A.cpl[2][czu];
@@ -265,12 +305,33 @@ __device__ __forceinline__ void pin(const GroupOperands &g) {
     sfp::pin(g.zhi);
     sfp::pin(g.czhi);
 }
-// The upper couplings at the grid's end.
-__device__ __forceinline__ void end_couplings(GroupOperands &g, Dims d, int i, int j, int k) {
-    const f4v z4 = {0.f, 0.f, 0.f, 0.f};
-    if (!(i + 1 < d.nx)) g.cxp = z4;
-    if (!(j + 1 < d.ny)) g.cyp = z4;
-    if (!(k + 4 < d.nz)) g.czhi = 0.f;
+// What lies past the array put to 0: the upper couplings and (kAny) the cells of
+// groups that cross its ends.
+template <bool kAny>
+__device__ __forceinline__ void end_cells(GroupOperands &g, Dims d, unsigned c) {
+    const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy, left = (unsigned)d.cells() - c;
+    if constexpr (kAny) {
+        const unsigned xu = left > sx ? left - sx : 0, yu = left > sy ? left - sy : 0;  // cells there are
+        g.cxp = first_cells(g.cxp, xu);
+        g.xp = first_cells(g.xp, xu);
+        g.cyp = first_cells(g.cyp, yu);
+        g.yp = first_cells(g.yp, yu);
+        const unsigned xd = c < sx ? sx - c : 0, yd = c < sy ? sy - c : 0;  // (from 4 on: none, coupled with 0)
+        if (__any((xd - 1 < 3) | (yd - 1 < 3))) {
+            g.xm = moved_up(g.xm, xd);
+            g.ym = moved_up(g.ym, yd);
+        }
+        g.xc = first_cells(g.xc, left);
+        g.cx = first_cells(g.cx, left);
+        g.cy = first_cells(g.cy, left);
+        g.cz = first_cells(g.cz, left);
+        g.b = first_cells(g.b, left);
+    } else {
+        const f4v z4 = {0.f, 0.f, 0.f, 0.f};
+        if (!(left > sx)) g.cxp = z4;
+        if (!(left > sy)) g.cyp = z4;
+    }
+    if (!(left > 4)) g.czhi = 0.f;
 }
 
 // kEagerRun (levels of at most kEagerCells cells, where a launch is one round of
@@ -285,10 +346,10 @@ __device__ __forceinline__ void end_couplings(GroupOperands &g, Dims d, int i, i
 // copy rate being 31; its 128^3 level 11.8, 6.5 so).
 enum FlatRun { kBytesRun, kEagerRun, kListRun };
 // (wavefronts per SIMD the registers of a mode allow: blocks of a list run per CU)
-constexpr int list_waves(int mode) { return (mode & SM_PROLONG) ? 7 : 8; }
+constexpr int list_waves(int mode, bool any) { return (mode & SM_PROLONG) || any ? 7 : 8; }
 
-template <int MODE, bool kRowsum, FlatRun kRun>
-__global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE) : 1) void k_smooth_flat(
+template <int MODE, bool kRowsum, FlatRun kRun, bool kAny>
+__global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE, kAny) : 1) void k_smooth_flat(
                                                         Dims d, Op32 A, const float *__restrict__ b,
                                                         const float *__restrict__ xin,
                                                         float *__restrict__ xout, float *dvec,
@@ -301,30 +362,31 @@ __global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE) : 1) vo
     typedef float f2 __attribute__((ext_vector_type(2)));
     constexpr bool kEager = kRun == kEagerRun;
     static_assert(kRun != kListRun || !kRowsum, "no list where every cell is active");
+    static_assert(!kAny || !kProlong, "the prolongation reads z rows of whole groups");
     const double stop = load_gate(gate, A.diag);
-    const unsigned n = (unsigned)d.cells();  // a multiple of 4 below 2^32
+    const unsigned n = (unsigned)d.cells();  // below 2^32
     auto group = [&](unsigned ct) {  // the group of cells from ct on
         const bool on = ct < n;
-        const unsigned c = on ? ct : n - 4;
-        const bool rs = kRowsum && rowsum_group(A, c, d);  // every group there has an active cell
+        const unsigned c = on ? ct : (n - 1) & ~3u;
+        const bool rs = kRowsum && rowsum_group<kAny>(A, c, d);  // every group there has an active cell
         f4 dg = {0.f, 0.f, 0.f, 0.f};
-        if (!rs) dg = *(const f4 *)(A.diag + c);
+        if (!rs) dg = own_cells<kAny>(A.diag, c, n);
         if constexpr (kRun == kBytesRun) {
             if (stop != 0.0) return;
             const bool act = on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f);
             if (!__any(act)) return;
         }
-        // (i, j, k) of the first cell
-        const unsigned t = c / (unsigned)d.nz;
-        const int k = (int)(c - t * (unsigned)d.nz);
-        const unsigned iu = t / (unsigned)d.ny;
-        const int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny);
-        GroupOperands g = load_operands(A, b, xin, d, c, i, j, k);
+        GroupOperands g = load_operands<kAny>(A, b, xin, d, c);
         f4 dprev = {0.f, 0.f, 0.f, 0.f};
-        if constexpr ((MODE & SM_READ_D) != 0) dprev = *(const f4 *)(dvec + c);
+        if constexpr ((MODE & SM_READ_D) != 0) dprev = own_cells<kAny>(dvec, c, n);
         f2 ec, e_xm, e_xp, e_ym, e_yp;
         float ezlo = 0.f, ezhi = 0.f;
         if constexpr (kProlong) {
+            // (i, j, k) of the first cell (z rows of whole groups)
+            const unsigned t = c / (unsigned)d.nz;
+            const int k = (int)(c - t * (unsigned)d.nz);
+            const unsigned iu = t / (unsigned)d.ny;
+            const int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny);
             // coarse values of the group's two coarse cells in this row and in the
             // neighbouring rows and planes (16-byte aligned groups: k >> 1 even)
             const int kc = k >> 1, jl = max(j - 1, 0) >> 1, jh = min(j + 1, d.ny - 1) >> 1, il = max(i - 1, 0) >> 1,
@@ -349,7 +411,7 @@ __global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE) : 1) vo
             }
             if (stop != 0.0) return;
         }
-        end_couplings(g, d, i, j, k);
+        end_cells<kAny>(g, d, c);
         if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
         const f4 xin_c = g.xc;
         if constexpr (kProlong) {
@@ -384,8 +446,8 @@ __global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE) : 1) vo
             dno[q] = dn;
         }
         if (!on) return;
-        *(f4 *)(xout + c) = xo;
-        if constexpr ((MODE & SM_WRITE_D) != 0) *(f4 *)(dvec + c) = dno;
+        store_cells<kAny>(xout, c, n, xo);
+        if constexpr ((MODE & SM_WRITE_D) != 0) store_cells<kAny>(dvec, c, n, dno);
     };
     if constexpr (kRun == kListRun) {
         if (stop != 0.0) return;
@@ -885,20 +947,40 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
 // place, before a plain first post-smoothing step: on large grids this pass
 // and the step cost less than the step that adds the correction at every
 // neighbour it reads (the coarse values' gathers cost a third of that step).
-__global__ __launch_bounds__(kBlock) void k_prolong_add(CellGrid cg, Dims d, const float *__restrict__ diag32,
+// Groups of four cells over the flat cell index, as k_smooth_flat; kList: of the
+// listed chunks.
+template <bool kList>
+__global__ __launch_bounds__(kBlock) void k_prolong_add(Dims d, const unsigned *__restrict__ list,
+                                                        const float *__restrict__ diag32,
                                                         const float *__restrict__ e, Dims dc,
                                                         float *__restrict__ x, const double *gate) {
     if (gated(gate)) return;
-    int k, j, i0;
-    cell_tile(cg, k, j, i0);
-    if (k >= d.nz || j >= d.ny) return;
-    const Strides s(d);
-    const size_t dcsx = (size_t)dc.ny * dc.nz;
-    const size_t eo = dc.idx(0, j >> 1, k >> 1);
-    size_t c = d.idx(i0, j, k);
-    for (int i = i0, ie = min(i0 + cg.planes, d.nx); i < ie; i++, c += s.sx) {
-        if (!(diag32[c] > 0.f)) continue;
-        x[c] = x[c] + e[(size_t)(i >> 1) * dcsx + eo];
+    const unsigned n = (unsigned)d.cells();
+    auto group = [&](unsigned c) {
+        if (c >= n) return;
+        const f4v dg = own_cells<true>(diag32, c, n);
+        if (!(dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f)) return;
+        f4v v = own_cells<true>(x, c, n);
+        const unsigned t = c / (unsigned)d.nz, iu = t / (unsigned)d.ny;
+        int i = (int)iu, j = (int)(t - iu * (unsigned)d.ny), k = (int)(c - t * (unsigned)d.nz);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (dg[q] > 0.f) v[q] = v[q] + e[dc.idx(i >> 1, j >> 1, k >> 1)];
+            if (++k == d.nz) {  // the next row
+                k = 0;
+                if (++j == d.ny) {
+                    j = 0;
+                    i++;
+                }
+            }
+        }
+        store_cells<true>(x, c, n, v);
+    };
+    if constexpr (kList) {
+        const unsigned units = list[0], waves = flat_waves();
+        for (unsigned u = flat_wave(); u < units; u += waves) group(list_cell<4>(list, u));
+    } else {
+        group(blockIdx.x * kSmoothFlatCells + 4 * (unsigned)flat_tid());
     }
 }
 
@@ -984,8 +1066,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict(CellGrid cg, Dims df, Op32 
     }
 }
 
-// The same restriction over the flat cell index (grids with nz a multiple of
-// 4): a wavefront covers 64 cells of a z row in two rows and two planes, four
+// The same restriction over the flat cell index: a wavefront covers 64 cells of a z row in two rows and two planes, four
 // cells per lane (lanes 0-15: row j, plane i; 16-31: row j+1; 32-63: plane
 // i+1), so a coarse cell's children are added in k_restrict's order -- the z
 // pair in the lane, the y pair across lanes 16 apart, the x pair across lanes
@@ -995,7 +1076,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict(CellGrid cg, Dims df, Op32 
 // stores zeros.
 constexpr int kRestrictFlatZ = 64;  // z cells per wavefront
 
-template <bool kRowsum, bool kEager, bool kList>
+template <bool kRowsum, bool kEager, bool kList, bool kAny>
 __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const float *__restrict__ b,
                                                           const float *__restrict__ x, Dims dc,
                                                           float *__restrict__ bc, float *__restrict__ x0c,
@@ -1019,11 +1100,11 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
     const int kw = kRestrictFlatZ * (int)kz + 4 * (lane & 15);
     const bool on = iw < df.nx && jw < df.ny && kw < df.nz;
     // lanes outside the grid load the nearest cells and drop them
-    const int i = min(iw, df.nx - 1), j = min(jw, df.ny - 1), k = min(kw, df.nz - 4);
-    const unsigned c = (unsigned)df.idx(i, j, k);
-    const bool rs = kRowsum && rowsum_group(A, c, df);  // every group there has an active cell
+    const int i = min(iw, df.nx - 1), j = min(jw, df.ny - 1), k = min(kw, (df.nz - 1) & ~3);
+    const unsigned c = (unsigned)df.idx(i, j, k), n = (unsigned)df.cells();
+    const bool rs = kRowsum && rowsum_group<kAny>(A, c, df);  // every group there has an active cell
     f4 dg = {0.f, 0.f, 0.f, 0.f};
-    if (!rs) dg = *(const f4 *)(A.diag + c);
+    if (!rs) dg = own_cells<kAny>(A.diag, c, n);
     f4 r = {0.f, 0.f, 0.f, 0.f};
     bool any = true;
     if constexpr (!kEager && !kList) {
@@ -1031,13 +1112,13 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
         any = __any(on && (rs || dg.x > 0.f || dg.y > 0.f || dg.z > 0.f || dg.w > 0.f));
     }
     if (any) {
-        GroupOperands g = load_operands(A, b, x, df, c, i, j, k);
+        GroupOperands g = load_operands<kAny>(A, b, x, df, c);
         if constexpr (kEager) {
             pin(g);
             sfp::pin(dg);
             if (stop != 0.0) return;
         }
-        end_couplings(g, df, i, j, k);
+        end_cells<kAny>(g, df, c);
         if (rs) dg = rowsum_diag4(g.cx, g.cxp, g.cy, g.cyp, g.cz, g.czhi);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -1051,7 +1132,8 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
             off = fmaf(g.cz[q], xzm, off);
             off = fmaf(czp, xzp, off);
             const float rr = g.b[q] - fmaf(dg[q], g.xc[q], -off);
-            r[q] = on && dg[q] > 0.f ? rr : 0.f;
+            // (past the row: the next one's)
+            r[q] = on && (!kAny || kw + q < df.nz) && dg[q] > 0.f ? rr : 0.f;
         }
     }
     float s0 = r.x + r.y, s1 = r.z + r.w;  // z pairs
@@ -1067,13 +1149,22 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
         v.y += s1;
         v.y += o1;
         const size_t q = dc.idx((int)ip, (int)jp, k >> 1);
-        *(f2 *)(bc + q) = v;
-        if (x0c) {
-            const f2 dgc = *(const f2 *)(diag32c + q);
-            f2 x0;
-            x0.x = c0 * rcp_or_zero(dgc.x) * v.x;
-            x0.y = c0 * rcp_or_zero(dgc.y) * v.y;
-            *(f2 *)(x0c + q) = x0;
+        if constexpr (!kAny) {
+            *(f2 *)(bc + q) = v;
+            if (x0c) {
+                const f2 dgc = *(const f2 *)(diag32c + q);
+                f2 x0;
+                x0.x = c0 * rcp_or_zero(dgc.x) * v.x;
+                x0.y = c0 * rcp_or_zero(dgc.y) * v.y;
+                *(f2 *)(x0c + q) = x0;
+            }
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                if ((k >> 1) + h < dc.nz) {
+                    bc[q + h] = v[h];
+                    if (x0c) x0c[q + h] = c0 * rcp_or_zero(diag32c[q + h]) * v[h];
+                }
         }
     }
 }
@@ -1852,15 +1943,17 @@ unsigned restrict_quads(Dims d) {
            (unsigned)((d.nx + 1) / 2);
 }
 
-bool flat_step(Dims d) { return d.nz % 4 == 0 && d.cells() < (size_t(1) << 32); }
+bool flat_step(Dims d) { return d.cells() < (size_t(1) << 32) - 64; }
+bool whole_groups(Dims d) { return d.nz % 4 == 0 && flat_step(d); }
 
-// The flat step where it applies: no fused first step, z rows of whole
-// 4-cell groups, 16-byte aligned arrays (8-byte aligned coarse values). On
-// MI355X 12 % faster than x-plane tiles at 256^3, 17 % at 128^3.
+// The flat step where it applies: no fused first step, 16-byte aligned arrays;
+// with the prolongation z rows of whole 4-cell groups (8-byte aligned coarse
+// values). On MI355X 12 % faster than x-plane tiles at 256^3, 17 % at 128^3, and
+// 14.5 us instead of 26 at 131 x 129 x 133 (the restriction 13 instead of 29).
 static bool smooth_flat(Dims d, int mode, const double *r64, const float *ecoarse,
                         std::initializer_list<const float *> arrays) {
     if ((mode & SM_FIRST) || r64 || !flat_step(d)) return false;
-    if ((mode & SM_PROLONG) && (uintptr_t)ecoarse % 8) return false;
+    if ((mode & SM_PROLONG) && (!whole_groups(d) || (uintptr_t)ecoarse % 8)) return false;
     for (const float *a : arrays)
         if ((uintptr_t)a % 16) return false;
     return true;
@@ -1872,11 +1965,17 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
     if (smooth_flat(d, mode, r64, ecoarse, {A.diag, A.cpl[0], A.cpl[1], A.cpl[2], b, xin, xout, dvec})) {
         const unsigned nb = (unsigned)((d.cells() + kSmoothFlatCells - 1) / kSmoothFlatCells);
         const Dims dc = d.coarse();
-        const bool eager = d.cells() <= kEagerCells;
-#define SFP_FLAT_LAUNCH(M, RS, RUN)                                                                  \
-    hipLaunchKernelGGL((k_smooth_flat<M, RS, RUN>),                                                  \
-                       dim3(RUN == kListRun ? std::min(nb, 256u * list_waves(M)) : nb), dim3(kBlock), 0, st, d, A, b, \
+        const bool eager = d.cells() <= kEagerCells, any = !whole_groups(d);
+#define SFP_FLAT_RUN(M, RS, RUN, ANY)                                                                \
+    hipLaunchKernelGGL((k_smooth_flat<M, RS, RUN, ANY>),                                               \
+                       dim3(RUN == kListRun ? std::min(nb, 256u * list_waves(M, ANY)) : nb), dim3(kBlock), 0, st, d, A, b, \
                        xin, xout, dvec, cd, cr, ecoarse, dc, gate)
+#define SFP_FLAT_LAUNCH(M, RS, RUN)                                                                  \
+    do {                                                                                             \
+        if constexpr (((M) & SM_PROLONG) != 0) SFP_FLAT_RUN(M, RS, RUN, false);                      \
+        else if (any) SFP_FLAT_RUN(M, RS, RUN, true);                                                \
+        else SFP_FLAT_RUN(M, RS, RUN, false);                                                        \
+    } while (0)
 #define SFP_FLAT_CASE(M)                                                                           \
     case M:                                                                                        \
         if (A.pinned_rowsum) {                                                                     \
@@ -1901,6 +2000,7 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
         }
 #undef SFP_FLAT_CASE
 #undef SFP_FLAT_LAUNCH
+#undef SFP_FLAT_RUN
         SFP_LAUNCH_CHECK();
         return;
     }
@@ -1981,14 +2081,14 @@ void launch_row_activity(hipStream_t st, Dims d, const float *diag32, unsigned c
 }
 
 // flags[q]: whether chunk q (256 cells) holds an active cell. A wavefront per
-// chunk; cells() is a multiple of 4.
+// chunk.
 __global__ __launch_bounds__(kBlock) void k_chunk_flags(unsigned n, const float *__restrict__ diag32,
                                                         unsigned char *__restrict__ flags) {
     const unsigned q = (blockIdx.x * kBlock + threadIdx.x) / 64, lane = threadIdx.x & 63;
     const unsigned c = q * kChunk + 4 * lane;
     bool a = false;
     if (c < n) {
-        const f4v v = *(const f4v *)(diag32 + c);
+        const f4v v = own_cells<true>(diag32, c, n);
         a = v.x > 0.f || v.y > 0.f || v.z > 0.f || v.w > 0.f;
     }
     const unsigned long long m = __ballot(a);
@@ -2206,10 +2306,16 @@ void launch_smooth_restrict(hipStream_t st, Dims d, Op32 A, const float *b, cons
     SFP_LAUNCH_CHECK();
 }
 
-void launch_prolong_add(hipStream_t st, Dims d, const float *diag32, const float *ecoarse, float *x,
-                        const double *gate) {
-    Launch L = cell_launch(d, 0, 8);
-    hipLaunchKernelGGL(k_prolong_add, L.grid, L.block, 0, st, L.cg, d, diag32, ecoarse, d.coarse(), x, gate);
+void launch_prolong_add(hipStream_t st, Dims d, const float *diag32, const unsigned *list, const float *ecoarse,
+                        float *x, const double *gate) {
+    if (!flat_step(d)) throw ArgError("launch_prolong_add: grid too large");
+    const unsigned nb = (unsigned)((d.cells() + kSmoothFlatCells - 1) / kSmoothFlatCells);
+    if (list)
+        hipLaunchKernelGGL(k_prolong_add<true>, dim3(std::min(nb, 2048u)), dim3(kBlock), 0, st, d, list, diag32,
+                           ecoarse, d.coarse(), x, gate);
+    else
+        hipLaunchKernelGGL(k_prolong_add<false>, dim3(nb), dim3(kBlock), 0, st, d, list, diag32, ecoarse,
+                           d.coarse(), x, gate);
     SFP_LAUNCH_CHECK();
 }
 
@@ -2231,9 +2337,14 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
     if (flat) {
         const unsigned nb = (unsigned)(((size_t)restrict_quads(df) * 64 + kBlock - 1) / kBlock);
         const bool eager = df.cells() <= kEagerCells;
-#define SFP_RESTRICT_LAUNCH(RS, EA, LI)                                                            \
-    hipLaunchKernelGGL((k_restrict_flat<RS, EA, LI>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc,  \
+#define SFP_RESTRICT_RUN(RS, EA, LI, ANY)                                                              \
+    hipLaunchKernelGGL((k_restrict_flat<RS, EA, LI, ANY>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc, \
                        bc, x0c, diag32c, c0, gate)
+#define SFP_RESTRICT_LAUNCH(RS, EA, LI)                      \
+    do {                                                     \
+        if (whole_groups(df)) SFP_RESTRICT_RUN(RS, EA, LI, false); \
+        else SFP_RESTRICT_RUN(RS, EA, LI, true);             \
+    } while (0)
         if (A.pinned_rowsum) {
             if (eager) SFP_RESTRICT_LAUNCH(true, true, false); else SFP_RESTRICT_LAUNCH(true, false, false);
         } else if (A.chunks.quads) {
@@ -2242,6 +2353,7 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
             if (eager) SFP_RESTRICT_LAUNCH(false, true, false); else SFP_RESTRICT_LAUNCH(false, false, false);
         }
 #undef SFP_RESTRICT_LAUNCH
+#undef SFP_RESTRICT_RUN
         SFP_LAUNCH_CHECK();
         return;
     }
@@ -2256,7 +2368,7 @@ void launch_coarsen(hipStream_t st, Dims df, Op64 Af, const float *diag32f, Dims
                     double scale, double rs_scale, double *diag64c, double *const cpl64c[3],
                     float *diag32c, float *const cpl32c[3]) {
     MutFaces m{{cpl64c[0], cpl64c[1], cpl64c[2]}};
-    bool flat = flat_step(df) && (uintptr_t)diag32f % 16 == 0;
+    bool flat = whole_groups(df) && (uintptr_t)diag32f % 16 == 0;
     for (const double *a : {Af.diag, Af.cpl[0], Af.cpl[1], Af.cpl[2]}) flat = flat && (uintptr_t)a % 16 == 0;
     if (flat) {
         const size_t waves = (size_t)((df.nz + 63) / 64) * ((df.ny + 1) / 2) * ((df.nx + 1) / 2);

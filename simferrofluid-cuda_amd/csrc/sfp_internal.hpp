@@ -101,11 +101,6 @@ struct DevBuf {
 };
 
 // ------------------------------------------------------------------ operators
-// A 7-point symmetric operator on a cell grid:
-//   (A x)_c = diag_c x_c - sum_a ( cpl_a[c] x_{c-e_a} + cpl_a[c+e_a] x_{c+e_a} )
-// cpl_a[c] >= 0 couples c - e_a and c (0 on the lower boundary, at inactive
-// cells and across solid faces). Inactive cells are identity rows (diag 1)
-// with zero right-hand side and zero solution.
 // The chunks of 256 consecutive cells that hold an active cell (null: every
 // chunk is taken): list[0] is their number, list[1 ..] their indices,
 // ascending. The kernels over the flat cell index then run on the listed chunks
@@ -115,6 +110,12 @@ struct Chunks {
     const unsigned *list = nullptr, *quads = nullptr;
 };
 constexpr unsigned kChunk = 256;
+
+// A 7-point symmetric operator on a cell grid:
+//   (A x)_c = diag_c x_c - sum_a ( cpl_a[c] x_{c-e_a} + cpl_a[c+e_a] x_{c+e_a} )
+// cpl_a[c] >= 0 couples c - e_a and c (0 on the lower boundary, at inactive
+// cells and across solid faces). Inactive cells are identity rows (diag 1)
+// with zero right-hand side and zero solution.
 struct Op64 {
     const double *diag;
     const double *cpl[3];

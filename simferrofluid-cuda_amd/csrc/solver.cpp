@@ -80,6 +80,11 @@ KernelTimer::~KernelTimer() {
 }
 
 // ---------------------------------------------------------------- System
+// Levels whose steps run in pairs: large ones, and of those with a list of
+// active chunks the ones the row-pair kernel takes (131 x 129 x 133 pool: two
+// listed steps 15 us, the x-plane pair 24).
+static bool pairs(const Level &L) { return pair_pays(L.d) && (!L.sparse || pair_segments_max(L.d) > 0); }
+
 // Grids whose kernels are bound by launch latency rather than bytes.
 static bool small_grid(Dims d) { return d.cells() <= ((size_t)1 << 19); }
 
@@ -410,7 +415,7 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
     // the last step and the restriction run as one pass where the grid pays
     // for the pass's tile overlap
     const bool fuse_restrict =
-        deg >= 3 && (((ws.fused_pairs & 1) && pair_pays(L.d)) || ((ws.fused_pairs & 4) && small_grid(L.d)));
+        deg >= 3 && (((ws.fused_pairs & 1) && pairs(L)) || ((ws.fused_pairs & 4) && small_grid(L.d)));
     if (deg == 1) {
         launch_smooth_first(st, L.d, A, r64, L.b.p, cur, cb.cr[0], ws.gate);
     } else {
@@ -420,7 +425,7 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
         // at degree 3 the two passes from the stored first iterate can run as
         // one: the iterate is also step 1's previous direction
         const bool pre_pair = deg == 3 && !fuse_restrict && first == SM_XFIRST &&
-                              (ws.fused_pairs & 16) && pair_pays(L.d);
+                              (ws.fused_pairs & 16) && pairs(L);
         if (pre_pair) {
             // reads x0, b, diag, 3 couplings; writes x
             if (fine && ws.profiling) ws.timers[K_SMOOTH_PAIR].begin(st, (24.0 + pair_diag_bytes) * cells);
@@ -495,13 +500,13 @@ float *System::post_smooth(Workspace &ws, const Smoothing &sm, int l, float *cur
     // the last two steps run as one pass where the grid is large enough to
     // pay for the pass's tile overlap (the direction they leave is not stored:
     // nothing reads it before the next cycle rewrites it)
-    const int fused = (deg >= 3 && (((ws.fused_pairs & 2) && pair_pays(L.d)) ||
+    const int fused = (deg >= 3 && (((ws.fused_pairs & 2) && pairs(L)) ||
                                     ((ws.fused_pairs & 8) && small_grid(L.d)))) ? 2 : 0;
     // step 0 adds the coarse correction: in the flat step's gathers, else on
     // large grids by its own pointwise pass before a plain step (cheaper than
     // the x-plane tiles' gathers at every neighbour); equal values every way
-    const bool add_first = !flat_step(L.d) && pair_pays(L.d);
-    if (add_first) launch_prolong_add(st, L.d, L.diag32.p, e, cur, ws.gate);
+    const bool add_first = !whole_groups(L.d) && !small_grid(L.d);
+    if (add_first) launch_prolong_add(st, L.d, L.diag32.p, A.chunks.list, e, cur, ws.gate);
     for (int s = 0; s < deg - fused; s++) {
         // step 0 adds the prolonged correction; the fine-level steps are timed
         const int mode = (s == 0 ? (add_first ? 0 : SM_PROLONG) : SM_READ_D) | (s < deg - 1 ? SM_WRITE_D : 0);

@@ -14,8 +14,11 @@ EVERY = 18 + 32  # the default step pairs, no lists
 
 # chunks of whole z rows, of several and across them; a last chunk in part; the
 # row-pair kernel's segments (193 to 256 cells per row, one and several tile
-# columns, more planes than one activity mask holds)
-GRIDS = [(96, 90, 64), (84, 82, 80), (67, 83, 100), (36, 80, 200), (96, 90, 256), (160, 72, 196)]
+# columns, more planes than one activity mask holds); groups of four and pairs
+# of cells that cross z rows, planes and the array's ends (nz = 1, 2, 3 mod 4,
+# with and without whole groups in a plane and in the grid)
+GRIDS = [(96, 90, 64), (84, 82, 80), (67, 83, 100), (36, 80, 200), (96, 90, 256), (160, 72, 196),
+         (83, 89, 91), (82, 80, 81), (81, 81, 82), (75, 85, 87), (82, 84, 86)]
 
 
 @pytest.mark.parametrize("n", GRIDS)
@@ -45,7 +48,7 @@ def test_lists_change_nothing(n):
         np.testing.assert_allclose(x, y, rtol=0, atol=1e-9 * np.abs(b[1]).max())
 
 
-@pytest.mark.parametrize("n", [(84, 82, 80), (36, 80, 200)])
+@pytest.mark.parametrize("n", [(84, 82, 80), (36, 80, 200), (83, 89, 91)])
 def test_a_new_active_set(n):
     """Solves of other liquids before leave nothing behind: the same bits as a
     new context's, from an empty container, a full one and other pools."""
