@@ -69,8 +69,7 @@ sfp_status sfp_test_set_vcycle_tail(sfp_context ctx, int enable);
  * pre-smoothing passes of a degree-3 cycle on large grids, or each as
  * separate launches. Bit 5 (from the next assembly on): run the kernels over
  * the flat cell index on every chunk of cells instead of the active ones'
- * list. A V-cycle's results are the same bit for bit; with bit 5 the solver's
- * FP64 sums take another order. */
+ * list. Results are the same bit for bit. */
 sfp_status sfp_test_set_fused_pairs(sfp_context ctx, int mask); /* default 18 */
 /* Let the stencil kernels of the magnetic system (FCG matvec, smoothing
  * steps, restriction) rebuild the FP64 and FP32 diagonals from the couplings

@@ -50,11 +50,16 @@ void launch_smooth_pair(hipStream_t s, Dims d, Op32 A, const float *b, const flo
                         const double *gate = nullptr, const unsigned char *rowact = nullptr,
                         const int *segments = nullptr);
 bool row_pair(Dims d);
-// The lists of a level's active chunks and restriction units (see Chunks; flags:
-// a byte for each, lists: an entry for each and one more).
+// The lists of a level's active chunks, restriction units and FCG blocks (see
+// Chunks; flags: a byte for each, lists: an entry for each and one more).
 unsigned restrict_quads(Dims d);
-void launch_active_chunks(hipStream_t s, Dims d, const float *diag32, unsigned char *flags, unsigned *list,
-                          unsigned char *quad_flags, unsigned *quads);
+struct ActiveLists {
+    unsigned char *flags, *quad_flags, *block_flags;
+    unsigned *list, *quads, *blocks;
+};
+void launch_active_chunks(hipStream_t s, Dims d, const float *diag32, const ActiveLists &a);
+// Doubles of Chunks::sums.
+size_t list_sums(Dims d);
 // k_smooth_pair_rows' work on a level with inactive rows: segments[0] runs of x
 // planes of a tile column, each (column, first plane, end) from segments[1 + 3 q]
 // on. pair_segments_max: the most of them, 0 where they are not used.
@@ -230,7 +235,7 @@ void launch_fcg_matvec(hipStream_t s, Dims d, Op64 A, const float *active, const
 // `active`. fold: the scalars are formed from the matvec's partials in the
 // kernel, and of rr only the partial sums (launch_fcg_norm, or the next cycle's
 // first launch, adds them).
-void launch_fcg_update(hipStream_t s, Dims d, const float *active, const unsigned *chunks, const double *w, double *q, double *r,
+void launch_fcg_update(hipStream_t s, Dims d, const float *active, const Chunks &chunks, const double *w, double *q, double *r,
                        float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate = nullptr,
                        hipEvent_t kernel_done = nullptr, KrylovScalars *host = nullptr);

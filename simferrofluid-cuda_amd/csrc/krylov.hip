@@ -31,61 +31,201 @@ __device__ __forceinline__ void st_stream(T *a, T v) {
 typedef double double2v __attribute__((ext_vector_type(2)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 
-// The stencil kernels run over the flat cell index, two consecutive cells per
-// lane: 16-byte loads of the FP64 operator and vectors at the pair and at its x
-// and y neighbour pairs, one extra value and z coupling at each end. A pair may
-// lie across the end of a z row: a neighbour is sx, sy or 1 cells on in the array
-// wherever rows and planes end, the coupling to it being 0 there as stored (the
-// lower coupling of the first cell across). The off-diagonal sum has the order
-// x-, x+, y-, y+, z-, z+; a row-sum diagonal is rebuilt from the couplings (the
-// same sums in the same order as the assembly's, so the same bits), except in
-// the pairs that hold cell 0 or its upper neighbours.
-typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
-typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
-// kAny (nz odd): a neighbour pair is at any address of its type. One that
-// crosses the array's end is loaded past it (an allocation reaches 64 bytes past
-// its array) and one that crosses its start is loaded from the start and moved;
-// the cell outside is put to 0. Else only a missing upper neighbour's couplings
-// are (a missing neighbour's value is any other, coupled with 0).
-template <bool kAny>
+// The x-plane stencils, for grids with odd nz whose sums keep their order: the
+// constant mode of a magnetic potential hangs on one pinned cell, which carries
+// the last bits of an iteration's sums into it 10^5 times larger (131 x 129 x
+// 133: the flat kernels' order moves the field at the pin by 2e-8 of its rms).
+// The stencil kernels below march over the block's x planes with the
+// x-neighbours in registers and take the z-neighbours (value and z coupling)
+// from the adjacent lanes of the tile row; only the row's end lanes load
+// them. The off-diagonal sum keeps the order x-, x+, y-, y+, z-, z+.
+__global__ __launch_bounds__(kBlock) void k_residual64(CellGrid cg, Dims d, Op64 A,
+                                                       const double *__restrict__ b,
+                                                       const double *__restrict__ x,
+                                                       double *__restrict__ r,
+                                                       double *__restrict__ partials,
+                                                       float *__restrict__ b32,
+                                                       float *__restrict__ x0,
+                                                       const float *__restrict__ diag32,
+                                                       float c0, const double *need) {
+    if (need && *need == 0.0) return;
+    int k, j, i0;
+    cell_tile(cg, k, j, i0);
+    const Strides s(d);
+    const int tz = blockDim.x, lane = threadIdx.x;
+    const bool on = k < d.nz && j < d.ny && i0 < d.nx;
+    const bool zlo = k > 0, zhi = k + 1 < d.nz;
+    const int ie = min(i0 + cg.planes, d.nx);
+    double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
+    size_t c = on ? d.idx(i0, j, k) : 0;
+    // the FP32 copy of r and the cycle's first iterate (the FCG update's arithmetic)
+    auto store32 = [&](size_t q, double rq) {
+        const float dq = diag32 ? diag32[q] : 0.f;
+        if (dq > 0.f) v[2] += 1.0;
+        if (!b32) return;
+        const float bf = (float)rq;
+        b32[q] = bf;
+        if (x0) x0[q] = c0 * rcp_or_zero(dq) * bf;
+    };
+    if (!x) {
+        if (on)
+            for (int i = i0; i < ie; i++, c += s.sx) {
+                const double bc = b[c];
+                if (r) r[c] = bc;
+                store32(c, bc);
+                v[0] += bc * bc;
+                v[1] += bc * bc;
+            }
+        block_partials<3>(v, partials);
+        return;
+    }
+    double xm = (on && i0 > 0) ? x[c - s.sx] : 0.0;
+    double xc = on ? x[c] : 0.0;
+    double cxc = on ? A.cpl[0][c] : 0.0;
+    for (int i = i0; i < ie; i++, c += s.sx) {
+        const bool up = i + 1 < d.nx;
+        const double xp = (on && up) ? x[c + s.sx] : 0.0;
+        const double cxp = (on && up) ? A.cpl[0][c + s.sx] : 0.0;
+        const double czm = on ? A.cpl[2][c] : 0.0;
+        double xzm = __shfl_up(xc, 1, tz);
+        double xzp = __shfl_down(xc, 1, tz);
+        double czp = __shfl_down(czm, 1, tz);
+        if (lane == 0) xzm = (on && zlo) ? x[c - 1] : 0.0;
+        if (lane == tz - 1) {
+            xzp = (on && zhi) ? x[c + 1] : 0.0;
+            czp = (on && zhi) ? A.cpl[2][c + 1] : 0.0;
+        }
+        if (on) {
+            double off = 0.0;
+            if (i > 0) off += cxc * xm;
+            if (up) off += cxp * xp;
+            if (j > 0) off += A.cpl[1][c] * x[c - s.sy];
+            if (j + 1 < d.ny) off += A.cpl[1][c + s.sy] * x[c + s.sy];
+            if (zlo) off += czm * xzm;
+            if (zhi) off += czp * xzp;
+            const double bc = b[c];
+            const double rc = bc - (A.diag[c] * xc - off);
+            if (r) r[c] = rc;
+            store32(c, rc);
+            v[0] += rc * rc;
+            v[1] += bc * bc;
+        }
+        xm = xc;
+        xc = xp;
+        cxc = cxp;
+    }
+    block_partials<3>(v, partials);
+}
+
+__global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64 A,
+                                                       const float *__restrict__ active,
+                                                       const float *__restrict__ z,
+                                                       const double *__restrict__ r,
+                                                       const double *__restrict__ qprev,
+                                                       double *__restrict__ w, int first,
+                                                       double *__restrict__ partials,
+                                                       const double *gate) {
+    if (gated(gate)) return;
+    int k, j, i0;
+    cell_tile(cg, k, j, i0);
+    const Strides s(d);
+    const int tz = blockDim.x, lane = threadIdx.x;
+    const bool on = k < d.nz && j < d.ny && i0 < d.nx;
+    const bool zlo = k > 0, zhi = k + 1 < d.nz, ylo = on && j > 0, yhi = on && j + 1 < d.ny;
+    const int ie = min(i0 + cg.planes, d.nx);
+    double v[3] = {0.0, 0.0, 0.0};  // z.w, z.q_prev, z.r
+    size_t c = on ? d.idx(i0, j, k) : 0;
+    float zm = 0.f, zc = 0.f;
+    double cxc = 0.0;
+    bool primed = false;  // zm, zc, cxc hold this plane's values
+    float act_next = (active && on) ? active[c] : 0.f;
+    for (int i = i0; i < ie; i++, c += s.sx) {
+        float act = 1.f;
+        if (active) {
+            act = act_next;
+            act_next = (on && i + 1 < ie) ? active[c + s.sx] : 0.f;
+            if (!__any(on && act > 0.f)) {
+                primed = false;
+                continue;
+            }
+        }
+        if (!primed) {
+            zm = (on && i > 0) ? z[c - s.sx] : 0.f;
+            zc = on ? z[c] : 0.f;
+            cxc = on ? A.cpl[0][c] : 0.0;
+            primed = true;
+        }
+        const bool up = i + 1 < d.nx;
+        const float zp = (on && up) ? z[c + s.sx] : 0.f;
+        const double cxp = (on && up) ? A.cpl[0][c + s.sx] : 0.0;
+        const double czm = on ? A.cpl[2][c] : 0.0;
+        const double cym = ylo ? A.cpl[1][c] : 0.0;
+        const double cyp = yhi ? A.cpl[1][c + s.sy] : 0.0;
+        const float zym = ylo ? z[c - s.sy] : 0.f;
+        const float zyp = yhi ? z[c + s.sy] : 0.f;
+        const double dg = on ? A.diag[c] : 0.0;
+        const double qp = (on && !first) ? ld_stream(qprev + c) : 0.0;
+        const double rc = on ? ld_stream(r + c) : 0.0;
+        float zzm = __shfl_up(zc, 1, tz);
+        float zzp = __shfl_down(zc, 1, tz);
+        double czp = __shfl_down(czm, 1, tz);
+        if (lane == 0) zzm = (on && zlo) ? z[c - 1] : 0.f;
+        if (lane == tz - 1) {
+            zzp = (on && zhi) ? z[c + 1] : 0.f;
+            czp = (on && zhi) ? A.cpl[2][c + 1] : 0.0;
+        }
+        if (on) {
+            double off = 0.0;
+            if (i > 0) off += cxc * (double)zm;
+            if (up) off += cxp * (double)zp;
+            if (j > 0) off += cym * (double)zym;
+            if (j + 1 < d.ny) off += cyp * (double)zyp;
+            if (zlo) off += czm * (double)zzm;
+            if (zhi) off += czp * (double)zzp;
+            const double zd = act > 0.f ? (double)zc : 0.0;
+            const double wc = dg * zd - off;
+            st_stream(w + c, wc);
+            v[0] += zd * wc;
+            if (!first) v[1] += zd * qp;
+            v[2] += zd * rc;
+        }
+        zm = zc;
+        zc = zp;
+        cxc = cxp;
+    }
+    block_partials<3>(v, partials);
+}
+
+// The flat stencils run over the flat cell index, two consecutive cells of one z
+// row per lane (nz even): 16-byte loads of the FP64 operator and vectors at the
+// pair and at its x and y neighbour pairs, one extra value and z coupling at
+// each end. A neighbour is sx, sy or 1 cells on in the array also where a row or
+// a plane ends: the coupling to it is 0 there as stored (the lower coupling of
+// the first cell across), and only a neighbour past the array has its couplings
+// put to 0 (its value is any other). The off-diagonal sum has the order x-, x+,
+// y-, y+, z-, z+; a row-sum diagonal is rebuilt from the couplings (the same
+// sums in the same order as the assembly's, so the same bits), except in the
+// pairs that hold cell 0 or its upper neighbours.
 struct PairAt {
     unsigned n, sx, sy, c;
     __device__ __forceinline__ PairAt(Dims d, size_t cell)
         : n((unsigned)d.cells()), sx((unsigned)d.ny * (unsigned)d.nz), sy((unsigned)d.nz), c((unsigned)cell) {}
-    // a at the pair k cells before and after this one
-    template <class V2, class U2, class T>
-    __device__ __forceinline__ V2 below(const T *__restrict__ a, unsigned k) const {
-        V2 v = *(const U2 *)(a + (c >= k ? c - k : 0));
-        if constexpr (kAny) {
-            v.y = c >= k ? v.y : c + 1 == k ? v.x : 0;
-            v.x = c >= k ? v.x : 0;
-        }
-        return v;
-    }
-    template <class V2, class U2, class T>
-    __device__ __forceinline__ V2 above(const T *__restrict__ a, unsigned k) const {
-        const unsigned left = n - c;
-        V2 v = *(const U2 *)(a + (left > k ? c + k : c));
-        if constexpr (kAny) {
-            v.x = left > k ? v.x : 0;
-            v.y = left > k + 1 ? v.y : 0;
-        }
-        return v;
-    }
+    // a at this pair and at the pair k cells before and after it
+    __device__ __forceinline__ double2v at(const double *__restrict__ a) const { return *(const double2v *)(a + c); }
+    __device__ __forceinline__ float2v at(const float *__restrict__ a) const { return *(const float2v *)(a + c); }
     __device__ __forceinline__ double2v below(const double *__restrict__ a, unsigned k) const {
-        return below<double2v, double2u>(a, k);
+        return *(const double2v *)(a + (c >= k ? c - k : 0));
     }
     __device__ __forceinline__ float2v below(const float *__restrict__ a, unsigned k) const {
-        return below<float2v, float2u>(a, k);
+        return *(const float2v *)(a + (c >= k ? c - k : 0));
     }
     __device__ __forceinline__ double2v above(const double *__restrict__ a, unsigned k) const {
-        return above<double2v, double2u>(a, k);
+        return *(const double2v *)(a + (n - c > k ? c + k : c));
     }
     __device__ __forceinline__ float2v above(const float *__restrict__ a, unsigned k) const {
-        return above<float2v, float2u>(a, k);
+        return *(const float2v *)(a + (n - c > k ? c + k : c));
     }
-    // the cell below the pair's first, and the one above its second (any other
-    // cell's where there is none)
+    // the cell below the pair's first, and the one above its second
     template <class T>
     __device__ __forceinline__ T one_below(const T *__restrict__ a) const {
         return a[c > 0 ? c - 1 : 0];
@@ -94,47 +234,29 @@ struct PairAt {
     __device__ __forceinline__ T one_above(const T *__restrict__ a) const {
         return a[n - c > 2 ? c + 2 : c];
     }
-    // a coupling of the pair k cells on, 0 past the array
-    __device__ __forceinline__ double2v upper(const double *__restrict__ a, unsigned k) const {
-        double2v v = above(a, k);
-        if (!kAny && !(n - c > k)) v = double2v{0.0, 0.0};
-        return v;
-    }
-    // this pair's own cells of a vector (streamed)
-    __device__ __forceinline__ double2v own(const double *a) const {
-        double2v v = ld_stream((const double2v *)(a + c));
-        if constexpr (kAny) v.y = n - c > 1 ? v.y : 0.0;
-        return v;
-    }
-    __device__ __forceinline__ void store(double *a, double2v v) const {
-        if (!kAny || n - c > 1) st_stream((double2v *)(a + c), v);
-        else a[c] = v.x;
-    }
-    __device__ __forceinline__ void store(float *a, float2v v) const {
-        if (!kAny || n - c > 1) *(float2v *)(a + c) = v;
-        else a[c] = v.x;
-    }
     // whether the pair holds a cell whose diagonal is not the row sum (0, 1, nz, nz*ny)
-    __device__ __forceinline__ bool pinned() const { return c <= 1 || sy - c < 2 || sx - c < 2; }
+    __device__ __forceinline__ bool pinned() const { return c == 0 || c == sy || c == sx; }
 };
 // The operator at a pair: its couplings and diagonal.
 struct PairOperator {
     double2v cxm, cxp, cym, cyp, cz, dg;
     double czp;
-    template <bool kAny>
-    __device__ __forceinline__ PairOperator(const Op64 &A, const PairAt<kAny> &P) {
-        cxm = P.above(A.cpl[0], 0);
-        cxp = P.upper(A.cpl[0], P.sx);
-        cym = P.above(A.cpl[1], 0);
-        cyp = P.upper(A.cpl[1], P.sy);
-        cz = P.above(A.cpl[2], 0);   // below each cell of the pair
+    __device__ __forceinline__ PairOperator(const Op64 &A, const PairAt &P) {
+        cxm = P.at(A.cpl[0]);
+        cxp = P.above(A.cpl[0], P.sx);
+        cym = P.at(A.cpl[1]);
+        cyp = P.above(A.cpl[1], P.sy);
+        cz = P.at(A.cpl[2]);          // below each cell of the pair
         czp = P.one_above(A.cpl[2]);  // above the second
-        czp = P.n - P.c > 2 ? czp : 0.0;
+        const unsigned left = P.n - P.c;
+        if (!(left > P.sx)) cxp = double2v{0.0, 0.0};
+        if (!(left > P.sy)) cyp = double2v{0.0, 0.0};
+        if (!(left > 2)) czp = 0.0;
         if (A.pinned_rowsum && !P.pinned()) {
             dg.x = ((((cxm.x + cxp.x) + cym.x) + cyp.x) + cz.x) + cz.y;
             dg.y = ((((cxm.y + cxp.y) + cym.y) + cyp.y) + cz.y) + czp;
         } else {
-            dg = P.above(A.diag, 0);
+            dg = P.at(A.diag);
         }
     }
     // (A v) of the pair, whose values are vc, the neighbours' the rest
@@ -158,120 +280,111 @@ struct PairOperator {
 };
 __device__ __forceinline__ double2v widen(float2v v) { return double2v{(double)v.x, (double)v.y}; }
 
-// r = b - A x (x null: b) with the sums of r.r, b.b and the active cells
-// (diag32). r, and b32 with x0 (the FP32 copy of r and the cycle's first
-// iterate, in the FCG update's arithmetic), may be null (then not stored: a
-// convergence check needs only the sums, and with kList takes them over the
-// listed chunks: b and x are 0 in the others).
-constexpr unsigned kResidualCells = 2 * kBlock;
+// The same residual (r, and b32 with x0, may be null: then not stored; a
+// convergence check needs only the sums, and with kList takes them of the listed
+// blocks, as the matvec below).
+constexpr unsigned kResidualCells = kListCells;
 
-template <bool kList, bool kAny>
-__global__ __launch_bounds__(kBlock, kList ? 7 : 1) void k_residual64_flat(Dims d, Op64 A,
-                                                            const double *__restrict__ b,
+template <bool kList>
+__global__ __launch_bounds__(kBlock) void k_residual64_flat(Dims d, Op64 A, const double *__restrict__ b,
                                                             const double *__restrict__ x,
-                                                            double *__restrict__ r,
-                                                            double *__restrict__ partials,
-                                                            float *__restrict__ b32,
-                                                            float *__restrict__ x0,
-                                                            const float *__restrict__ diag32,
-                                                            float c0, const double *need) {
+                                                            double *__restrict__ r, double *__restrict__ partials,
+                                                            float *__restrict__ b32, float *__restrict__ x0,
+                                                            const float *__restrict__ diag32, float c0,
+                                                            unsigned nb, const double *need) {
     if (need && *need == 0.0) return;
-    double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
-    auto pair = [&](size_t c) {
-        const PairAt<kAny> P(d, c);
-        const double2v bc = P.own(b);
-        double2v rc = bc;
-        if (x) {
-            const double2v xc = P.above(x, 0), xxm = P.below(x, P.sx), xxp = P.above(x, P.sx),
-                           xym = P.below(x, P.sy), xyp = P.above(x, P.sy);
-            const double xzm = P.one_below(x), xzp = P.one_above(x);
-            const PairOperator op(A, P);
-            const double2v ax = op.apply(xc, xxm, xxp, xym, xyp, xzm, xzp);
-            rc.x = bc.x - ax.x;
-            rc.y = bc.y - ax.y;
+    const unsigned count = kList ? A.chunks.blocks[0] : nb;
+    for (unsigned u = blockIdx.x; u < count; u += kList ? gridDim.x : nb) {
+        const unsigned block = kList ? A.chunks.blocks[1 + u] : u;
+        const size_t c = (size_t)block * kResidualCells + 2 * (size_t)flat_tid();
+        double v[3] = {0.0, 0.0, 0.0};  // r.r, b.b, active cells (with diag32)
+        if (c < d.cells()) {            // cells() is even: then c + 1 is a cell too
+            const PairAt P(d, c);
+            const double2v bc = ld_stream((const double2v *)(b + c));
+            double2v rc = bc;
+            if (x) {
+                const double2v xc = P.at(x), xxm = P.below(x, P.sx), xxp = P.above(x, P.sx), xym = P.below(x, P.sy),
+                               xyp = P.above(x, P.sy);
+                const double xzm = P.one_below(x), xzp = P.one_above(x);
+                const PairOperator op(A, P);
+                const double2v ax = op.apply(xc, xxm, xxp, xym, xyp, xzm, xzp);
+                rc.x = bc.x - ax.x;
+                rc.y = bc.y - ax.y;
+            }
+            if (r) st_stream((double2v *)(r + c), rc);
+            const float2v dd = diag32 ? *(const float2v *)(diag32 + c) : float2v{0.f, 0.f};
+            v[2] = (dd.x > 0.f ? 1.0 : 0.0) + (dd.y > 0.f ? 1.0 : 0.0);
+            if (b32) {
+                const float2v bf = {(float)rc.x, (float)rc.y};
+                *(float2v *)(b32 + c) = bf;
+                if (x0) {
+                    const float2v xf = {c0 * rcp_or_zero(dd.x) * bf.x, c0 * rcp_or_zero(dd.y) * bf.y};
+                    *(float2v *)(x0 + c) = xf;
+                }
+            }
+            v[0] = rc.x * rc.x + rc.y * rc.y;
+            v[1] = bc.x * bc.x + bc.y * bc.y;
         }
-        if (r) P.store(r, rc);
-        const float2v dd = diag32 ? P.above(diag32, 0) : float2v{0.f, 0.f};
-        v[2] += (dd.x > 0.f ? 1.0 : 0.0) + (dd.y > 0.f ? 1.0 : 0.0);
-        if (b32) {
-            const float2v bf = {(float)rc.x, (float)rc.y};
-            P.store(b32, bf);
-            if (x0) P.store(x0, float2v{c0 * rcp_or_zero(dd.x) * bf.x, c0 * rcp_or_zero(dd.y) * bf.y});
-        }
-        v[0] += rc.x * rc.x + rc.y * rc.y;
-        v[1] += bc.x * bc.x + bc.y * bc.y;
-    };
-    const size_t n = d.cells();
-    if constexpr (kList) {
-        const unsigned units = A.chunks.list[0] * list_units<2>(), waves = flat_waves();
-        for (unsigned u = flat_wave(); u < units; u += waves) {
-            const unsigned c = list_cell<2>(A.chunks.list, u);
-            if (c < n) pair(c);
-        }
-    } else {
-        const size_t c = (size_t)blockIdx.x * kResidualCells + 2 * (size_t)flat_tid();
-        if (c < n) pair(c);
+        block_sum<3>(v);
+        if (flat_tid() == 0)
+#pragma unroll
+            for (int q = 0; q < 3; q++) partials[(size_t)q * nb + block] = v[q];
     }
-    block_partials<3>(v, partials);
 }
 
-// w = A z with the sums of z.w, z.q_prev and z.r, and z as FP64. `active` (the
-// FP32 diagonal, 0 = inactive cell) or null: with it, z counts as 0 at the
-// inactive cells (a z buffer may hold an earlier solve's values in groups that
-// its writer skips), and a wavefront whose 128 cells are all inactive is skipped
-// (the vectors it would write are never read by active cells). kList:
-// kListBlocks blocks share the listed chunks (256^3 pool, 26 % of the rows
-// active: 80 us a wavefront per 128 cells of the grid, 69 so, and its fewer
-// partial sums need one launch less).
-constexpr unsigned kMatvecCells = 2 * kBlock;
+// The same matvec. kList: the launch's blocks share the listed blocks of
+// kMatvecCells cells (Chunks::blocks), each with its own place among the partial
+// sums (0 in the others', as its cells would give), so the sums keep their order
+// to the bit. 256^3 pool, 26 % of the rows active: 70 us so, 80 with a block for
+// each (the list's bytes at the copy rate: 62).
+constexpr unsigned kMatvecCells = kListCells;
+static_assert(kMatvecCells == 2 * kBlock, "two cells per lane");
 
-template <bool kList, bool kAny>
-__global__ __launch_bounds__(kBlock, kList ? 7 : 1) void k_fcg_matvec_flat(Dims d, Op64 A,
+template <bool kList>
+__global__ __launch_bounds__(kBlock, kList ? 8 : 1) void k_fcg_matvec_flat(Dims d, Op64 A,
                                                             const float *__restrict__ active,
                                                             const float *__restrict__ z,
                                                             const double *__restrict__ r,
                                                             const double *__restrict__ qprev,
                                                             double *__restrict__ w, int first,
-                                                            double *__restrict__ partials,
+                                                            double *__restrict__ partials, unsigned nb,
                                                             const double *gate) {
     if (gated(gate)) return;
-    double v[3] = {0.0, 0.0, 0.0};  // z.w, z.q_prev, z.r
-    // one pair of cells (every lane of the wavefront comes here)
-    auto pair = [&](size_t c, bool on) {
-        const PairAt<kAny> P(d, on ? c : 0);
-        bool on0 = true, on1 = true;  // the pair's cells are active
+    const unsigned count = kList ? A.chunks.blocks[0] : nb;
+    for (unsigned u = blockIdx.x; u < count; u += kList ? gridDim.x : nb) {
+        const unsigned block = kList ? A.chunks.blocks[1 + u] : u;
+        const size_t c = (size_t)block * kMatvecCells + 2 * (size_t)flat_tid();
+        const bool on = c < d.cells();  // cells() is even: then c + 1 is a cell too
+        double v[3] = {0.0, 0.0, 0.0};  // z.w, z.q_prev, z.r
+        bool act = on, on0 = true, on1 = true;  // the pair's cells are active
         if (active && on) {
-            const float2v a = P.above(active, 0);
+            const float2v a = *(const float2v *)(active + c);
             on0 = a.x > 0.f;
             on1 = a.y > 0.f;
+            act = on0 || on1;
         }
-        if (!(on && (kList || __any(on && (on0 || on1))))) return;
-        const float2v zl = P.above(z, 0);
-        const float2v zxm = P.below(z, P.sx), zxp = P.above(z, P.sx), zym = P.below(z, P.sy),
-                      zyp = P.above(z, P.sy);
-        const float zzm = P.one_below(z), zzp = P.one_above(z);
-        const PairOperator op(A, P);
-        const double2v qp = first ? double2v{0.0, 0.0} : P.own(qprev);
-        const double2v rc = P.own(r);
-        const double2v zc = {on0 ? (double)zl.x : 0.0, on1 ? (double)zl.y : 0.0};
-        const double2v wc = op.apply(zc, widen(zxm), widen(zxp), widen(zym), widen(zyp), (double)zzm, (double)zzp);
-        P.store(w, wc);
-        v[0] += zc.x * wc.x + zc.y * wc.y;
-        if (!first) v[1] += zc.x * qp.x + zc.y * qp.y;
-        v[2] += zc.x * rc.x + zc.y * rc.y;
-    };
-    const size_t n = d.cells();
-    if constexpr (kList) {
-        const unsigned units = A.chunks.list[0] * list_units<2>(), waves = flat_waves();
-        for (unsigned u = flat_wave(); u < units; u += waves) {
-            const unsigned c = list_cell<2>(A.chunks.list, u);
-            pair(c, c < n);
+        if (__any(act) && on) {
+            const PairAt P(d, c);
+            const float2v zl = P.at(z);
+            const float2v zxm = P.below(z, P.sx), zxp = P.above(z, P.sx), zym = P.below(z, P.sy),
+                          zyp = P.above(z, P.sy);
+            const float zzm = P.one_below(z), zzp = P.one_above(z);
+            const PairOperator op(A, P);
+            const double2v qp = first ? double2v{0.0, 0.0} : ld_stream((const double2v *)(qprev + c));
+            const double2v rc = ld_stream((const double2v *)(r + c));
+            const double2v zc = {on0 ? (double)zl.x : 0.0, on1 ? (double)zl.y : 0.0};
+            const double2v wc =
+                op.apply(zc, widen(zxm), widen(zxp), widen(zym), widen(zyp), (double)zzm, (double)zzp);
+            st_stream((double2v *)(w + c), wc);
+            v[0] = zc.x * wc.x + zc.y * wc.y;
+            if (!first) v[1] = zc.x * qp.x + zc.y * qp.y;
+            v[2] = zc.x * rc.x + zc.y * rc.y;
         }
-    } else {
-        const size_t c = (size_t)blockIdx.x * kMatvecCells + 2 * (size_t)flat_tid();
-        pair(c, c < n);
+        block_sum<3>(v);
+        if (flat_tid() == 0)
+#pragma unroll
+            for (int q = 0; q < 3; q++) partials[(size_t)q * nb + block] = v[q];
     }
-    block_partials<3>(v, partials);
 }
 
 // The iteration's scalars from its dots: p = z - beta p_prev with beta =
@@ -406,9 +519,10 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(size_t n, const float *__
     block_partials<1>(v, partials);
 }
 
-// The same update on the listed chunks (kListBlocks blocks share them), the
-// scalars from a finalize launch.
-__global__ __launch_bounds__(kBlock) void k_fcg_update_list(unsigned n, const unsigned *__restrict__ list,
+// The same update on the listed blocks of kUpdateCells cells, as the matvec's
+// (256^3 pool: 46 us, 50 with a block for each; the list's bytes: 51).
+static_assert(kUpdateCells == kListCells, "the lists' blocks");
+__global__ __launch_bounds__(kBlock) void k_fcg_update_list(size_t n, const unsigned *__restrict__ blocks,
                                                             const float *__restrict__ active,
                                                             const double *__restrict__ w, double *__restrict__ q,
                                                             double *__restrict__ r, float *__restrict__ b32,
@@ -418,34 +532,54 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update_list(unsigned n, const un
                                                             const double *gate) {
     if (gated(gate)) return;
     const double alpha = sc->alpha[iter % kCoefs], beta = sc->beta[iter % kCoefs];
-    double v[1] = {0.0};
-    const unsigned units = list[0] * list_units<2>(), waves = flat_waves();
-    for (unsigned u = flat_wave(); u < units; u += waves) {
-        const unsigned c = list_cell<2>(list, u);
-        if (c >= n) continue;
-        const PairAt<true> P(Dims{1, 1, (int)n}, c);
-        const float2v dg = x0 ? P.above(active, 0) : float2v{0.f, 0.f};
-        const double2v wc = P.own(w), r0 = P.own(r);
-        double2v qc = wc;
-        if (!first) {
-            const double2v qq = P.own(q);
-            qc.x = wc.x - beta * qq.x;
-            qc.y = wc.y - beta * qq.y;
+    const unsigned count = blocks[0];
+    for (unsigned u = blockIdx.x; u < count; u += gridDim.x) {
+        const unsigned block = blocks[1 + u];
+        const size_t c = (size_t)block * kUpdateCells + 2 * (size_t)flat_tid();
+        const bool pair = c + 1 < n;  // else at most the grid's last cell
+        double v[1] = {0.0};
+        float2v dg = {0.f, 0.f};
+        if (pair) dg = *(const float2v *)(active + c);
+        else if (c < n) dg.x = active[c];
+        if (__any(dg.x > 0.f || dg.y > 0.f)) {
+            if (pair) {
+                const double2v wc = ld_stream((const double2v *)(w + c)), r0 = ld_stream((const double2v *)(r + c));
+                double2v qc = wc;
+                if (!first) {
+                    const double2v qq = ld_stream((const double2v *)(q + c));
+                    qc.x = wc.x - beta * qq.x;
+                    qc.y = wc.y - beta * qq.y;
+                }
+                double2v rc;
+                rc.x = r0.x - alpha * qc.x;
+                rc.y = r0.y - alpha * qc.y;
+                st_stream((double2v *)(q + c), qc);
+                st_stream((double2v *)(r + c), rc);
+                if (b32) {
+                    const float2v bf = {(float)rc.x, (float)rc.y};
+                    *(float2v *)(b32 + c) = bf;
+                    if (x0) {
+                        const float2v xf = {c0 * rcp_or_zero(dg.x) * bf.x, c0 * rcp_or_zero(dg.y) * bf.y};
+                        *(float2v *)(x0 + c) = xf;
+                    }
+                }
+                v[0] += rc.x * rc.x;
+                v[0] += rc.y * rc.y;
+            } else if (c < n) {
+                const double qc = first ? w[c] : w[c] - beta * q[c];
+                q[c] = qc;
+                const double rc = r[c] - alpha * qc;
+                r[c] = rc;
+                if (b32) {
+                    b32[c] = (float)rc;
+                    if (x0) x0[c] = c0 * rcp_or_zero(dg.x) * b32[c];
+                }
+                v[0] += rc * rc;
+            }
         }
-        double2v rc;
-        rc.x = r0.x - alpha * qc.x;
-        rc.y = r0.y - alpha * qc.y;
-        P.store(q, qc);
-        P.store(r, rc);
-        if (b32) {
-            const float2v bf = {(float)rc.x, (float)rc.y};
-            P.store(b32, bf);
-            if (x0) P.store(x0, float2v{c0 * rcp_or_zero(dg.x) * bf.x, c0 * rcp_or_zero(dg.y) * bf.y});
-        }
-        v[0] += rc.x * rc.x;
-        v[0] += rc.y * rc.y;
+        block_sum<1>(v);
+        if (flat_tid() == 0) partials[block] = v[0];
     }
-    block_partials<1>(v, partials);
 }
 
 // p = z_k - beta_k p, x += alpha_k p for K iterations (numbers i0 .. i0 + K - 1,
@@ -645,13 +779,20 @@ void finalize(hipStream_t st, int op, unsigned nb, int first, int iter, double *
 
 }  // namespace
 
-// The FP64 stencils run over the flat cell index (11 % faster than x-plane
-// tiles at 256^3 and 9 % at 384^3 on MI355X; 131 x 129 x 133 36 us -> 26).
-static unsigned matvec_blocks(Dims d) { return (unsigned)((d.cells() + kMatvecCells - 1) / kMatvecCells); }
-// Blocks of a kernel over the listed chunks: as many as run at once (seven of
-// four wavefronts per CU), or the grid's where that is less.
-constexpr unsigned kListBlocks = 7 * 256;
-static unsigned list_blocks(Dims d) { return std::min(kListBlocks, matvec_blocks(d)); }
+// FCG matvec: the flat kernel where z rows hold whole cell pairs (nz even;
+// 11 % faster than x-plane tiles at 256^3 and 9 % at 384^3 on MI355X), else
+// x-plane tiles of 4 planes per block (more blocks in flight than the 16 of the
+// other reductions: 6 % faster at 256^3). (With odd nz the flat order of the
+// sums is not for use: see the x-plane stencils.)
+static bool matvec_flat(Dims d) { return d.nz % 2 == 0; }
+static Launch matvec_launch(Dims d) { return cell_launch(d, 0, 4); }
+static unsigned matvec_blocks(Dims d) {
+    return matvec_flat(d) ? (unsigned)((d.cells() + kMatvecCells - 1) / kMatvecCells)
+                          : matvec_launch(d).blocks();
+}
+// Blocks of a launch over the listed ones: as many as run at once (eight of four
+// wavefronts per CU), or the grid's where that is less.
+static unsigned list_launch(unsigned nb) { return std::min(nb, 8u * 256); }
 static unsigned update_blocks(Dims d) { return (unsigned)((d.cells() + kUpdateCells - 1) / kUpdateCells); }
 
 size_t reduction_partials(Dims d) {
@@ -662,6 +803,8 @@ size_t reduction_partials(Dims d) {
                     3 * (size_t)matvec_blocks(d) + (size_t)update_blocks(d)) +
            3 * (size_t)kStageMaxBlocks;
 }
+
+size_t list_sums(Dims d) { return 3 * (size_t)matvec_blocks(d) + update_blocks(d) + 4 * (size_t)kStageMaxBlocks; }
 
 bool fold_pays(Dims d) { return std::max(matvec_blocks(d), update_blocks(d)) <= kFoldMax; }
 FoldArgs update_fold(Dims d, double *partials, KrylovScalars *sc) {
@@ -683,26 +826,33 @@ void launch_residual64(hipStream_t st, Dims d, Op64 A, const double *b, const do
         if ((uintptr_t)a % 16) throw ArgError("launch_residual64: FP64 array not 16-byte aligned");
     if ((uintptr_t)b32 % 8 || (uintptr_t)x0 % 8 || (uintptr_t)diag32 % 8)
         throw ArgError("launch_residual64: b32, x0 or the diagonal not 8-byte aligned");
-    const bool list = A.chunks.list && !r && !b32;  // (a residual that is stored covers every cell)
-    const unsigned nb = list ? list_blocks(d) : (unsigned)((d.cells() + kResidualCells - 1) / kResidualCells);
-#define SFP_RESIDUAL(LIST, ANY)                                                                              \
-    hipLaunchKernelGGL((k_residual64_flat<LIST, ANY>), dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials, \
-                       b32, x0, diag32, c0, need)
-    if (d.nz & 1) {
-        if (list) SFP_RESIDUAL(true, true); else SFP_RESIDUAL(false, true);
-    } else {
-        if (list) SFP_RESIDUAL(true, false); else SFP_RESIDUAL(false, false);
+    if (matvec_flat(d)) {
+        const unsigned nb = (unsigned)((d.cells() + kResidualCells - 1) / kResidualCells);
+        if (A.chunks.blocks && !r && !b32) {
+            partials = A.chunks.sums;
+            hipLaunchKernelGGL(k_residual64_flat<true>, dim3(list_launch(nb)), dim3(kBlock), 0, st, d, A, b, x, r,
+                               partials, b32, x0, diag32, c0, nb, need);
+        } else {
+            hipLaunchKernelGGL(k_residual64_flat<false>, dim3(nb), dim3(kBlock), 0, st, d, A, b, x, r, partials,
+                               b32, x0, diag32, c0, nb, need);
+        }
+        SFP_LAUNCH_CHECK();
+        finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host, need, tol);
+        return;
     }
-#undef SFP_RESIDUAL
+    const Launch L = cell_launch(d, kReducePlanes);
+    hipLaunchKernelGGL(k_residual64, L.grid, L.block, 0, st, L.cg, d, A, b, x, r, partials, b32, x0, diag32, c0,
+                       need);
     SFP_LAUNCH_CHECK();
-    finalize(st, FIN_RESIDUAL, nb, 0, 0, partials, sc, nullptr, host, need, tol);
+    finalize(st, FIN_RESIDUAL, L.blocks(), 0, 0, partials, sc, nullptr, host, need, tol);
 }
 
 void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, const float *z,
                        const double *r, const double *qprev, double *w, int first, int iter, bool fold,
                        double *partials, KrylovScalars *sc, const double *gate, hipEvent_t kernel_done) {
-    const bool list = A.chunks.list != nullptr;
-    const unsigned nb = list ? list_blocks(d) : matvec_blocks(d);
+    const bool list = A.chunks.blocks && matvec_flat(d);
+    const unsigned nb = matvec_blocks(d);
+    if (list) partials = A.chunks.sums;
     if (d.cells() >= (size_t(1) << 32) - 64) throw ArgError("launch_fcg_matvec: grid too large");
     // pairs of cells: 16-byte (8-byte for z and the flags) aligned vectors
     for (const void *a : {(const void *)A.diag, (const void *)A.cpl[0], (const void *)A.cpl[1],
@@ -710,21 +860,23 @@ void launch_fcg_matvec(hipStream_t st, Dims d, Op64 A, const float *active, cons
         if ((uintptr_t)a % 16) throw ArgError("launch_fcg_matvec: FP64 array not 16-byte aligned");
     if ((uintptr_t)z % 8 || (uintptr_t)active % 8)
         throw ArgError("launch_fcg_matvec: z or the diagonal not 8-byte aligned");
-#define SFP_MATVEC(LIST, ANY)                                                                               \
-    hipLaunchKernelGGL((k_fcg_matvec_flat<LIST, ANY>), dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r, qprev, \
-                       w, first, partials, gate)
-    if (d.nz & 1) {
-        if (list) SFP_MATVEC(true, true); else SFP_MATVEC(false, true);
+    if (list) {
+        hipLaunchKernelGGL(k_fcg_matvec_flat<true>, dim3(list_launch(nb)), dim3(kBlock), 0, st, d, A, active, z, r,
+                           qprev, w, first, partials, nb, gate);
+    } else if (matvec_flat(d)) {
+        hipLaunchKernelGGL(k_fcg_matvec_flat<false>, dim3(nb), dim3(kBlock), 0, st, d, A, active, z, r, qprev, w,
+                           first, partials, nb, gate);
     } else {
-        if (list) SFP_MATVEC(true, false); else SFP_MATVEC(false, false);
+        const Launch L = matvec_launch(d);
+        hipLaunchKernelGGL(k_fcg_matvec, L.grid, L.block, 0, st, L.cg, d, A, active, z, r, qprev, w, first,
+                           partials, gate);
     }
-#undef SFP_MATVEC
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
     if (!fold) finalize(st, FIN_MATVEC, nb, first, iter, partials, sc, gate);
 }
 
-void launch_fcg_update(hipStream_t st, Dims d, const float *active, const unsigned *chunks, const double *w, double *q, double *r,
+void launch_fcg_update(hipStream_t st, Dims d, const float *active, const Chunks &chunks, const double *w, double *q, double *r,
                        float *b32, float *x0, float c0, int first, int iter, bool fold, double *partials,
                        KrylovScalars *sc, const double *gate, hipEvent_t kernel_done, KrylovScalars *host) {
     // two cells per lane: 16-byte (8-byte for the FP32 ones) aligned vectors
@@ -733,13 +885,14 @@ void launch_fcg_update(hipStream_t st, Dims d, const float *active, const unsign
     if ((uintptr_t)active % 8 || (uintptr_t)b32 % 8 || (uintptr_t)x0 % 8)
         throw ArgError("launch_fcg_update: the diagonal, b32 or x0 not 8-byte aligned");
     if (x0 && (!b32 || !active)) throw ArgError("launch_fcg_update: x0 needs b32 and the diagonal");
-    if (chunks && fold) throw ArgError("launch_fcg_update: no list here");
+    if (chunks.blocks && (fold || !active)) throw ArgError("launch_fcg_update: no list here");
     const unsigned nb = update_blocks(d), nb_mv = matvec_blocks(d);
     double *out = partials + 3 * (size_t)nb_mv;
-    if (chunks)
-        hipLaunchKernelGGL(k_fcg_update_list, dim3(list_blocks(d)), dim3(kBlock), 0, st, (unsigned)d.cells(), chunks, active,
-                           w, q, r, b32, x0, c0, first, iter, out, sc, gate);
-    else if (fold)
+    if (chunks.blocks) {
+        out = chunks.sums + 3 * (size_t)nb_mv + 3 * kStageMaxBlocks;
+        hipLaunchKernelGGL(k_fcg_update_list, dim3(list_launch(nb)), dim3(kBlock), 0, st, d.cells(), chunks.blocks,
+                           active, w, q, r, b32, x0, c0, first, iter, out, sc, gate);
+    } else if (fold)
         hipLaunchKernelGGL(k_fcg_update<true>, dim3(nb), dim3(kBlock), 0, st, d.cells(), active, w, q, r, b32, x0,
                            c0, first, iter, partials, nb_mv, out, sc, gate);
     else
@@ -748,7 +901,7 @@ void launch_fcg_update(hipStream_t st, Dims d, const float *active, const unsign
     SFP_LAUNCH_CHECK();
     if (kernel_done) SFP_HIP(hipEventRecord(kernel_done, st));
     if (!fold)
-        finalize(st, FIN_UPDATE, chunks ? list_blocks(d) : nb, 0, 0, out, sc, gate, host);
+        finalize(st, FIN_UPDATE, nb, 0, 0, out, sc, gate, host);
 }
 
 void launch_fcg_norm(hipStream_t st, Dims d, double *partials, KrylovScalars *sc, const double *gate,

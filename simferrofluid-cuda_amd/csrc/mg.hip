@@ -2096,19 +2096,15 @@ __global__ __launch_bounds__(kBlock) void k_chunk_flags(unsigned n, const float 
 }
 
 // The set flags' indices in ascending order (so sums over the listed chunks
-// have a fixed order), list[0] their number. A block for either list: a thread counts a run
+// have a fixed order), list[0] their number. A block for each list: a thread counts a run
 // of flags, 16 at a time, the counts are summed over the threads before it, and
 // it writes its run's (65536 chunks of a 256^3 grid: 12 us, beside the clears).
 constexpr int kListThreads = 1024;
-__global__ __launch_bounds__(kListThreads) void k_chunk_list(unsigned nch, const unsigned char *__restrict__ flags,
-                                                             unsigned *__restrict__ list, unsigned nq,
-                                                             const unsigned char *__restrict__ quad_flags,
-                                                             unsigned *__restrict__ quads) {
-    if (blockIdx.x == 1) {
-        nch = nq;
-        flags = quad_flags;
-        list = quads;
-    }
+__global__ __launch_bounds__(kListThreads) void k_chunk_list(unsigned nch, unsigned nq, unsigned nbl, ActiveLists a) {
+    if (blockIdx.x == 1) nch = nq;
+    if (blockIdx.x == 2) nch = nbl;
+    const unsigned char *const flags = blockIdx.x == 0 ? a.flags : blockIdx.x == 1 ? a.quad_flags : a.block_flags;
+    unsigned *const list = blockIdx.x == 0 ? a.list : blockIdx.x == 1 ? a.quads : a.blocks;
     __shared__ unsigned sums[kListThreads / 64];
     const unsigned tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const unsigned per = ((nch + kListThreads - 1) / kListThreads + 15) / 16 * 16;
@@ -2143,11 +2139,15 @@ __global__ __launch_bounds__(kListThreads) void k_chunk_list(unsigned nch, const
 }
 
 // flags[u]: whether quad u of the restriction (k_restrict_flat's 64 cells of z
-// in two rows and two planes) meets an active chunk.
-__global__ __launch_bounds__(kBlock) void k_quad_flags(Dims d, unsigned quads,
+// in two rows and two planes) meets an active chunk; then whether an FCG block
+// (two chunks) holds one.
+__global__ __launch_bounds__(kBlock) void k_unit_flags(Dims d, unsigned quads, unsigned blocks, unsigned nch,
                                                        const unsigned char *__restrict__ chunk_flags,
-                                                       unsigned char *__restrict__ flags) {
+                                                       unsigned char *__restrict__ quad_flags,
+                                                       unsigned char *__restrict__ block_flags) {
+    static_assert(kListCells == 2 * kChunk, "an FCG block is two chunks");
     const unsigned u = blockIdx.x * kBlock + threadIdx.x;
+    if (u < blocks) block_flags[u] = chunk_flags[2 * u] | (2 * u + 1 < nch ? chunk_flags[2 * u + 1] : 0);
     if (u >= quads) return;
     const unsigned zch = (unsigned)(d.nz + kRestrictFlatZ - 1) / kRestrictFlatZ, yp = (unsigned)(d.ny + 1) / 2;
     const int k0 = kRestrictFlatZ * (int)(u % zch), k1 = min(k0 + kRestrictFlatZ, d.nz) - 1;
@@ -2158,19 +2158,20 @@ __global__ __launch_bounds__(kBlock) void k_quad_flags(Dims d, unsigned quads,
         const int i = min(i0 + (q >> 1), d.nx - 1), j = min(j0 + (q & 1), d.ny - 1);
         a |= chunk_flags[(unsigned)d.idx(i, j, k0) / kChunk] | chunk_flags[(unsigned)d.idx(i, j, k1) / kChunk];
     }
-    flags[u] = a;
+    quad_flags[u] = a;
 }
 
-void launch_active_chunks(hipStream_t st, Dims d, const float *diag32, unsigned char *flags, unsigned *list,
-                          unsigned char *quad_flags, unsigned *quads) {
+void launch_active_chunks(hipStream_t st, Dims d, const float *diag32, const ActiveLists &a) {
     if (!flat_step(d)) throw ArgError("launch_active_chunks: not a flat level");
-    const unsigned n = (unsigned)d.cells(), nch = (n + kChunk - 1) / kChunk, nq = restrict_quads(d);
+    const unsigned n = (unsigned)d.cells(), nch = (n + kChunk - 1) / kChunk, nq = restrict_quads(d),
+                   nbl = (n + kListCells - 1) / kListCells;
     hipLaunchKernelGGL(k_chunk_flags, dim3((nch + kBlock / 64 - 1) / (kBlock / 64)), dim3(kBlock), 0, st, n, diag32,
-                       flags);
+                       a.flags);
     SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_quad_flags, dim3((nq + kBlock - 1) / kBlock), dim3(kBlock), 0, st, d, nq, flags, quad_flags);
+    hipLaunchKernelGGL(k_unit_flags, dim3((std::max(nq, nbl) + kBlock - 1) / kBlock), dim3(kBlock), 0, st, d, nq, nbl,
+                       nch, a.flags, a.quad_flags, a.block_flags);
     SFP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_chunk_list, dim3(2), dim3(kListThreads), 0, st, nch, flags, list, nq, quad_flags, quads);
+    hipLaunchKernelGGL(k_chunk_list, dim3(3), dim3(kListThreads), 0, st, nch, nq, nbl, a);
     SFP_LAUNCH_CHECK();
 }
 

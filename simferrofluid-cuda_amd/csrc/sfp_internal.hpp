@@ -105,11 +105,15 @@ struct DevBuf {
 // chunk is taken): list[0] is their number, list[1 ..] their indices,
 // ascending. The kernels over the flat cell index then run on the listed chunks
 // only: an inactive chunk's cells are 0 and stay so. quads: the same of the
-// restriction's units of 64 cells in two rows and two planes.
+// restriction's units of 64 cells in two rows and two planes; blocks: of the
+// FCG kernels' blocks of kListCells cells, whose partial sums are in `sums` (the
+// matvec's, then the update's, each followed by the two-stage finalize's room; 0
+// at the blocks that are not listed).
 struct Chunks {
-    const unsigned *list = nullptr, *quads = nullptr;
+    const unsigned *list = nullptr, *quads = nullptr, *blocks = nullptr;
+    double *sums = nullptr;
 };
-constexpr unsigned kChunk = 256;
+constexpr unsigned kChunk = 256, kListCells = 512;
 
 // A 7-point symmetric operator on a cell grid:
 //   (A x)_c = diag_c x_c - sum_a ( cpl_a[c] x_{c-e_a} + cpl_a[c+e_a] x_{c+e_a} )
@@ -148,11 +152,14 @@ struct Level {
     // whole rows; null elsewhere and where every row is active)
     DevBuf<unsigned char> rowact;
     // the active chunks (sparse: kept and used), and the step pairs' segments
-    DevBuf<unsigned> chunk_list, quad_list;
-    DevBuf<unsigned char> chunk_flags, quad_flags;
+    DevBuf<unsigned> chunk_list, quad_list, block_list;
+    DevBuf<unsigned char> chunk_flags, quad_flags, block_flags;
+    DevBuf<double> list_sums;
     DevBuf<int> segments;
     bool sparse = false;
-    Chunks chunks() const { return sparse ? Chunks{chunk_list.p, quad_list.p} : Chunks{}; }
+    Chunks chunks() const {
+        return sparse ? Chunks{chunk_list.p, quad_list.p, block_list.p, list_sums.p} : Chunks{};
+    }
     // both operators have the row-sum structure of Op64::pinned_rowsum and
     // Op32::pinned_rowsum, and kernels may rebuild the diagonals
     bool pinned_rowsum = false;

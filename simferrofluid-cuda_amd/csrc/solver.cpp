@@ -193,13 +193,19 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
         // hold an active cell (small grids' launches cost the same either way)
         L.sparse = sparse_ && !(ws.fused_pairs & 32) && flat_step(L.d) && !small_grid(L.d);
         if (L.sparse) {
-            const size_t nch = (L.d.cells() + kChunk - 1) / kChunk;
+            const size_t nch = (L.d.cells() + kChunk - 1) / kChunk, nq = restrict_quads(L.d);
+            const size_t nbl = (L.d.cells() + kListCells - 1) / kListCells;
             L.chunk_flags.ensure(nch);
             L.chunk_list.ensure(nch + 1);
-            L.quad_flags.ensure(restrict_quads(L.d));
-            L.quad_list.ensure(restrict_quads(L.d) + 1);
-            launch_active_chunks(side, L.d, L.diag32.p, L.chunk_flags.p, L.chunk_list.p, L.quad_flags.p,
-                                 L.quad_list.p);
+            L.quad_flags.ensure(nq);
+            L.quad_list.ensure(nq + 1);
+            L.block_flags.ensure(nbl);
+            L.block_list.ensure(nbl + 1);
+            launch_active_chunks(side, L.d, L.diag32.p,
+                                 ActiveLists{L.chunk_flags.p, L.quad_flags.p, L.block_flags.p, L.chunk_list.p,
+                                             L.quad_list.p, L.block_list.p});
+            L.list_sums.ensure(list_sums(L.d));
+            SFP_HIP(hipMemsetAsync(L.list_sums.p, 0, list_sums(L.d) * sizeof(double), side));
             if (const unsigned segs = L.pinned_rowsum ? 0 : pair_segments_max(L.d)) {
                 L.segments.ensure(1 + 3 * (size_t)segs);
                 launch_pair_segments(side, L.d, L.rowact.p, L.segments.p);
@@ -762,7 +768,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             ws.x0_level = -1;
             // (a cycle whose first launch folds forms its first iterate itself)
             float *const x0_next = fold ? nullptr : x0;
-            launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, A.chunks.list, w_.p, q_.p, r_.p, b32, x0_next, c0,
+            launch_fcg_update(st, d, x0_next ? lv_[level].diag32.p : flags, A.chunks, w_.p, q_.p, r_.p, b32, x0_next, c0,
                               first ? 1 : 0, iter + it, fold, ws.partials.p, ws.scalars.p, ws.gate, done,
                               it + 1 == batch ? ws.host_sc : nullptr);
             if (profiling) ws.timers[K_UPDATE64].end_recorded();
