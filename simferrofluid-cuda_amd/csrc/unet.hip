@@ -4,8 +4,8 @@
 // uint16), activation gradients FP32, master weights FP32 with BF16 copies
 // [tap][cout][cin] for the convolutions.
 //
-// k_conv3r is an implicit GEMM: M = output voxels (z rows of 16), N = output
-// channels (blocks of 16), K = 27 taps x input channels, on
+// k_conv3r is an implicit GEMM: M = output channels (blocks of 16), N = output
+// voxels (z rows of 16), K = 27 taps x input channels, on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation. Lane layouts (checked on
 // the device): A[m][k] from lane m%16 + 16*(k/8), B[k][n] from lane
 // n + 16*(k/8), D[m][n] in lane n + 16*(m/4), element m%4.
@@ -55,12 +55,15 @@ struct ConvArgs {
 // outputs are at most 2 GiB).
 constexpr unsigned kInLimit = 0x40000000u, kInOutside = 0x40000000u, kOutOutside = 0x80000000u;
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+typedef uint16_t h4v __attribute__((ext_vector_type(4)));
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ int ch_of(int nb, int r16) { return nb * 16 + r16; }
-__device__ __forceinline__ uint16_t bf16_bits(float f) {  // round to nearest even (v_cvt_pk_bf16_f32)
-    return __builtin_bit_cast(uint16_t, (__bf16)f);
+// four values as BF16 bits, rounded to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ u2v bf16_bits4(v4f f) {
+    return __builtin_bit_cast(u2v, v4bf{(__bf16)f[0], (__bf16)f[1], (__bf16)f[2], (__bf16)f[3]});
 }
 
 // The 3x3x3 convolution (zero padding), optionally reading its input
@@ -76,7 +79,16 @@ __device__ __forceinline__ uint16_t bf16_bits(float f) {  // round to nearest ev
 // one plane ahead of their use, and each fragment feeds the MFMAs of up to 9
 // output rows: planes gx + 1, gx, gx - 1 (dx = 0, 1, 2) times the rows it
 // neighbours in y. Accumulators of three output planes rotate; plane gx - 1
-// is complete after the step and goes through the epilogue.
+// is complete after the step and goes through the epilogue. The weights are
+// operand A, so a lane's four results are four channels of one voxel: one
+// 8-byte store (16 for FP32) and one load of the skip or mask tensor instead of
+// four of 2 bytes each.
+// Small volumes are bound by the march's chain of loads (a step of 36 MFMAs
+// waits about 1 us for the next plane), large ones by the MFMAs and their
+// fragments. 16 -> 16 channels on 8 crops of 32^3: 13.4 -> 11.7 us with these
+// stores and the wavefront's indices in scalar registers. Measured and not
+// taken: fragments two planes ahead (25.9 us), a march rolled to one step per
+// iteration (16.7), twice the wavefronts (17.3).
 template <int CIN>
 constexpr int kchunks() {
     return CIN == 8 ? 1 : CIN == 16 ? 2 : CIN == 32 ? 3 : 6;
@@ -187,7 +199,8 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
     const int X = a.X, Y = a.Y, Z = a.Z;
     const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
     const int ypn = (Y + PY - 1) / PY, zbn = (Z + 15) / 16;
-    unsigned w = blockIdx.x * 4 + (threadIdx.x >> 6);
+    // (in scalar registers, as all that follows from it)
+    unsigned w = blockIdx.x * 4 + (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nb = (int)(w % NB);
     w /= NB;
     const int yp = (int)(w % (unsigned)ypn);
@@ -200,7 +213,7 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
     const int y0 = yp * PY, z0 = zb * 16, xa = xr * run;
     if (xa >= X) return;
     const int xe = min(xa + run, X);
-    // weights [dx][dy][kc]: B[k][n] of lane n + 16 (k / 8)
+    // weights [dx][dy][kc]: A[m][k] of lane m + 16 (k / 8), m the output channel
     v8bf wf[3][3][KC];
 #pragma unroll
     for (int dx = 0; dx < 3; dx++)
@@ -216,8 +229,8 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
                 wf[dx][dy][kc] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(p));
             }
     // this lane's input voxel (z) and channel byte offset per chunk within an
-    // (x, y) row of the (possibly half-resolution) input: A[m][k] of lane
-    // m + 16 (k / 8), m = z - z0 of the output row
+    // (x, y) row of the (possibly half-resolution) input: B[k][n] of lane
+    // n + 16 (k / 8), n = z - z0 of the output row
     const int up = UP ? 1 : a.up;
     const int Xs = up ? X >> 1 : X, Ys = up ? Y >> 1 : Y, Zs = up ? Z >> 1 : Z;
     const auto rin = buf_rsrc(a.in, a.in_bytes);
@@ -249,30 +262,22 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
         }
     }
     const unsigned row_bytes = (unsigned)(Zs * CIN * 2);
-    // Offsets that do not change along the march, per lane: the input rows
-    // y0 - 1 .. y0 + PY (their y part plus the z/channel part; kInOutside
-    // parts where outside the volume), and the output values' (y, z, channel)
-    // part (kOutOutside outside). Each step adds its plane's part, a value
-    // common to the wavefront.
-    unsigned rzc[PY + 2][NC], rzh[PY + 2][NC];
+    // Offsets that do not change along the march: the input rows y0 - 1 .. y0 +
+    // PY (kInOutside where outside the volume; scalars), and per lane the
+    // output values' (y, z, channel) part (kOutOutside outside). Each step adds
+    // its plane's part, a scalar too: one vector add per load or store.
+    unsigned ry[PY + 2];
 #pragma unroll
     for (int iy = 0; iy < PY + 2; iy++) {
         const int gy = y0 + iy - 1;
-        const unsigned ry = gy >= 0 && gy < Y ? (unsigned)(up ? gy >> 1 : gy) * row_bytes : kInOutside;
-#pragma unroll
-        for (int q = 0; q < NC; q++) {
-            rzc[iy][q] = ry + zc[q];
-            rzh[iy][q] = ry + zh[q];
-        }
+        ry[iy] = gy >= 0 && gy < Y ? (unsigned)(up ? gy >> 1 : gy) * row_bytes : kInOutside;
     }
-    unsigned ob[PY][4];  // byte offsets of the 16-bit outputs within a plane
+    unsigned ob[PY];  // byte offsets of the 16-bit outputs within a plane: voxel z0 + r16, channels 4 g .. 4 g + 3
 #pragma unroll
-    for (int oy = 0; oy < PY; oy++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int gy = y0 + oy, gz = z0 + 4 * g + j;
-            ob[oy][j] = gy < Y && gz < Z ? (unsigned)((gy * Z + gz) * COUT + ch_of(nb, r16)) * 2 : kOutOutside;
-        }
+    for (int oy = 0; oy < PY; oy++) {
+        const int gy = y0 + oy, gz = z0 + r16;
+        ob[oy] = gy < Y && gz < Z ? (unsigned)((gy * Z + gz) * COUT + nb * 16 + 4 * g) * 2 : kOutOutside;
+    }
     v4f acc[3][PY];
 #pragma unroll
     for (int s = 0; s < 3; s++)
@@ -292,14 +297,17 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
 #pragma unroll
             for (int q = 0; q < NC; q++) {
                 if (src_row<PY, UP>(iy) != iy) continue;  // (known after unrolling)
-                fc[iy][q] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rin, po + rzc[iy][q], 0, 0));
+                fc[iy][q] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rin, po + ry[iy] + zc[q], 0, 0));
                 if constexpr (kDpp)
                     fh[iy][q] =
-                        __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rin, po + rzh[iy][q], 0, 0));
+                        __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rin, po + ry[iy] + zh[q], 0, 0));
             }
     };
-    const int ch = nb * 16 + r16;
-    const float bias = a.bias ? a.bias[ch] : 0.f;
+    v4f bias = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) bias[j] = a.bias[nb * 16 + 4 * g + j];
+    }
     const auto rskip = buf_rsrc(a.skip, a.skip ? 2 * a.out_elems : 0);
     const auto rout = buf_rsrc(a.out, a.out ? 2 * a.out_elems : 0);
     const auto rout32 = buf_rsrc(a.out32, a.out32 ? 4 * a.out_elems : 0);
@@ -324,13 +332,11 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
         const unsigned pb = (unsigned)((b * X + (gx - 1)) * Y * Z * COUT) * 2;
         // the skip values of that plane, loaded before the next plane's
         // fragments so that waiting for them leaves those in flight
-        uint16_t skv[PY][4];
+        u2v skv[PY];
         if (has_skip && t >= 2) {
 #pragma unroll
             for (int oy = 0; oy < PY; oy++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    skv[oy][j] = __builtin_amdgcn_raw_buffer_load_b16(rskip, pb + ob[oy][j], 0, 0);
+                skv[oy] = __builtin_bit_cast(u2v, __builtin_amdgcn_raw_buffer_load_b64(rskip, pb + ob[oy], 0, 0));
         }
         if constexpr (L) load_plane(fc[1 - P], fh[1 - P], gx + 1);  // (one past the run at the end: unused)
 #pragma unroll
@@ -350,7 +356,7 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
 #pragma unroll
                     for (int kc = 0; kc < KC; kc++)
                         acc[(U - dx + 3) % 3][oy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            ck[kc], wf[dx][dy][kc], acc[(U - dx + 3) % 3][oy], 0, 0, 0);
+                            wf[dx][dy][kc], ck[kc], acc[(U - dx + 3) % 3][oy], 0, 0, 0);
                 }
         }
         // planes before the run (gx + 1 - dx < xa) took contributions in
@@ -367,22 +373,27 @@ __global__ __launch_bounds__(256, WPS) void k_conv3r(ConvArgs a, int run, int xr
             constexpr int S = (U + 1) % 3;
 #pragma unroll
             for (int oy = 0; oy < PY; oy++) {
+                const unsigned o = pb + ob[oy];  // past the buffers where outside the volume
+                v4f v = acc[S][oy] + bias;
+                if (relu)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const unsigned o = pb + ob[oy][j];  // past the buffers where outside the volume
-                    float v = acc[S][oy][j] + bias;
-                    if (relu) v = v > 0.f ? v : 0.f;
-                    if (has_relu_copy) __builtin_amdgcn_raw_buffer_store_b16(bf16_bits(v), rrelu, o, 0, 0);
-                    if (has_skip && !mask) v += bf2f(skv[oy][j]);
-                    if (mask)
-                        __builtin_amdgcn_raw_buffer_store_b16(
-                            bf2f(skv[oy][j]) > 0.f ? bf16_bits(v) : (uint16_t)0, rout, o, 0, 0);
-                    if (f32)  // (FP32 output: twice the 16-bit offset)
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rout32,
-                                                              ob[oy][j] == kOutOutside ? kOutOutside : 2 * o, 0, 0);
-                    else if (!mask)
-                        __builtin_amdgcn_raw_buffer_store_b16(bf16_bits(v), rout, o, 0, 0);
+                    for (int j = 0; j < 4; j++) v[j] = v[j] > 0.f ? v[j] : 0.f;
+                if (has_relu_copy) __builtin_amdgcn_raw_buffer_store_b64(bf16_bits4(v), rrelu, o, 0, 0);
+                const h4v sk = __builtin_bit_cast(h4v, skv[oy]);
+                if (has_skip && !mask)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] += bf2f(sk[j]);
+                if (mask) {
+                    h4v m = __builtin_bit_cast(h4v, bf16_bits4(v));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) m[j] = bf2f(sk[j]) > 0.f ? m[j] : (uint16_t)0;
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, m), rout, o, 0, 0);
                 }
+                if (f32)  // (FP32 output: twice the 16-bit offset)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, v), rout32,
+                                                           ob[oy] == kOutOutside ? kOutOutside : 2 * o, 0, 0);
+                else if (!mask)
+                    __builtin_amdgcn_raw_buffer_store_b64(bf16_bits4(v), rout, o, 0, 0);
                 acc[S][oy] = v4f{0.f, 0.f, 0.f, 0.f};
             }
         }
@@ -892,9 +903,11 @@ void conv_dispatch(hipStream_t st, const ConvArgs &a) {
     // 216)
     constexpr int PY = CIN == 8 ? 4 : COUT == 64 ? 1 : 2;
     constexpr int WPS = CIN <= 32 ? 2 : 1;
-    // x runs: about two wavefronts per SIMD of the 256 CUs
+    // x runs: WPS wavefronts per SIMD of the 256 CUs. With 64 input channels
+    // one fits, and a second round of them loads its weights (54 KB each) again:
+    // 64 -> 64 on 8 volumes of 8^3 in 21.6 us with 2048 wavefronts, 13.3 with 1024
     const long long base = (long long)a.B * ((a.Z + 15) / 16) * ((a.Y + PY - 1) / PY) * (COUT / 16);
-    const long long target = 2048;
+    const long long target = 1024 * WPS;
     int xruns = (int)std::min<long long>(a.X, std::max<long long>(1, (target + base - 1) / base));
     const int run = (a.X + xruns - 1) / xruns;
     xruns = (a.X + run - 1) / run;
