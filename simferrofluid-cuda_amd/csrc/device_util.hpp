@@ -130,6 +130,12 @@ __device__ __forceinline__ void block_partials(double (&v)[N], double *partials)
     }
 }
 
+// A raw buffer over `bytes` bytes from p: a load at an offset past them reads 0
+// and a store there is dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+
 // Inside a one-block kernel of T threads: totals of nb block partials, valid
 // in thread 0. Each thread keeps U running sums so U loads per sum are in
 // flight at a time (tens of thousands of partials in a few microseconds);

@@ -677,12 +677,10 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
 // SM_XFIRST | SM_WRITE_D when d1 is x1 (kDx), then SM_READ_D), bit for bit.
 //
 // Each iteration of the march, for plane i:
-//   1. puts x1 and cpl_y of plane i + 2 (loaded one iteration earlier) in
-//      LDS, with the out-of-tile rows next to the tile (rows 0 and
-//      kRowPairRows - 1 load them);
-//   2. issues the loads of x1, cpl_x, cpl_y of plane i + 3 and of cpl_z, b,
-//      d1 and the diagonal of plane i + 2, so one iteration hides their
-//      latency;
+//   1. puts x1, cpl_x and cpl_y of plane i + 2 (loaded kEarlyAhead - 2
+//      iterations earlier) in LDS, with the out-of-tile rows next to the tile;
+//   2. issues the loads of x1, cpl_x, cpl_y of plane i + kEarlyAhead and of
+//      cpl_z, b, d1 and the diagonal of plane i + kRestAhead;
 //   3. computes step A on plane i + 1 (x1 of the rows above and below and
 //      their cpl_y from LDS) and puts x2 in LDS; one barrier;
 //   4. computes step B on plane i (x2 of the three planes and of the rows
@@ -690,14 +688,22 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
 // LDS rings: x1 two planes deep (written an iteration before it is read, and
 // rewritten only after the next barrier), x2 three (written before the
 // barrier that precedes its readers, which a wavefront one barrier ahead must
-// not disturb) and cpl_y four (read by step A in one iteration and by step B
-// in the next). `rowact` (null: every row active) marks the (plane, row) z
-// rows holding an active cell: the others load nothing and stay 0, as the
-// vectors hold there.
+// not disturb), cpl_y four (read by step A in one iteration and by step B
+// in the next) and cpl_x three (read by the wavefront that wrote it only).
+// `rowact` (null: every row active) marks the (plane, row) z rows holding an
+// active cell: the others load nothing and stay 0, as the vectors hold there.
+//
+// One block per CU (152 KB of LDS, 160 registers) has to keep enough loads in
+// flight for its share of the memory's rate: what bounds it is their latency.
+// 256^3, every row active: 94 us a pair (28 B per cell) and 87 with d1 = x1
+// (24 B), 5.1-5.5 TB/s with the rows read twice; 110 and 108 with the loads
+// behind branches and one plane ahead, 99 and 94 one plane ahead.
 constexpr int kRowPairRows = 12;
 constexpr int kRowPairY = kRowPairRows - 2;  // interior rows: the tiles' stride in y
 // the out-of-tile rows take one value per thread: 3 parts of 256 z values
-static_assert(64 * kRowPairRows >= 3 * 256, "k_smooth_pair_rows: too few threads for the halo rows");
+static_assert(64 * kRowPairRows == 3 * 256, "k_smooth_pair_rows: the halo rows take every thread");
+// A byte offset past every run's planes; two of them add up without wrapping.
+constexpr unsigned kPairOut = 0x40000000u;
 
 template <bool kRowsum, bool kDx>
 __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
@@ -706,12 +712,17 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     float crB, const unsigned char *__restrict__ rowact, const int *__restrict__ segments, int planes,
     unsigned ytiles, const double *gate) {
     typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
     if (gated(gate)) return;
     const unsigned runs = segments ? (unsigned)segments[0] : gridDim.x;
     if (blockIdx.x >= runs) return;
     __shared__ f4 sx1[2][kRowPairRows + 2][64];  // x1 of rows -1 .. kRowPairRows (index row + 1)
     __shared__ f4 scy[4][kRowPairRows + 1][64];  // cpl_y of rows 0 .. kRowPairRows
     __shared__ f4 sx2[3][kRowPairRows][64];      // x2 of rows 0 .. kRowPairRows - 1
+    // the stored diagonal of lane 0's group on planes 0 and 1: a row-sum
+    // diagonal is rebuilt but in the groups of cells 1, nz and nz*ny
+    __shared__ f4 sdg[2][kRowsum ? kRowPairRows : 1];
+    __shared__ f4 scx[3][kRowPairRows][64];      // cpl_x, read by the wavefront that wrote it
     // logical tiles run y fastest; each XCD (block b goes to XCD b % 8) takes
     // a contiguous run of them, so the rows two tiles share meet in one L2
     unsigned L = blockIdx.x;
@@ -727,7 +738,7 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
         ie = segments[3 + 3 * L];
     }
     if (i0 >= d.nx) return;  // uniform over the block
-    const int lane = threadIdx.x, row = threadIdx.y;
+    const int lane = threadIdx.x, row = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int k = 4 * lane;
     const int j = (int)by * kRowPairY - 1 + row;
     const bool zon = k < d.nz;
@@ -740,21 +751,33 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     // past the row's end read its last group (a cache hit) and drop it
     const unsigned c0 = yin ? (unsigned)d.idx(0, j, min(k, d.nz - 4)) : 0u;
     const unsigned sx = (unsigned)s.sx;
+    // Every load is a buffer load over planes p0 .. of the run, issued on every
+    // row and lane: one that has nothing to load (an inactive row, a plane
+    // outside, a lane past the row) passes an offset past the buffer, which
+    // reads 0 and moves nothing. (Behind branches, or with a select on what
+    // they loaded, the loads were waited for where they were issued: the
+    // compiler cannot count those in flight. 256^3: 110 us a pair so.)
+    const int p0 = max(i0 - 2, 0);
+    const unsigned plane_bytes = 4 * sx;
+    const unsigned run_bytes = (unsigned)(min(ie + 6, d.nx) - p0) * plane_bytes;  // (< kPairOut)
+    auto rsrc = [&](const float *p) { return buf_rsrc(p + (size_t)p0 * sx, run_bytes); };
+    const auto rx1 = rsrc(x1), rcx = rsrc(A.cpl[0]), rcy = rsrc(A.cpl[1]), rcz = rsrc(A.cpl[2]), rb = rsrc(b),
+               rd1 = rsrc(d1), rdg = rsrc(A.diag), rxo = rsrc(xo);
+    const unsigned o0 = yin && zon ? 4 * c0 : kPairOut;  // bytes within a plane
     // the out-of-tile rows next to the tile (x1 of rows j0 - 1 and
     // j0 + kRowPairRows - 2, cpl_y of the latter), one value per thread: thread
     // t of the block takes z = t mod 256 of part t / 256
-    const int t = row * 64 + lane;
-    const int hpart = t >> 8, hz = t & 255;  // part 3: nothing
+    const int hpart = row >> 2, hz = (row & 3) * 64 + lane;
     const int jt = (int)by * kRowPairY - 1;  // the tile's row 0
     const int jh = hpart == 0 ? jt - 1 : jt + kRowPairRows;
-    const bool hon_any = hpart < 3 && jh >= 0 && jh < d.ny;  // uniform over the wavefront
-    const unsigned ch = hon_any ? (unsigned)d.idx(0, jh, min(hz, d.nz - 1)) : 0u;
+    const bool hon_any = jh >= 0 && jh < d.ny;  // uniform over the wavefront
+    const unsigned oh = hon_any && hz < d.nz ? 4 * (unsigned)d.idx(0, jh, hz) : kPairOut;
     const f4 z4 = {0.f, 0.f, 0.f, 0.f};
     // activity of this row and of the out-of-tile row for planes i0 - 2 ..
     // i0 + 61 (bit q - i0 + 2), one lane per plane, read once
     auto row_mask = [&](int jj) -> unsigned long long {
         const int q = i0 - 2 + lane;
-        const bool a = q >= 0 && q < d.nx && jj >= 0 && jj < d.ny &&
+        const bool a = q >= 0 && q < d.nx && q <= ie + 1 && jj >= 0 && jj < d.ny &&
                        (!rowact || rowact[(size_t)q * d.ny + jj] != 0);
         return __ballot(a);
     };
@@ -762,7 +785,10 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     const unsigned long long hmask_lo = row_mask(jt - 1), hmask_hi = row_mask(jt + kRowPairRows);
     const unsigned long long hmask = hpart == 0 ? hmask_lo : hmask_hi;
     auto active = [&](int q, unsigned long long m) { return ((m >> (q - i0 + 2)) & 1ull) != 0; };
-    auto ld = [&](const float *p) { return zon ? *(const f4 *)p : z4; };
+    auto at = [&](int q, unsigned long long m) { return active(q, m) ? (unsigned)(q - p0) * plane_bytes : kPairOut; };
+    auto ld = [&](__amdgpu_buffer_rsrc_t p, unsigned o) {
+        return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(p, o0 + o, 0, 0));
+    };
 
     struct Early {
         f4 x, cx, cy;  // x1, cpl_x, cpl_y
@@ -771,41 +797,33 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     struct Rest {
         f4 cz, bv, dv, dg;
     };
-    // loads branch on the wavefront's row activity only (uniform)
     auto load_early = [&](int q) {
-        Early e{z4, z4, z4, 0.f};
-        if (active(q, amask)) {
-            const unsigned c = c0 + (unsigned)q * sx;
-            e.x = ld(x1 + c);
-            e.cx = ld(A.cpl[0] + c);
-            e.cy = ld(A.cpl[1] + c);
-        }
-        if (hon_any && active(q, hmask)) {
-            const unsigned h = ch + (unsigned)q * sx;
-            const float v = hpart == 2 ? A.cpl[1][h] : x1[h];
-            e.h = hz < d.nz ? v : 0.f;
-        }
+        Early e;
+        const unsigned o = at(q, amask);
+        e.x = ld(rx1, o);
+        e.cx = ld(rcx, o);
+        e.cy = ld(rcy, o);
+        e.h = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(hpart == 2 ? rcy : rx1,
+                                                                             oh + at(q, hmask), 0, 0));
         return e;
     };
     auto load_rest = [&](int q) {
-        Rest r{z4, z4, z4, z4};
-        if (active(q, amask)) {
-            const unsigned c = c0 + (unsigned)q * sx;
-            r.cz = ld(A.cpl[2] + c);
-            r.bv = ld(b + c);
-            if (!kDx) r.dv = ld(d1 + c);
-            // a row-sum diagonal is rebuilt; the groups of cells 1, nz and
-            // nz*ny (on planes 0 and 1, rows 0 and 1) read it
-            if (!kRowsum || !A.pinned_rowsum || (q <= 1 && j <= 1)) r.dg = ld(A.diag + c);
-        }
+        Rest r;
+        const unsigned o = at(q, amask);
+        r.cz = ld(rcz, o);
+        r.bv = ld(rb, o);
+        r.dv = r.dg = z4;
+        if constexpr (!kDx) r.dv = ld(rd1, o);
+        if constexpr (!kRowsum) r.dg = ld(rdg, o);
         return r;
     };
     auto put_early = [&](int q, const Early &e) {
         sx1[q & 1][row + 1][lane] = e.x;
         scy[q & 3][row][lane] = e.cy;
+        scx[(q + 3) % 3][row][lane] = e.cx;
         if (hpart == 0) ((float *)&sx1[q & 1][0][0])[hz] = e.h;
         else if (hpart == 1) ((float *)&sx1[q & 1][kRowPairRows + 1][0])[hz] = e.h;
-        else if (hpart == 2) ((float *)&scy[q & 3][kRowPairRows][0])[hz] = e.h;
+        else ((float *)&scy[q & 3][kRowPairRows][0])[hz] = e.h;
     };
     // one Chebyshev step of the four cells at plane q from iterate xc (x
     // neighbours xm, xp; y neighbours and couplings given), direction dp
@@ -838,11 +856,14 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     // the diagonal at plane q: loaded, or rebuilt from the couplings
     auto diag_at = [&](int q, f4 cxc, f4 cxp, f4 cym, f4 cyp, const Rest &r) {
         f4 dg = r.dg;
-        if (kRowsum && A.pinned_rowsum) {
-            const unsigned c = c0 + (unsigned)q * sx;
+        if constexpr (kRowsum) {
             const float czdn = __shfl_down(r.cz.x, 1, 64);  // all lanes (see cheb)
             const float czhi = zh ? czdn : 0.f;
-            if (rowsum_group(A, c, d)) dg = rowsum_diag4(cxc, cxp, cym, cyp, r.cz, czhi);
+            dg = rowsum_diag4(cxc, cxp, cym, cyp, r.cz, czhi);
+            if (q <= 1 && j <= 1) {  // uniform
+                const f4 stored = sdg[q & 1][row];
+                if (!rowsum_group(A, c0 + (unsigned)q * sx, d)) dg = stored;
+            }
         }
         return dg;
     };
@@ -851,66 +872,75 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     // plane's diagonal and its reciprocal again from the same operands (bit
     // for bit the same values): carried in registers for an iteration they
     // made the kernel spill.
-    auto step_a = [&](int q, f4 xm, const Early &e, f4 cxp, const Rest &r, f4 &d2) {
-        const f4 xc = sx1[q & 1][row + 1][lane], xp = sx1[(q + 1) & 1][row + 1][lane];
-        const f4 xym = sx1[q & 1][row][lane], xyp = sx1[q & 1][row + 2][lane];
+    auto step_a = [&](int q, f4 xm, const Rest &r, f4 &d2, f4 &xc) {
         const f4 cym = scy[q & 3][row][lane], cyp = scy[q & 3][row + 1][lane];
-        const f4 dg = diag_at(q, e.cx, cxp, cym, cyp, r);
+        const f4 cxc = scx[(q + 3) % 3][row][lane], cxp = scx[(q + 4) % 3][row][lane];
+        const f4 dg = diag_at(q, cxc, cxp, cym, cyp, r);
+        // (the FP64 row sums' registers are free again before x1 is read)
+        if constexpr (kRowsum) __builtin_amdgcn_sched_barrier(0);
+        xc = sx1[q & 1][row + 1][lane];
+        const f4 xp = sx1[(q + 1) & 1][row + 1][lane];
+        const f4 xym = sx1[q & 1][row][lane], xyp = sx1[q & 1][row + 2][lane];
         f4 rdg;
 #pragma unroll
         for (int k = 0; k < 4; k++) rdg[k] = rcp_or_zero(dg[k]);
         d2 = z4;
         if (!active(q, amask)) return z4;  // uniform over the wavefront
-        f4 x2 = cheb(xc, xm, xp, xym, xyp, e.cx, cxp, cym, cyp, r.cz, r.bv, dg, rdg, kDx ? xc : r.dv,
+        f4 x2 = cheb(xc, xm, xp, xym, xyp, cxc, cxp, cym, cyp, r.cz, r.bv, dg, rdg, kDx ? xc : r.dv,
                      cdA, crA, d2);
         if (!zon) x2 = z4;
         return x2;
     };
 
     // ---- prologue: planes i0 - 1 and i0 through step A, plane i0 + 1 in LDS
+    // E: planes i + 2 and i + 3 in flight, by the parity of i - i0; R: planes i
+    // and i + 1 and, in flight, i + 2, by their distance from i0 mod 4; D: the
+    // direction of planes i and i + 1 from step A. (The march is unrolled by
+    // four, so every index is a constant and nothing in flight is copied.)
+    // (three planes ahead for R beside the diagonal, or four for E beside d1, spills)
+    constexpr int kEarlyAhead = kDx ? 4 : 3, kRestAhead = kRowsum ? 3 : 2;
+    if constexpr (kRowsum) {
+        if (i0 <= 2 && yin && j <= 1 && lane == 0)
+            for (int q = 0; q < min(2, d.nx); q++) sdg[q][row] = *(const f4 *)(A.diag + c0 + (size_t)q * sx);
+    }
+    Early E[2];
+    Rest R[4];
+    f4 D[2];
     const f4 xpre = load_early(i0 - 2).x;
-    Early em = load_early(i0 - 1), e0 = load_early(i0), e1 = load_early(i0 + 1);
-    Early e2 = load_early(i0 + 2);
-    Rest rm = load_rest(i0 - 1), r0 = load_rest(i0), r1 = load_rest(i0 + 1);
+    const Early em = load_early(i0 - 1), e0 = load_early(i0), e1 = load_early(i0 + 1);
+    R[3] = load_rest(i0 - 1);
+    R[0] = load_rest(i0);
+    E[0] = load_early(i0 + 2);
+    R[1] = load_rest(i0 + 1);
+    if constexpr (kEarlyAhead == 4) E[1] = load_early(i0 + 3);
+    if constexpr (kRestAhead == 3) R[2] = load_rest(i0 + 2);
     // step A at i0 - 1 reads planes i0 - 1 and i0 from the x1 ring, step A at
     // i0 planes i0 and i0 + 1 (which takes the buffer of i0 - 1)
     put_early(i0 - 1, em);
     put_early(i0, e0);
     __syncthreads();
-    f4 dtmp, d2c;
-    const f4 x2m = step_a(i0 - 1, xpre, em, e0.cx, rm, dtmp);
+    f4 xa, xb;  // x1 at planes i and i + 1 (this row)
+    f4 x2prev = step_a(i0 - 1, xpre, R[3], D[0], xa);  // x2 at plane i - 1 (this row)
     __syncthreads();
     put_early(i0 + 1, e1);
     __syncthreads();
-    const f4 x2c = step_a(i0, em.x, e0, e1.cx, r0, d2c);
-    sx2[(i0 + 2) % 3][row][lane] = x2m;  // (i0 - 1) mod 3
-    sx2[i0 % 3][row][lane] = x2c;
+    {
+        const f4 x2c = step_a(i0, xa, R[0], D[0], xb);
+        sx2[(i0 + 2) % 3][row][lane] = x2prev;  // (i0 - 1) mod 3
+        sx2[i0 % 3][row][lane] = x2c;
+    }
+    xa = xb;
     __syncthreads();
-    // Rings indexed by plane - i0 mod 3 (the march is unrolled by three, so
-    // every index is a constant and nothing is copied between iterations):
-    // E holds x1 / cpl_x / cpl_y of planes i + 1 and i + 2 and receives plane
-    // i + 3 in the slot of plane i; R the rest of planes i, i + 1 (and i + 2,
-    // loaded into the slot of plane i - 1); D2 the direction of planes i and
-    // i + 1 from step A.
-    Early E[3] = {e0, e1, e2};
-    Rest R[3] = {r0, r1, Rest{z4, z4, z4, z4}};
-    f4 D2[3];
-    D2[0] = d2c;
-    f4 xa = e0.x;     // x1 at plane i
-    f4 cxa = e0.cx;   // cpl_x at plane i
-    f4 x2prev = x2m;  // x2 at plane i - 1 (this row)
-    (void)x2c;
     auto iter = [&](auto Uc, int i) {
-        constexpr int U = decltype(Uc)::value, U1 = (U + 1) % 3, U2 = (U + 2) % 3;
-        // 1. loads for the next iteration, in flight during this one's two
-        // steps: their slots hold planes i and i - 1, which this iteration
-        // no longer reads (plane i's x1 and cpl_x are in xa, cxa)
-        E[U] = load_early(i + 3);
-        R[U2] = load_rest(i + 2);
-        // 2. x1 and cpl_y of plane i + 2 into LDS
-        put_early(i + 2, E[U2]);
+        constexpr int U = decltype(Uc)::value;
+        // 1. what was loaded two iterations ago: x1 and the couplings of plane
+        // i + 2 into LDS
+        put_early(i + 2, E[U & 1]);
+        // 2. loads into registers just read, in flight for two iterations
+        E[(U + kEarlyAhead) & 1] = load_early(i + kEarlyAhead);
+        R[(U + kRestAhead) & 3] = load_rest(i + kRestAhead);
         // 3. step A on plane i + 1
-        const f4 x2n = step_a(i + 1, xa, E[U1], E[U2].cx, R[U1], D2[U1]);
+        const f4 x2n = step_a(i + 1, xa, R[(U + 1) & 3], D[(U + 1) & 1], xb);
         sx2[(i + 1) % 3][row][lane] = x2n;
         __syncthreads();
         // 4. step B on plane i (the tile's interior rows)
@@ -918,28 +948,32 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
             const int bi = i % 3;
             const f4 xc = sx2[bi][row][lane];
             if (active(i, amask)) {
+                const Rest &r = R[U];
                 const f4 xym = sx2[bi][row - 1][lane], xyp = sx2[bi][row + 1][lane];
                 const f4 cym = scy[i & 3][row][lane], cyp = scy[i & 3][row + 1][lane];
-                const f4 dgB = diag_at(i, cxa, E[U1].cx, cym, cyp, R[U]);
+                const f4 cxc = scx[bi][row][lane], cxp = scx[(i + 1) % 3][row][lane];
+                const f4 dgB = diag_at(i, cxc, cxp, cym, cyp, r);
                 f4 rdgB;
 #pragma unroll
                 for (int k = 0; k < 4; k++) rdgB[k] = rcp_or_zero(dgB[k]);
                 f4 dn;
-                const f4 x3 = cheb(xc, x2prev, x2n, xym, xyp, cxa, E[U1].cx, cym, cyp, R[U].cz, R[U].bv, dgB,
-                                   rdgB, D2[U], cdB, crB, dn);
-                if (zon) *(f4 *)(xo + c0 + (unsigned)i * sx) = x3;
+                const f4 x3 = cheb(xc, x2prev, x2n, xym, xyp, cxc, cxp, cym, cyp, r.cz, r.bv, dgB, rdgB, D[U & 1],
+                                   cdB, crB, dn);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x3), rxo,
+                                                       o0 + (unsigned)(i - p0) * plane_bytes, 0, 0);
             }
             x2prev = xc;
         }
-        xa = E[U1].x;
-        cxa = E[U1].cx;
+        xa = xb;
     };
-    for (int i = i0; i < ie; i += 3) {  // uniform over the block
+    for (int i = i0; i < ie; i += 4) {  // uniform over the block
         iter(std::integral_constant<int, 0>{}, i);
         if (i + 1 >= ie) break;
         iter(std::integral_constant<int, 1>{}, i + 1);
         if (i + 2 >= ie) break;
         iter(std::integral_constant<int, 2>{}, i + 2);
+        if (i + 3 >= ie) break;
+        iter(std::integral_constant<int, 3>{}, i + 3);
     }
 }
 
@@ -2043,7 +2077,12 @@ Launch pair_launch(Dims d, bool even_planes) {
     return L;
 }
 
-bool row_pair(Dims d) { return d.nz % 4 == 0 && d.nz > 192 && d.nz <= 256 && d.cells() < (size_t(1) << 32); }
+// (k_smooth_pair_rows addresses a run's planes, at most 64 with their
+// neighbours, by byte offsets below kPairOut)
+bool row_pair(Dims d) {
+    return d.nz % 4 == 0 && d.nz > 192 && d.nz <= 256 && d.cells() < (size_t(1) << 32) &&
+           64 * 4 * (size_t)d.ny * d.nz < kPairOut;
+}
 
 // Compute units of the current device (cached per device).
 static int device_cus() {

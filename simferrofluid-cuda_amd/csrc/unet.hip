@@ -58,9 +58,6 @@ typedef unsigned u4v __attribute__((ext_vector_type(4)));
 typedef unsigned u2v __attribute__((ext_vector_type(2)));
 typedef uint16_t h4v __attribute__((ext_vector_type(4)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, unsigned bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
-}
 // four values as BF16 bits, rounded to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ u2v bf16_bits4(v4f f) {
     return __builtin_bit_cast(u2v, v4bf{(__bf16)f[0], (__bf16)f[1], (__bf16)f[2], (__bf16)f[3]});
