@@ -94,10 +94,10 @@ HOT_KERNELS = {
                  "flexible-CG w = A z with the FP64 operator and its 3 inner products "
                  "(two cells of a z row per lane): reads z, 3 FP64 couplings (the magnetic "
                  "diagonal rebuilt from them, no activity flags), r, q_prev, writes w"),
-    "update64": ("k_fcg_update", 80.0,
-                 "flexible-CG update of p, q, r (FP64) with r.r, the FP32 copy b of r and the next "
-                 "cycle's first iterate c0 D^-1 b; x read and written every other iteration "
-                 "(88 B then 72 B per cell)"),
+    "update64": ("k_fcg_update", 52.0,
+                 "flexible-CG update of q, r (FP64) with r.r, the FP32 copy b of r and the next "
+                 "cycle's first iterate c0 D^-1 b: reads w, q, r, diag, writes q, r, b, x0 (x and p "
+                 "are formed from the kept z of several iterations in one pass, k_fcg_flush)"),
     "restrict": ("k_restrict_flat", 21.5, "fine-level FP32 residual summed over 2x2x2 children, "
                  "with the coarse level's first Chebyshev iterate"),
 }
@@ -135,7 +135,7 @@ def summarize_profiles(d, n=256):
     alg = bpc * cells
     avg = statistics.mean(fine)
     lines = [f"# {sym} at {n}^3: rocprofv3 kernel trace", "", f"{what}.", "",
-             "Commands (GPU box, repo root):", "",
+             "Commands (repo root):", "",
              "    python3 bench.py > gpurun_out/bench_full.json",
              "    rocprofv3 --kernel-trace --stats -f csv -d gpurun_out/prof_trace -o trace -- \\",
              "        python3 bench.py --no-cpu-baseline --no-profile --no-learned --steps 4 --warmup 0 --systems m2,m8",
@@ -184,7 +184,7 @@ def summarize_profiles(d, n=256):
            "traffic_over_algorithmic": (rd + wr) / alg}
     json.dump(res, open(os.path.join(out_dir, f"traffic_{name}_{n}.json"), "w"), indent=1)
     md = [f"# {sym} at {n}^3: HBM traffic from FETCH_SIZE / WRITE_SIZE", "",
-          "Commands (GPU box, repo root), one counter per pass:", "",
+          "Commands (repo root), one counter per pass:", "",
           "    python3 bench.py > gpurun_out/bench_full.json",
           "    rocprofv3 --pmc FETCH_SIZE -f csv -d gpurun_out/prof_fetch -o fetch -- \\",
           "        python3 bench.py --no-cpu-baseline --no-profile --no-learned --steps 2 --warmup 0 --systems m2,m8",
@@ -252,7 +252,7 @@ def summarize_profiles(d, n=256):
         unet = [r for r in st if "k_conv" in r["Name"] or "k_pool" in r["Name"] or "k_up2" in r["Name"]
                 or "k_head" in r["Name"] or "k_pack" in r["Name"] or "k_corr" in r["Name"]]
         lm = [f"# Learned leg at {n}^3 (network on the {n // 2}^3 first coarse level): rocprofv3 kernel trace",
-              "", "Command (GPU box, repo root):", "",
+              "", "Command (repo root):", "",
               "    rocprofv3 --kernel-trace --stats -f csv -d gpurun_out/prof_learned -o learned -- \\",
               "        python3 bench.py --no-cpu-baseline --no-profile --steps 2 --warmup 1 --systems p", "",
               "The run holds both legs (plain MG-PCG, then the learned preconditioner) of 3 pressure",
