@@ -34,22 +34,26 @@ void launch_smooth(hipStream_t s, int mode, Dims d, Op32 A, const double *r64, f
 // from x1. Same results as the two launch_smooth calls, bit for bit.
 // With x1 == d1 (the stored zero-start iterate, which is also the previous
 // direction) the pair is the first two steps of a cycle.
-// pair_pays: grids on which it beats the two launches on MI355X (its 64 x 16
-// tiles overlap by one cell per side; measured equal at 128^3, faster above).
-inline bool pair_pays(Dims d) { return d.nz >= 64 && d.cells() > ((size_t)1 << 21); }
+// pair_pays: grids on which it beats the two launches on MI355X. The 64 x 16
+// tiles overlap by one cell per side: equal at 128^3, faster above. Whole rows
+// of 97..128 cells: 20 us against 23 at 128^3, 45 against 82 at 256 x 256 x 128
+// (magnetic solves 1.03x and 1.1x), 1.01x at 100 x 105 x 100.
+bool row_pair(Dims d);
+inline bool pair_pays(Dims d) {
+    return d.nz >= 64 && d.cells() > ((size_t)1 << (row_pair(d) && d.nz <= 128 ? 20 : 21));
+}
 // Grids on which launch_smooth runs its steps (all but the fused first step)
 // over the flat cell index: fewer than 2^32 cells. whole_groups: with the
 // prolongation too (nz a multiple of 4).
 bool flat_step(Dims d);
 bool whole_groups(Dims d);
-// Grids with z rows of 193..256 cells in groups of four run it over whole
-// rows (k_smooth_pair_rows); rowact (null: all active) marks the z rows
+// Grids with z rows of 97..128 or 193..256 cells in groups of four run it over
+// whole rows (k_smooth_pair_rows); rowact (null: all active) marks the z rows
 // holding an active cell (launch_row_activity), whose loads the others skip.
 void launch_smooth_pair(hipStream_t s, Dims d, Op32 A, const float *b, const float *x1, float *x3,
                         const float *d1, float cdA, float crA, float cdB, float crB,
                         const double *gate = nullptr, const unsigned char *rowact = nullptr,
                         const int *segments = nullptr);
-bool row_pair(Dims d);
 // The lists of a level's active chunks, restriction units and FCG blocks (see
 // Chunks; flags: a byte for each, lists: an entry for each and one more).
 unsigned restrict_quads(Dims d);

@@ -669,10 +669,10 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
 
 // The same pair of steps (step A, then step B with kRestrict false) on grids
 // whose z rows hold at most 256 cells, in groups of four: a lane holds four
-// consecutive cells of a z row (16-byte accesses), a wavefront a whole row,
-// a block kRowPairRows rows of y, and the block marches over its run of x
+// consecutive cells of a z row (16-byte accesses), a wavefront a whole row or
+// two, a block kRows rows of y, and the block marches over its run of x
 // planes. Tiles overlap by one row on each side in y (rows 0 and
-// kRowPairRows - 1 are step A's halo) and not at all in z. The per-cell
+// kRows - 1 are step A's halo) and not at all in z. The per-cell
 // arithmetic is k_smooth_flat's (two launches: SM_READ_D | SM_WRITE_D, or
 // SM_XFIRST | SM_WRITE_D when d1 is x1 (kDx), then SM_READ_D), bit for bit.
 //
@@ -698,15 +698,20 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
 // 256^3, every row active: 94 us a pair (28 B per cell) and 87 with d1 = x1
 // (24 B), 5.1-5.5 TB/s with the rows read twice; 110 and 108 with the loads
 // behind branches and one plane ahead, 99 and 94 one plane ahead.
-constexpr int kRowPairRows = 12;
-constexpr int kRowPairY = kRowPairRows - 2;  // interior rows: the tiles' stride in y
-// the out-of-tile rows take one value per thread: 3 parts of 256 z values
-static_assert(64 * kRowPairRows == 3 * 256, "k_smooth_pair_rows: the halo rows take every thread");
+//
+// kSub: z rows a wavefront holds, each in 64 / kSub lanes (2 where rows hold at
+// most 128 cells). 128^3: 20 us a pair, 22 with a row a wavefront and half its
+// lanes idle, two flat steps 23; runs of 4 planes a block, so the loads of the
+// two planes around them and the first step's latency are half of it. Listed
+// levels (pressure, 128^3, 26 % of the rows active) keep their flat steps: 13
+// us for two, 20-23 a pair.
+constexpr int kRowPairWaves = 12;
+constexpr int row_pair_y(int sub) { return kRowPairWaves * sub - 2; }  // interior rows: the tiles' stride in y
 // A byte offset past every run's planes; two of them add up without wrapping.
 constexpr unsigned kPairOut = 0x40000000u;
 
-template <bool kRowsum, bool kDx>
-__global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
+template <bool kRowsum, bool kDx, int kSub>
+__global__ __launch_bounds__(64 * kRowPairWaves, 1) void k_smooth_pair_rows(
     Dims d, Op32 A, const float *__restrict__ b, const float *__restrict__ x1,
     float *__restrict__ xo, const float *__restrict__ d1, float cdA, float crA, float cdB,
     float crB, const unsigned char *__restrict__ rowact, const int *__restrict__ segments, int planes,
@@ -714,15 +719,19 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     if (gated(gate)) return;
+    constexpr int kLanes = 64 / kSub, kRows = kRowPairWaves * kSub, kRowsY = row_pair_y(kSub);
+    // the out-of-tile rows take one value per thread: 3 parts of 4 kLanes z values
+    constexpr int kHaloWaves = 4 / kSub;
+    static_assert(3 * kHaloWaves <= kRowPairWaves, "too few wavefronts for the halo rows");
     const unsigned runs = segments ? (unsigned)segments[0] : gridDim.x;
     if (blockIdx.x >= runs) return;
-    __shared__ f4 sx1[2][kRowPairRows + 2][64];  // x1 of rows -1 .. kRowPairRows (index row + 1)
-    __shared__ f4 scy[4][kRowPairRows + 1][64];  // cpl_y of rows 0 .. kRowPairRows
-    __shared__ f4 sx2[3][kRowPairRows][64];      // x2 of rows 0 .. kRowPairRows - 1
+    __shared__ f4 sx1[2][kRows + 2][kLanes];  // x1 of rows -1 .. kRows (index row + 1)
+    __shared__ f4 scy[4][kRows + 1][kLanes];  // cpl_y of rows 0 .. kRows
+    __shared__ f4 sx2[3][kRows][kLanes];      // x2 of rows 0 .. kRows - 1
     // the stored diagonal of lane 0's group on planes 0 and 1: a row-sum
     // diagonal is rebuilt but in the groups of cells 1, nz and nz*ny
-    __shared__ f4 sdg[2][kRowsum ? kRowPairRows : 1];
-    __shared__ f4 scx[3][kRowPairRows][64];      // cpl_x, read by the wavefront that wrote it
+    __shared__ f4 sdg[2][kRowsum ? kRows : 1];
+    __shared__ f4 scx[3][kRows][kLanes];      // cpl_x, read by the wavefront that wrote it
     // logical tiles run y fastest; each XCD (block b goes to XCD b % 8) takes
     // a contiguous run of them, so the rows two tiles share meet in one L2
     unsigned L = blockIdx.x;
@@ -738,12 +747,13 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
         ie = segments[3 + 3 * L];
     }
     if (i0 >= d.nx) return;  // uniform over the block
-    const int lane = threadIdx.x, row = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y), wlane = threadIdx.x;
+    const int lane = wlane % kLanes, sub = kSub > 1 ? wlane / kLanes : 0, row = kSub * wave + sub;
     const int k = 4 * lane;
-    const int j = (int)by * kRowPairY - 1 + row;
+    const int j = (int)by * kRowsY - 1 + row;
     const bool zon = k < d.nz;
     const bool yin = j >= 0 && j < d.ny;
-    const bool interior = row >= 1 && row <= kRowPairY;
+    const bool interior = row >= 1 && row <= kRowsY;
     const bool ylo = j > 0, yhi = j + 1 < d.ny;
     const bool zl = k > 0, zh = k + 4 < d.nz;
     const Strides s(d);
@@ -765,26 +775,36 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
                rd1 = rsrc(d1), rdg = rsrc(A.diag), rxo = rsrc(xo);
     const unsigned o0 = yin && zon ? 4 * c0 : kPairOut;  // bytes within a plane
     // the out-of-tile rows next to the tile (x1 of rows j0 - 1 and
-    // j0 + kRowPairRows - 2, cpl_y of the latter), one value per thread: thread
+    // j0 + kRows - 2, cpl_y of the latter), one value per thread: thread
     // t of the block takes z = t mod 256 of part t / 256
-    const int hpart = row >> 2, hz = (row & 3) * 64 + lane;
-    const int jt = (int)by * kRowPairY - 1;  // the tile's row 0
-    const int jh = hpart == 0 ? jt - 1 : jt + kRowPairRows;
-    const bool hon_any = jh >= 0 && jh < d.ny;  // uniform over the wavefront
+    const int hpart = wave / kHaloWaves, hz = wave % kHaloWaves * 64 + wlane;
+    const int jt = (int)by * kRowsY - 1;  // the tile's row 0
+    const int jh = hpart == 0 ? jt - 1 : jt + kRows;
+    const bool hon_any = hpart < 3 && jh >= 0 && jh < d.ny;  // uniform over the wavefront
     const unsigned oh = hon_any && hz < d.nz ? 4 * (unsigned)d.idx(0, jh, hz) : kPairOut;
     const f4 z4 = {0.f, 0.f, 0.f, 0.f};
     // activity of this row and of the out-of-tile row for planes i0 - 2 ..
     // i0 + 61 (bit q - i0 + 2), one lane per plane, read once
     auto row_mask = [&](int jj) -> unsigned long long {
-        const int q = i0 - 2 + lane;
+        const int q = i0 - 2 + wlane;
         const bool a = q >= 0 && q < d.nx && q <= ie + 1 && jj >= 0 && jj < d.ny &&
                        (!rowact || rowact[(size_t)q * d.ny + jj] != 0);
         return __ballot(a);
     };
-    const unsigned long long amask = row_mask(j);
-    const unsigned long long hmask_lo = row_mask(jt - 1), hmask_hi = row_mask(jt + kRowPairRows);
+    // (of the wavefront's rows: its first and, kSub 2, its second)
+    const int jw = (int)by * kRowsY - 1 + kSub * wave;
+    const unsigned long long amask = row_mask(jw), amask2 = kSub > 1 ? row_mask(jw + 1) : 0ull;
+    const unsigned long long hmask_lo = row_mask(jt - 1), hmask_hi = row_mask(jt + kRows);
     const unsigned long long hmask = hpart == 0 ? hmask_lo : hmask_hi;
     auto active = [&](int q, unsigned long long m) { return ((m >> (q - i0 + 2)) & 1ull) != 0; };
+    auto mine = [&](int q) { return sub ? active(q, amask2) : active(q, amask); };
+    auto any_active = [&](int q) { return active(q, amask | amask2); };
+    auto at_row = [&](int q) {
+        const unsigned o = active(q, amask) ? (unsigned)(q - p0) * plane_bytes : kPairOut;
+        if constexpr (kSub == 1) return o;
+        const unsigned o2 = active(q, amask2) ? (unsigned)(q - p0) * plane_bytes : kPairOut;
+        return sub ? o2 : o;
+    };
     auto at = [&](int q, unsigned long long m) { return active(q, m) ? (unsigned)(q - p0) * plane_bytes : kPairOut; };
     auto ld = [&](__amdgpu_buffer_rsrc_t p, unsigned o) {
         return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(p, o0 + o, 0, 0));
@@ -799,7 +819,7 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     };
     auto load_early = [&](int q) {
         Early e;
-        const unsigned o = at(q, amask);
+        const unsigned o = at_row(q);
         e.x = ld(rx1, o);
         e.cx = ld(rcx, o);
         e.cy = ld(rcy, o);
@@ -809,7 +829,7 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
     };
     auto load_rest = [&](int q) {
         Rest r;
-        const unsigned o = at(q, amask);
+        const unsigned o = at_row(q);
         r.cz = ld(rcz, o);
         r.bv = ld(rb, o);
         r.dv = r.dg = z4;
@@ -822,8 +842,8 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
         scy[q & 3][row][lane] = e.cy;
         scx[(q + 3) % 3][row][lane] = e.cx;
         if (hpart == 0) ((float *)&sx1[q & 1][0][0])[hz] = e.h;
-        else if (hpart == 1) ((float *)&sx1[q & 1][kRowPairRows + 1][0])[hz] = e.h;
-        else ((float *)&scy[q & 3][kRowPairRows][0])[hz] = e.h;
+        else if (hpart == 1) ((float *)&sx1[q & 1][kRows + 1][0])[hz] = e.h;
+        else if (hpart == 2) ((float *)&scy[q & 3][kRows][0])[hz] = e.h;
     };
     // one Chebyshev step of the four cells at plane q from iterate xc (x
     // neighbours xm, xp; y neighbours and couplings given), direction dp
@@ -860,7 +880,7 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
             const float czdn = __shfl_down(r.cz.x, 1, 64);  // all lanes (see cheb)
             const float czhi = zh ? czdn : 0.f;
             dg = rowsum_diag4(cxc, cxp, cym, cyp, r.cz, czhi);
-            if (q <= 1 && j <= 1) {  // uniform
+            if (q <= 1 && jw <= 1) {  // uniform
                 const f4 stored = sdg[q & 1][row];
                 if (!rowsum_group(A, c0 + (unsigned)q * sx, d)) dg = stored;
             }
@@ -885,10 +905,10 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
 #pragma unroll
         for (int k = 0; k < 4; k++) rdg[k] = rcp_or_zero(dg[k]);
         d2 = z4;
-        if (!active(q, amask)) return z4;  // uniform over the wavefront
+        if (!any_active(q)) return z4;  // uniform over the wavefront
         f4 x2 = cheb(xc, xm, xp, xym, xyp, cxc, cxp, cym, cyp, r.cz, r.bv, dg, rdg, kDx ? xc : r.dv,
                      cdA, crA, d2);
-        if (!zon) x2 = z4;
+        if (!zon || (kSub > 1 && !mine(q))) x2 = z4;
         return x2;
     };
 
@@ -944,12 +964,13 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
         sx2[(i + 1) % 3][row][lane] = x2n;
         __syncthreads();
         // 4. step B on plane i (the tile's interior rows)
-        if (interior) {
+        if (kSub > 1 || interior) {
             const int bi = i % 3;
             const f4 xc = sx2[bi][row][lane];
-            if (active(i, amask)) {
+            if (any_active(i)) {
                 const Rest &r = R[U];
-                const f4 xym = sx2[bi][row - 1][lane], xyp = sx2[bi][row + 1][lane];
+                const int rb = kSub > 1 ? max(row - 1, 0) : row - 1, ra = kSub > 1 ? min(row + 1, kRows - 1) : row + 1;
+                const f4 xym = sx2[bi][rb][lane], xyp = sx2[bi][ra][lane];
                 const f4 cym = scy[i & 3][row][lane], cyp = scy[i & 3][row + 1][lane];
                 const f4 cxc = scx[bi][row][lane], cxp = scx[(i + 1) % 3][row][lane];
                 const f4 dgB = diag_at(i, cxc, cxp, cym, cyp, r);
@@ -960,7 +981,9 @@ __global__ __launch_bounds__(64 * kRowPairRows, 1) void k_smooth_pair_rows(
                 const f4 x3 = cheb(xc, x2prev, x2n, xym, xyp, cxc, cxp, cym, cyp, r.cz, r.bv, dgB, rdgB, D[U & 1],
                                    cdB, crB, dn);
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x3), rxo,
-                                                       o0 + (unsigned)(i - p0) * plane_bytes, 0, 0);
+                                                       kSub == 1 ? o0 + (unsigned)(i - p0) * plane_bytes
+                                                                 : interior ? o0 + at_row(i) : kPairOut,
+                                                       0, 0);
             }
             x2prev = xc;
         }
@@ -2077,10 +2100,13 @@ Launch pair_launch(Dims d, bool even_planes) {
     return L;
 }
 
-// (k_smooth_pair_rows addresses a run's planes, at most 64 with their
-// neighbours, by byte offsets below kPairOut)
+// Rows that fill at least three quarters of a wavefront's lanes, or of half a
+// wavefront's (row_pair_sub 2). k_smooth_pair_rows addresses a run's planes, at
+// most 64 with their neighbours, by byte offsets below kPairOut.
+static int row_pair_sub(Dims d) { return d.nz <= 128 ? 2 : 1; }
 bool row_pair(Dims d) {
-    return d.nz % 4 == 0 && d.nz > 192 && d.nz <= 256 && d.cells() < (size_t(1) << 32) &&
+    const bool rows = (d.nz > 96 && d.nz <= 128) || (d.nz > 192 && d.nz <= 256);
+    return d.nz % 4 == 0 && rows && d.cells() < (size_t(1) << 32) &&
            64 * 4 * (size_t)d.ny * d.nz < kPairOut;
 }
 
@@ -2222,11 +2248,12 @@ void launch_active_chunks(hipStream_t st, Dims d, const float *diag32, const Act
 // P the least with which there are no more runs than CUs.
 constexpr int kSegTiles = 128, kSegPlanes = 1024, kSegMin = 8, kSegMax = 56;
 unsigned pair_segments_max(Dims d) {
-    const unsigned ytiles = (unsigned)((d.ny + kRowPairY - 1) / kRowPairY);
-    if (!row_pair(d) || ytiles > (unsigned)kSegTiles || d.nx > kSegPlanes) return 0;
+    const int rows = row_pair_y(row_pair_sub(d));
+    const unsigned ytiles = (unsigned)((d.ny + rows - 1) / rows);
+    if (!row_pair(d) || row_pair_sub(d) > 1 || ytiles > (unsigned)kSegTiles || d.nx > kSegPlanes) return 0;
     return ytiles * (unsigned)((d.nx + kSegMin - 1) / kSegMin);
 }
-__global__ __launch_bounds__(kListThreads) void k_pair_segments(Dims d, int ytiles, int cus,
+__global__ __launch_bounds__(kListThreads) void k_pair_segments(Dims d, int ytiles, int rows, int cus,
                                                                 const unsigned char *__restrict__ rowact,
                                                                 int *__restrict__ segments) {
     __shared__ unsigned long long mask[kSegTiles][kSegPlanes / 64];
@@ -2238,10 +2265,10 @@ __global__ __launch_bounds__(kListThreads) void k_pair_segments(Dims d, int ytil
     __syncthreads();
     for (int e = wave; e < ytiles * words; e += kListThreads / 64) {
         const int by = e / words, w = e % words, q = 64 * w + lane;
-        const int j1 = min((by + 1) * kRowPairY, d.ny);
+        const int j1 = min((by + 1) * rows, d.ny);
         bool a = false;
         if (q < d.nx)
-            for (int j = by * kRowPairY; j < j1; j++) a |= rowact[(size_t)q * d.ny + j] != 0;
+            for (int j = by * rows; j < j1; j++) a |= rowact[(size_t)q * d.ny + j] != 0;
         const unsigned long long m = __ballot(a);
         if (lane == 0) {
             mask[by][w] = m;
@@ -2284,9 +2311,9 @@ __global__ __launch_bounds__(kListThreads) void k_pair_segments(Dims d, int ytil
     }
 }
 void launch_pair_segments(hipStream_t st, Dims d, const unsigned char *rowact, int *segments) {
-    const int ytiles = (d.ny + kRowPairY - 1) / kRowPairY;
+    const int rows = row_pair_y(row_pair_sub(d)), ytiles = (d.ny + rows - 1) / rows;
     if (!pair_segments_max(d)) throw ArgError("launch_pair_segments: not a row-pair level");
-    hipLaunchKernelGGL(k_pair_segments, dim3(1), dim3(kListThreads), 0, st, d, ytiles, device_cus(), rowact,
+    hipLaunchKernelGGL(k_pair_segments, dim3(1), dim3(kListThreads), 0, st, d, ytiles, rows, device_cus(), rowact,
                        segments);
     SFP_LAUNCH_CHECK();
 }
@@ -2302,21 +2329,26 @@ void launch_smooth_pair(hipStream_t st, Dims d, Op32 A, const float *b, const fl
         // one block per compute unit, in one round: as many x runs per tile
         // column as the columns leave CUs for (at most 56 planes a run, the
         // activity masks' reach)
-        const unsigned ytiles = (unsigned)((d.ny + kRowPairY - 1) / kRowPairY);
+        const int sub = row_pair_sub(d), ty = row_pair_y(sub);
+        const unsigned ytiles = (unsigned)((d.ny + ty - 1) / ty);
         const int runs_max = std::max(1, device_cus() / (int)ytiles);
         int planes = std::min(56, std::max(1, (d.nx + runs_max - 1) / runs_max));
         const unsigned runs = (unsigned)((d.nx + planes - 1) / planes);
         const bool dx = d1 == x1;
         const unsigned char *ra = A.pinned_rowsum ? nullptr : rowact;
         const int *sg = ra ? segments : nullptr;
-        const dim3 grid(sg ? pair_segments_max(d) : ytiles * runs), block(64, kRowPairRows);
+        const dim3 grid(sg ? pair_segments_max(d) : ytiles * runs), block(64, kRowPairWaves);
 #define SFP_ROWPAIR(RS, DX)                                                                      \
-    hipLaunchKernelGGL((k_smooth_pair_rows<RS, DX>), grid, block, 0, st, d, A, b, x1, x3, d1, cdA, \
-                       crA, cdB, crB, ra, sg, planes, ytiles, gate)
+    if (sub == 2)                                                                                \
+        hipLaunchKernelGGL((k_smooth_pair_rows<RS, DX, 2>), grid, block, 0, st, d, A, b, x1, x3, \
+                           d1, cdA, crA, cdB, crB, ra, sg, planes, ytiles, gate);                \
+    else                                                                                         \
+        hipLaunchKernelGGL((k_smooth_pair_rows<RS, DX, 1>), grid, block, 0, st, d, A, b, x1, x3, \
+                           d1, cdA, crA, cdB, crB, ra, sg, planes, ytiles, gate)
         if (A.pinned_rowsum) {
-            if (dx) SFP_ROWPAIR(true, true); else SFP_ROWPAIR(true, false);
+            if (dx) { SFP_ROWPAIR(true, true); } else { SFP_ROWPAIR(true, false); }
         } else {
-            if (dx) SFP_ROWPAIR(false, true); else SFP_ROWPAIR(false, false);
+            if (dx) { SFP_ROWPAIR(false, true); } else { SFP_ROWPAIR(false, false); }
         }
 #undef SFP_ROWPAIR
         SFP_LAUNCH_CHECK();

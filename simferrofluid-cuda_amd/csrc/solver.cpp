@@ -441,8 +441,20 @@ float *System::vlevel(Workspace &ws, const Smoothing &sm, int l, const double *r
             std::swap(cur, oth);
         } else {
             smooth(first | (deg > 2 ? SM_WRITE_D : 0), cb.cd[1], cb.cr[1], r64, nullptr);
-            for (int s = 2; s < deg - (fuse_restrict ? 1 : 0); s++)
+            // from degree 4 the last two steps can (the first of them reads the
+            // direction the step before stored)
+            const bool last_pair = deg >= 4 && !fuse_restrict && (ws.fused_pairs & 16) && pairs(L);
+            for (int s = 2; s < deg - (fuse_restrict ? 1 : last_pair ? 2 : 0); s++)
                 smooth(SM_READ_D | (s < deg - 1 ? SM_WRITE_D : 0), cb.cd[s], cb.cr[s], nullptr, nullptr);
+            if (last_pair) {
+                // reads x, b, d, diag, 3 couplings; writes x
+                if (fine && ws.profiling) ws.timers[K_SMOOTH_PAIR].begin(st, (28.0 + pair_diag_bytes) * cells);
+                launch_smooth_pair(st, L.d, A, L.b.p, cur, oth, L.dv.p, cb.cd[deg - 2], cb.cr[deg - 2],
+                                   cb.cd[deg - 1], cb.cr[deg - 1], ws.gate, L.rowact.p,
+                                   L.sparse ? L.segments.p : nullptr);
+                if (fine && ws.profiling) ws.timers[K_SMOOTH_PAIR].end(st);
+                std::swap(cur, oth);
+            }
         }
     }
     bool store_x0 = false;  // the restriction stores the coarse level's first iterate

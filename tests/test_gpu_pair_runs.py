@@ -1,6 +1,6 @@
 """GPU test of the row-tiled pair of Chebyshev steps (csrc/mg.hip,
 k_smooth_pair_rows) over runs of x planes of every length modulo its unrolled
-march, and on both sides of the plane size up to which it addresses a run by
+march, of rows a wavefront or half of one holds, and on both sides of the plane size up to which it addresses a run by
 32-bit byte offsets (the x-plane tiles above): bit-identical to two flat
 steps."""
 import numpy as np
@@ -14,10 +14,12 @@ pytestmark = pytest.mark.gpu
 
 # 129 tile columns of y leave one run a column: of all planes up to 56, then two
 @pytest.mark.parametrize("n", [(1, 1290, 196), (2, 1290, 196), (3, 1290, 200), (4, 1290, 196), (5, 1290, 196),
-                               (56, 1290, 196), (57, 1290, 196), (3, 16380, 256), (3, 16388, 256)])
+                               (56, 1290, 196), (57, 1290, 196), (3, 16380, 256), (3, 16388, 256),
+                               # two rows a wavefront: 22 of a tile's, a tile of one, odd counts, short rows
+                               (40, 22, 128), (41, 23, 128), (60, 67, 100), (3, 133, 124), (128, 128, 128)])
 @pytest.mark.parametrize("pre", [False, True])
 def test_runs_match_two_steps(n, pre):
-    for kind in ("magnetic", "pressure") if n[0] in (3, 5) and n[1] < 2000 else ("magnetic",):
+    for kind in ("magnetic", "pressure") if (n[0] in (3, 5) or n[2] <= 128) and n[1] < 2000 else ("magnetic",):
         print(f"[case] pair runs {kind} {n} pre {pre}", flush=True)
         sc = scenes.random_pressure_scene(n, seed=3) if kind == "pressure" else scenes.magnetic_scene(n, seed=3)
         which = 0 if kind == "pressure" else 1
