@@ -36,8 +36,8 @@ void launch_smooth(hipStream_t s, int mode, Dims d, Op32 A, const double *r64, f
 // direction) the pair is the first two steps of a cycle.
 // pair_pays: grids on which it beats the two launches on MI355X. The 64 x 16
 // tiles overlap by one cell per side: equal at 128^3, faster above. Whole rows
-// of 97..128 cells: 20 us against 23 at 128^3, 45 against 82 at 256 x 256 x 128
-// (magnetic solves 1.03x and 1.1x), 1.01x at 100 x 105 x 100.
+// of 80..128 cells: 20 us against 23 at 128^3, 45 against 82 at 256 x 256 x 128
+// (magnetic solves 1.03x and 1.17x), 1.01x at 100 x 105 x 100.
 bool row_pair(Dims d);
 inline bool pair_pays(Dims d) {
     return d.nz >= 64 && d.cells() > ((size_t)1 << (row_pair(d) && d.nz <= 128 ? 20 : 21));
@@ -47,8 +47,7 @@ inline bool pair_pays(Dims d) {
 // prolongation too (nz a multiple of 4).
 bool flat_step(Dims d);
 bool whole_groups(Dims d);
-// Grids with z rows of 97..128 or 193..256 cells in groups of four run it over
-// whole rows (k_smooth_pair_rows); rowact (null: all active) marks the z rows
+// Grids with z rows of 80..256 cells in groups of four run it over whole rows (k_smooth_pair_rows); rowact (null: all active) marks the z rows
 // holding an active cell (launch_row_activity), whose loads the others skip.
 void launch_smooth_pair(hipStream_t s, Dims d, Op32 A, const float *b, const float *x1, float *x3,
                         const float *d1, float cdA, float crA, float cdB, float crB,

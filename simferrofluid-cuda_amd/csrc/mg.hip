@@ -2100,13 +2100,13 @@ Launch pair_launch(Dims d, bool even_planes) {
     return L;
 }
 
-// Rows that fill at least three quarters of a wavefront's lanes, or of half a
-// wavefront's (row_pair_sub 2). k_smooth_pair_rows addresses a run's planes, at
+// Rows of a wavefront, or of half a wavefront (row_pair_sub 2) from 80 cells: 180
+// x 180 x 132 to 192 magnetic solves 1.04-1.11x against the x-plane pair, 120 x
+// 124 x 80 1.02x and x 72 0.98x against flat steps. k_smooth_pair_rows addresses a run's planes, at
 // most 64 with their neighbours, by byte offsets below kPairOut.
 static int row_pair_sub(Dims d) { return d.nz <= 128 ? 2 : 1; }
 bool row_pair(Dims d) {
-    const bool rows = (d.nz > 96 && d.nz <= 128) || (d.nz > 192 && d.nz <= 256);
-    return d.nz % 4 == 0 && rows && d.cells() < (size_t(1) << 32) &&
+    return d.nz % 4 == 0 && d.nz >= 80 && d.nz <= 256 && d.cells() < (size_t(1) << 32) &&
            64 * 4 * (size_t)d.ny * d.nz < kPairOut;
 }
 

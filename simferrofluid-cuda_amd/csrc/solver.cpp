@@ -183,15 +183,19 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     }
     bool lists = false;
     for (Level &L : lv_) {
-        // the row-tiled step pairs skip the loads of z rows without active cells
-        if (row_pair(L.d) && !L.pinned_rowsum) {
-            L.rowact.ensure((size_t)L.d.nx * L.d.ny);
-            launch_row_activity(side, L.d, L.diag32.p, L.rowact.p);
-            lists = true;
-        }
         // a system of part of the grid: the flat kernels run on the chunks that
         // hold an active cell (small grids' launches cost the same either way)
         L.sparse = sparse_ && !(ws.fused_pairs & 32) && flat_step(L.d) && !small_grid(L.d);
+        // and the row-tiled step pairs skip the loads of z rows without one
+        // (on levels of rows up to 128 cells only where there are such pairs:
+        // the launch took 35 us of 180 x 180 x 72's 1740)
+        if (sparse_ && row_pair(L.d) && (L.d.nz > 128 || pairs(L))) {
+            L.rowact.ensure((size_t)L.d.nx * L.d.ny);
+            launch_row_activity(side, L.d, L.diag32.p, L.rowact.p);
+            lists = true;
+        } else {
+            L.rowact.release();
+        }
         if (L.sparse) {
             const size_t nch = (L.d.cells() + kChunk - 1) / kChunk, nq = restrict_quads(L.d);
             const size_t nbl = (L.d.cells() + kListCells - 1) / kListCells;
@@ -206,7 +210,7 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
                                              L.quad_list.p, L.block_list.p});
             L.list_sums.ensure(list_sums(L.d));
             SFP_HIP(hipMemsetAsync(L.list_sums.p, 0, list_sums(L.d) * sizeof(double), side));
-            if (const unsigned segs = L.pinned_rowsum ? 0 : pair_segments_max(L.d)) {
+            if (const unsigned segs = pair_segments_max(L.d)) {
                 L.segments.ensure(1 + 3 * (size_t)segs);
                 launch_pair_segments(side, L.d, L.rowact.p, L.segments.p);
             }

@@ -16,10 +16,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n", [(1, 1290, 196), (2, 1290, 196), (3, 1290, 200), (4, 1290, 196), (5, 1290, 196),
                                (56, 1290, 196), (57, 1290, 196), (3, 16380, 256), (3, 16388, 256),
                                # two rows a wavefront: 22 of a tile's, a tile of one, odd counts, short rows
-                               (40, 22, 128), (41, 23, 128), (60, 67, 100), (3, 133, 124), (128, 128, 128)])
+                               (40, 22, 128), (41, 23, 128), (60, 67, 100), (3, 133, 124), (128, 128, 128),
+                               (61, 45, 80), (41, 23, 132), (20, 41, 160)])
 @pytest.mark.parametrize("pre", [False, True])
 def test_runs_match_two_steps(n, pre):
-    for kind in ("magnetic", "pressure") if (n[0] in (3, 5) or n[2] <= 128) and n[1] < 2000 else ("magnetic",):
+    for kind in ("magnetic", "pressure") if (n[0] in (3, 5) or n[2] <= 160) and n[1] < 2000 else ("magnetic",):
         print(f"[case] pair runs {kind} {n} pre {pre}", flush=True)
         sc = scenes.random_pressure_scene(n, seed=3) if kind == "pressure" else scenes.magnetic_scene(n, seed=3)
         which = 0 if kind == "pressure" else 1
