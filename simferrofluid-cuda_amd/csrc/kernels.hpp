@@ -139,16 +139,6 @@ bool tail_fits(const Dims *lv, int nlev);
 void launch_vcycle_tail(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
 // The buffer that holds the tail's result for its first level.
 inline float *tail_result(const TailArgs &t) { return t.lv[0].x1; }
-// The tail with every array of its levels (8 each, unpadded) in LDS: the one
-// for hierarchies whose coarsest level has 2 (mod 4) cells (18, of 2 x 3 x 3),
-// for which its staging of the dense inverse leaves the entries (r, 0) and
-// (r, 1) of odd rows r unset. The cycle it computes there is not the
-// level-by-level one, solves take one or two iterations more, and their
-// iterates are kept as they are.
-constexpr size_t kTailLdsMaxCells = 4096;
-constexpr size_t kTailLdsBytes = 149504;
-inline size_t tail_lds_bytes(Dims d) { return 8 * sizeof(float) * d.cells(); }
-void launch_vcycle_tail_lds(hipStream_t s, const TailArgs &t, const double *gate = nullptr);
 
 // Several Chebyshev steps of one level in one launch, over overlapping tiles
 // held in registers and LDS. start:

@@ -252,30 +252,22 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     if (ws.side && lists) SFP_HIP(hipStreamWaitEvent(ws.stream, ws.side_lists, 0));
 }
 
-// (see launch_vcycle_tail_lds)
-static bool lds_tail(Dims coarsest) { return coarsest.cells() % 4 == 2; }
-
 bool System::tail_at(const Workspace &ws, int l) const {
     const int nlev = (int)lv_.size() - l;
     if (!ws.vcycle_tail || nlev < 2 || nlev > kTailMaxLevels) return false;
     Dims dims[kTailMaxLevels];
     for (int q = 0; q < nlev; q++) dims[q] = lv_[l + q].d;
-    if (!lds_tail(dims[nlev - 1])) return tail_fits(dims, nlev);
-    size_t bytes = 0;
-    for (int q = 0; q < nlev; q++) bytes += tail_lds_bytes(dims[q]);
-    return dims[0].cells() <= kTailLdsMaxCells && bytes <= kTailLdsBytes;
+    return tail_fits(dims, nlev);
 }
 
 bool System::fold_at(const Workspace &ws, const Smoothing &sm, int l) {
     if (!fold_pays(lv_[l].d) || l + 1 >= (int)lv_.size()) return false;
-    if (tail_at(ws, l)) return !lds_tail(lv_.back().d);
-    return tile_stages(ws, l, sm.at(l).degree - 1, true).n > 0;
+    return tail_at(ws, l) || tile_stages(ws, l, sm.at(l).degree - 1, true).n > 0;
 }
 
 float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
     if (!tail_at(ws, l)) return nullptr;
     const int nlev = (int)lv_.size() - l;
-    const bool lds = lds_tail(lv_.back().d);
     TailArgs t;
     t.nlev = nlev;
     for (int q = 0; q < nlev; q++) {
@@ -292,10 +284,9 @@ float *System::vcycle_tail(Workspace &ws, const Smoothing &sm, int l) {
     }
     t.lv[0].x1 = last_out(ws, l, t.lv[0].x1);
     t.ainv = ainv_.p;
-    if (!lds && l == ws.z_level) t.fold = ws.fold;
+    if (l == ws.z_level) t.fold = ws.fold;
     join_ainv(ws);
-    if (lds) launch_vcycle_tail_lds(ws.stream, t, ws.gate);
-    else launch_vcycle_tail(ws.stream, t, ws.gate);
+    launch_vcycle_tail(ws.stream, t, ws.gate);
     return tail_result(t);
 }
 
