@@ -164,7 +164,9 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64
         const float zym = ylo ? z[c - s.sy] : 0.f;
         const float zyp = yhi ? z[c + s.sy] : 0.f;
         const double dg = on ? A.diag[c] : 0.0;
-        const double qp = (on && !first) ? ld_stream(qprev + c) : 0.0;
+        // (an inactive cell's q may be an earlier system's: the update skips
+        // groups of 128 cells of the array, not of this row)
+        const double qp = (on && act > 0.f && !first) ? ld_stream(qprev + c) : 0.0;
         const double rc = on ? ld_stream(r + c) : 0.0;
         float zzm = __shfl_up(zc, 1, tz);
         float zzp = __shfl_down(zc, 1, tz);

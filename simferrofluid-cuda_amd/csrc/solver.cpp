@@ -230,9 +230,10 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     // the inactive cells (values left on cells that were active before would
     // otherwise leak into z, w, q and the inner products). Active cells are
     // written before they are read in every cycle; q is written at every cell
-    // of the update's groups by the first iteration and read in those groups
-    // only. The ring of z needs none: z counts as 0 at inactive cells wherever
-    // it is read for its own cell, and elsewhere couples with weight 0.
+    // of the update's groups by the first iteration, and read in those groups
+    // (the flat matvec's are the same) or, by the x-plane matvec, at active
+    // cells only. The ring of z needs none: z counts as 0 at inactive cells
+    // wherever it is read for its own cell, and elsewhere couples with weight 0.
     if (lv_.size() > (size_t)kClearMaxLevels) throw ArgError("too many multigrid levels");
     ClearArgs ca;
     ca.nlev = (int)lv_.size();

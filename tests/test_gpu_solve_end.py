@@ -106,3 +106,29 @@ def test_non_finite_input_leaves_nothing_behind(n):
     np.testing.assert_array_equal(p, want_p)
     for a, b in zip(vel, want_v):
         np.testing.assert_array_equal(a, b)
+
+
+# odd nz: the matvec's rows and the update's groups of cells are not the same
+@pytest.mark.parametrize("n", [(19, 21, 23), (83, 89, 91)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_non_finite_input_leaves_nothing_behind_on_odd_rows(n, value):
+    """As above, and after infinities: the next projection and re-projection
+    are those of a new context."""
+    print(f"[case] solve end after {value} {n}", flush=True)
+    pool = scenes.random_pressure_scene(n, 9)
+    full = dict(pool, phi=np.full_like(pool["phi"], -1.0), velocity=[np.full_like(v, value) for v in pool["velocity"]])
+
+    def both(ctx):
+        return [ctx.pressure_project(pool, reproject=again) for again in (False, True)]
+
+    with sfp.Context.for_scene(pool, tol=1e-8) as ctx:
+        want = both(ctx)
+    with sfp.Context.for_scene(pool, tol=1e-8, max_iters=5) as ctx:
+        assert not ctx.pressure_project(full)[2]["converged"]
+        ctx.set_params(max_iters=200)
+        got = both(ctx)
+    for (vel, p, st), (want_v, want_p, want_st) in zip(got, want):
+        assert st["converged"] and st["iterations"] == want_st["iterations"]
+        np.testing.assert_array_equal(p, want_p)
+        for a, b in zip(vel, want_v):
+            np.testing.assert_array_equal(a, b)
