@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_fcg_matvec(CellGrid cg, Dims d, Op64
         const double dg = on ? A.diag[c] : 0.0;
         // (an inactive cell's q may be an earlier system's: the update skips
         // groups of 128 cells of the array, not of this row)
-        const double qp = (on && act > 0.f && !first) ? ld_stream(qprev + c) : 0.0;
+        const double qp = (on & (act > 0.f) & !first) ? ld_stream(qprev + c) : 0.0;
         const double rc = on ? ld_stream(r + c) : 0.0;
         float zzm = __shfl_up(zc, 1, tz);
         float zzp = __shfl_down(zc, 1, tz);
@@ -237,7 +237,7 @@ struct PairAt {
         return a[n - c > 2 ? c + 2 : c];
     }
     // whether the pair holds a cell whose diagonal is not the row sum (0, 1, nz, nz*ny)
-    __device__ __forceinline__ bool pinned() const { return c == 0 || c == sy || c == sx; }
+    __device__ __forceinline__ bool pinned() const { return (c == 0) | (c == sy) | (c == sx); }
 };
 // The operator at a pair: its couplings and diagonal.
 struct PairOperator {
@@ -254,7 +254,9 @@ struct PairOperator {
         if (!(left > P.sx)) cxp = double2v{0.0, 0.0};
         if (!(left > P.sy)) cyp = double2v{0.0, 0.0};
         if (!(left > 2)) czp = 0.0;
-        if (A.pinned_rowsum && !P.pinned()) {
+        // (one condition, by bit operations: a short circuit between its uniform
+        // and its lanes' part has been compiled to loads at undefined addresses)
+        if ((A.pinned_rowsum != 0) & !P.pinned()) {
             dg.x = ((((cxm.x + cxp.x) + cym.x) + cyp.x) + cz.x) + cz.y;
             dg.y = ((((cxm.y + cxp.y) + cym.y) + cyp.y) + cz.y) + czp;
         } else {

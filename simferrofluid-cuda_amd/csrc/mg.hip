@@ -222,12 +222,15 @@ __device__ __forceinline__ f4v rowsum_diag4(f4v cxc, f4v cxp, f4v cym, f4v cyp, 
     return dg;
 }
 // The group of four cells from c on holds none of the cells whose diagonal is
-// not the row sum (0, 1, nz, nz*ny); kAny: it may start at any cell.
+// not the row sum (0, 1, nz, nz*ny); kAny: it may start at any cell. For
+// operators of Op32::pinned_rowsum only (the kernels' kRowsum): the condition
+// guards a load, so it holds nothing uniform beside the lane's part, and no
+// branch of its own (see load_operands).
 template <bool kAny = false>
-__device__ __forceinline__ bool rowsum_group(const Op32 &A, size_t c, Dims d) {
-    if constexpr (!kAny) return A.pinned_rowsum && c != 0 && c != (size_t)d.nz && c != (size_t)d.ny * d.nz;
+__device__ __forceinline__ bool rowsum_group(size_t c, Dims d) {
+    if constexpr (!kAny) return (c != 0) & (c != (size_t)d.nz) & (c != (size_t)d.ny * d.nz);
     const unsigned sy = (unsigned)d.nz, sx = (unsigned)d.ny * sy, cu = (unsigned)c;
-    return A.pinned_rowsum && cu > 1 && sy - cu >= 4 && sx - cu >= 4;  // (differences below 0 are large)
+    return (cu > 1) & (sy - cu >= 4) & (sx - cu >= 4);  // (differences below 0 are large)
 }
 
 // The operands of one group, which (kAny: nz no multiple of 4) need not lie
@@ -368,7 +371,7 @@ __global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE, kAny) :
     auto group = [&](unsigned ct) {  // the group of cells from ct on
         const bool on = ct < n;
         const unsigned c = on ? ct : (n - 1) & ~3u;
-        const bool rs = kRowsum && rowsum_group<kAny>(A, c, d);  // every group there has an active cell
+        const bool rs = kRowsum && rowsum_group<kAny>(c, d);  // every group there has an active cell
         f4 dg = {0.f, 0.f, 0.f, 0.f};
         if (!rs) dg = own_cells<kAny>(A.diag, c, n);
         if constexpr (kRun == kBytesRun) {
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
         if (q >= d.nx) return P;
         const size_t c = c0 + q * s.sx;
         // a row-sum diagonal is rebuilt below (cells 1, nz and nz*ny read it)
-        const bool rs = kRowsum && on && A.pinned_rowsum && c != 1 && c != (size_t)d.nz && c != s.sx;
+        const bool rs = kRowsum && (on & (c != 1) & (c != (size_t)d.nz) & (c != s.sx));
         float dg = (on && !rs) ? A.diag[c] : 0.f;
         P.live = __any(on && (rs || dg > 0.f));
         if (!P.live) {
@@ -882,7 +885,7 @@ __global__ __launch_bounds__(64 * kRowPairWaves, 1) void k_smooth_pair_rows(
             dg = rowsum_diag4(cxc, cxp, cym, cyp, r.cz, czhi);
             if (q <= 1 && jw <= 1) {  // uniform
                 const f4 stored = sdg[q & 1][row];
-                if (!rowsum_group(A, c0 + (unsigned)q * sx, d)) dg = stored;
+                if (!rowsum_group(c0 + (unsigned)q * sx, d)) dg = stored;
             }
         }
         return dg;
@@ -1159,7 +1162,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_flat(Dims df, Op32 A, const
     // lanes outside the grid load the nearest cells and drop them
     const int i = min(iw, df.nx - 1), j = min(jw, df.ny - 1), k = min(kw, (df.nz - 1) & ~3);
     const unsigned c = (unsigned)df.idx(i, j, k), n = (unsigned)df.cells();
-    const bool rs = kRowsum && rowsum_group<kAny>(A, c, df);  // every group there has an active cell
+    const bool rs = kRowsum && rowsum_group<kAny>(c, df);  // every group there has an active cell
     f4 dg = {0.f, 0.f, 0.f, 0.f};
     if (!rs) dg = own_cells<kAny>(A.diag, c, n);
     f4 r = {0.f, 0.f, 0.f, 0.f};

@@ -255,3 +255,27 @@ def test_fused_pairs_match_separate_launches(kind):
                     np.testing.assert_array_equal(p, q)
             elif u is not None:
                 np.testing.assert_array_equal(u, v)
+
+
+# the cells whose diagonal is not the row sum (0, 1, nz, nz ny) at every place of
+# a group of four: rows of 5 to 9 cells, one row, one plane, planes of 1 to 3 cells
+# past a group; the last, the x-plane pair
+@pytest.mark.parametrize("n", [(9, 7, 5), (8, 5, 6), (7, 3, 7), (6, 4, 8), (5, 9, 9), (9, 1, 7), (1, 8, 11),
+                               (131, 129, 133)])
+def test_rowsum_diagonals_wherever_the_pin_lies(n):
+    """Level by level (no tiles, no tail): the same bits with the diagonals
+    rebuilt and read."""
+    print(f"[case] row-sum diagonals {n}", flush=True)
+    sc = scenes.magnetic_scene(n, seed=5)
+    out = []
+    with sfp.Context.for_scene(sc, max_iters=3) as ctx:
+        ctx.set_vcycle_tail(False)
+        for on in (True, False):
+            ctx.set_rowsum_diagonal(on)
+            ctx.reset_warm_start()
+            pot, _, _ = ctx.magnetic_solve(sc)
+            r = np.random.default_rng(2).standard_normal(n)
+            out.append((pot, ctx.precondition(1, r)))
+    assert np.abs(out[0][1]).max() > 0
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
