@@ -46,29 +46,43 @@ sfp_params to_params(const SolverConfig &c) {
     return p;
 }
 
+// After an exception: work enqueued before it may still use the caller's arrays
+// or raise the input-error flag, which belongs to the failed call, as do the
+// pointers a solve keeps in the workspace for its batch.
+void abandon(sfp_context ctx) {
+    Workspace &ws = ctx->ws;
+    (void)hipStreamSynchronize(ws.stream);
+    if (ws.side) (void)hipStreamSynchronize(ws.side);
+    *ws.host_err = 0;
+    ws.gate = nullptr;
+    ws.x0_level = -1;
+    ws.zout = nullptr;
+    ws.fold = FoldArgs{};
+}
+
 template <class F>
 sfp_status guarded(sfp_context ctx, F &&f) {
     if (!ctx) return SFP_ERR_ARGUMENT;
+    const auto failed = [&](const std::exception &e, sfp_status st) {
+        abandon(ctx);
+        ctx->last_error = e.what();
+        return st;
+    };
     try {
         SFP_HIP(hipSetDevice(ctx->device));
         f();
         ctx->last_error.clear();
         return SFP_OK;
     } catch (const ArgError &e) {
-        ctx->last_error = e.what();
-        return SFP_ERR_ARGUMENT;
+        return failed(e, SFP_ERR_ARGUMENT);
     } catch (const InputError &e) {
-        ctx->last_error = e.what();
-        return SFP_ERR_INPUT;
+        return failed(e, SFP_ERR_INPUT);
     } catch (const StateError &e) {
-        ctx->last_error = e.what();
-        return SFP_ERR_STATE;
+        return failed(e, SFP_ERR_STATE);
     } catch (const HipError &e) {
-        ctx->last_error = e.what();
-        return SFP_ERR_HIP;
+        return failed(e, SFP_ERR_HIP);
     } catch (const std::exception &e) {
-        ctx->last_error = e.what();
-        return SFP_ERR_ARGUMENT;
+        return failed(e, SFP_ERR_ARGUMENT);
     }
 }
 
@@ -98,10 +112,7 @@ void fill_stats(sfp_stats *st, const SolveInfo &info, long long unknowns, float 
 
 void check_err(sfp_context ctx, const char *msg) {
     ctx->ws.wait();
-    if (*ctx->ws.host_err) {
-        *ctx->ws.host_err = 0;
-        throw InputError(msg);
-    }
+    if (*ctx->ws.host_err) throw InputError(msg);  // (guarded() clears the flag)
 }
 
 // whether two arrays share memory (null: no)
@@ -126,6 +137,8 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     System &sys = ctx->pressure;
     sys.allocate(d);
     sys.sparse_ = true;
+    sys.input_err_ = ctx->ws.host_err;
+    *ctx->ws.host_err = 0;  // (the streams are idle between calls)
     ctx->liquid.ensure(d.cells());
     const Faces F{{frac[0], frac[1], frac[2]}}, V{{vel[0], vel[1], vel[2]}}, U{{us[0], us[1], us[2]}};
     Faces J{{nullptr, nullptr, nullptr}};

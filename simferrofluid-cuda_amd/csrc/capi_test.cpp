@@ -318,4 +318,8 @@ sfp_status sfp_test_set_rowsum_diagonal(sfp_context ctx, int enable) {
     return run(ctx, [&] { ctx->ws.rowsum_diag = enable != 0; });
 }
 
+sfp_status sfp_test_raise_input_error(sfp_context ctx) {
+    return run(ctx, [&] { *ctx->ws.host_err = 1; });
+}
+
 }  // extern "C"

@@ -799,9 +799,10 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             known = true;
             info.active = (long long)h.active;
             // (launches that returned at once are no measurement)
-            if (profiling && (h.iters == 0.0 || *ws.host_err))
+            const bool bad_input = input_err_ && *input_err_;
+            if (profiling && (h.iters == 0.0 || bad_input))
                 for (auto &t : ws.timers) t.used = 0;
-            if (*ws.host_err) {
+            if (bad_input) {
                 info.input_error = true;
                 clear_ring(ws);
                 return info;

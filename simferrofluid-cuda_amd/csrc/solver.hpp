@@ -211,6 +211,9 @@ class System {
     // Inactive cells are expected (the air of a pressure system): levels over
     // the flat cell index keep the list of their active chunks.
     bool sparse_ = false;
+    // The flag that the system's assembly raises on invalid input (null: it
+    // raises none), read with the solve's first residual.
+    const int *input_err_ = nullptr;
 
   private:
     enum Cycle { kCycleLearned, kCycleSmooth, kCycleRestrictOnly };

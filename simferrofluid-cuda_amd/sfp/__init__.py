@@ -45,7 +45,8 @@ EXPORTS = {
                    "sfp_test_residual", "sfp_test_solve",
                    "sfp_test_restrict_smoothed", "sfp_test_smooth_pair",
                    "sfp_test_smooth_restrict", "sfp_test_set_vcycle_tail",
-                   "sfp_test_set_fused_pairs", "sfp_test_set_rowsum_diagonal"],
+                   "sfp_test_set_fused_pairs", "sfp_test_set_rowsum_diagonal",
+                   "sfp_test_raise_input_error"],
     "sfp_learned.h": ["sfp_unet_param_count", "sfp_set_network", "sfp_learned_features",
                       "sfp_unet_create", "sfp_unet_destroy", "sfp_unet_set_params",
                       "sfp_unet_get_params", "sfp_unet_init_params", "sfp_unet_forward",
@@ -167,6 +168,8 @@ def lib():
         L.sfp_test_set_fused_pairs.argtypes = [vp, C.c_int]
         L.sfp_test_set_rowsum_diagonal.restype = C.c_int
         L.sfp_test_set_rowsum_diagonal.argtypes = [vp, C.c_int]
+        L.sfp_test_raise_input_error.restype = C.c_int
+        L.sfp_test_raise_input_error.argtypes = [vp]
         L.sfp_test_smooth_restrict.restype = C.c_int
         L.sfp_test_smooth_restrict.argtypes = [vp, C.c_int, C.c_int, _fp, _fp, _fp, C.c_float,
                                                C.c_float, _fp, _fp, _fp, _fp]
@@ -596,6 +599,10 @@ class Context:
         (False), from the next magnetic solve on; the results are the same bit
         for bit."""
         self._check(lib().sfp_test_set_rowsum_diagonal(self._h, 1 if enable else 0))
+
+    def raise_input_error(self):
+        """Leave the input-error flag up, as a call that failed before reading it."""
+        self._check(lib().sfp_test_raise_input_error(self._h))
 
     def smooth_restrict(self, which, level, b, x1, d1, cd, cr):
         """The last pre-smoothing step and the restriction on a level, from

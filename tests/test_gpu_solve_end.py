@@ -132,3 +132,33 @@ def test_non_finite_input_leaves_nothing_behind_on_odd_rows(n, value):
         np.testing.assert_array_equal(p, want_p)
         for a, b in zip(vel, want_v):
             np.testing.assert_array_equal(a, b)
+
+
+def test_input_error_of_a_failed_call_stays_its_own():
+    """The flag left up by a call that failed before reading it (the hook
+    raises it from the host) changes neither a magnetic solve nor a
+    projection; an open boundary face is still reported, each time."""
+    print("[case] input error left behind", flush=True)
+    sc = scenes.magnetic_scene((24, 20, 28), seed=9)
+    with sfp.Context.for_scene(sc, tol=1e-8) as ctx:
+        want = ctx.magnetic_solve(sc)
+        ctx.raise_input_error()
+        ctx.reset_warm_start()
+        x, field, st = ctx.magnetic_solve(sc)
+    assert st["converged"] and st["iterations"] == want[2]["iterations"]
+    for a, b in zip([x, *field], [want[0], *want[1]]):
+        np.testing.assert_array_equal(a, b)
+    sc = scenes.random_pressure_scene((19, 21, 23), 9)
+    broken = dict(sc, phi=np.full_like(sc["phi"], -1.0), fraction=[np.zeros_like(f) for f in sc["fraction"]])
+    with sfp.Context.for_scene(sc, tol=1e-8) as ctx:
+        want = ctx.pressure_project(sc)
+        for _ in range(2):
+            with pytest.raises(sfp.SfpError):
+                ctx.pressure_project(broken)
+            with pytest.raises(sfp.SfpError):
+                ctx.pressure_project(sc, reproject=True)
+            ctx.raise_input_error()
+            vel, p, st = ctx.pressure_project(sc)
+            assert st["iterations"] == want[2]["iterations"]
+            for a, b in zip([p, *vel], [want[1], *want[0]]):
+                np.testing.assert_array_equal(a, b)
