@@ -91,11 +91,12 @@ __global__ __launch_bounds__(kBlock) void k_pressure_assemble(CellGrid cg,
     Dims d, const double *__restrict__ phi, Faces frac, Faces vel, Faces us, Faces jump,
     int has_jump, double vol_error, double *__restrict__ diag64, MutFaces cpl64,
     double *__restrict__ rhs, float *__restrict__ diag32, float *cpl32x, float *cpl32y,
-    float *cpl32z, unsigned char *__restrict__ liquid, int *err) {
+    float *cpl32z, unsigned char *__restrict__ liquid, int *err, RowsFlag rows) {
     int k, j, i0;
     cell_tile(cg, k, j, i0);
     if (k >= d.nz || j >= d.ny) return;
     float *cpl32[3] = {cpl32x, cpl32y, cpl32z};
+    bool row = false;
     for (int i = i0, ie = min(i0 + cg.planes, d.nx); i < ie; i++) {
         const size_t c = d.idx(i, j, k);
         const double pc = phi[c];
@@ -156,12 +157,15 @@ __global__ __launch_bounds__(kBlock) void k_pressure_assemble(CellGrid cg,
             const double dg = diag != 0 ? diag : 1.;
             diag64[c] = dg;
             diag32[c] = (float)dg;
+            row = row || (float)dg > 0.f;
         }
         for (int a = 0; a < 3; a++) {
             cpl64.a[a][c] = low[a];
             cpl32[a][c] = (float)low[a];
         }
     }
+    const unsigned long long m = __ballot(row);
+    if (m != 0ull && (flat_tid() & 63) == __ffsll(m) - 1) *rows.seen = rows.epoch;
 }
 
 __global__ __launch_bounds__(kBlock) void k_pressure_rhs(CellGrid cg, Dims d,
@@ -399,13 +403,13 @@ __global__ __launch_bounds__(kBlock) void k_vertex_pressures(Dims d, MagGeom g, 
 void launch_pressure_assemble(hipStream_t st, Dims d, const double *phi, Faces frac, Faces vel,
                               Faces us, const Faces *jump, double vol_error, double *diag64,
                               double *const cpl64[3], double *rhs, float *diag32,
-                              float *const cpl32[3], unsigned char *liquid, int *err) {
+                              float *const cpl32[3], unsigned char *liquid, int *err, RowsFlag rows) {
     Launch L = cell_launch(d, 0, kAssemblyPlanes);
     Faces j = jump ? *jump : Faces{{nullptr, nullptr, nullptr}};
     MutFaces c{{cpl64[0], cpl64[1], cpl64[2]}};
     hipLaunchKernelGGL(k_pressure_assemble, L.grid, L.block, 0, st, L.cg, d, phi, frac, vel, us, j,
                        jump ? 1 : 0, vol_error, diag64, c, rhs, diag32, cpl32[0], cpl32[1],
-                       cpl32[2], liquid, err);
+                       cpl32[2], liquid, err, rows);
     SFP_LAUNCH_CHECK();
 }
 

@@ -144,6 +144,12 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     Faces J{{nullptr, nullptr, nullptr}};
     if (jump) J = Faces{{jump[0], jump[1], jump[2]}};
     Level &L = sys.fine();
+    const auto nothing = [&] {  // no unknowns: Pressure::Project returns early
+        ctx->pressure_ready = true;
+        if (pressure) SFP_HIP(hipMemsetAsync(pressure, 0, d.cells() * sizeof(double), s));
+        SFP_HIP(hipStreamSynchronize(s));
+        fill_stats(st, SolveInfo{0, 0.0, true, 0, ctx->cfg.precond}, 0, 0.f, 0.f, 0.f);
+    };
     SFP_HIP(hipEventRecord(ctx->ev[0], s));
     if (!reproject) {
         // the assembly overwrites the liquid mask and the fine operator: until
@@ -151,13 +157,18 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
         // reprojection has nothing consistent to reuse
         ctx->pressure_ready = false;
         ctx->pressure_unknowns = 0;
+        ctx->ws.rows.epoch++;
         double *c64[3] = {L.cpl64[0].p, L.cpl64[1].p, L.cpl64[2].p};
         float *c32[3] = {L.cpl32[0].p, L.cpl32[1].p, L.cpl32[2].p};
         launch_pressure_assemble(s, d, phi, F, V, U, jump ? &J : nullptr, vol_error, L.diag64.p, c64,
-                                 sys.rhs().p, L.diag32.p, c32, ctx->liquid.p, ctx->ws.host_err);
-        // (its input errors and the number of unknowns are read with the
-        // solve's first residual: nothing before that needs them)
-        sys.build_hierarchy(ctx->ws, ctx->cfg.for_pressure());
+                                 sys.rhs().p, L.diag32.p, c32, ctx->liquid.p, ctx->ws.host_err,
+                                 ctx->ws.rows);
+        // (the number of unknowns, and input errors raised late, are read with
+        // the solve's first residual: nothing before that needs them)
+        if (!sys.build_hierarchy(ctx->ws, ctx->cfg.for_pressure(), false)) {
+            check_err(ctx, kOpenFace);
+            return nothing();
+        }
     } else {
         if (!ctx->pressure_ready) throw StateError("reproject before project");
         if (ctx->pressure_unknowns == 0) {
@@ -189,12 +200,7 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     if (!reproject) {
         ctx->pressure_unknowns = info.active;
         ctx->pressure_ready = true;
-        if (info.active == 0) {  // Pressure::Project returns early
-            if (pressure) SFP_HIP(hipMemsetAsync(pressure, 0, d.cells() * sizeof(double), s));
-            SFP_HIP(hipStreamSynchronize(s));
-            fill_stats(st, SolveInfo{0, 0.0, true, 0, ctx->cfg.precond}, 0, 0.f, 0.f, 0.f);
-            return;
-        }
+        if (info.active == 0) return nothing();
     }
     if (!info.finished) apply(nullptr);
     if (pressure && !apart) SFP_HIP(hipMemcpyAsync(pressure, sys.x().p, nb, hipMemcpyDeviceToDevice, s));
@@ -556,6 +562,11 @@ sfp_status sfp_create(sfp_context *out, int nx, int ny, int nz, double spacing,
         SFP_HIP(hipHostMalloc((void **)&ctx->ws.host_err, sizeof(int), hipHostMallocDefault));
         *ctx->ws.host_sc = KrylovScalars{};
         *ctx->ws.host_err = 0;
+        SFP_HIP(hipHostMalloc((void **)&ctx->ws.rows.host, sizeof(unsigned), hipHostMallocDefault));
+        *ctx->ws.rows.host = 0;
+        ctx->ws.rows_seen.ensure(1);
+        SFP_HIP(hipMemset(ctx->ws.rows_seen.p, 0, sizeof(unsigned)));
+        ctx->ws.rows.seen = ctx->ws.rows_seen.p;
     } catch (const std::exception &e) {
         g_create_error = e.what();
         sfp_destroy(ctx);
@@ -576,6 +587,7 @@ void sfp_destroy(sfp_context ctx) {
         if (e) (void)hipEventDestroy(e);
     if (ctx->ws.host_sc) (void)hipHostFree(ctx->ws.host_sc);
     if (ctx->ws.host_err) (void)hipHostFree(ctx->ws.host_err);
+    if (ctx->ws.rows.host) (void)hipHostFree(ctx->ws.rows.host);
     hipStream_t s = ctx->ws.stream, side = ctx->ws.side;
     ctx->ws.stream = nullptr;
     ctx->ws.side = nullptr;

@@ -90,10 +90,10 @@ void launch_restrict(hipStream_t s, Dims df, Op32 A, const float *b, const float
 // Galerkin coarsening by 2x2x2 aggregation, scaled: writes the coarse FP64
 // and FP32 operators, the couplings scaled by `scale` and each row's sum
 // (diagonal minus couplings) by `rs_scale` (scale: scale * P^T A P).
+// (rows: of the assembly before it, which it tells the host of as it starts)
 void launch_coarsen(hipStream_t s, Dims df, Op64 Af, const float *diag32f, Dims dc,
                     double scale, double rs_scale, double *diag64c, double *const cpl64c[3],
-                    float *diag32c,
-                    float *const cpl32c[3]);
+                    float *diag32c, float *const cpl32c[3], RowsFlag rows = {});
 // Dense inverse of the coarsest operator (n = cells <= kMaxCoarse) into ainv (n*n floats).
 constexpr int kMaxCoarse = 64;
 
@@ -282,7 +282,7 @@ MagGeom mag_geometry(Dims d, double spacing, const double origin[3]);
 void launch_pressure_assemble(hipStream_t s, Dims d, const double *phi, Faces frac, Faces vel,
                               Faces us, const Faces *jump, double vol_error, double *diag64,
                               double *const cpl64[3], double *rhs, float *diag32,
-                              float *const cpl32[3], unsigned char *liquid, int *err);
+                              float *const cpl32[3], unsigned char *liquid, int *err, RowsFlag rows);
 // Pressure::SetRightHandSide on the stored unknowns.
 void launch_pressure_rhs(hipStream_t s, Dims d, const unsigned char *liquid, Faces frac,
                          Faces vel, Faces us, double vol_error, double *rhs);

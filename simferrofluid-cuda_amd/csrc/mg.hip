@@ -1249,6 +1249,17 @@ __global__ __launch_bounds__(kBlock) void k_clear_inactive(ClearArgs a) {
     if (l == 0 && a.w) a.w[c] = 0.0;
 }
 
+// Whether the assembly before the launch has formed rows (see RowsFlag; null:
+// it has), which one thread tells the host.
+__device__ __forceinline__ bool tell_rows(const RowsFlag &rows) {
+    if (!rows.host) return true;
+    const bool any = *rows.seen == rows.epoch;  // uniform
+    if (blockIdx.x == 0 && flat_tid() == 0)
+        __hip_atomic_store(rows.host, 2u * rows.epoch + (any ? 1u : 0u), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    return any;
+}
+
 // Galerkin coarsening over the fine grid (the mapping of k_restrict): each
 // fine cell forms its contributions to its aggregate -- the active cell's
 // row sum diag - (its 6 couplings), its lower-face couplings where it lies on
@@ -1265,7 +1276,8 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_fine(CellGrid cg, Dims df, O
                                                          double scale, double rs_scale, double *diag64c,
                                                          MutFaces cpl64c, float *diag32c,
                                                          float *cpl32c0, float *cpl32c1,
-                                                         float *cpl32c2) {
+                                                         float *cpl32c2, RowsFlag rows) {
+    if (!tell_rows(rows)) return;
     __shared__ double sh[kCoarsenSums][kBlock];
     int k, j, i0;
     cell_tile(cg, k, j, i0);
@@ -1363,7 +1375,8 @@ __global__ __launch_bounds__(kBlock) void k_coarsen_flat(Dims df, Op64 Af, const
                                                          Dims dc, double scale, double rs_scale,
                                                          double *diag64c, MutFaces cpl64c,
                                                          float *diag32c, float *cpl32c0, float *cpl32c1,
-                                                         float *cpl32c2) {
+                                                         float *cpl32c2, RowsFlag rows) {
+    if (!tell_rows(rows)) return;
     typedef double d2 __attribute__((ext_vector_type(2)));
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x & 63;
@@ -2039,7 +2052,7 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
 
 void launch_coarsen(hipStream_t st, Dims df, Op64 Af, const float *diag32f, Dims dc,
                     double scale, double rs_scale, double *diag64c, double *const cpl64c[3],
-                    float *diag32c, float *const cpl32c[3]) {
+                    float *diag32c, float *const cpl32c[3], RowsFlag rows) {
     MutFaces m{{cpl64c[0], cpl64c[1], cpl64c[2]}};
     bool flat = whole_groups(df) && (uintptr_t)diag32f % 16 == 0;
     for (const double *a : {Af.diag, Af.cpl[0], Af.cpl[1], Af.cpl[2]}) flat = flat && (uintptr_t)a % 16 == 0;
@@ -2047,7 +2060,7 @@ void launch_coarsen(hipStream_t st, Dims df, Op64 Af, const float *diag32f, Dims
         const size_t waves = (size_t)((df.nz + 63) / 64) * ((df.ny + 1) / 2) * ((df.nx + 1) / 2);
         const unsigned nb = (unsigned)((waves * 64 + kBlock - 1) / kBlock);
         hipLaunchKernelGGL(k_coarsen_flat, dim3(nb), dim3(kBlock), 0, st, df, Af, diag32f, dc, scale, rs_scale,
-                           diag64c, m, diag32c, cpl32c[0], cpl32c[1], cpl32c[2]);
+                           diag64c, m, diag32c, cpl32c[0], cpl32c[1], cpl32c[2], rows);
         SFP_LAUNCH_CHECK();
         return;
     }
@@ -2055,7 +2068,7 @@ void launch_coarsen(hipStream_t st, Dims df, Op64 Af, const float *diag32f, Dims
     Launch L = cell_launch(df, 0, 8);
     if (L.cg.planes & 1) L = cell_launch(df, L.cg.planes + 1);
     hipLaunchKernelGGL(k_coarsen_fine, L.grid, L.block, 0, st, L.cg, df, Af, diag32f, dc, scale, rs_scale,
-                       diag64c, m, diag32c, cpl32c[0], cpl32c[1], cpl32c[2]);
+                       diag64c, m, diag32c, cpl32c[0], cpl32c[1], cpl32c[2], rows);
     SFP_LAUNCH_CHECK();
 }
 

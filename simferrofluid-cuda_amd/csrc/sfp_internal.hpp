@@ -176,6 +176,14 @@ struct Level {
 // iterations whose coefficients are kept.
 constexpr int kRing = 12, kCoefs = 2 * kRing;
 
+// Where an assembly notes that it has formed a row: `seen` (on the device) is
+// then `epoch`, the projection's number. The launch after it tells the host, in
+// pinned memory, 2 epoch + whether it has.
+struct RowsFlag {
+    unsigned *seen = nullptr, *host = nullptr;
+    unsigned epoch = 0;
+};
+
 // Scalars of the flexible-CG recurrences, resident on the device.
 struct KrylovScalars {
     double zw, zq, zr;           // dots of the current iteration

@@ -134,7 +134,24 @@ void System::join_ainv(Workspace &ws) {
     ainv_pending_ = false;
 }
 
-void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
+// The assembly is known to have formed no row, or to have raised an error: a
+// look at pinned memory, whose answer may still be on its way.
+bool System::nothing_to_solve(const Workspace &ws) const {
+    return input_err_ && (__atomic_load_n(input_err_, __ATOMIC_ACQUIRE) != 0 ||
+                          __atomic_load_n(ws.rows.host, __ATOMIC_ACQUIRE) == 2u * ws.rows.epoch);
+}
+
+// Waits for that answer (or the end of the stream's work, failed or not).
+void System::await_rows(const Workspace &ws) const {
+    for (unsigned look = 1; __atomic_load_n(ws.rows.host, __ATOMIC_ACQUIRE) >> 1 != ws.rows.epoch % 0x80000000u; look++)
+        if (look % (1u << 22) == 0) {  // every few milliseconds
+            const hipError_t e = hipStreamQuery(ws.stream);
+            (void)hipGetLastError();
+            if (e != hipErrorNotReady) return;
+        }
+}
+
+bool System::build_hierarchy(Workspace &ws, const SolverConfig &cfg, bool known_rows) {
     // an inverse still being formed reads the coarsest operator rebuilt below
     join_ainv(ws);
     const int coarsest = std::max(2, std::min(cfg.coarsest, 4));
@@ -170,7 +187,8 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
         double *c64[3] = {C.cpl64[0].p, C.cpl64[1].p, C.cpl64[2].p};
         float *c32[3] = {C.cpl32[0].p, C.cpl32[1].p, C.cpl32[2].p};
         launch_coarsen(ws.stream, F.d, F.op64(), F.diag32.p, C.d, cfg.coarse_scale,
-                       pinned_ ? 1.0 : cfg.coarse_scale, C.diag64.p, c64, C.diag32.p, c32);
+                       pinned_ ? 1.0 : cfg.coarse_scale, C.diag64.p, c64, C.diag32.p, c32,
+                       l == 1 && !known_rows ? ws.rows : RowsFlag{});
     }
     // On the side stream, overlapping the clears below: which rows and chunks of
     // cells are active (one-block kernels but for the flags), then the dense
@@ -180,6 +198,17 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     if (ws.side) {
         SFP_HIP(hipEventRecord(ws.side_in, ws.stream));
         SFP_HIP(hipStreamWaitEvent(side, ws.side_in, 0));
+    }
+    // Large systems wait for the assembly here, hidden by the coarsening (0.1 ms
+    // at 256^3), so that an empty one costs no more than these launches; on smaller
+    // ones the host is the slower, and only looks, here and in the first batch. A
+    // projection without liquid at 20^3, 64^3, 128^3 and 256^3: 60, 66, 90 and
+    // 360 us (210, 240, 370 and 1015 with the whole set-up and a batch before the
+    // host knew); with liquid as fast as without the look, where 20^3 and 64^3
+    // took 50 us longer if they waited here.
+    if (!known_rows) {
+        if (lv_[0].d.cells() > (size_t)1 << 21) await_rows(ws);
+        if (nothing_to_solve(ws)) return false;
     }
     bool lists = false;
     for (Level &L : lv_) {
@@ -251,6 +280,7 @@ void System::build_hierarchy(Workspace &ws, const SolverConfig &cfg) {
     ca.w = w_.p;
     launch_clear_inactive(ws.stream, ca);
     if (ws.side && lists) SFP_HIP(hipStreamWaitEvent(ws.stream, ws.side_lists, 0));
+    return true;
 }
 
 bool System::tail_at(const Workspace &ws, int l) const {
@@ -739,6 +769,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             ws.gate = &ws.scalars.p->stop;
         }
         for (int it = 0; it < batch; it++) {
+            if (!known && nothing_to_solve(ws)) break;  // (found below)
             const double *r64 = b_ready ? nullptr : r_.p;  // null: the cycle reads b
             ws.x0_level = b_ready ? level : -1;
             ws.zout = zring_.p + (size_t)(pending + it) * zring_stride_;

@@ -101,6 +101,9 @@ struct Workspace {
     // input-error flag of the assembly and the velocity update
     KrylovScalars *host_sc = nullptr;
     int *host_err = nullptr;
+    // whether the last projection's assembly has formed a row
+    DevBuf<unsigned> rows_seen;
+    RowsFlag rows;  // (rows.host: pinned)
     bool profiling = false;
     std::array<KernelTimer, K_COUNT> timers;
     // learned preconditioner: the context's network and the level set and
@@ -168,7 +171,11 @@ class System {
     Level &level(int l) { return lv_[l]; }
 
     // Coarsen the fine operator into the hierarchy and invert the coarsest level.
-    void build_hierarchy(Workspace &ws, const SolverConfig &cfg);
+    // The levels of the fine operator assembled on ws.stream. known_rows false:
+    // that assembly reports to ws.rows and input_err_ and may have formed no
+    // system; where that is seen in time, false is returned and the levels are
+    // half made.
+    bool build_hierarchy(Workspace &ws, const SolverConfig &cfg, bool known_rows = true);
     // One preconditioner application z = B r (FP32 result, fine grid): the
     // V-cycle, Jacobi, or (cfg.precond 3) the learned cycle with a zero
     // correction in place of the network's.
@@ -260,6 +267,8 @@ class System {
     // the dense inverse is being formed on ws.side: join before reading it
     // (or before the coarsest operator it reads is rewritten)
     bool ainv_pending_ = false;
+    bool nothing_to_solve(const Workspace &ws) const;
+    void await_rows(const Workspace &ws) const;
     void join_ainv(Workspace &ws);
     int built_coarsest_ = -1;
 };
