@@ -72,8 +72,8 @@ __global__ __launch_bounds__(kBlock) void k_smooth_first(CellGrid cg, Dims d, Op
 //                stencil point (b read from r64 and rounded when r64 != null,
 //                which also stores b); the previous direction equals it
 //   SM_PROLONG : xin + P e (piecewise-constant coarse correction)
-//   otherwise  : xin
-// Every lane of a row takes part in the shuffles, so lanes past the grid
+// (the other modes run over the flat cell index, k_smooth_flat, as SM_PROLONG
+// does where z rows hold whole groups). Every lane of a row takes part in the shuffles, so lanes past the grid
 // edge stay in the loop with their loads and stores masked.
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
     if (gated(gate)) return;
     constexpr bool kFirst = (MODE & SM_FIRST) != 0;
     constexpr bool kProlong = (MODE & SM_PROLONG) != 0;
-    constexpr bool kXFirst = (MODE & SM_XFIRST) != 0;
+    static_assert(kFirst != kProlong && (MODE & ~(SM_FIRST | SM_PROLONG | SM_WRITE_D)) == 0, "k_smooth's modes");
     int k, j, i0;
     cell_tile(cg, k, j, i0);
     const int tz = blockDim.x;
@@ -112,10 +112,8 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
     auto xval = [&](size_t q, int qi, size_t ecol) -> float {
         if constexpr (kFirst) {
             return c0 * rcp_or_zero(A.diag[q]) * bval(q);
-        } else if constexpr (kProlong) {
-            return xin[q] + e[(size_t)(qi >> 1) * dcsx + ecol];
         } else {
-            return xin[q];
+            return xin[q] + e[(size_t)(qi >> 1) * dcsx + ecol];
         }
     };
     const int ie = min(i0 + cg.planes, d.nx);
@@ -154,7 +152,6 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
             bc = on ? b[c] : 0.f;
         }
         float dprev = 0.f;
-        if constexpr ((MODE & SM_READ_D) != 0) dprev = on ? dvec[c] : 0.f;
         float xin_c = 0.f;
         if constexpr (kProlong) xin_c = on ? xin[c] : 0.f;
         float xzm = __shfl_up(xc, 1, tz);
@@ -180,7 +177,7 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
                 if (!(dg > 0.f)) x0 = xin_c;
             }
             const float r = bc - fmaf(dg, x0, -off);
-            if constexpr (kFirst || kXFirst) dprev = x0;
+            if constexpr (kFirst) dprev = x0;
             const float dn = fmaf(cd, dprev, cr * rcp_or_zero(dg) * r);
             xout[c] = x0 + dn;
             if constexpr ((MODE & SM_WRITE_D) != 0) dvec[c] = dn;
@@ -191,15 +188,17 @@ __global__ __launch_bounds__(kBlock) void k_smooth(CellGrid cg, Dims d, Op32 A,
     }
 }
 
-// The same step (modes without SM_FIRST) over the flat cell index, four
-// consecutive cells of one z row per lane (grids with nz a multiple of 4):
-// 16-byte loads of every array at the cell, its x and y neighbours and the
-// upper x and y couplings, one more iterate value and z coupling at each end
-// of the group. With SM_PROLONG the coarse correction (two coarse cells per
-// group and row) is added to every iterate value read and, on active cells,
-// to the centre, as k_prolong_add followed by a plain step would. Every cell's
-// arithmetic is k_smooth's (same operands, same order), so the two give the
-// same bits. A wavefront whose 256 cells are all inactive writes nothing.
+// The step in every mode but SM_FIRST over the flat cell index, four
+// consecutive cells per lane (of one z row where nz is a multiple of 4; else
+// wherever they lie, kAny): 16-byte loads of every array at the cell, its x and
+// y neighbours and the upper x and y couplings, one more iterate value and z
+// coupling at each end of the group. With SM_XFIRST the iterate is the
+// zero-start first step and the previous direction too; with SM_PROLONG the
+// coarse correction (two coarse cells per group and row) is added to every
+// iterate value read and, on active cells, to the centre, as k_prolong_add
+// followed by a plain step would. A cell's off-diagonal sum has the order x-,
+// x+, y-, y+, z-, z+ (one fmaf each, the first two products paired), as
+// k_smooth's. A wavefront whose 256 cells are all inactive writes nothing, or 0.
 constexpr unsigned kSmoothFlatCells = 4 * kBlock;
 constexpr size_t kEagerCells = (size_t)1 << 21;
 
@@ -468,9 +467,9 @@ __global__ __launch_bounds__(kBlock, kRun == kListRun ? list_waves(MODE, kAny) :
 //   x3 = x2 + cdB d2 + crB D^{-1} (b - A x2)   (written to xo; d2 not stored),
 // and with kRestrict true the restriction of the residual of x2,
 //   bc = R (b - A x2)   (x2 written to xo),
-// with the per-cell arithmetic of the separate launches (k_smooth with
-// SM_READ_D | SM_WRITE_D, then SM_READ_D; or k_smooth with SM_READ_D, then
-// k_restrict), so results agree bit for bit.
+// with the per-cell arithmetic of the separate launches (k_smooth_flat with
+// SM_READ_D | SM_WRITE_D, then SM_READ_D; or with SM_READ_D, then
+// k_restrict_flat), so results agree bit for bit.
 //
 // A block of 64 lanes (z) x kPairRows wavefronts (y) marches over x planes,
 // computing x2 on its whole 64 x kPairRows tile one plane ahead of step B;
@@ -635,7 +634,7 @@ __global__ __launch_bounds__(64 * kPairRows, 8) void k_smooth_pair(
             }
         } else {
             // residual of x2 on the interior's active cells (the operand
-            // order of k_restrict), then the 2 x 2 x 2 sums
+            // order of k_restrict_flat), then the 2 x 2 x 2 sums
             float r = 0.f;
             if (pc.live) {
                 const float xzm = __shfl_up(pc.x2, 1, 64);
@@ -1045,94 +1044,13 @@ __global__ __launch_bounds__(kBlock) void k_prolong_add(Dims d, const unsigned *
 }
 
 // Residual b - A x on the fine grid, summed over each coarse cell's (up to 8)
-// children. Threads map to fine cells like the smoother (coalesced rows,
-// x-neighbours in registers, z-neighbours from adjacent lanes); the children
-// are added pairwise: z through the lane pair, y through LDS (rows 2m and
-// 2m+1 of a block), x over the block's plane pairs. The block's plane count
-// is even and starts on an even plane, and tz, ty are even (or tz = 1).
-__global__ __launch_bounds__(kBlock) void k_restrict(CellGrid cg, Dims df, Op32 A, const float *__restrict__ b,
-                                                     const float *__restrict__ x, Dims dc,
-                                                     float *__restrict__ bc, float *__restrict__ x0c,
-                                                     const float *__restrict__ diag32c, float c0,
-                                                     const double *gate) {
-    if (gated(gate)) return;
-    __shared__ float sh[kBlock];
-    int k, j, i0;
-    cell_tile(cg, k, j, i0);
-    const int tz = blockDim.x, lane = threadIdx.x, row = threadIdx.y;
-    if (i0 >= df.nx) return;  // uniform over the block
-    const bool on = k < df.nz && j < df.ny;
-    const bool writer = on && (k & 1) == 0 && (j & 1) == 0;
-    const Strides s(df);
-    const int ie = min(i0 + cg.planes, df.nx);
-    const bool zlo = k > 0, zhi = k + 1 < df.nz;
-    size_t c = on ? df.idx(i0, j, k) : 0;
-    float xm = 0.f, xc = 0.f, cxc = 0.f;
-    bool primed = false;  // xm, xc, cxc hold this plane's values
-    float acc = 0.f;
-    for (int i = i0; i < ie; i++, c += s.sx) {
-        const bool up = i + 1 < df.nx;
-        const float dg = on ? A.diag[c] : 0.f;
-        float r = 0.f;
-        // a wavefront whose cells are all inactive contributes 0: skip its loads
-        if (__any(on && dg > 0.f)) {
-            if (!primed) {
-                xm = (on && i > 0) ? x[c - s.sx] : 0.f;
-                xc = on ? x[c] : 0.f;
-                cxc = on ? A.cpl[0][c] : 0.f;
-                primed = true;
-            }
-            const float xp = (on && up) ? x[c + s.sx] : 0.f;
-            const float cxp = (on && up) ? A.cpl[0][c + s.sx] : 0.f;
-            const float czm = on ? A.cpl[2][c] : 0.f;
-            float xzm = __shfl_up(xc, 1, tz);
-            float xzp = __shfl_down(xc, 1, tz);
-            float czp = __shfl_down(czm, 1, tz);
-            if (lane == 0) xzm = (on && zlo) ? x[c - 1] : 0.f;
-            if (lane == tz - 1) {
-                xzp = (on && zhi) ? x[c + 1] : 0.f;
-                czp = (on && zhi) ? A.cpl[2][c + 1] : 0.f;
-            }
-            if (on && dg > 0.f) {
-                float off = 0.f;
-                if (i > 0) off = fmaf(cxc, xm, off);
-                if (up) off = fmaf(cxp, xp, off);
-                if (j > 0) off = fmaf(A.cpl[1][c], x[c - s.sy], off);
-                if (j + 1 < df.ny) off = fmaf(A.cpl[1][c + s.sy], x[c + s.sy], off);
-                if (zlo) off = fmaf(czm, xzm, off);
-                if (zhi) off = fmaf(czp, xzp, off);
-                r = b[c] - fmaf(dg, xc, -off);
-            }
-            xm = xc;
-            xc = xp;
-            cxc = cxp;
-        } else {
-            primed = false;
-        }
-        if (tz > 1) r += __shfl_xor(r, 1, tz);  // z pair
-        sh[row * tz + lane] = r;
-        __syncthreads();
-        if ((row & 1) == 0) r += sh[(row + 1) * tz + lane];  // y pair
-        __syncthreads();
-        acc += r;  // x pair
-        if ((i & 1) == 1 || !up) {
-            if (writer) {
-                const size_t q = dc.idx(i >> 1, j >> 1, k >> 1);
-                bc[q] = acc;
-                if (x0c) x0c[q] = c0 * rcp_or_zero(diag32c[q]) * acc;
-            }
-            acc = 0.f;
-        }
-    }
-}
-
-// The same restriction over the flat cell index: a wavefront covers 64 cells of a z row in two rows and two planes, four
-// cells per lane (lanes 0-15: row j, plane i; 16-31: row j+1; 32-63: plane
-// i+1), so a coarse cell's children are added in k_restrict's order -- the z
-// pair in the lane, the y pair across lanes 16 apart, the x pair across lanes
-// 32 apart, onto a zero -- and the first 16 lanes store two coarse values
-// each. Each active cell's residual is k_restrict's arithmetic, so the two
-// give the same values. A wavefront whose 256 cells are all inactive only
+// children, over the flat cell index: a wavefront covers 64 cells of a z row in
+// two rows and two planes, four cells per lane (lanes 0-15: row j, plane i;
+// 16-31: row j+1; 32-63: plane i+1). The children are added as the z pairs (in
+// the lane), the y pairs (across lanes 16 apart) and the x pair (32 apart) onto
+// a zero, and the first 16 lanes store two coarse values each. A residual's
+// off-diagonal sum has the order x-, x+, y-, y+, z-, z+, one fmaf each. A
+// wavefront whose 256 cells are all inactive only
 // stores zeros.
 constexpr int kRestrictFlatZ = 64;  // z cells per wavefront
 
@@ -1260,7 +1178,7 @@ __device__ __forceinline__ bool tell_rows(const RowsFlag &rows) {
     return any;
 }
 
-// Galerkin coarsening over the fine grid (the mapping of k_restrict): each
+// Galerkin coarsening over the fine grid (the mapping of k_smooth): each
 // fine cell forms its contributions to its aggregate -- the active cell's
 // row sum diag - (its 6 couplings), its lower-face couplings where it lies on
 // the aggregate's lower layer of an axis, its upper-face couplings where it
@@ -1687,16 +1605,10 @@ void launch_smooth(hipStream_t st, int mode, Dims d, Op32 A, const double *r64, 
     switch (mode) {
         SFP_SMOOTH_CASE(SM_FIRST)
         SFP_SMOOTH_CASE(SM_FIRST | SM_WRITE_D)
-        SFP_SMOOTH_CASE(SM_XFIRST)
-        SFP_SMOOTH_CASE(SM_XFIRST | SM_WRITE_D)
-        SFP_SMOOTH_CASE(SM_READ_D)
-        SFP_SMOOTH_CASE(SM_READ_D | SM_WRITE_D)
         SFP_SMOOTH_CASE(SM_PROLONG)
         SFP_SMOOTH_CASE(SM_PROLONG | SM_WRITE_D)
-        SFP_SMOOTH_CASE(0)
-        SFP_SMOOTH_CASE(SM_WRITE_D)
-        default:
-            throw ArgError("unsupported smoother mode");
+        default:  // (a flat mode on arrays or a grid it does not take)
+            throw ArgError("unsupported smoother mode, arrays or grid");
     }
 #undef SFP_SMOOTH_CASE
     SFP_LAUNCH_CHECK();
@@ -2020,9 +1932,9 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
     bool flat = flat_step(df) && (uintptr_t)bc % 8 == 0 && (uintptr_t)x0c % 8 == 0 &&
                 (uintptr_t)diag32c % 8 == 0;
     for (const float *a : {A.diag, A.cpl[0], A.cpl[1], A.cpl[2], b, x}) flat = flat && (uintptr_t)a % 16 == 0;
-    if (flat) {
-        const unsigned nb = (unsigned)(((size_t)restrict_quads(df) * 64 + kBlock - 1) / kBlock);
-        const bool eager = df.cells() <= kEagerCells;
+    if (!flat) throw ArgError("launch_restrict: grid too large or arrays not aligned");
+    const unsigned nb = (unsigned)(((size_t)restrict_quads(df) * 64 + kBlock - 1) / kBlock);
+    const bool eager = df.cells() <= kEagerCells;
 #define SFP_RESTRICT_RUN(RS, EA, LI, ANY)                                                              \
     hipLaunchKernelGGL((k_restrict_flat<RS, EA, LI, ANY>), dim3(nb), dim3(kBlock), 0, st, df, A, b, x, dc, \
                        bc, x0c, diag32c, c0, gate)
@@ -2031,22 +1943,15 @@ void launch_restrict(hipStream_t st, Dims df, Op32 A, const float *b, const floa
         if (whole_groups(df)) SFP_RESTRICT_RUN(RS, EA, LI, false); \
         else SFP_RESTRICT_RUN(RS, EA, LI, true);             \
     } while (0)
-        if (A.pinned_rowsum) {
-            if (eager) SFP_RESTRICT_LAUNCH(true, true, false); else SFP_RESTRICT_LAUNCH(true, false, false);
-        } else if (A.chunks.quads) {
-            SFP_RESTRICT_LAUNCH(false, false, true);
-        } else {
-            if (eager) SFP_RESTRICT_LAUNCH(false, true, false); else SFP_RESTRICT_LAUNCH(false, false, false);
-        }
+    if (A.pinned_rowsum) {
+        if (eager) SFP_RESTRICT_LAUNCH(true, true, false); else SFP_RESTRICT_LAUNCH(true, false, false);
+    } else if (A.chunks.quads) {
+        SFP_RESTRICT_LAUNCH(false, false, true);
+    } else {
+        if (eager) SFP_RESTRICT_LAUNCH(false, true, false); else SFP_RESTRICT_LAUNCH(false, false, false);
+    }
 #undef SFP_RESTRICT_LAUNCH
 #undef SFP_RESTRICT_RUN
-        SFP_LAUNCH_CHECK();
-        return;
-    }
-    Launch L = cell_launch(df, 0, 8);
-    if (L.cg.planes & 1) L = cell_launch(df, L.cg.planes + 1);  // plane pairs stay in one block
-    hipLaunchKernelGGL(k_restrict, L.grid, L.block, 0, st, L.cg, df, A, b, x, dc, bc, x0c, diag32c, c0,
-                       gate);
     SFP_LAUNCH_CHECK();
 }
 

@@ -15,8 +15,8 @@
 // of every cell is also in LDS, twice (a step reads one copy and writes the
 // other, so one barrier a step). Outside the grid and in the padding the
 // couplings, the diagonal and the values are 0, which leaves every sum as the
-// separate launches form it: each cell's arithmetic is k_smooth's,
-// k_restrict's and k_coarse_solve's, in their order, and the results agree
+// separate launches form it: each cell's arithmetic is k_smooth_flat's,
+// k_restrict_flat's and k_coarse_solve's, in their order, and the results agree
 // bit for bit.
 #include "device_util.hpp"
 #include "kernels.hpp"
@@ -147,7 +147,7 @@ __device__ __forceinline__ void place_group(Groups<G> &g, int q, int t, const Ge
 }
 
 // The off-diagonal sums and the step of one group from the iterate in X:
-// d = cd d + cr D^-1 (b - A x), x += d (k_smooth's arithmetic).
+// d = cd d + cr D^-1 (b - A x), x += d (k_smooth_flat's arithmetic).
 __device__ __forceinline__ void cheb_group(const f4 &cx, const f4 &cxp, const f4 &cy, const f4 &cyp, const f4 &cz,
                                            float czp, const f4 &dg, const f4 &rd, const f4 &b, f4 &d, f4 &x, f4 xm,
                                            f4 xp, f4 ym, f4 yp, float zl, float zh, float cd, float cr) {
@@ -169,7 +169,7 @@ __device__ __forceinline__ void cheb_group(const f4 &cx, const f4 &cxp, const f4
     x = xn;
 }
 
-// The residual's z-pair sums of one group (k_restrict's residual, 0 on
+// The residual's z-pair sums of one group (k_restrict_flat's residual, 0 on
 // inactive cells).
 __device__ __forceinline__ f2 residual_pairs(const f4 &cx, const f4 &cxp, const f4 &cy, const f4 &cyp, const f4 &cz,
                                              float czp, const f4 &dg, const f4 &b, const f4 &x, f4 xm, f4 xp, f4 ym,
@@ -231,7 +231,7 @@ __device__ __forceinline__ void residual_groups(const Groups<G> &g, const float 
 }
 
 // Sum of a coarse cell's children: its z-pair sums S at the fine (or tile)
-// rows (i, j) and (i, j + 1) of planes i and i + 1 (k_restrict's order: the y
+// rows (i, j) and (i, j + 1) of planes i and i + 1 (k_restrict_flat's order: the y
 // pair, then the x pair onto 0).
 __device__ __forceinline__ float child_sum(const float *S, int i, int j, int K, int nx, int ny, int zh) {
     const float *p = S + (i * ny + j) * zh + K;
