@@ -77,6 +77,10 @@ sfp_status sfp_test_set_fused_pairs(sfp_context ctx, int mask); /* default 18 */
  * instead of reading them, or read them. Results are the same bit for bit.
  * Takes effect at the next magnetic solve. */
 sfp_status sfp_test_set_rowsum_diagonal(sfp_context ctx, int enable); /* default 1 */
+/* Keep the preconditioned residuals of at most `vectors` (1 to 12) iterations
+ * before the solution is brought up to date, as where memory is short. Results
+ * are the same bit for bit. */
+sfp_status sfp_test_set_ring(sfp_context ctx, int vectors); /* default 12 */
 /* Raise the flag by which a projection's kernels report invalid input, as a
  * call that ended by an exception before it was read would leave it. */
 sfp_status sfp_test_raise_input_error(sfp_context ctx);

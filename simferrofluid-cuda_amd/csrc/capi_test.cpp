@@ -318,6 +318,13 @@ sfp_status sfp_test_set_rowsum_diagonal(sfp_context ctx, int enable) {
     return run(ctx, [&] { ctx->ws.rowsum_diag = enable != 0; });
 }
 
+sfp_status sfp_test_set_ring(sfp_context ctx, int vectors) {
+    return run(ctx, [&] {
+        if (vectors < 1 || vectors > kRing) throw ArgError("ring: 1 to 12 vectors");
+        ctx->ws.ring_limit = vectors;
+    });
+}
+
 sfp_status sfp_test_raise_input_error(sfp_context ctx) {
     return run(ctx, [&] { *ctx->ws.host_err = 1; });
 }

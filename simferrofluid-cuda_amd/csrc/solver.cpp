@@ -120,10 +120,23 @@ void System::allocate(Dims d) {
     q_.ensure(n);
     w_.ensure(n);
     for (auto *v : {&r_, &q_, &w_}) SFP_HIP(hipMemset(v->p, 0, n * sizeof(double)));
+    // The ring (48 B per cell) and the direction p, which a solve of more than
+    // ring_ iterations needs, are allocated here, so that no solve runs out of
+    // memory on the way. Where memory is short the ring takes fewer vectors, and
+    // p and x are formed more often (the same bits): it and p leave three quarters
+    // of what is free to the coarse levels, the other system and the caller.
     zring_stride_ = (n + 63) / 64 * 64;
-    zring_.ensure(kRing * zring_stride_);
-    SFP_HIP(hipMemset(zring_.p, 0, kRing * zring_stride_ * sizeof(float)));
-    p_.release();
+    const auto ring_bytes = [&](int slots) { return slots * zring_stride_ * sizeof(float) + n * sizeof(double); };
+    ring_ = kRing;
+    if (ring_bytes(kRing) > (size_t)1 << 30) {  // (the query takes as long as a small solve)
+        size_t free_bytes = 0, total_bytes = 0;
+        SFP_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
+        for (int slots : {kBatch, 1})
+            if (ring_bytes(ring_) > free_bytes / 4) ring_ = slots;
+    }
+    zring_.ensure(ring_ * zring_stride_);
+    SFP_HIP(hipMemset(zring_.p, 0, ring_ * zring_stride_ * sizeof(float)));
+    p_.ensure(n);
     SFP_HIP(hipMemset(x_.p, 0, n * sizeof(double)));
     built_coarsest_ = -1;
 }
@@ -658,7 +671,7 @@ const float *System::restrict_smoothed(Workspace &ws, const SolverConfig &cfg, c
 // skips writing them, their neighbours couple with weight 0, and 0 times them
 // is NaN.
 void System::clear_ring(Workspace &ws) {
-    SFP_HIP(hipMemsetAsync(zring_.p, 0, kRing * zring_stride_ * sizeof(float), ws.stream));
+    SFP_HIP(hipMemsetAsync(zring_.p, 0, ring_ * zring_stride_ * sizeof(float), ws.stream));
 }
 
 SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool warm, const Finish &finish) {
@@ -704,7 +717,8 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     // learned iteration runs alone: it decides whether the network pays,
     // and iterations enqueued behind a stall would still launch every
     // kernel of the learned cycle (each returning at once)
-    int next_batch = learned ? 1 : kBatch;
+    const int ring = std::min(ring_, ws.ring_limit), full_batch = std::min(kBatch, ring);
+    int next_batch = learned ? 1 : full_batch;
     bool predicted = false;  // next_batch is expected to reach the tolerance
     // iterations whose z is in the ring and whose alpha p is not yet in x, and
     // the number of the next iteration (its scalars' place)
@@ -713,7 +727,6 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
     const float *flags = A.pinned_rowsum ? nullptr : lv_[level].diag32.p;
     auto bring_x_up_to_date = [&](bool keep_p) {
         if (pending > 0) {
-            if (keep_p) p_.ensure(d_.cells());
             launch_fcg_flush(st, d, flags, zring_.p, zring_stride_, pending, iter - pending, p_.p,
                              has_p, keep_p, x_.p, zero_x, ws.scalars.p);
             zero_x = false;
@@ -756,7 +769,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
         // iteration reduced ||r|| by less than stall_ratio, and every kernel
         // of the remaining iterations of the batch then returns at once
         // (profiled launches among them are dropped from the timings).
-        if (pending + next_batch > kRing) bring_x_up_to_date(true);
+        if (pending + next_batch > ring) bring_x_up_to_date(true);
         const int batch = std::min(next_batch, cfg.max_iters - info.iterations);
         // Behind a batch expected to be the last, the check above and what
         // follows the solve are enqueued too, behind the stop flag and the
@@ -879,12 +892,12 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
         // so there a batch is kBatch at most and the host waits again. A wait
         // costs some 20 us, as do the check and the Finish behind a batch that
         // then needs another.
-        next_batch = kBatch;
+        next_batch = full_batch;
         predicted = false;
         if (done > 0 && rel > 0.0 && rel < prev) {
             const double rate = std::pow(rel / prev, 1.0 / done);
             const double left = std::log(cfg.tol / rel) / std::log(rate);
-            const int cap = small_grid(d) ? kRing : kBatch;
+            const int cap = small_grid(d) ? ring : full_batch;
             if (left <= cap) next_batch = std::max(1, (int)std::ceil(left));
             predicted = left <= 1.5 * next_batch;
         }
@@ -900,7 +913,7 @@ SolveInfo System::fcg(Workspace &ws, const SolverConfig &cfg, int level, bool wa
             const float c0_plain = first_coef(false);
             if (c0_plain != c0) b_ready = false;
             c0 = c0_plain;
-            next_batch = kBatch;
+            next_batch = full_batch;
             predicted = false;
         }
     }

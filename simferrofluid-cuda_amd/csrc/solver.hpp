@@ -134,6 +134,7 @@ struct Workspace {
     // the level's own iterates)
     float *zout = nullptr;
     int z_level = 0;
+    int ring_limit = kRing;  // (vectors of the ring a solve uses)
     // the ||r||^2 the cycle's first launch adds (fold.nb 0: none)
     FoldArgs fold;
     // a second stream (default priority) on which the coarsest level's dense
@@ -257,9 +258,10 @@ class System {
     Dims d_{};
     std::vector<Level> lv_;
     DevBuf<double> rhs_, x_, r_, q_, w_;
-    // the z of the iterations whose update of x is pending: kRing vectors,
-    // zring_stride_ apart; p_ (formed only where more than kRing iterations
+    // the z of the iterations whose update of x is pending: ring_ vectors,
+    // zring_stride_ apart; p_ (formed only where more than ring_ iterations
     // are pending): the direction before them
+    int ring_ = kRing;
     DevBuf<float> zring_;
     size_t zring_stride_ = 0;
     DevBuf<double> p_;

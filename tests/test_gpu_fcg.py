@@ -4,6 +4,7 @@ time, against the textbook recurrence in numpy around the library's own
 preconditioner and operator."""
 import numpy as np
 import pytest
+import torch
 
 import sfp
 from sfp import scenes
@@ -64,3 +65,34 @@ def test_iterates_match_the_recurrence(kind, n):
         np.testing.assert_allclose(x, want[k - 1], rtol=0, atol=1e-7 * scale)
     # a planted mistake in the recurrence (a direction left out) is caught
     assert np.abs(want[1] - want[0]).max() > 100 * 1e-7 * scale
+
+
+# rings shorter than, equal to and of no whole number of batches of four; small
+# grids (batches of any length) and larger ones; solves of up to three rings
+@pytest.mark.parametrize("kind,n", [("pressure", (19, 21, 23)), ("magnetic", (24, 20, 28)),
+                                    ("pressure", (83, 89, 91)), ("magnetic", (90, 88, 86))])
+def test_short_rings_give_the_same_solution(kind, n):
+    """Fewer kept residuals (as where memory is short): the same bits, however
+    often the solution is brought up to date, from a warm start too, and no
+    memory is allocated by a solve longer than the ring."""
+    print(f"[case] ring {kind} {n}", flush=True)
+    sc = scenes.random_pressure_scene(n, 9) if kind == "pressure" else scenes.magnetic_scene(n, seed=9)
+    out = {}
+    with sfp.Context.for_scene(sc, tol=1e-12, max_iters=4) as ctx:
+        run = ctx.pressure_project if kind == "pressure" else ctx.magnetic_solve
+        run(sc)
+        free = torch.cuda.mem_get_info()[0]
+        for tol, most in ((1e-12, 100), (1e-300, 14)):
+            ctx.set_params(tol=tol, max_iters=most)
+            for ring in (12, 1, 3, 4, 7):
+                ctx.set_ring(ring)
+                ctx.reset_warm_start()
+                passes = [run(sc), run(sc, reproject=True) if kind == "pressure" else run(sc)]
+                out[ring] = [(p[2]["iterations"], p[0], p[1]) for p in passes]
+                for (it, *arrays), (it0, *arrays0) in zip(out[ring], out[12]):
+                    assert it == it0
+                    for a, b in zip(arrays, arrays0):
+                        for x, y in zip(a, b):
+                            np.testing.assert_array_equal(x, y)
+            assert out[12][0][0] > 7  # longer than every short ring
+        assert torch.cuda.mem_get_info()[0] == free
