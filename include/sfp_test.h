@@ -81,6 +81,9 @@ sfp_status sfp_test_set_rowsum_diagonal(sfp_context ctx, int enable); /* default
  * before the solution is brought up to date, as where memory is short. Results
  * are the same bit for bit. */
 sfp_status sfp_test_set_ring(sfp_context ctx, int vectors); /* default 12 */
+/* Let a device allocation of the calling thread fail, after `after` of them that
+ * do not (negative: none fails). */
+sfp_status sfp_test_fail_allocation(int after);
 /* Raise the flag by which a projection's kernels report invalid input, as a
  * call that ended by an exception before it was read would leave it. */
 sfp_status sfp_test_raise_input_error(sfp_context ctx);

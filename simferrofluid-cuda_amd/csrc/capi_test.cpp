@@ -318,6 +318,11 @@ sfp_status sfp_test_set_rowsum_diagonal(sfp_context ctx, int enable) {
     return run(ctx, [&] { ctx->ws.rowsum_diag = enable != 0; });
 }
 
+sfp_status sfp_test_fail_allocation(int after) {
+    fail_allocation(after);
+    return SFP_OK;
+}
+
 sfp_status sfp_test_set_ring(sfp_context ctx, int vectors) {
     return run(ctx, [&] {
         if (vectors < 1 || vectors > kRing) throw ArgError("ring: 1 to 12 vectors");

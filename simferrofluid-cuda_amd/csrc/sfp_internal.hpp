@@ -71,6 +71,10 @@ struct Launch {
 Launch cell_launch(Dims d, int planes = 0, int max_planes = 16);
 
 // ------------------------------------------------------------------ device memory
+// Whether a test wants this allocation of the calling thread to fail
+// (sfp_test_fail_allocation).
+bool allocation_fails();
+
 template <class T>
 struct DevBuf {
     T *p = nullptr;
@@ -90,7 +94,7 @@ struct DevBuf {
         if (count == 0) return;
         // (64 bytes more: a 16-byte access at an array's last elements may
         // reach past them)
-        SFP_HIP(hipMalloc(&p, count * sizeof(T) + 64));
+        SFP_HIP(hipMalloc(&p, allocation_fails() ? (size_t)1 << 60 : count * sizeof(T) + 64));
         n = count;
     }
     void release() {

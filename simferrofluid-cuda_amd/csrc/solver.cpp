@@ -13,8 +13,13 @@ namespace sfp {
 void hip_fail(hipError_t e, const char *what, const char *file, int line) {
     char buf[512];
     std::snprintf(buf, sizeof(buf), "%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
+    (void)hipGetLastError();  // (else the next launch's check would report it again)
     throw HipError(buf);
 }
+
+static thread_local int t_fail_after = -1;
+void fail_allocation(int after) { t_fail_after = after; }
+bool allocation_fails() { return t_fail_after >= 0 && t_fail_after-- == 0; }
 
 // ---------------------------------------------------------------- Chebyshev
 Cheby Cheby::make(int degree, double ratio) {
@@ -97,7 +102,7 @@ static void zero_vectors(Level &L) {
 
 void System::allocate(Dims d) {
     if (d_.nx == d.nx && d_.ny == d.ny && d_.nz == d.nz && !lv_.empty()) return;
-    d_ = d;
+    d_ = Dims{};  // (of a system whose every vector is there)
     lv_.clear();
     lv_.emplace_back();
     Level &L = lv_[0];
@@ -139,6 +144,7 @@ void System::allocate(Dims d) {
     p_.ensure(n);
     SFP_HIP(hipMemset(x_.p, 0, n * sizeof(double)));
     built_coarsest_ = -1;
+    d_ = d;
 }
 
 void System::join_ainv(Workspace &ws) {
@@ -169,6 +175,7 @@ bool System::build_hierarchy(Workspace &ws, const SolverConfig &cfg, bool known_
     join_ainv(ws);
     const int coarsest = std::max(2, std::min(cfg.coarsest, 4));
     if (built_coarsest_ != coarsest) {
+        built_coarsest_ = -1;
         lv_.resize(1);
         while (true) {
             Dims dl = lv_.back().d;

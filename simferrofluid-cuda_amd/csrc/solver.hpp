@@ -12,6 +12,10 @@
 
 namespace sfp {
 
+// Device allocations of the calling thread from now until one fails (negative:
+// none does).
+void fail_allocation(int after);
+
 // FCG iterations enqueued before the host first reads the residual (and later
 // where their number cannot be predicted).
 constexpr int kBatch = 4;

@@ -46,7 +46,7 @@ EXPORTS = {
                    "sfp_test_restrict_smoothed", "sfp_test_smooth_pair",
                    "sfp_test_smooth_restrict", "sfp_test_set_vcycle_tail",
                    "sfp_test_set_fused_pairs", "sfp_test_set_rowsum_diagonal",
-                   "sfp_test_set_ring", "sfp_test_raise_input_error"],
+                   "sfp_test_set_ring", "sfp_test_fail_allocation", "sfp_test_raise_input_error"],
     "sfp_learned.h": ["sfp_unet_param_count", "sfp_set_network", "sfp_learned_features",
                       "sfp_unet_create", "sfp_unet_destroy", "sfp_unet_set_params",
                       "sfp_unet_get_params", "sfp_unet_init_params", "sfp_unet_forward",
@@ -170,6 +170,8 @@ def lib():
         L.sfp_test_set_rowsum_diagonal.argtypes = [vp, C.c_int]
         L.sfp_test_set_ring.restype = C.c_int
         L.sfp_test_set_ring.argtypes = [vp, C.c_int]
+        L.sfp_test_fail_allocation.restype = C.c_int
+        L.sfp_test_fail_allocation.argtypes = [C.c_int]
         L.sfp_test_raise_input_error.restype = C.c_int
         L.sfp_test_raise_input_error.argtypes = [vp]
         L.sfp_test_smooth_restrict.restype = C.c_int
