@@ -558,15 +558,12 @@ sfp_status sfp_create(sfp_context *out, int nx, int ny, int nz, double spacing,
         ctx->ws.partials.ensure(reduction_partials(ctx->d));
         ctx->ws.scalars.ensure(1);
         SFP_HIP(hipMemset(ctx->ws.scalars.p, 0, sizeof(KrylovScalars)));
-        SFP_HIP(hipHostMalloc((void **)&ctx->ws.host_sc, sizeof(KrylovScalars), hipHostMallocDefault));
-        SFP_HIP(hipHostMalloc((void **)&ctx->ws.host_err, sizeof(int), hipHostMallocDefault));
-        *ctx->ws.host_sc = KrylovScalars{};
-        *ctx->ws.host_err = 0;
-        SFP_HIP(hipHostMalloc((void **)&ctx->ws.rows.host, sizeof(unsigned), hipHostMallocDefault));
-        *ctx->ws.rows.host = 0;
-        ctx->ws.rows_seen.ensure(1);
-        SFP_HIP(hipMemset(ctx->ws.rows_seen.p, 0, sizeof(unsigned)));
-        ctx->ws.rows.seen = ctx->ws.rows_seen.p;
+        Workspace &ws = ctx->ws;
+        SFP_HIP(hipHostMalloc((void **)&ws.pinned, sizeof(Workspace::Pinned), hipHostMallocDefault));
+        *ws.pinned = Workspace::Pinned{};
+        ws.host_sc = &ws.pinned->sc;
+        ws.host_err = &ws.pinned->err;
+        ws.rows = RowsFlag{&ws.scalars.p->rows_seen, &ws.pinned->rows, 0};
     } catch (const std::exception &e) {
         g_create_error = e.what();
         sfp_destroy(ctx);
@@ -585,9 +582,7 @@ void sfp_destroy(sfp_context ctx) {
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : {ctx->ws.side_in, ctx->ws.side_out, ctx->ws.side_lists})
         if (e) (void)hipEventDestroy(e);
-    if (ctx->ws.host_sc) (void)hipHostFree(ctx->ws.host_sc);
-    if (ctx->ws.host_err) (void)hipHostFree(ctx->ws.host_err);
-    if (ctx->ws.rows.host) (void)hipHostFree(ctx->ws.rows.host);
+    if (ctx->ws.pinned) (void)hipHostFree(ctx->ws.pinned);
     hipStream_t s = ctx->ws.stream, side = ctx->ws.side;
     ctx->ws.stream = nullptr;
     ctx->ws.side = nullptr;

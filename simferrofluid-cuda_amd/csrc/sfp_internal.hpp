@@ -92,9 +92,12 @@ struct DevBuf {
         if (count <= n && p) return;
         release();
         if (count == 0) return;
-        // (64 bytes more: a 16-byte access at an array's last elements may
-        // reach past them)
-        SFP_HIP(hipMalloc(&p, allocation_fails() ? (size_t)1 << 60 : count * sizeof(T) + 64));
+        // (64 bytes more: a 16-byte access at the last elements of a list, of
+        // flags or of an FP32 array may reach past them. FP64 arrays hold a pair at
+        // least and no access goes past: the 2 MiB of a 64^3 vector and a few bytes
+        // take ten times as long to allocate and free as 2 MiB)
+        const size_t bytes = sizeof(T) < 8 ? count * sizeof(T) + 64 : (count < 2 ? 2 : count) * sizeof(T);
+        SFP_HIP(hipMalloc(&p, allocation_fails() ? (size_t)1 << 60 : bytes));
         n = count;
     }
     void release() {
@@ -204,6 +207,7 @@ struct KrylovScalars {
     // learned preconditioner in a batch: an update whose ||r||^2 exceeds
     // stall_rr times the previous one raises `stalled` and `stop` (0: off)
     double stall_rr, stalled;
+    unsigned rows_seen, unused;  // (RowsFlag::seen)
     // of iteration number i, at i mod kCoefs
     double alpha[kCoefs], beta[kCoefs], pq[kCoefs];
 };

@@ -103,11 +103,15 @@ struct Workspace {
     DevBuf<KrylovScalars> scalars;
     // pinned, and written by kernels: the scalars the host reads, and the
     // input-error flag of the assembly and the velocity update
+    struct Pinned {
+        KrylovScalars sc;
+        int err;
+        unsigned rows;
+    };
+    Pinned *pinned = nullptr;
     KrylovScalars *host_sc = nullptr;
     int *host_err = nullptr;
-    // whether the last projection's assembly has formed a row
-    DevBuf<unsigned> rows_seen;
-    RowsFlag rows;  // (rows.host: pinned)
+    RowsFlag rows;  // whether the last projection's assembly has formed a row
     bool profiling = false;
     std::array<KernelTimer, K_COUNT> timers;
     // learned preconditioner: the context's network and the level set and
@@ -263,12 +267,12 @@ class System {
     std::vector<Level> lv_;
     DevBuf<double> rhs_, x_, r_, q_, w_;
     // the z of the iterations whose update of x is pending: ring_ vectors,
-    // zring_stride_ apart; p_ (formed only where more than ring_ iterations
-    // are pending): the direction before them
+    // zring_stride_ apart, and after them p_ (formed only where more than ring_
+    // iterations are pending): the direction before them
     int ring_ = kRing;
     DevBuf<float> zring_;
     size_t zring_stride_ = 0;
-    DevBuf<double> p_;
+    double *p_ = nullptr;
     DevBuf<float> ainv_;
     // the dense inverse is being formed on ws.side: join before reading it
     // (or before the coarsest operator it reads is rewritten)
