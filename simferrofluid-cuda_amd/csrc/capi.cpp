@@ -135,7 +135,7 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
     const hipStream_t s = ctx->ws.stream;
     const Dims d = ctx->d;
     System &sys = ctx->pressure;
-    sys.allocate(d);
+    sys.allocate(d, s);
     sys.sparse_ = true;
     sys.input_err_ = ctx->ws.host_err;
     *ctx->ws.host_err = 0;  // (the streams are idle between calls)
@@ -218,7 +218,7 @@ void magnetic_dev(sfp_context ctx, const double *phi, const double *const hext[3
     const hipStream_t s = ctx->ws.stream;
     const Dims d = ctx->d;
     System &sys = ctx->magnetic;
-    sys.allocate(d);
+    sys.allocate(d, s);
     for (int a = 0; a < 3; a++) {
         ctx->mu[a].ensure(face_count(d, a));
         ctx->htot[a].ensure(face_count(d, a));
@@ -557,7 +557,7 @@ sfp_status sfp_create(sfp_context *out, int nx, int ny, int nz, double spacing,
         for (auto &e : ctx->ev) SFP_HIP(hipEventCreate(&e));
         ctx->ws.partials.ensure(reduction_partials(ctx->d));
         ctx->ws.scalars.ensure(1);
-        SFP_HIP(hipMemset(ctx->ws.scalars.p, 0, sizeof(KrylovScalars)));
+        SFP_HIP(hipMemsetAsync(ctx->ws.scalars.p, 0, sizeof(KrylovScalars), ctx->ws.stream));
         Workspace &ws = ctx->ws;
         SFP_HIP(hipHostMalloc((void **)&ws.pinned, sizeof(Workspace::Pinned), hipHostMallocDefault));
         *ws.pinned = Workspace::Pinned{};

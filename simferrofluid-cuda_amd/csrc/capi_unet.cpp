@@ -60,7 +60,7 @@ sfp_status sfp_set_network(sfp_context ctx, const float *params, long long count
         SFP_HIP(hipSetDevice(ctx->device));
         if (!params) throw ArgError("null parameters");
         check_count(count);
-        if (!ctx->net) ctx->net = std::make_unique<UNet>();
+        if (!ctx->net) ctx->net = std::make_unique<UNet>(ctx->ws.stream);
         ctx->net->set_params(ctx->ws.stream, params);
         ctx->ws.net = ctx->net.get();
         ctx->last_error.clear();
@@ -135,7 +135,7 @@ sfp_status sfp_unet_create(sfp_unet *out, int device, int batch, int nx, int ny,
     try {
         SFP_HIP(hipSetDevice(device));
         SFP_HIP(hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking));
-        n->net = new UNet();
+        n->net = new UNet(n->stream);
         n->net->ensure(n->shape, n->training);
         const size_t nv = n->shape.voxels(0);
         n->in.ensure(nv * 4);

@@ -95,12 +95,12 @@ static bool small_grid(Dims d) { return d.cells() <= ((size_t)1 << 19); }
 
 // The stencil kernels skip wavefront rows whose cells are all inactive; the
 // skipped cells of the level vectors then keep the zeros written here.
-static void zero_vectors(Level &L) {
+static void zero_vectors(Level &L, hipStream_t st) {
     const size_t n = L.d.cells();
-    for (auto *v : {&L.x0, &L.x1, &L.dv, &L.b}) SFP_HIP(hipMemset(v->p, 0, n * sizeof(float)));
+    for (auto *v : {&L.x0, &L.x1, &L.dv, &L.b}) SFP_HIP(hipMemsetAsync(v->p, 0, n * sizeof(float), st));
 }
 
-void System::allocate(Dims d) {
+void System::allocate(Dims d, hipStream_t st) {
     if (d_.nx == d.nx && d_.ny == d.ny && d_.nz == d.nz && !lv_.empty()) return;
     d_ = Dims{};  // (of a system whose every vector is there)
     lv_.clear();
@@ -118,13 +118,13 @@ void System::allocate(Dims d) {
     L.x1.ensure(n);
     L.dv.ensure(n);
     L.b.ensure(n);
-    zero_vectors(L);
+    zero_vectors(L, st);
     rhs_.ensure(n);
     x_.ensure(n);
     r_.ensure(n);
     q_.ensure(n);
     w_.ensure(n);
-    for (auto *v : {&r_, &q_, &w_}) SFP_HIP(hipMemset(v->p, 0, n * sizeof(double)));
+    for (auto *v : {&r_, &q_, &w_}) SFP_HIP(hipMemsetAsync(v->p, 0, n * sizeof(double), st));
     // The ring (48 B per cell) and the direction p, which a solve of more than
     // ring_ iterations needs, are allocated here, so that no solve runs out of
     // memory on the way. Where memory is short the ring takes fewer vectors, and
@@ -142,8 +142,8 @@ void System::allocate(Dims d) {
     // (one allocation: each costs some 0.3 ms above 2 MiB)
     zring_.ensure(ring_ * zring_stride_ + 2 * n);
     p_ = (double *)(zring_.p + ring_ * zring_stride_);
-    SFP_HIP(hipMemset(zring_.p, 0, ring_ * zring_stride_ * sizeof(float)));
-    SFP_HIP(hipMemset(x_.p, 0, n * sizeof(double)));
+    SFP_HIP(hipMemsetAsync(zring_.p, 0, ring_ * zring_stride_ * sizeof(float), st));
+    SFP_HIP(hipMemsetAsync(x_.p, 0, n * sizeof(double), st));
     built_coarsest_ = -1;
     d_ = d;
 }
@@ -194,7 +194,7 @@ bool System::build_hierarchy(Workspace &ws, const SolverConfig &cfg, bool known_
             L.x1.ensure(n);
             L.dv.ensure(n);
             L.b.ensure(n);
-            zero_vectors(L);
+            zero_vectors(L, ws.stream);
             lv_.push_back(std::move(L));
         }
         if ((int)lv_.back().d.cells() > kMaxCoarse) throw ArgError("coarsest level too large");

@@ -171,7 +171,9 @@ using Finish = std::function<void(const double *need)>;
 
 class System {
   public:
-    void allocate(Dims d);
+    // (the vectors are cleared on st, which the system's work has to run on: a
+    // hipMemset is on the null stream and is not waited for)
+    void allocate(Dims d, hipStream_t st);
     Dims dims() const { return d_; }
     Level &fine() { return lv_[0]; }
     DevBuf<double> &rhs() { return rhs_; }

@@ -91,7 +91,7 @@ struct UNetShape {
 
 class UNet {
   public:
-    UNet();
+    explicit UNet(hipStream_t st);  // the parameters cleared on st
     // parameters (host FP32, unet_param_count() values)
     void set_params(hipStream_t st, const float *host);
     void get_params(hipStream_t st, float *host) const;

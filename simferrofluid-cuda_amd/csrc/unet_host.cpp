@@ -13,7 +13,7 @@ long long unet_param_count() {
     return n + 16 + 1;
 }
 
-UNet::UNet() {
+UNet::UNet(hipStream_t st) {
     long long o = 0;
     for (int k = 0; k < kUNetConvs; k++) {
         off_w_[k] = o;
@@ -27,10 +27,7 @@ UNet::UNet() {
     grad_.ensure(n);
     m_.ensure(n);
     v_.ensure(n);
-    SFP_HIP(hipMemset(w_.p, 0, n * sizeof(float)));
-    SFP_HIP(hipMemset(m_.p, 0, n * sizeof(float)));
-    SFP_HIP(hipMemset(v_.p, 0, n * sizeof(float)));
-    SFP_HIP(hipMemset(grad_.p, 0, n * sizeof(float)));
+    for (auto *b : {&w_, &m_, &v_, &grad_}) SFP_HIP(hipMemsetAsync(b->p, 0, n * sizeof(float), st));
     for (int k = 0; k < kUNetConvs; k++) {
         wf_[k].ensure((size_t)conv_taps(kConvCin[k]) * kConvCin[k] * kConvCout[k]);
         wt_[k].ensure((size_t)conv_taps(kConvCout[k]) * kConvCin[k] * kConvCout[k]);
