@@ -13,12 +13,12 @@ pytestmark = pytest.mark.gpu
 
 
 class Busy:
-    """Some 50 ms of clears of 4 GiB on the null stream of the library's runtime."""
+    """Some 0.15 s of clears of 4 GiB on the null stream of the library's runtime."""
 
     def __enter__(self):
         self.hip, self.p, self.n = sfp.lib(), C.c_void_p(), 4 << 30
         assert self.hip.hipMalloc(C.byref(self.p), C.c_size_t(self.n)) == 0
-        for _ in range(60):
+        for _ in range(150):
             assert self.hip.hipMemsetAsync(self.p, C.c_int(0), C.c_size_t(self.n), None) == 0
         return self
 
