@@ -171,10 +171,7 @@ void pressure_dev(sfp_context ctx, double *const vel[3], const double *phi,
         }
     } else {
         if (!ctx->pressure_ready) throw StateError("reproject before project");
-        if (ctx->pressure_unknowns == 0) {
-            fill_stats(st, SolveInfo{0, 0.0, true, 0, ctx->cfg.precond}, 0, 0.f, 0.f, 0.f);
-            return;
-        }
+        if (ctx->pressure_unknowns == 0) return nothing();
         launch_pressure_rhs(s, d, ctx->liquid.p, F, V, U, vol_error, sys.rhs().p);
     }
     SFP_HIP(hipEventRecord(ctx->ev[1], s));

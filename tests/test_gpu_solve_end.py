@@ -228,3 +228,18 @@ def test_empty_projections_between_full_ones(n):
                 assert st[key] == want[k][2][key]
             for a, b in zip([p, *vel], [want[k][1], *want[k][0]]):
                 np.testing.assert_array_equal(a, b)
+
+
+def test_reprojection_without_unknowns_has_no_pressure():
+    """Its pressure is 0, as the projection's before it, not what an earlier
+    call left in the library's buffers."""
+    print("[case] re-projection without unknowns", flush=True)
+    pool = scenes.random_pressure_scene((24, 20, 28), 9)
+    air = dict(pool, phi=np.ones_like(pool["phi"]))
+    with sfp.Context.for_scene(pool, tol=1e-8) as ctx:
+        assert ctx.pressure_project(pool)[1].any()
+        ctx.pressure_project(air, want_pressure=False)
+        vel, p, st = ctx.pressure_project(air, reproject=True)
+    assert st["unknowns"] == 0 and st["converged"] and not p.any()
+    for a, b in zip(vel, air["velocity"]):
+        np.testing.assert_array_equal(a, b)
